@@ -297,7 +297,7 @@ __device__ __forceinline__ void givens_d_solve(bool f64, const double* D, int l,
 
 // d_ldlt_1x1_step (kernels :538-585)
 template<typename VT>
-__device__ void step_1x1(VT* T, double* tri, int p, int len)
+__device__ bool step_1x1(VT* T, double* tri, int p, int len)
 {
     const int lane = lane_id();
     const int j = lane & 31, half = lane >> 5;
@@ -329,6 +329,7 @@ __device__ void step_1x1(VT* T, double* tri, int p, int len)
     if(mod && lane == 0) T[32 * p + p] = 1;
     if(lane < 3) tri[3 * p + lane] = (lane == 1) ? (double) d : 0.0;
     wave_sync();
+    return fabs(d) < (VT) INFINITY;   // D is finite
 }
 
 // d_ldlt_2x2_step (kernels :589-675): Givens rotation of the 2x2 pivot.
@@ -337,7 +338,7 @@ __device__ void step_1x1(VT* T, double* tri, int p, int len)
 // products with the FP64-exact row factors r1, r2. A replaced near-singular
 // pivot is (VT) 1e-6 on the diagonal in both forms.
 template<typename VT, typename AT>
-__device__ void step_2x2(VT* T, double* tri, int p, int len)
+__device__ bool step_2x2(VT* T, double* tri, int p, int len)
 {
     const int lane = lane_id();
     const int j = lane & 31, half = lane >> 5;
@@ -395,6 +396,7 @@ __device__ void step_2x2(VT* T, double* tri, int p, int len)
         tri[3 * (p + 1) + lane] = (lane == 0) ? (double) d12 : ((lane == 1) ? (double) d22 : 0.0);
     }
     wave_sync();
+    return fabs(d11) + fabs(d12) + fabs(d22) < (AT) INFINITY;   // D is finite
 }
 
 template<typename VT>
@@ -666,6 +668,36 @@ __device__ void dense_pivot_op(VT* T, int32_t* perm, int len, int pa, int pb)
     wave_sync();
 }
 
+// ---------------------------------------------------------------------------
+// Which Schur pairs do anything. The product of a pair (k, i), (k, j) is
+// sum_l R[l][j] (A' D)[c][l] over the rows l of block row k: a pair whose
+// blocks share no row adds exact zeros. At level-0 fill nearly every pair is
+// such a pair (blocks of 1-3 entries in 32 rows: 97 % at kkt-400k, about
+// 70 % at n = 2,000), and walking one costs a chain of four dependent
+// loads, so each stored block leaves a 32-bit mask of its rows and a pair's
+// masks are compared first. A 2x2 pivot couples neighbouring rows (the mask
+// is widened by one row each way), and a non-finite entry or D makes the
+// products of unmatched rows NaN (the mask ALL_ROWS matches every block).
+constexpr uint32_t ALL_ROWS = 0xffffffffu;
+constexpr int32_t ROW_2X2 = 1, ROW_NONFINITE = 2;
+
+template<typename T>
+__device__ __forceinline__ bool finite_value(T v) { return fabs(v) < (T) INFINITY; }
+
+// the mask of a stored block with entries in the rows m (dense blocks:
+// ALL_ROWS), any_bad: one of them is not finite; flag: its row's row_flag
+__device__ __forceinline__ uint32_t store_row_mask(uint32_t m, bool any_bad, int32_t flag)
+{
+    if(any_bad || (flag & ROW_NONFINITE)) return ALL_ROWS;
+    if(flag & ROW_2X2) m |= (m << 1) | (m >> 1);
+    return m;
+}
+
+__device__ __forceinline__ bool pair_matches(uint32_t mi, uint32_t mj)
+{
+    return (mi & mj) != 0u || mi == ALL_ROWS || mj == ALL_ROWS;
+}
+
 // k_factor_pivot_blocks (kernels :1146-1283) for the pivot block at level
 // position q, one wave
 template<typename VT>
@@ -774,6 +806,7 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     double* tri = a.tri + 3 * (int64_t) fr;
     int32_t* fpiv = a.is_piv + fr;
     int32_t* bperm = a.perm + fr;
+    int32_t rflag = 0;
     int p = 0;
     while(p < len) {
         int order, p0 = p, p1 = p + 1;
@@ -782,15 +815,16 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
         else order = (p < len - 1 && !fpiv[p + 1]) ? 2 : 1;
         if(order == 1) {
             if(a.pivoting && p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
-            step_1x1(T0, tri, p, len);
+            if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
             if(a.pivoting && lane == 0) fpiv[p] = 1;
         } else {
             if(a.pivoting) {
                 if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
                 dense_pivot_op(T0, bperm, len, p + 1, p1);
             }
-            if(a.piv64) step_2x2<VT, double>(T0, tri, p, len);
-            else step_2x2<VT, VT>(T0, tri, p, len);
+            const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
+                                     : step_2x2<VT, VT>(T0, tri, p, len);
+            rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
             if(a.pivoting && lane == 0) {
                 fpiv[p] = 1;
                 fpiv[p + 1] = 0;
@@ -820,6 +854,7 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     if(lane == 0) {
         a.if_cnt[q] = len * len;
         a.piv_loc[i] = q;
+        a.row_flag[i] = rflag;
     }
 }
 
@@ -863,20 +898,29 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
     tile_load(s.T, m, a.bs, a.ix_in, a.val_in);
     for(int c0 = 0; c0 < np; c0 += 64) {
         Dep mi{}, mj{};
+        bool hit = false;
         if(c0 + lane < np) {
-            mi = load_dep(a.bout, a.bs, a.upd_ki[p0 + c0 + lane]);
-            mj = load_dep(a.bout, a.bs, a.upd_kj[p0 + c0 + lane]);
+            const int ki = a.upd_ki[p0 + c0 + lane], kj = a.upd_kj[p0 + c0 + lane];
+            hit = pair_matches(a.row_mask[ki], a.row_mask[kj]);
+            if(hit) {
+                mi = load_dep(a.bout, a.bs, ki);
+                mj = load_dep(a.bout, a.bs, kj);
+            }
         }
-        const int cnt = min(64, np - c0);
-        Dep ci = bcast(mi, 0), cj = bcast(mj, 0);
+        uint64_t hits = wave_ballot(hit);
+        if(!hits) continue;
+        int d = __ffsll((long long) hits) - 1;
+        Dep ci = bcast(mi, d), cj = bcast(mj, d);
         Pre<VT> pi = prefetch(ci, a.ix_out, a.val_out, a.tri, true);
         Pre<VT> pj = prefetch(cj, a.ix_out, a.val_out, a.tri, false);
-        for(int d = 0; d < cnt; ++d) {
+        while(hits) {
+            hits &= hits - 1;
             Dep ni = ci, nj = cj;
             Pre<VT> qi = pi, qj = pj;
-            if(d + 1 < cnt) {
-                ni = bcast(mi, d + 1);
-                nj = bcast(mj, d + 1);
+            if(hits) {
+                d = __ffsll((long long) hits) - 1;
+                ni = bcast(mi, d);
+                nj = bcast(mj, d);
                 qi = prefetch(ni, a.ix_out, a.val_out, a.tri, true);
                 qj = prefetch(nj, a.ix_out, a.val_out, a.tri, false);
             }
@@ -1116,25 +1160,33 @@ __device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr,
     // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order
     for(int e0 = 0; e0 < np; e0 += 64) {
         Dep mi{}, mj{};
+        bool hit = false;
         if(e0 + lane < np) {
             const int4 pr = pairs[e0 + lane];
-            mi = dep_meta(a.bout, pr.x, pr.z, pr.w);
-            mj = dep_meta(a.bout, pr.y, pr.z, pr.w);
+            hit = pair_matches(a.row_mask[pr.x], a.row_mask[pr.y]);
+            if(hit) {
+                mi = dep_meta(a.bout, pr.x, pr.z, pr.w);
+                mj = dep_meta(a.bout, pr.y, pr.z, pr.w);
+            }
         }
-        if(wave_ballot(e0 + lane < np && !small_sparse<VT>(mj))) {
+        uint64_t hits = wave_ballot(hit);
+        if(!hits) continue;
+        if(wave_ballot(hit && !small_sparse<VT>(mj))) {
             if(lane == 0) a.defer_list[atomicAdd(a.defer_cnt + lr.level, 1)] = q;
             return;
         }
-        const int cnt = min(64, np - e0);
-        Dep ci = bcast(mi, 0), cj = bcast(mj, 0);
+        int d = __ffsll((long long) hits) - 1;
+        Dep ci = bcast(mi, d), cj = bcast(mj, d);
         Pre<VT> pi = prefetch(ci, a.ix_out, a.val_out, a.tri, true);
         Pre<VT> pj = prefetch(cj, a.ix_out, a.val_out, a.tri, false);
-        for(int d = 0; d < cnt; ++d) {
+        while(hits) {
+            hits &= hits - 1;
             Dep ni = ci, nj = cj;
             Pre<VT> qi = pi, qj = pj;
-            if(d + 1 < cnt) {
-                ni = bcast(mi, d + 1);
-                nj = bcast(mj, d + 1);
+            if(hits) {
+                d = __ffsll((long long) hits) - 1;
+                ni = bcast(mi, d);
+                nj = bcast(mj, d);
                 qi = prefetch(ni, a.ix_out, a.val_out, a.tri, true);
                 qj = prefetch(nj, a.ix_out, a.val_out, a.tri, false);
             }
@@ -1251,6 +1303,7 @@ __device__ __forceinline__ void offdiag_body(const FactorArgs<VT>& a, const Leve
 // zeros in the wave form are skipped).
 constexpr int TINY_E = 8;
 constexpr int TINY_T = 32;
+constexpr int TINY_F = 4;   // pairs whose row masks are fetched together
 
 template<typename VT>
 struct TinyLds {
@@ -1271,11 +1324,9 @@ struct TinyMeta {
     int nnz_i, cp_i, vp_i, nnz_j, cp_j, vp_j;
 };
 
-__device__ __forceinline__ TinyMeta tiny_meta(const BlockMeta* bout, int4 pp, bool valid)
+__device__ __forceinline__ TinyMeta tiny_meta(const BlockMeta* bout, int4 pp)
 {
-    TinyMeta t{};
-    t.ok = true;
-    if(!valid) return t;
+    TinyMeta t;
     const BlockMeta mi = bout[pp.x], mj = bout[pp.y];
     t.ok = mi.format == FMT_SPARSE && mi.nnz <= TINY_E && mj.format == FMT_SPARSE &&
         mj.nnz <= TINY_E;
@@ -1355,159 +1406,165 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
         V(n) = a.val_in[(int64_t) t1.w + e];
         ++n;
     }
-    // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order. Loads run
-    // ahead of the arithmetic: while pair pr is computed, the entries of
-    // pair pr + 1, the metadata of pair pr + 2 and the pair record of pair
-    // pr + 3 are in flight.
-    auto rec = [&](int k) { return k < np ? pairs[k] : make_int4(0, 0, 0, 0); };
-    int4 pc = rec(0), p1 = rec(1), p2 = rec(2);
-    TinyMeta mc = tiny_meta(a.bout, pc, np > 0), m1 = tiny_meta(a.bout, p1, np > 1);
-    TinyRaw<VT> rc;
-    tiny_raw(a.ix_out, a.val_out, mc, rc);
-    for(int pr = 0; pr < np; ++pr) {
-        if(!mc.ok) {
-            to_wave_form(a, lr, q);
-            return;
-        }
-        // next entries, metadata and record
-        TinyRaw<VT> rn;
-        tiny_raw(a.ix_out, a.val_out, m1, rn);
-        const TinyMeta m2 = tiny_meta(a.bout, p2, pr + 2 < np);
-        const int4 p3 = rec(pr + 3);
-        const int rb = pc.z;
-        // U_ki: rows l of block k, columns c (rows of block i), width hgt
-        int al[TINY_E], ac[TINY_E];
-        VT av[TINY_E];
+    // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order: the row masks
+    // of TINY_F pairs are fetched together, and of the pairs that match (few)
+    // the metadata, entries and D are read one pair after the other
+    for(int p0 = 0; p0 < np; p0 += TINY_F) {
+        uint32_t hits = 0;
+        {
+            int2 pr[TINY_F];
+            uint32_t mi[TINY_F], mj[TINY_F];
 #pragma unroll
-        for(int e = 0; e < TINY_E; ++e) {
-            al[e] = -4; ac[e] = -1; av[e] = 0;
-            if(e < mc.nnz_i) {
-                const int ix = rc.ixi[e];
-                al[e] = ix / hgt;
-                ac[e] = ix - al[e] * hgt;
-                av[e] = rc.vi[e];
+            for(int u = 0; u < TINY_F; ++u) {
+                const int4 r = pairs[min(p0 + u, np - 1)];
+                pr[u] = make_int2(r.x, r.y);
             }
-        }
-        // U_kj: rows l, columns j, width wid; nonzero entries by (column, row)
-        int rl[TINY_E], rj[TINY_E];
-        VT rv[TINY_E];
 #pragma unroll
-        for(int e = 0; e < TINY_E; ++e) {
-            rl[e] = 0; rj[e] = 64; rv[e] = 0;
-            if(e < mc.nnz_j) {
-                const int ix = rc.ixj[e];
-                const VT v = rc.vj[e];
-                if(v != (VT) 0) {
-                    rl[e] = ix / wid;
-                    rj[e] = ix - rl[e] * wid;
-                    rv[e] = v;
+            for(int u = 0; u < TINY_F; ++u) {
+                mi[u] = a.row_mask[pr[u].x];
+                mj[u] = a.row_mask[pr[u].y];
+            }
+#pragma unroll
+            for(int u = 0; u < TINY_F; ++u)
+                if(p0 + u < np && pair_matches(mi[u], mj[u])) hits |= 1u << u;
+        }
+        for(; hits; hits &= hits - 1) {
+            const int4 pc = pairs[p0 + __ffs(hits) - 1];
+            const TinyMeta mc = tiny_meta(a.bout, pc);
+            if(!mc.ok) {
+                to_wave_form(a, lr, q);
+                return;
+            }
+            TinyRaw<VT> rc;
+            tiny_raw(a.ix_out, a.val_out, mc, rc);
+            const int rb = pc.z;
+            // U_ki: rows l of block k, columns c (rows of block i), width hgt
+            int al[TINY_E], ac[TINY_E];
+            VT av[TINY_E];
+    #pragma unroll
+            for(int e = 0; e < TINY_E; ++e) {
+                al[e] = -4; ac[e] = -1; av[e] = 0;
+                if(e < mc.nnz_i) {
+                    const int ix = rc.ixi[e];
+                    al[e] = ix / hgt;
+                    ac[e] = ix - al[e] * hgt;
+                    av[e] = rc.vi[e];
                 }
             }
-        }
-        const bool one_one = mc.nnz_i == 1 && mc.nnz_j == 1;
-        rc = rn;
-        mc = m1;
-        m1 = m2;
-        pc = p1;
-        p1 = p2;
-        p2 = p3;
-        if(one_one) {
-            // one entry on each side (nearly every pair at level-0 fill):
-            // the general form below reduces to one product for the single
-            // element (column of U_ki's entry, column of U_kj's entry), with
-            // the same operations
-            if(rj[0] < 64) {
-                const int l = rl[0];
-                const double* td = a.tri + 3 * (int64_t) (rb + l);
-                const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
-                const VT left = (al[0] == l - 1) ? av[0] : (VT) 0;
-                const VT mid = (al[0] == l) ? av[0] : (VT) 0;
-                const VT right = (al[0] == l + 1) ? av[0] : (VT) 0;
-                const VT lt = fma(sub, right, fma(dia, mid, sup * left));
-                const VT acc = fma(rv[0], lt, (VT) 0);
-                const int idx = 32 * ac[0] + rj[0];
-                int k = find(idx);
-                if(k < 0) {
-                    if(acc == (VT) 0) continue;
-                    if(n == TINY_T) { to_wave_form(a, lr, q); return; }
-                    k = n++;
-                    I(k) = (int16_t) idx;
-                    V(k) = 0;
+            // U_kj: rows l, columns j, width wid; nonzero entries by (column, row)
+            int rl[TINY_E], rj[TINY_E];
+            VT rv[TINY_E];
+    #pragma unroll
+            for(int e = 0; e < TINY_E; ++e) {
+                rl[e] = 0; rj[e] = 64; rv[e] = 0;
+                if(e < mc.nnz_j) {
+                    const int ix = rc.ixj[e];
+                    const VT v = rc.vj[e];
+                    if(v != (VT) 0) {
+                        rl[e] = ix / wid;
+                        rj[e] = ix - rl[e] * wid;
+                        rv[e] = v;
+                    }
                 }
-                V(k) -= acc;
             }
-            continue;
-        }
-        int key[TINY_E], rank[TINY_E];
-#pragma unroll
-        for(int e = 0; e < TINY_E; ++e) key[e] = rj[e] * 32 + rl[e];
-#pragma unroll
-        for(int e = 0; e < TINY_E; ++e) {
-            int rk = 0;
-#pragma unroll
-            for(int f = 0; f < TINY_E; ++f) rk += (key[f] < key[e]) || (key[f] == key[e] && f < e);
-            rank[e] = rk;
-        }
-        // distinct columns of U_ki
-        int dc[TINY_E];
-#pragma unroll
-        for(int e = 0; e < TINY_E; ++e) {
-            bool seen = ac[e] < 0;
-#pragma unroll
-            for(int f = 0; f < e; ++f) seen = seen || (ac[f] == ac[e]);
-            dc[e] = -1;
-            if(!seen) dc[e] = ac[e];
-        }
-        // columns j in ascending order; within a column, rows ascending
-        VT acc[TINY_E];
-        int curj = -1;
-        for(int rk = 0; rk <= TINY_E; ++rk) {
-            int e = -1;
-#pragma unroll
-            for(int f = 0; f < TINY_E; ++f)
-                if(rank[f] == rk) e = f;
-            const int j = (rk < TINY_E && e >= 0) ? rj[e] : 64;
-            if(j != curj && curj >= 0 && curj < 64) {
-                // column curj done: T[c][curj] -= acc[c]
-#pragma unroll
-                for(int f = 0; f < TINY_E; ++f) {
-                    if(dc[f] < 0) continue;
-                    const int idx = 32 * dc[f] + curj;
+            if(mc.nnz_i == 1 && mc.nnz_j == 1) {
+                // one entry on each side (nearly every pair at level-0 fill):
+                // the general form below reduces to one product for the single
+                // element (column of U_ki's entry, column of U_kj's entry), with
+                // the same operations
+                if(rj[0] < 64) {
+                    const int l = rl[0];
+                    const double* td = a.tri + 3 * (int64_t) (rb + l);
+                    const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
+                    const VT left = (al[0] == l - 1) ? av[0] : (VT) 0;
+                    const VT mid = (al[0] == l) ? av[0] : (VT) 0;
+                    const VT right = (al[0] == l + 1) ? av[0] : (VT) 0;
+                    const VT lt = fma(sub, right, fma(dia, mid, sup * left));
+                    const VT acc = fma(rv[0], lt, (VT) 0);
+                    const int idx = 32 * ac[0] + rj[0];
                     int k = find(idx);
                     if(k < 0) {
-                        if(acc[f] == (VT) 0) continue;
+                        if(acc == (VT) 0) continue;
                         if(n == TINY_T) { to_wave_form(a, lr, q); return; }
                         k = n++;
                         I(k) = (int16_t) idx;
                         V(k) = 0;
                     }
-                    V(k) -= acc[f];
+                    V(k) -= acc;
                 }
+                continue;
             }
-            if(j >= 64) break;
-            if(j != curj) {
-                curj = j;
-#pragma unroll
-                for(int f = 0; f < TINY_E; ++f) acc[f] = 0;
+            int key[TINY_E], rank[TINY_E];
+    #pragma unroll
+            for(int e = 0; e < TINY_E; ++e) key[e] = rj[e] * 32 + rl[e];
+    #pragma unroll
+            for(int e = 0; e < TINY_E; ++e) {
+                int rk = 0;
+    #pragma unroll
+                for(int f = 0; f < TINY_E; ++f) rk += (key[f] < key[e]) || (key[f] == key[e] && f < e);
+                rank[e] = rk;
             }
-            const int l = rl[e];
-            const VT r = rv[e];
-            const double* td = a.tri + 3 * (int64_t) (rb + l);
-            const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
-#pragma unroll
-            for(int f = 0; f < TINY_E; ++f) {
-                if(dc[f] < 0) continue;
-                const int c = dc[f];
-                VT left = 0, mid = 0, right = 0;
-#pragma unroll
-                for(int g = 0; g < TINY_E; ++g) {
-                    if(ac[g] != c) continue;
-                    if(al[g] == l - 1) left = av[g];
-                    if(al[g] == l) mid = av[g];
-                    if(al[g] == l + 1) right = av[g];
+            // distinct columns of U_ki
+            int dc[TINY_E];
+    #pragma unroll
+            for(int e = 0; e < TINY_E; ++e) {
+                bool seen = ac[e] < 0;
+    #pragma unroll
+                for(int f = 0; f < e; ++f) seen = seen || (ac[f] == ac[e]);
+                dc[e] = -1;
+                if(!seen) dc[e] = ac[e];
+            }
+            // columns j in ascending order; within a column, rows ascending
+            VT acc[TINY_E];
+            int curj = -1;
+            for(int rk = 0; rk <= TINY_E; ++rk) {
+                int e = -1;
+    #pragma unroll
+                for(int f = 0; f < TINY_E; ++f)
+                    if(rank[f] == rk) e = f;
+                const int j = (rk < TINY_E && e >= 0) ? rj[e] : 64;
+                if(j != curj && curj >= 0 && curj < 64) {
+                    // column curj done: T[c][curj] -= acc[c]
+    #pragma unroll
+                    for(int f = 0; f < TINY_E; ++f) {
+                        if(dc[f] < 0) continue;
+                        const int idx = 32 * dc[f] + curj;
+                        int k = find(idx);
+                        if(k < 0) {
+                            if(acc[f] == (VT) 0) continue;
+                            if(n == TINY_T) { to_wave_form(a, lr, q); return; }
+                            k = n++;
+                            I(k) = (int16_t) idx;
+                            V(k) = 0;
+                        }
+                        V(k) -= acc[f];
+                    }
                 }
-                const VT lt = fma(sub, right, fma(dia, mid, sup * left));
-                acc[f] = fma(r, lt, acc[f]);
+                if(j >= 64) break;
+                if(j != curj) {
+                    curj = j;
+    #pragma unroll
+                    for(int f = 0; f < TINY_E; ++f) acc[f] = 0;
+                }
+                const int l = rl[e];
+                const VT r = rv[e];
+                const double* td = a.tri + 3 * (int64_t) (rb + l);
+                const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
+    #pragma unroll
+                for(int f = 0; f < TINY_E; ++f) {
+                    if(dc[f] < 0) continue;
+                    const int c = dc[f];
+                    VT left = 0, mid = 0, right = 0;
+    #pragma unroll
+                    for(int g = 0; g < TINY_E; ++g) {
+                        if(ac[g] != c) continue;
+                        if(al[g] == l - 1) left = av[g];
+                        if(al[g] == l) mid = av[g];
+                        if(al[g] == l + 1) right = av[g];
+                    }
+                    const VT lt = fma(sub, right, fma(dia, mid, sup * left));
+                    acc[f] = fma(r, lt, acc[f]);
+                }
             }
         }
     }
@@ -1975,8 +2032,18 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
     VT* out_v = a.val_out + mo.val_ptr;
     if(mo.format == FMT_DENSE) {
         for(int e = lane; e < h * w; e += 64) out_v[e] = vals[e];
+        if(lane == 0) a.row_mask[b] = ALL_ROWS;
         return;
     }
+    const int32_t rflag = a.row_flag[mo.block_row];
+    uint32_t rows = 0;
+    bool bad = false;
+    auto keep_mask = [&]() {
+#pragma unroll
+        for(int o = WAVE / 2; o > 0; o >>= 1) rows |= (uint32_t) __shfl_xor((int) rows, o, WAVE);
+        const bool any_bad = wave_ballot(bad) != 0ull;
+        if(lane == 0) a.row_mask[b] = store_row_mask(rows, any_bad, rflag);
+    };
     const uint16_t* ixs = a.if_idx + (int64_t) q * 1024;
     int32_t* out_i = a.ix_out + mo.col_ptr;
     if(lane < h) nrm[lane] = drop_norm(a.rn[fr + lane]);
@@ -1999,9 +2066,12 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
                 const int pos = base + lanes_below(mask);
                 out_i[pos] = (ix >> 5) * w + (ix & 31);
                 out_v[pos] = v;
+                rows |= 1u << (ix >> 5);
+                bad = bad || !finite_value(v);
             }
             base += __popcll(mask);
         }
+        keep_mask();
         return;
     }
     // over capacity: keep the max_nnz largest |v|, ties to the lower tile
@@ -2026,8 +2096,11 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
         if(rank < mo.max_nnz) {
             out_i[rank] = (ie >> 5) * w + (ie & 31);
             out_v[rank] = vals[e];
+            rows |= 1u << (ie >> 5);
+            bad = bad || !finite_value(vals[e]);
         }
     }
+    keep_mask();
 }
 
 // the positions k_store_tiny leaves to the wave form, grid-stride
@@ -2069,6 +2142,9 @@ __device__ __forceinline__ void store_tiny_body(const FactorArgs<VT>& a, const L
     const uint16_t* ixs = a.if_idx + (int64_t) q * 1024;
     VT* out_v = a.val_out + mo.val_ptr;
     int32_t* out_i = a.ix_out + mo.col_ptr;
+    const int32_t rflag = a.row_flag[mo.block_row];
+    uint32_t rows = 0;
+    bool bad = false;
     VT key[STORE_TINY];
     int ixk[STORE_TINY];
 #pragma unroll
@@ -2081,6 +2157,7 @@ __device__ __forceinline__ void store_tiny_body(const FactorArgs<VT>& a, const L
             const bool k = !(fabs(v) < a.threshold * drop_norm(a.rn[fr + (ix >> 5)]));
             key[e] = k ? (VT) fabs(v) : (VT) -1;
             ixk[e] = ix;
+            bad = bad || (k && !finite_value(v));
         }
     }
     if(!a.overflow[q]) {
@@ -2090,9 +2167,11 @@ __device__ __forceinline__ void store_tiny_body(const FactorArgs<VT>& a, const L
             if(key[e] >= (VT) 0) {
                 out_i[pos] = (ixk[e] >> 5) * w + (ixk[e] & 31);
                 out_v[pos] = vals[e];
+                rows |= 1u << (ixk[e] >> 5);
                 ++pos;
             }
         }
+        a.row_mask[b] = store_row_mask(rows, bad, rflag);
         return;
     }
 #pragma unroll
@@ -2105,8 +2184,10 @@ __device__ __forceinline__ void store_tiny_body(const FactorArgs<VT>& a, const L
         if(rank < mo.max_nnz) {
             out_i[rank] = (ixk[e] >> 5) * w + (ixk[e] & 31);
             out_v[rank] = vals[e];
+            rows |= 1u << (ixk[e] >> 5);
         }
     }
+    a.row_mask[b] = store_row_mask(rows, bad, rflag);
 }
 
 // k_pivot_col_blocks (kernels :1352-1418) with d_col_pivot_block

@@ -52,6 +52,11 @@ struct FactorArgs {
     int32_t* granted = nullptr;           // leftover space granted per position
     uint8_t* overflow = nullptr;
     int32_t* piv_loc = nullptr;           // nb
+    // rows of each factored off-diagonal block that can contribute to a
+    // Schur product (store_row_mask), and per block row what its pivots add
+    // to that (ROW_2X2, ROW_NONFINITE)
+    uint32_t* row_mask = nullptr;         // per coarse block
+    int32_t* row_flag = nullptr;          // nb
     // static, in level-list order: capacity of a sparse block (max_nnz >= 0)
     // or -1 - rows * cols for a dense block; first fine row of its block row
     const int32_t* lq_cap = nullptr;

@@ -173,6 +173,8 @@ void Bildlt::upload_pattern(hipStream_t st)
     d_overflow.ensure(mlb);
     d_piv_loc.ensure(sizeof(int32_t) * s.nb);
     d_carry.ensure(sizeof(int32_t) * 8);
+    d_row_mask.ensure(sizeof(uint32_t) * (size_t) std::max(1, K));
+    d_row_flag.ensure(sizeof(int32_t) * (size_t) std::max(1, s.nb));
     for(int q = 0; q < 4; ++q) d_ptr[q].ensure(sizeof(int32_t) * (size_t) (n + 1));
     for(int q = 0; q < 2; ++q) d_task[q].ensure(sizeof(int32_t) * 8 * (size_t) s.nb);
     d_totals.ensure(sizeof(int32_t) * 4);
@@ -249,6 +251,8 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.granted = d_granted.as<int32_t>();
     a.overflow = d_overflow.as<uint8_t>();
     a.piv_loc = d_piv_loc.as<int32_t>();
+    a.row_mask = d_row_mask.as<uint32_t>();
+    a.row_flag = d_row_flag.as<int32_t>();
     a.lq_cap = d_lq_cap.as<int32_t>();
     a.lq_fr = d_lq_fr.as<int32_t>();
     a.chunk = d_chunk.as<int64_t>();
@@ -652,7 +656,7 @@ int64_t Bildlt::numeric_bytes() const
             &d_if_val, &d_if_idx, &d_if_cnt, &d_rn_part, &d_drop_cnt, &d_overflow, &d_piv_loc,
             &d_carry, &d_totals, &d_task[0], &d_task[1], &d_keep, &d_granted, &d_chunk,
             &d_scan_tmp, &d_piv_umask, &d_defer_list, &d_defer_cnt, &d_wave_list, &d_wave_cnt,
-            &d_store_list, &d_store_cnt,
+            &d_store_list, &d_store_cnt, &d_row_mask, &d_row_flag,
             &d_chain_pub, &d_jac[0], &d_jac[1], &d_jac[2]})
         b += (int64_t) d->bytes;
     for(int q = 0; q < 4; ++q)
@@ -674,6 +678,7 @@ int64_t Bildlt::numeric_bytes_estimate(bool with_layout) const
     b += r16(8 * (int64_t) s.value_slot.size()) + 2 * r16(v * s.val_space) + r16(36 * K);
     b += r16(4 * s.ix_space) + 24 * n + v * n;
     b += v * 1024 * mlb + 2048 * mlb + 4 * mlb + v * 32 * mlb + 4 * mlb + mlb;
+    b += r16(4 * K) + r16(4 * nb);   // row masks and flags
     b += 4 * nb + 32 + 4 * 4 * (n + 1) + 2 * 32 * nb + 16 + 4 * ((int64_t) scan_tmp_ints(s.n));
     b += 16 * std::max<int64_t>(1, n) + 4;   // single-launch solves' published values, error
     b += 2 * r16(4 * mlb) + 2 * r16(4 * std::max(1, s.num_levels));   // wave / store lists

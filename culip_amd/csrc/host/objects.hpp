@@ -163,6 +163,7 @@ struct Bildlt final : Precond {
     DevBuf d_keep, d_granted, d_chunk;
     DevBuf d_piv_umask, d_defer_list, d_defer_cnt, d_wave_list, d_wave_cnt, d_store_list,
         d_store_cnt;
+    DevBuf d_row_mask, d_row_flag;
     // solve layout
     DevBuf d_ptr[4], d_col[4], d_val[4], d_lr[4], d_task[2];
     DevBuf d_totals, d_scan_tmp;
