@@ -15,12 +15,11 @@
 //               A_ij), per-row partial sums of squares; the result leaves as
 //               a dense tile or as a compact (index, value) list of the
 //               entries with |v| > 1e-10
-//   k_rownorm   one wave per block row: row sums of squares in a fixed order
-//   k_level_scan
-//               chunked scan in level-list order: entries surviving the
-//               threshold, leftover-space pool, granted extra space, output
-//               offsets and the factored metadata
-//   k_store     one wave per block: compacted final storage
+//   k_drop      one workgroup per row group: row sums of squares in a fixed
+//               order, entries surviving the threshold, leftover-space pool in
+//               level-list order, granted extra space, the factored metadata
+//               and the final storage of blocks with few entries
+//   k_store     one wave per remaining block: compacted final storage
 //
 // The dependency blocks of a tile are walked with their metadata fetched
 // lane-parallel up front. In the pivot blocks a block whose nonzero entries share
@@ -66,27 +65,25 @@ __device__ __forceinline__ void tile_copy(VT* dst, const VT* src)
     for(int t = 0; t < 16; ++t) dst[64 * t + lane] = src[64 * t + lane];
 }
 
-// d_load_block (kernels :22-81) for an input block: zero, then fill
+// d_load_block (kernels :22-81) for an input block of h x w, m its {format,
+// nnz, col_ptr, val_ptr}: zero, then fill
 template<typename VT>
-__device__ void tile_load(VT* T, const BlockMeta& m, const int32_t* bs, const int32_t* ixs,
-    const VT* vals)
+__device__ void tile_load(VT* T, int4 m, int h, int w, const int32_t* ixs, const VT* vals)
 {
     const int lane = lane_id();
-    const int h = bs[m.block_row + 1] - bs[m.block_row];
-    const int w = bs[m.block_col + 1] - bs[m.block_col];
     tile_zero(T);
     wave_sync();
-    if(m.format == FMT_DENSE) {
+    if(m.x == FMT_DENSE) {
 #pragma unroll
         for(int t = 0; t < 16; ++t) {
             const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
-            if(r < h && c < w) T[idx] = vals[(int64_t) m.val_ptr + r * w + c];
+            if(r < h && c < w) T[idx] = vals[(int64_t) m.w + r * w + c];
         }
     } else {
-        for(int e = lane; e < m.nnz; e += 64) {
-            const int ix = ixs[(int64_t) m.col_ptr + e];
+        for(int e = lane; e < m.y; e += 64) {
+            const int ix = ixs[(int64_t) m.z + e];
             const int r = ix / w, c = ix - r * w;
-            T[32 * r + c] = vals[(int64_t) m.val_ptr + e];
+            T[32 * r + c] = vals[(int64_t) m.w + e];
         }
     }
     wave_sync();
@@ -705,13 +702,16 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     PivLds<VT>& s)
 {
     const int lane = lane_id();
-    const int b = a.lvlb_idx[lr.lo + q];
-    const BlockMeta m = a.bin[b];
-    const int i = m.block_row;
-    const int fr = a.bs[i];
-    const int len = a.bs[i + 1] - fr;
-    const int cb0 = a.csc_off[i];
-    const int nd = a.csc_off[i + 1] - 1 - cb0;
+    const int4 t0 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q)];
+    const int4 t1 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q) + 1];
+    const int4 t2 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q) + 2];
+    // the pool before the level: its pivot blocks come first in it
+    const int32_t pool = a.carry[4 * (lr.level & 1)];
+    const int i = t0.w;
+    const int fr = t0.y;
+    const int len = t0.z;
+    const int cb0 = t2.x;
+    const int nd = t2.y;
     const int j = lane & 31, cq = lane >> 5;
     // metadata of the first 64 dependency blocks, in flight during the tile
     // load; later chunks are fetched while the previous one is walked
@@ -719,7 +719,7 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     if(lane < nd) nxt = load_dep(a.bout, a.bs, a.csc_idx[cb0 + lane]);
     // the pivot tile in registers (rows cq + 2t of column j)
     VT* T0 = s.X[0];
-    tile_load(T0, m, a.bs, a.ix_in, a.val_in);
+    tile_load(T0, t1, len, len, a.ix_in, a.val_in);
     VT T[16];
 #pragma unroll
     for(int t = 0; t < 16; ++t) T[t] = T0[32 * (cq + 2 * t) + j];
@@ -846,16 +846,82 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     // and whether there is any such column at all (one word per tile)
     const bool um_some = wave_ballot(um != 0u) != 0ull;
     if(lane == 0) a.piv_any[q] = um_some ? 1u : 0u;
+    // the tile for the level's off-diagonal blocks, and its final storage:
+    // dense blocks keep their size, so the offset follows from the pool alone
+    // (k_drop)
     VT* out = a.if_val + (int64_t) q * 1024;
+    VT* fin = a.val_out + ((int64_t) t1.w - pool);
     for(int e = lane; e < len * len; e += 64) {
         const int r = e / len, c = e - r * len;
-        out[e] = T0[32 * r + c];
+        const VT v = T0[32 * r + c];
+        out[e] = v;
+        fin[e] = v;
     }
     if(lane == 0) {
-        a.if_cnt[q] = len * len;
         a.piv_loc[i] = q;
         a.row_flag[i] = rflag;
     }
+}
+
+// the entry list of position q holding cnt entries
+template<typename VT>
+struct EntryList {
+    VT* v;
+    uint16_t* ix;
+};
+
+template<typename VT>
+__device__ __forceinline__ EntryList<VT> entry_list(const FactorArgs<VT>& a, int q, int cnt)
+{
+    if(cnt <= LIST_C) return {a.c_val + (int64_t) q * LIST_C, a.c_idx + (int64_t) q * LIST_C};
+    return {a.if_val + (int64_t) q * 1024, a.if_idx + (int64_t) q * 1024};
+}
+
+// a scaled off-diagonal tile X (one wave, stride 32) as position q leaves
+// it: row sums of squares, and the dense tile or the entries above NZ_EPS
+template<typename VT>
+__device__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int hgt, int wid,
+    int format)
+{
+    const int lane = lane_id();
+    const VT ssq = (lane < hgt) ? row_ssq(X, lane, wid) : (VT) 0;
+    const uint64_t rows = wave_ballot(!(ssq == (VT) 0));
+    if((rows >> lane) & 1ull) {
+        const int j = lanes_below(rows);
+        if(j == 0) a.rn_first[q] = ssq;
+        else a.rn_part[(int64_t) q * 32 + j] = ssq;
+    }
+    if(lane == 0) a.part_mask[q] = (uint32_t) rows;
+    if(format == FMT_DENSE) {
+        VT* oval = a.if_val + (int64_t) q * 1024;
+        for(int e = lane; e < hgt * wid; e += 64) {
+            const int r = e / wid, c = e - r * wid;
+            oval[e] = X[32 * r + c];
+        }
+        if(lane == 0) a.if_cnt[q] = hgt * wid;
+        return;
+    }
+    auto live = [&](int t) {
+        const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
+        return r < hgt && c < wid && fabs((double) X[idx]) > NZ_EPS;
+    };
+    int cnt = 0;
+#pragma unroll
+    for(int t = 0; t < 16; ++t) cnt += __popcll(wave_ballot(live(t)));
+    const EntryList<VT> o = entry_list(a, q, cnt);
+    int base = 0;
+#pragma unroll
+    for(int t = 0; t < 16; ++t) {
+        const bool pred = live(t);
+        const uint64_t msk = wave_ballot(pred);
+        if(pred) {
+            const int pos = base + lanes_below(msk);
+            o.ix[pos] = (uint16_t) (64 * t + lane);
+            o.v[pos] = X[64 * t + lane];
+        }
+        base += __popcll(msk);
+    }
+    if(lane == 0) a.if_cnt[q] = cnt;
 }
 
 // k_update_scale_offdiagonal_blocks (kernels :1628-1803) with
@@ -895,7 +961,7 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
     tile_zero(s.A);
     if(lane < 32) { s.mask[lane] = 0; s.umask[lane] = 0; }
     if(np > 0) tile_zero(s.R);
-    tile_load(s.T, m, a.bs, a.ix_in, a.val_in);
+    tile_load(s.T, make_int4(m.format, m.nnz, m.col_ptr, m.val_ptr), hgt, wid, a.ix_in, a.val_in);
     for(int c0 = 0; c0 < np; c0 += 64) {
         Dep mi{}, mj{};
         bool hit = false;
@@ -1004,33 +1070,7 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
         }
     }
     wave_sync();
-    if(lane < hgt) a.rn_part[(int64_t) q * 32 + lane] = row_ssq(s.T, lane, wid);
-
-    VT* oval = a.if_val + (int64_t) q * 1024;
-    if(m.format == FMT_DENSE) {
-        for(int e = lane; e < hgt * wid; e += 64) {
-            const int r = e / wid, c = e - r * wid;
-            oval[e] = s.T[32 * r + c];
-        }
-        if(lane == 0) a.if_cnt[q] = hgt * wid;
-    } else {
-        uint16_t* oix = a.if_idx + (int64_t) q * 1024;
-        int base = 0;
-#pragma unroll
-        for(int t = 0; t < 16; ++t) {
-            const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
-            const VT v = s.T[idx];
-            const bool pred = r < hgt && c < wid && fabs((double) v) > NZ_EPS;
-            const uint64_t msk = wave_ballot(pred);
-            if(pred) {
-                const int pos = base + lanes_below(msk);
-                oix[pos] = (uint16_t) idx;
-                oval[pos] = v;
-            }
-            base += __popcll(msk);
-        }
-        if(lane == 0) a.if_cnt[q] = base;
-    }
+    offdiag_output(a, q, s.T, hgt, wid, m.format);
 }
 
 // ---------------------------------------------------------------------------
@@ -1247,33 +1287,7 @@ __device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr,
         }
     }
     wave_sync();
-    if(lane < hgt) a.rn_part[(int64_t) q * 32 + lane] = row_ssq(s.X, lane, wid);
-
-    VT* oval = a.if_val + (int64_t) q * 1024;
-    if(t1.x == FMT_DENSE) {
-        for(int e = lane; e < hgt * wid; e += 64) {
-            const int r = e / wid, c = e - r * wid;
-            oval[e] = s.X[32 * r + c];
-        }
-        if(lane == 0) a.if_cnt[q] = hgt * wid;
-    } else {
-        uint16_t* oix = a.if_idx + (int64_t) q * 1024;
-        int base = 0;
-#pragma unroll
-        for(int t = 0; t < 16; ++t) {
-            const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
-            const VT v = s.X[idx];
-            const bool pred = r < hgt && c < wid && fabs((double) v) > NZ_EPS;
-            const uint64_t msk = wave_ballot(pred);
-            if(pred) {
-                const int pos = base + lanes_below(msk);
-                oix[pos] = (uint16_t) idx;
-                oval[pos] = v;
-            }
-            base += __popcll(msk);
-        }
-        if(lane == 0) a.if_cnt[q] = base;
-    }
+    offdiag_output(a, q, s.X, hgt, wid, t1.x);
 }
 
 // the positions k_offdiag_tiny leaves to the wave form, grid-stride
@@ -1569,11 +1583,10 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
         }
     }
     // the tile list for the second phase
-    VT* lv = a.if_val + (int64_t) q * 1024;
-    uint16_t* li = a.if_idx + (int64_t) q * 1024;
+    const EntryList<VT> o = entry_list(a, q, n);
     for(int k = 0; k < n; ++k) {
-        li[k] = (uint16_t) I(k);
-        lv[k] = V(k);
+        o.ix[k] = (uint16_t) I(k);
+        o.v[k] = V(k);
     }
     a.if_cnt[q] = n;
 }
@@ -1611,11 +1624,10 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
         return -1;
     };
     {
-        const VT* lv = a.if_val + (int64_t) q * 1024;
-        const uint16_t* li = a.if_idx + (int64_t) q * 1024;
+        const EntryList<VT> o = entry_list(a, q, n);
         for(int k = 0; k < n; ++k) {
-            I(k) = (int16_t) li[k];
-            V(k) = lv[k];
+            I(k) = (int16_t) o.ix[k];
+            V(k) = o.v[k];
         }
     }
     // U_ii' forward substitution over the rows in ascending order
@@ -1670,30 +1682,33 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
         I(m + 1) = ik;
         V(m + 1) = vk;
     }
-    // row partial sums of squares (columns ascending) of the rows with
-    // entries; the others stay at the zero the first phase stored (a row
-    // without entries sums to +0)
-    VT* rp = a.rn_part + (int64_t) q * 32;
-    int k = 0;
-    while(k < n) {
+    // row sums of squares (columns ascending) and the compact list
+    uint32_t rows = 0;
+    int nr = 0, cnt = 0;
+    for(int k = 0; k < n;) {
         const int r = I(k) >> 5;
         VT ssq = 0;
         while(k < n && (I(k) >> 5) == r) {
             ssq = fma(V(k), V(k), ssq);
+            cnt += fabs((double) V(k)) > NZ_EPS;
             ++k;
         }
-        rp[r] = ssq;
+        if(!(ssq == (VT) 0)) {
+            if(nr == 0) a.rn_first[q] = ssq;
+            else a.rn_part[(int64_t) q * 32 + nr] = ssq;
+            rows |= 1u << r;
+            ++nr;
+        }
     }
-    // and the compact list
-    VT* oval = a.if_val + (int64_t) q * 1024;
-    uint16_t* oix = a.if_idx + (int64_t) q * 1024;
-    int cnt = 0;
+    a.part_mask[q] = rows;
+    const EntryList<VT> o = entry_list(a, q, cnt);
+    int pos = 0;
     for(int m = 0; m < n; ++m) {
         const VT v = V(m);
         if(fabs((double) v) > NZ_EPS) {
-            oix[cnt] = (uint16_t) I(m);
-            oval[cnt] = v;
-            ++cnt;
+            o.ix[pos] = (uint16_t) I(m);
+            o.v[pos] = v;
+            ++pos;
         }
     }
     a.if_cnt[q] = cnt;
@@ -1717,13 +1732,7 @@ __device__ __forceinline__ void pivots_pairs_body(const FactorArgs<VT>& a, const
         pivots_one<VT>(a, lr, w, u.piv);
         return;
     }
-    // the workgroup's positions' row partial sums start at zero, stored
-    // coalesced here (the second phase writes only the rows with entries;
-    // the other off-diagonal kernels write every row of theirs)
     const int q0 = lr.npiv + (w - lr.npiv) * TINY_TPB;
-    const int q1 = min(q0 + TINY_TPB, lr.size);
-    VT* rp = a.rn_part + (int64_t) q0 * 32;
-    for(int e = (int) threadIdx.x; e < (q1 - q0) * 32; e += TINY_TPB) rp[e] = (VT) 0;
     tiny_pairs_one<VT>(a, lr, q0 + (int) threadIdx.x, (int) threadIdx.x, u.tiny);
 }
 
@@ -1731,42 +1740,14 @@ __device__ __forceinline__ void pivots_pairs_body(const FactorArgs<VT>& a, const
 template<typename VT>
 __device__ __forceinline__ VT drop_norm(VT rn) { return (VT) sqrtf((float) rn); }
 
-// row sums of squares: pivot block first, then the off-diagonal blocks of
-// the row by block id (contiguous in the level list at row_first_block_offset)
-template<typename VT>
-__device__ __forceinline__ void rownorm_body(const FactorArgs<VT>& a, const LevelRange& lr,
-    int bid_, int nblk_)
-{
-    const int lane = lane_id();
-    const int b = a.lvlb_idx[lr.lo + bid_];
-    const int i = a.bin[b].block_row;
-    const int fr = a.bs[i];
-    const int h = a.bs[i + 1] - fr;
-    const int nblk = a.csr_off[i + 1] - a.csr_off[i] - 1;
-    if(lane >= h) return;
-    VT acc = a.rn[fr + lane];
-    if(nblk > 0) {
-        const VT* part = a.rn_part + (int64_t) (lr.npiv + a.rfo[i]) * 32 + lane;
-        // sixteen loads in flight per pass; the sum stays in block order
-        int t = 0;
-        for(; t + 16 <= nblk; t += 16) {
-            VT v[16];
-#pragma unroll
-            for(int u = 0; u < 16; ++u) v[u] = part[32 * (t + u)];
-#pragma unroll
-            for(int u = 0; u < 16; ++u) acc += v[u];
-        }
-        for(; t < nblk; ++t) acc += part[32 * t];
-    }
-    a.rn[fr + lane] = acc;
-}
-
-// Leftover pool, granted extra space and output offsets of a level's blocks
-// in level-list order (kernels :1948-2008 with the atomics serialised in
-// that order). The pool after a sparse block is max(pool + max_nnz - kept,
-// 0); such maps p -> max(p + a, b) compose associatively, so the pool
-// sequence is a scan (k_level_scan): each chunk's composed map, then the
-// pools and grants, then the output offsets from the chunks' size sums.
+// Leftover pool and granted extra space of a level's blocks in level-list
+// order (kernels :1948-2008 with the atomics serialised in that order). The
+// pool after a sparse block is max(pool + max_nnz - kept candidates, 0); such
+// maps p -> max(p + a, b) compose associatively, so the pool sequence is a
+// scan. A block stores cap + (pool before) - (pool after) entries whatever
+// it was granted, so the sizes stored before a position add up to the
+// capacities before it (a static prefix sum) minus the pool at it: output
+// offsets need no scan of their own.
 struct PoolMap {
     int64_t a, b;
     __device__ static PoolMap shfl_up(const PoolMap& m, int o)
@@ -1787,232 +1768,373 @@ __device__ __forceinline__ int64_t map_apply(const PoolMap& m, int64_t p)
     const int64_t v = p + m.a;
     return v > m.b ? v : m.b;
 }
-struct Sizes {
-    int64_t x, v;   // index and value entries
-    __device__ static Sizes shfl_up(const Sizes& s, int o)
-    {
-        return {__shfl_up(s.x, o, WAVE), __shfl_up(s.v, o, WAVE)};
-    }
-};
-struct SumOp {
-    __device__ Sizes operator()(const Sizes& p, const Sizes& q) const { return {p.x + q.x, p.v + q.v}; }
-};
-
-constexpr int SC_TPB = 256;
-constexpr int SC_IPT = SCAN_CHUNK / SC_TPB;
-constexpr int SC_NW = SC_TPB / WAVE;
+constexpr int DR_TPB = GROUP_BLOCKS;
+constexpr int DR_NW = DR_TPB / WAVE;
+constexpr int DR_RUNS = 512;        // row sums a wave lays out at once
 constexpr int32_t CAP_NONE = -0x7fffffff;
+constexpr int STORE_TINY = 16;      // entries of a block stored by one lane
+constexpr int GROUP_SPIN_LIMIT = 1 << 22;
 
-// in-order combination of load(0 .. count-1) over the workgroup
-template<typename V, typename Op, typename Load>
-__device__ V block_prefix(int count, Load load, Op op, const V& id, V* sh)
+template<typename VT>
+struct DropLds {
+    VT val[DR_NW][DR_RUNS];                            // row sums, in block order
+    uint32_t rows[DR_NW][GROUP_ROWS][DR_RUNS / 32 + 1];   // per fine row: which are its own
+    int32_t runs[DR_NW];
+    VT nrm[GROUP_ROWS];
+    int32_t frow[GROUP_ROWS], rflag[GROUP_ROWS];
+    PoolMap sh[DR_NW];
+    int64_t pool;
+    int32_t ticket;
+};
+
+// Words of a row group's state: each carries its own validity in the low two
+// bits, so that readers need no ordering between them (relaxed 8-byte
+// agent-coherent stores and loads, no fences).
+__device__ __forceinline__ void publish(int64_t* p, int64_t v)
 {
-    const int per = (count + SC_TPB - 1) / SC_TPB;
-    V v = id;
-    for(int k = 0; k < per; ++k) {
-        const int i = (int) threadIdx.x * per + k;
-        if(i < count) v = op(v, load(i));
-    }
-    V tot;
-    (void) block_exclusive_scan<V, Op, SC_NW>(v, op, id, sh, &tot);
-    return tot;
+    __hip_atomic_store(p, (int64_t) ((uint64_t) v << 2) | 1, __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One launch per level, in chunks of SCAN_CHUNK positions. A workgroup
-// takes its chunk from a ticket counter, so every chunk it later waits for
-// belongs to a workgroup that is already running, whatever the dispatch
-// order. Every chunk runs the threshold counts, publishes its pool map
-// (release store of its flag), waits for the maps of the chunks before it
-// (acquire loads), runs the pools and grants, publishes its sizes, waits
-// for the sizes before it and writes the factored metadata. The waits are
-// bounded only as a guard against a hang; given the tickets they end as
-// soon as the earlier chunks have published.
-constexpr int SCAN_SPIN_LIMIT = 1 << 22;
-
-__device__ __forceinline__ int64_t load_published(const int64_t* p)
+__device__ __forceinline__ int64_t published_word(const int64_t* p)
 {
     return __hip_atomic_load(const_cast<int64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the first wave polls the flags of chunks [0, c); then the workgroup goes
-// on together. A wait that gives up records 2 in *err and goes on.
-__device__ void wait_chunk_flags(const int32_t* flags, int c, int32_t* err)
+// The pool before row group g of a level (one wave): the groups before it are
+// looked at 64 at a time, nearest first, until one whose pool is known or the
+// level's start (pool0); the maps in between are composed in order. A wait
+// that gives up records 2 in *err and goes on.
+__device__ int64_t pool_before(const int64_t* st, int g, int64_t pool0, int32_t* err)
 {
-    if(threadIdx.x < WAVE) {
-        int spins = 0;
+    const int lane = lane_id();
+    PoolMap acc{0, 0};
+    int spins = 0;
+    for(int base = g - 1;; base -= WAVE) {
+        const int idx = base - lane;
+        int64_t wa = 0, wb = 0, wp = 0;
+        bool known = idx < 0, have = known;
+        int near;
         for(;;) {
-            bool set = true;
-            for(int i = (int) threadIdx.x; i < c; i += WAVE)
-                set = set && __hip_atomic_load(const_cast<int32_t*>(flags + i), __ATOMIC_ACQUIRE,
-                    __HIP_MEMORY_SCOPE_AGENT) != 0;
-            if(wave_ballot(!set) == 0ull) break;
+            if(!have) {
+                wp = published_word(st + 3 * (int64_t) idx + 2);
+                wa = published_word(st + 3 * (int64_t) idx);
+                wb = published_word(st + 3 * (int64_t) idx + 1);
+                known = wp != 0;
+                have = known || (wa != 0 && wb != 0);
+            }
+            const uint64_t km = wave_ballot(known);
+            near = km ? __ffsll((long long) km) - 1 : WAVE;
+            const uint64_t need = near < WAVE ? (1ull << near) - 1 : ~0ull;
+            if((wave_ballot(!have) & need) == 0ull) break;
             __builtin_amdgcn_s_sleep(1);
-            if(++spins > SCAN_SPIN_LIMIT) {
-                if(threadIdx.x == 0 && err)
+            if(++spins > GROUP_SPIN_LIMIT) {
+                if(lane == 0 && err)
                     __hip_atomic_store(err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 break;
             }
         }
+        // lane 0 holds the latest group of the window
+        PoolMap m{0, 0};
+        if(lane < near) m = PoolMap{wa >> 2, wb >> 2};
+#pragma unroll
+        for(int o = 1; o < WAVE; o <<= 1) {
+            const PoolMap u{__shfl_down(m.a, o, WAVE), __shfl_down(m.b, o, WAVE)};
+            if(lane + o < WAVE) m = MapOp()(u, m);
+        }
+        acc = MapOp()(PoolMap{__shfl(m.a, 0, WAVE), __shfl(m.b, 0, WAVE)}, acc);
+        if(near < WAVE) {
+            const int64_t p = __shfl(idx < 0 ? pool0 : wp >> 2, near, WAVE);
+            return map_apply(acc, p);
+        }
     }
-    __syncthreads();
 }
 
+// the position a thread of k_drop works on
 template<typename VT>
-__device__ __forceinline__ void level_scan_body(const FactorArgs<VT>& a, const LevelRange& lr,
-    int bid_, int nblk_)
+struct DropPos {
+    int cap, row0, w, col, val, blk, cnt;
+    VT v[LIST_C];
+    int ix[LIST_C];
+};
+
+template<typename VT>
+__device__ __forceinline__ void drop_load(const FactorArgs<VT>& a, const LevelRange& lr, int q,
+    bool in, DropPos<VT>& p)
 {
-    __shared__ PoolMap shm[SC_NW];
-    __shared__ Sizes shs[SC_NW];
-    __shared__ int ticket;
-    int32_t* fmap = a.scan_flags + (int64_t) lr.level * (2 * a.scan_maxch + 1);
-    int32_t* fsize = fmap + a.scan_maxch;
-    if(threadIdx.x == 0) ticket = atomicAdd(fsize + a.scan_maxch, 1);
+    p.cap = CAP_NONE;
+    p.row0 = p.w = p.col = p.val = p.blk = p.cnt = 0;
+#pragma unroll
+    for(int e = 0; e < LIST_C; ++e) { p.v[e] = (VT) 0; p.ix[e] = 0; }
+    if(in) {
+        const int4 l = a.lq[lr.lo + q];
+        p.cap = l.x;
+        p.row0 = l.y;
+        p.w = l.z;
+        p.col = l.w;
+        p.val = a.lq_val[lr.lo + q];
+        p.blk = a.lvlb_idx[lr.lo + q];
+        p.cnt = a.if_cnt[q];
+        // beyond cnt (or for longer lists) these are not used
+#pragma unroll
+        for(int e = 0; e < LIST_C; ++e) {
+            p.v[e] = a.c_val[(int64_t) q * LIST_C + e];
+            p.ix[e] = a.c_idx[(int64_t) q * LIST_C + e];
+        }
+    }
+}
+
+// entries of a sparse position that survive |v| >= tau * sqrtf(norm)
+// (kernels :1919-1946); lists over STORE_TINY entries by the whole wave
+template<typename VT>
+__device__ __forceinline__ int drop_count(const FactorArgs<VT>& a, int q, const DropPos<VT>& p,
+    const VT* nrm)
+{
+    auto keeps = [&](VT v, VT n) { return !(fabs(v) < a.threshold * n); };
+    int keep = 0;
+    const bool big = p.cap >= 0 && p.cnt > STORE_TINY;
+    if(p.cap >= 0 && !big) {
+        if(p.cnt <= LIST_C) {
+#pragma unroll
+            for(int e = 0; e < LIST_C; ++e)
+                if(e < p.cnt) keep += keeps(p.v[e], nrm[p.row0 + (p.ix[e] >> 5)]);
+        } else {
+            const EntryList<VT> l = entry_list(a, q, p.cnt);
+            for(int e = 0; e < p.cnt; ++e) keep += keeps(l.v[e], nrm[p.row0 + (l.ix[e] >> 5)]);
+        }
+    }
+    for(uint64_t bm = wave_ballot(big); bm; bm &= bm - 1) {
+        const int src = __ffsll((long long) bm) - 1;
+        const int bq = __shfl(q, src), bc = __shfl(p.cnt, src), br = __shfl(p.row0, src);
+        const EntryList<VT> l = entry_list(a, bq, bc);
+        int k = 0;
+        for(int e0 = 0; e0 < bc; e0 += WAVE) {
+            const int e = e0 + lane_id();
+            const bool s = e < bc && keeps(l.v[min(e, bc - 1)], nrm[br + (l.ix[min(e, bc - 1)] >> 5)]);
+            k += __popcll(wave_ballot(s));
+        }
+        if(lane_id() == src) keep = k;
+    }
+    return keep;
+}
+
+// Final storage of a sparse block with at most STORE_TINY entries by one
+// lane (the selection and order of store_one), and its row mask
+template<typename VT>
+__device__ void drop_store(const FactorArgs<VT>& a, int q, const DropPos<VT>& p, const VT* nrm,
+    int px, int pv, bool overflow, int max_nnz, int32_t rflag)
+{
+    VT* out_v = a.val_out + pv;
+    int32_t* out_i = a.ix_out + px;
+    uint32_t rows = 0;
+    bool bad = false;
+    auto kept = [&](VT v, int ix) { return !(fabs(v) < a.threshold * nrm[p.row0 + (ix >> 5)]); };
+    auto write = [&](int pos, VT v, int ix) {
+        out_i[pos] = (ix >> 5) * p.w + (ix & 31);
+        out_v[pos] = v;
+        rows |= 1u << (ix >> 5);
+    };
+    int pos = 0;
+    if(p.cnt <= LIST_C && !overflow) {
+#pragma unroll
+        for(int e = 0; e < LIST_C; ++e) {
+            if(e < p.cnt && kept(p.v[e], p.ix[e])) {
+                bad = bad || !finite_value(p.v[e]);
+                if(fabs(p.v[e]) >= (VT) 0) write(pos++, p.v[e], p.ix[e]);
+            }
+        }
+    } else {
+        const EntryList<VT> l = entry_list(a, q, p.cnt);
+        for(int e = 0; e < p.cnt; ++e) {
+            const VT v = l.v[e];
+            const int ix = l.ix[e];
+            if(!kept(v, ix)) continue;
+            bad = bad || !finite_value(v);
+            const VT key = fabs(v);
+            if(!(key >= (VT) 0)) continue;
+            if(!overflow) { write(pos++, v, ix); continue; }
+            // over capacity: the max_nnz largest, ties to the lower index
+            int rank = 0;
+            for(int f = 0; f < p.cnt; ++f) {
+                const VT u = l.v[f];
+                const int fx = l.ix[f];
+                rank += kept(u, fx) && ((VT) fabs(u) > key || ((VT) fabs(u) == key && fx < ix));
+            }
+            if(rank < max_nnz) write(rank, v, ix);
+        }
+    }
+    a.row_mask[p.blk] = store_row_mask(rows, bad, rflag);
+}
+
+// One launch per level, one workgroup per row group (its ticket's, so every
+// group it waits for belongs to a workgroup that is already running). The
+// row sums of its blocks, published by the off-diagonal kernels as (row mask,
+// sums), are laid out in block order in LDS and added up per fine row in that
+// order; each thread then counts what survives of its block, the group's pool
+// map goes out, the pool before the group comes from the groups before it,
+// and each thread writes its block's metadata and entries.
+// Bound by latency: about eight dependent memory round trips. It replaced a
+// row-norm launch, a chunked scan with two waits and a store launch (11.6 +
+// 36 + 8 us per level at n = 400,000, 5 + 44 + 18 us at n = 2,000).
+template<typename VT>
+__device__ __forceinline__ void drop_body(const FactorArgs<VT>& a, const LevelRange& lr)
+{
+    __shared__ DropLds<VT> s;
+    const int t = (int) threadIdx.x;
+    const int lane = lane_id(), wv = t / WAVE;
+    const int64_t pool0 = a.carry[4 * (lr.level & 1)];
+    if(t == 0) s.ticket = atomicAdd(a.grp_ticket + lr.level, 1);
     __syncthreads();
-    const int c = ticket;
-    const int32_t* cin = a.carry + 4 * (lr.level & 1);
-    int32_t* cout = a.carry + 4 * ((lr.level + 1) & 1);
-    // -- entries of a sparse position that survive |v| >= tau * sqrtf(norm)
-    // (kernels :1919-1946); the thread's positions are read in three rounds
-    // of independent loads (capacity / first row / entry count, then each
-    // block's first entry, then that entry's row norm) instead of one
-    // dependent chain per position; further entries (rare at level-0 fill)
-    // are read in order
-    int capk[SC_IPT], frk[SC_IPT], cntk[SC_IPT];
-#pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        const int q = c * SCAN_CHUNK + (int) threadIdx.x * SC_IPT + k;
-        capk[k] = CAP_NONE;
-        frk[k] = 0;
-        cntk[k] = 0;
-        if(q < lr.size) {
-            capk[k] = a.lq_cap[lr.lo + q];
-            frk[k] = a.lq_fr[lr.lo + q];
-            cntk[k] = a.if_cnt[q];
+    const int g = s.ticket;
+    const int4 grp = a.groups[lr.grp_lo + g];
+    const int pp0 = grp.x, np = grp.y, q0 = grp.z, nblk = grp.w;
+    int64_t* state = a.grp_state + 3 * (int64_t) lr.grp_lo;
+    DropPos<VT> pos;
+    drop_load(a, lr, q0 + t, t < nblk, pos);
+    // the group's block rows: fine rows, flags, pivot block metadata
+    if(t < GROUP_ROWS) s.frow[t] = -1;
+    __syncthreads();
+    if(t < np) {
+        const int64_t p = (int64_t) lr.lo + pp0 + t;
+        const int4 r = ((const int4*) a.off_task)[3 * p];   // {block, first row, rows, block row}
+        const int4 l = a.lq[p];
+        const int32_t fl = a.row_flag[r.w];
+        for(int k = 0; k < r.z; ++k) {
+            s.frow[l.y + k] = r.y + k;
+            s.rflag[l.y + k] = fl;
         }
+        BlockMeta& o = a.bout[r.x];
+        o.nnz = 0;
+        o.col_ptr = (int32_t) (l.w - pool0);
+        o.val_ptr = (int32_t) (a.lq_val[p] - pool0);
     }
-    int ix0[SC_IPT];
-    VT v0[SC_IPT];
+    __syncthreads();
+    const int frow = (t < GROUP_ROWS) ? s.frow[t] : -1;
+    VT acc = (frow >= 0) ? a.rn[frow] : (VT) 0;
+    // row sums of squares: pivot block, then the off-diagonal blocks by id
+    for(int c0 = 0; c0 < nblk; c0 += DR_TPB) {
+        const int q = q0 + c0 + t;
+        const bool in = c0 + t < nblk;
+        const uint32_t m = in ? a.part_mask[q] : 0u;
+        const VT first = in ? a.rn_first[q] : (VT) 0;
+        const int row0 = in ? a.lq[lr.lo + q].y : 0;
+        const int n = __popc(m);
+        int off = n;
 #pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        const int q = c * SCAN_CHUNK + (int) threadIdx.x * SC_IPT + k;
-        ix0[k] = 0;
-        v0[k] = (VT) 0;
-        if(capk[k] >= 0 && cntk[k] > 0) {
-            ix0[k] = a.if_idx[(int64_t) q * 1024];
-            v0[k] = a.if_val[(int64_t) q * 1024];
+        for(int o = 1; o < WAVE; o <<= 1) {
+            const int u = __shfl_up(off, o, WAVE);
+            if(lane >= o) off += u;
         }
-    }
-    VT n0[SC_IPT];
-#pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        n0[k] = (VT) 0;
-        if(capk[k] >= 0 && cntk[k] > 0) n0[k] = a.rn[frk[k] + (ix0[k] >> 5)];
-    }
-    int dcnt[SC_IPT];
-    PoolMap m{0, 0};
-#pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        const int q = c * SCAN_CHUNK + (int) threadIdx.x * SC_IPT + k;
-        dcnt[k] = 0;
-        if(capk[k] >= 0) {
-            int keep = 0;
-            if(cntk[k] > 0) {
-                keep = !(fabs(v0[k]) < a.threshold * drop_norm(n0[k]));
-                const VT* vals = a.if_val + (int64_t) q * 1024;
-                const uint16_t* ixs = a.if_idx + (int64_t) q * 1024;
-                for(int e = 1; e < cntk[k]; ++e) {
-                    const VT nrm = drop_norm(a.rn[frk[k] + (ixs[e] >> 5)]);
-                    keep += !(fabs(vals[e]) < a.threshold * nrm);
+        const int total = __shfl(off, WAVE - 1, WAVE);
+        off -= n;
+        // all lanes at once, or sixteen (at most DR_RUNS sums) at a time, one
+        // wave after the other
+        const bool split = __syncthreads_or(total > DR_RUNS) != 0;
+        for(int step = 0; step < (split ? 4 * DR_NW : 1); ++step) {
+            const int l0 = split ? 16 * (step & 3) : 0;
+            const bool mine = !split || step / 4 == wv;
+            const int base = __shfl(off, l0, WAVE);
+            const int end = (split && l0 < 48) ? __shfl(off, min(l0 + 16, WAVE - 1), WAVE) : total;
+            for(int k = lane; k < GROUP_ROWS * (DR_RUNS / 32); k += WAVE)
+                s.rows[wv][k / (DR_RUNS / 32)][k % (DR_RUNS / 32)] = 0u;
+            if(lane == 0) s.runs[wv] = mine ? end - base : 0;
+            wave_sync();
+            if(mine && (!split || lane / 16 == l0 / 16)) {
+                int j = 0;
+                for(uint32_t bits = m; bits; bits &= bits - 1, ++j) {
+                    const int at = off - base + j;
+                    s.val[wv][at] = (j == 0) ? first : a.rn_part[(int64_t) q * 32 + j];
+                    atomicOr(&s.rows[wv][row0 + __ffs(bits) - 1][at >> 5], 1u << (at & 31));
                 }
             }
-            a.drop_cnt[q] = keep;
-            dcnt[k] = keep;
-            m = MapOp()(m, PoolMap{(int64_t) capk[k] - keep, 0});
+            __syncthreads();
+            if(t < GROUP_ROWS)
+                for(int u = 0; u < DR_NW; ++u)
+                    for(int wd = 0; 32 * wd < s.runs[u]; ++wd)
+                        for(uint32_t bits = s.rows[u][t][wd]; bits; bits &= bits - 1)
+                            acc += s.val[u][32 * wd + __ffs(bits) - 1];
+            __syncthreads();
         }
     }
-    PoolMap mtot;
-    const PoolMap mex = block_exclusive_scan<PoolMap, MapOp, SC_NW>(m, MapOp(), PoolMap{0, 0}, shm,
-        &mtot);
-    if(threadIdx.x == 0) {
-        a.chunk[4 * c + 0] = mtot.a;
-        a.chunk[4 * c + 1] = mtot.b;
-        __hip_atomic_store(fmap + c, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if(t < GROUP_ROWS) {
+        if(frow >= 0) a.rn[frow] = acc;
+        s.nrm[t] = drop_norm(acc);
     }
-    wait_chunk_flags(fmap, c, a.err);
-    // -- pools, grants and kept counts
-    const int64_t* ch = a.chunk;
-    const PoolMap before = block_prefix<PoolMap>(c,
-        [ch](int i) { return PoolMap{load_published(ch + 4 * i), load_published(ch + 4 * i + 1)}; },
-        MapOp(), PoolMap{0, 0}, shm);
-    const int64_t pool_c = map_apply(before, cin[0]);
-    int64_t pl = map_apply(mex, pool_c);
-    int kp[SC_IPT], gr[SC_IPT];
-    Sizes sz{0, 0};
-#pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        const int q = c * SCAN_CHUNK + (int) threadIdx.x * SC_IPT + k;
-        kp[k] = 0;
-        gr[k] = 0;
-        if(capk[k] >= 0) {
-            int64_t g = 0;
-            if(dcnt[k] > capk[k]) {
-                const int64_t e = (int64_t) dcnt[k] - capk[k];
-                g = e < pl ? e : pl;
+    __syncthreads();
+    // survivors and the group's pool map
+    PoolMap tot{0, 0}, ex{0, 0};
+    int dcnt = 0;
+    for(int c0 = 0; c0 < nblk; c0 += DR_TPB) {
+        const int q = q0 + c0 + t;
+        const bool in = c0 + t < nblk;
+        if(c0) drop_load(a, lr, q, in, pos);
+        dcnt = drop_count(a, q, pos, s.nrm);
+        if(nblk > DR_TPB && in) a.drop_cnt[q] = dcnt;
+        const PoolMap m = pos.cap >= 0 ? PoolMap{(int64_t) pos.cap - dcnt, 0} : PoolMap{0, 0};
+        PoolMap ctot;
+        ex = block_exclusive_scan<PoolMap, MapOp, DR_NW>(m, MapOp(), PoolMap{0, 0}, s.sh, &ctot);
+        tot = MapOp()(tot, ctot);
+    }
+    if(t == 0) {
+        publish(state + 3 * (int64_t) g, tot.a);
+        publish(state + 3 * (int64_t) g + 1, tot.b);
+    }
+    if(wv == 0) {
+        const int64_t before = pool_before(state, g, pool0, a.err);
+        if(t == 0) {
+            const int64_t after = map_apply(tot, before);
+            publish(state + 3 * (int64_t) g + 2, after);
+            s.pool = before;
+            if(g == lr.ngrp - 1) {
+                int32_t* cout = a.carry + 4 * ((lr.level + 1) & 1);
+                cout[0] = (int32_t) after;
+                cout[1] = (int32_t) (lr.end_ix - after);
+                cout[2] = (int32_t) (lr.end_val - after);
             }
-            const int64_t room = capk[k] + g;
-            kp[k] = (int32_t) (dcnt[k] < room ? dcnt[k] : room);
-            gr[k] = (int32_t) g;
-            const int64_t np = pl + capk[k] - dcnt[k];
-            pl = np > 0 ? np : 0;
-            a.keep[q] = kp[k];
-            a.granted[q] = gr[k];
-            sz.x += kp[k];
-            sz.v += kp[k];
-        } else if(capk[k] != CAP_NONE) {
-            sz.v += -1 - capk[k];
         }
     }
-    Sizes stot;
-    const Sizes sex = block_exclusive_scan<Sizes, SumOp, SC_NW>(sz, SumOp(), Sizes{0, 0}, shs, &stot);
-    if(threadIdx.x == 0) {
-        a.chunk[4 * c + 2] = stot.x;
-        a.chunk[4 * c + 3] = stot.v;
-        __hip_atomic_store(fsize + c, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    wait_chunk_flags(fsize, c, a.err);
-    // -- output offsets and factored metadata
-    const Sizes sbefore = block_prefix<Sizes>(c,
-        [ch](int i) { return Sizes{load_published(ch + 4 * i + 2), load_published(ch + 4 * i + 3)}; },
-        SumOp(), Sizes{0, 0}, shs);
-    int64_t px = cin[1] + sbefore.x + sex.x, pv = cin[2] + sbefore.v + sex.v;
-#pragma unroll
-    for(int k = 0; k < SC_IPT; ++k) {
-        if(capk[k] == CAP_NONE) continue;
-        const int q = c * SCAN_CHUNK + (int) threadIdx.x * SC_IPT + k;
-        const int b = a.lvlb_idx[lr.lo + q];
-        BlockMeta o = a.bin[b];
-        int64_t nv;
-        if(capk[k] >= 0) {
-            o.nnz = kp[k];
-            o.max_nnz = capk[k] + gr[k];
-            if(dcnt[k] > capk[k]) o.got_extra = gr[k];
-            a.overflow[q] = (uint8_t) (dcnt[k] > capk[k] + gr[k]);
-            nv = kp[k];
-        } else {
-            o.nnz = 0;
-            a.overflow[q] = 0;
-            nv = -1 - capk[k];
+    __syncthreads();
+    // pools, grants, metadata and storage
+    int64_t pool = s.pool;
+    for(int c0 = 0; c0 < nblk; c0 += DR_TPB) {
+        const int q = q0 + c0 + t;
+        const bool in = c0 + t < nblk;
+        if(nblk > DR_TPB) {
+            drop_load(a, lr, q, in, pos);
+            dcnt = in ? a.drop_cnt[q] : 0;
+            const PoolMap m = pos.cap >= 0 ? PoolMap{(int64_t) pos.cap - dcnt, 0} : PoolMap{0, 0};
+            PoolMap ctot;
+            ex = block_exclusive_scan<PoolMap, MapOp, DR_NW>(m, MapOp(), PoolMap{0, 0}, s.sh,
+                &ctot);
+            tot = ctot;
         }
-        o.col_ptr = (int32_t) px;
-        o.val_ptr = (int32_t) pv;
-        px += (capk[k] >= 0) ? kp[k] : 0;
-        pv += nv;
-        a.bout[o.id] = o;
-    }
-    if(threadIdx.x == 0 && c == nblk_ - 1) {
-        cout[0] = (int32_t) map_apply(mtot, pool_c);
-        cout[1] = (int32_t) (cin[1] + sbefore.x + stot.x);
-        cout[2] = (int32_t) (cin[2] + sbefore.v + stot.v);
+        if(in) {
+            const int64_t pl = map_apply(ex, pool);
+            const int32_t px = (int32_t) (pos.col - pl), pv = (int32_t) (pos.val - pl);
+            BlockMeta& o = a.bout[pos.blk];
+            o.col_ptr = px;
+            o.val_ptr = pv;
+            bool wave_form = true, overflow = false;
+            if(pos.cap >= 0) {
+                const int64_t e = (int64_t) dcnt - pos.cap;
+                const int32_t gr = (int32_t) (e > 0 ? (e < pl ? e : pl) : 0);
+                const int32_t room = pos.cap + gr;
+                overflow = dcnt > room;
+                o.nnz = overflow ? room : dcnt;
+                o.max_nnz = room;
+                o.got_extra = gr;
+                wave_form = pos.cnt > STORE_TINY;
+                if(!wave_form)
+                    drop_store(a, q, pos, s.nrm, px, pv, overflow, room, s.rflag[pos.row0]);
+            } else {
+                o.nnz = 0;
+            }
+            if(wave_form) {
+                a.overflow[q] = overflow ? 1 : 0;
+                a.store_list[atomicAdd(a.store_cnt + lr.level, 1)] = q;
+            }
+        }
+        pool = map_apply(tot, pool);
     }
 }
 
@@ -2028,7 +2150,7 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
     const int fr = a.bs[mo.block_row];
     const int h = a.bs[mo.block_row + 1] - fr;
     const int w = a.bs[mo.block_col + 1] - a.bs[mo.block_col];
-    const VT* vals = a.if_val + (int64_t) q * 1024;
+    const VT* vals = a.if_val + (int64_t) q * 1024;   // more than LIST_C entries
     VT* out_v = a.val_out + mo.val_ptr;
     if(mo.format == FMT_DENSE) {
         for(int e = lane; e < h * w; e += 64) out_v[e] = vals[e];
@@ -2103,7 +2225,7 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
     keep_mask();
 }
 
-// the positions k_store_tiny leaves to the wave form, grid-stride
+// the positions k_drop leaves to the wave form, grid-stride
 template<typename VT>
 __device__ __forceinline__ void store_body(const FactorArgs<VT>& a, const LevelRange& lr,
     int bid_, int nblk_)
@@ -2116,78 +2238,6 @@ __device__ __forceinline__ void store_body(const FactorArgs<VT>& a, const LevelR
         store_one(a, lr, a.store_list[t], nrm, key, kix);
         wave_sync();
     }
-}
-
-// one lane per sparse block with at most STORE_TINY pre-drop entries, the
-// same selection and order as store_one; the rest go to the wave form
-constexpr int STORE_TINY = 16;
-
-template<typename VT>
-__device__ __forceinline__ void store_tiny_body(const FactorArgs<VT>& a, const LevelRange& lr,
-    int bid_, int nblk_)
-{
-    const int q = bid_ * 256 + (int) threadIdx.x;
-    if(q >= lr.size) return;
-    const int cap = a.lq_cap[lr.lo + q];
-    const int cnt = a.if_cnt[q];
-    if(cap < 0 || cnt > STORE_TINY) {
-        a.store_list[atomicAdd(a.store_cnt + lr.level, 1)] = q;
-        return;
-    }
-    const int b = a.lvlb_idx[lr.lo + q];
-    const BlockMeta mo = a.bout[b];
-    const int fr = a.lq_fr[lr.lo + q];
-    const int w = a.bs[mo.block_col + 1] - a.bs[mo.block_col];
-    const VT* vals = a.if_val + (int64_t) q * 1024;
-    const uint16_t* ixs = a.if_idx + (int64_t) q * 1024;
-    VT* out_v = a.val_out + mo.val_ptr;
-    int32_t* out_i = a.ix_out + mo.col_ptr;
-    const int32_t rflag = a.row_flag[mo.block_row];
-    uint32_t rows = 0;
-    bool bad = false;
-    VT key[STORE_TINY];
-    int ixk[STORE_TINY];
-#pragma unroll
-    for(int e = 0; e < STORE_TINY; ++e) {
-        key[e] = (VT) -1;
-        ixk[e] = 0;
-        if(e < cnt) {
-            const VT v = vals[e];
-            const int ix = ixs[e];
-            const bool k = !(fabs(v) < a.threshold * drop_norm(a.rn[fr + (ix >> 5)]));
-            key[e] = k ? (VT) fabs(v) : (VT) -1;
-            ixk[e] = ix;
-            bad = bad || (k && !finite_value(v));
-        }
-    }
-    if(!a.overflow[q]) {
-        int pos = 0;
-#pragma unroll
-        for(int e = 0; e < STORE_TINY; ++e) {
-            if(key[e] >= (VT) 0) {
-                out_i[pos] = (ixk[e] >> 5) * w + (ixk[e] & 31);
-                out_v[pos] = vals[e];
-                rows |= 1u << (ixk[e] >> 5);
-                ++pos;
-            }
-        }
-        a.row_mask[b] = store_row_mask(rows, bad, rflag);
-        return;
-    }
-#pragma unroll
-    for(int e = 0; e < STORE_TINY; ++e) {
-        if(key[e] < (VT) 0) continue;
-        int rank = 0;
-#pragma unroll
-        for(int f = 0; f < STORE_TINY; ++f)
-            rank += (f < cnt) && ((key[f] > key[e]) || (key[f] == key[e] && ixk[f] < ixk[e]));
-        if(rank < mo.max_nnz) {
-            out_i[rank] = (ixk[e] >> 5) * w + (ixk[e] & 31);
-            out_v[rank] = vals[e];
-            rows |= 1u << (ixk[e] >> 5);
-        }
-    }
-    a.row_mask[b] = store_row_mask(rows, bad, rflag);
 }
 
 // k_pivot_col_blocks (kernels :1352-1418) with d_col_pivot_block
@@ -2221,27 +2271,15 @@ __global__ __launch_bounds__(64) void k_pivots_pairs(FactorArgs<VT> a, LevelRang
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64) void k_rownorm(FactorArgs<VT> a, LevelRange lr)
+__global__ __launch_bounds__(DR_TPB) void k_drop(FactorArgs<VT> a, LevelRange lr)
 {
-    rownorm_body<VT>(a, lr, blockIdx.x, gridDim.x);
-}
-
-template<typename VT>
-__global__ __launch_bounds__(SC_TPB) void k_level_scan(FactorArgs<VT> a, LevelRange lr)
-{
-    level_scan_body<VT>(a, lr, blockIdx.x, gridDim.x);
+    drop_body<VT>(a, lr);
 }
 
 template<typename VT>
 __global__ __launch_bounds__(64) void k_store(FactorArgs<VT> a, LevelRange lr)
 {
     store_body<VT>(a, lr, blockIdx.x, gridDim.x);
-}
-
-template<typename VT>
-__global__ __launch_bounds__(256) void k_store_tiny(FactorArgs<VT> a, LevelRange lr)
-{
-    store_tiny_body<VT>(a, lr, blockIdx.x, gridDim.x);
 }
 
 template<typename VT>
@@ -2315,9 +2353,7 @@ __global__ void bk_factor_begin(const FactorSys<VT>* fs, const int2* items)
         a.perm[g] = (int32_t) g;
     }
     if(g < F.val_space) F.val_in[g] = (VT) 0;
-    const int64_t nf = (a.num_levels > 0 && a.scan_maxch > 0)
-        ? (int64_t) (2 * a.scan_maxch + 1) * a.num_levels : 0;
-    if(g < nf) a.scan_flags[g] = 0;
+    if(g < a.state_words) ((int32_t*) a.grp_state)[g] = 0;
     if(g < a.num_levels) {
         a.defer_cnt[g] = 0;
         a.wave_cnt[g] = 0;
@@ -2377,33 +2413,12 @@ __global__ __launch_bounds__(64) void bk_offdiag_general(const FactorSys<VT>* fs
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64) void bk_rownorm(const FactorSys<VT>* fs, const int2* items,
+__global__ __launch_bounds__(DR_TPB) void bk_drop(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
-    const int2 it = items[blockIdx.x];
-    const FactorSys<VT>& F = fs[it.x];
+    const FactorSys<VT>& F = fs[items[blockIdx.x].x];
     const LevelRange lr = F.lr[level];
-    rownorm_body<VT>(F.a, lr, it.y, lr.npiv);
-}
-
-template<typename VT>
-__global__ __launch_bounds__(SC_TPB) void bk_level_scan(const FactorSys<VT>* fs, const int2* items,
-    int32_t level)
-{
-    const int2 it = items[blockIdx.x];
-    const FactorSys<VT>& F = fs[it.x];
-    const LevelRange lr = F.lr[level];
-    level_scan_body<VT>(F.a, lr, it.y, fl_grid_level_scan(lr));
-}
-
-template<typename VT>
-__global__ __launch_bounds__(256) void bk_store_tiny(const FactorSys<VT>* fs, const int2* items,
-    int32_t level)
-{
-    const int2 it = items[blockIdx.x];
-    const FactorSys<VT>& F = fs[it.x];
-    const LevelRange lr = F.lr[level];
-    store_tiny_body<VT>(F.a, lr, it.y, fl_grid_store_tiny(lr));
+    drop_body<VT>(F.a, lr);
 }
 
 template<typename VT>
@@ -2413,7 +2428,7 @@ __global__ __launch_bounds__(64) void bk_store(const FactorSys<VT>* fs, const in
     const int2 it = items[blockIdx.x];
     const FactorSys<VT>& F = fs[it.x];
     const LevelRange lr = F.lr[level];
-    store_body<VT>(F.a, lr, it.y, fl_grid_tasks(lr.size, BATCH_TASK_GRID));
+    store_body<VT>(F.a, lr, it.y, fl_grid_tasks(lr.size - lr.npiv, BATCH_TASK_GRID));
 }
 
 }  // namespace
@@ -2449,10 +2464,9 @@ void factor_begin(const FactorArgs<VT>& a, void* stream)
 {
     hipStream_t st = (hipStream_t) stream;
     k_zero_carry<VT><<<1, 64, 0, st>>>(a.carry);
-    if(a.num_levels > 0 && a.scan_maxch > 0) {
-        const int64_t nf = (int64_t) (2 * a.scan_maxch + 1) * a.num_levels;
-        k_zero<int32_t><<<(unsigned) ((nf + 255) / 256), 256, 0, st>>>(a.scan_flags, nf);
-    }
+    if(a.state_words > 0)
+        k_zero<int32_t><<<(unsigned) ((a.state_words + 255) / 256), 256, 0, st>>>(
+            (int32_t*) a.grp_state, a.state_words);
     if(a.num_levels > 0) {
         const unsigned g = (unsigned) ((a.num_levels + 255) / 256);
         k_zero<int32_t><<<g, 256, 0, st>>>(a.defer_cnt, a.num_levels);
@@ -2476,10 +2490,8 @@ void factor_level(const FactorArgs<VT>& a, const LevelRange& r, void* stream)
         k_offdiag_general<VT><<<grid, 64, 0, st>>>(a, r);
     }
     if(a.pivoting && r.npiv > 0) k_pivot_cols<VT><<<r.npiv, 64, 0, st>>>(a, r);
-    if(r.npiv > 0) k_rownorm<VT><<<r.npiv, 64, 0, st>>>(a, r);
-    k_level_scan<VT><<<fl_grid_level_scan(r), SC_TPB, 0, st>>>(a, r);
-    k_store_tiny<VT><<<fl_grid_store_tiny(r), 256, 0, st>>>(a, r);
-    k_store<VT><<<fl_grid_tasks(r.size, 2048), 64, 0, st>>>(a, r);
+    if(r.ngrp > 0) k_drop<VT><<<r.ngrp, DR_TPB, 0, st>>>(a, r);
+    if(noff > 0) k_store<VT><<<fl_grid_tasks(noff, 2048), 64, 0, st>>>(a, r);
 }
 
 template void gather_values<double>(const double*, const int64_t*, int64_t, double*, int64_t, void*);
@@ -2491,11 +2503,10 @@ template void factor_level<float>(const FactorArgs<float>&, const LevelRange&, v
 
 
 int64_t factor_batch_chunks(int32_t n, int64_t nnz, int64_t val_space, int32_t num_levels,
-    int32_t scan_maxch)
+    int32_t state_words)
 {
     int64_t m = std::max<int64_t>(std::max<int64_t>(n, nnz), std::max<int64_t>(val_space, 1));
-    if(num_levels > 0 && scan_maxch > 0)
-        m = std::max<int64_t>(m, (int64_t) (2 * scan_maxch + 1) * num_levels);
+    m = std::max<int64_t>(m, state_words);
     m = std::max<int64_t>(m, num_levels);
     return (m + 255) / 256;
 }
@@ -2521,9 +2532,7 @@ void factor_batch_level(const FactorSys<VT>* fs, const FactorBatchLevel& L, int3
         bk_offdiag<VT><<<grid(L.off), 64, 0, st>>>(fs, L.off.items, level);
         bk_offdiag_general<VT><<<grid(L.off), 64, 0, st>>>(fs, L.off.items, level);
     }
-    if(L.rn.count) bk_rownorm<VT><<<grid(L.rn), 64, 0, st>>>(fs, L.rn.items, level);
-    if(L.sc.count) bk_level_scan<VT><<<grid(L.sc), SC_TPB, 0, st>>>(fs, L.sc.items, level);
-    if(L.stt.count) bk_store_tiny<VT><<<grid(L.stt), 256, 0, st>>>(fs, L.stt.items, level);
+    if(L.dr.count) bk_drop<VT><<<grid(L.dr), DR_TPB, 0, st>>>(fs, L.dr.items, level);
     if(L.st.count) bk_store<VT><<<grid(L.st), 64, 0, st>>>(fs, L.st.items, level);
 }
 

@@ -35,7 +35,6 @@ struct FactorArgs {
     const int32_t* lvlb_idx = nullptr;    // level block list
     const int32_t* block_in_lvl = nullptr;
     const int32_t* lvl_rows = nullptr;
-    const int32_t* rfo = nullptr;         // row_first_block_offset
     const int32_t* ix_in = nullptr;       // input stores
     const VT* val_in = nullptr;
     int32_t* ix_out = nullptr;            // output stores
@@ -43,13 +42,20 @@ struct FactorArgs {
     double* tri = nullptr;                // 3n, tridiagonal D
     VT* rn = nullptr;                     // n, row sums of squares
     // per level position scratch
+    // the entries of a position before dropping: LIST_C or fewer in c_val /
+    // c_idx (contiguous over the positions, so that neighbouring positions
+    // share cache lines), more in if_val / if_idx; dense tiles in if_val
     VT* if_val = nullptr;                 // 1024 per position
     uint16_t* if_idx = nullptr;           // 1024 per position
+    VT* c_val = nullptr;                  // LIST_C per position
+    uint16_t* c_idx = nullptr;            // LIST_C per position
     int32_t* if_cnt = nullptr;
+    // row sums of squares of a position: the rows with a nonzero sum, the
+    // first such row's sum, and the j-th's at rn_part[32 q + j]
+    uint32_t* part_mask = nullptr;
+    VT* rn_first = nullptr;
     VT* rn_part = nullptr;                // 32 per position
     int32_t* drop_cnt = nullptr;
-    int32_t* keep = nullptr;              // entries kept per position
-    int32_t* granted = nullptr;           // leftover space granted per position
     uint8_t* overflow = nullptr;
     int32_t* piv_loc = nullptr;           // nb
     // rows of each factored off-diagonal block that can contribute to a
@@ -57,19 +63,26 @@ struct FactorArgs {
     // to that (ROW_2X2, ROW_NONFINITE)
     uint32_t* row_mask = nullptr;         // per coarse block
     int32_t* row_flag = nullptr;          // nb
-    // static, in level-list order: capacity of a sparse block (max_nnz >= 0)
-    // or -1 - rows * cols for a dense block; first fine row of its block row
-    const int32_t* lq_cap = nullptr;
-    const int32_t* lq_fr = nullptr;
-    int64_t* chunk = nullptr;             // per scan chunk: pool map (2), sizes (2)
-    // per level: two flags per scan chunk (pool map, sizes published) and a
-    // chunk ticket counter (2 scan_maxch + 1 words); zeroed at the start of
-    // every factor
-    int32_t* scan_flags = nullptr;
-    int32_t scan_maxch = 0;
-    // pinned host flag: 2 when a scan chunk's bounded wait gave up
+    // static, in level-list order: {capacity of a sparse block (max_nnz >= 0)
+    // or -1 - rows * cols of a dense one, the first of its rows within its
+    // row group, its width, its offset in the index store when every block
+    // keeps its capacity}, and that offset in the value store
+    const int4* lq = nullptr;
+    const int32_t* lq_val = nullptr;
+    // static, row groups of the levels: {first pivot position, block rows,
+    // first off-diagonal position, off-diagonal blocks}
+    const int4* groups = nullptr;
+    // per row group: published pool map (2 words) and pool (1 word), then
+    // one ticket counter per level; state_words 32-bit words in all, zeroed
+    // at the start of every factor
+    int64_t* grp_state = nullptr;
+    int32_t* grp_ticket = nullptr;
+    int32_t state_words = 0;
+    // pinned host flag: 2 when a row group's bounded wait gave up
     int32_t* err = nullptr;
-    // static, per level-list position of an off-diagonal block, 12 int32:
+    // static, per level-list position of an off-diagonal block, 12 int32
+    // (of a pivot block {block, first row, rows, block row}, {format, nnz,
+    // col_ptr, val_ptr}, {first block of its column, blocks above it}):
     // {block, first row, rows | cols << 8 | all-1x1 << 16, pivot position},
     // {input format, nnz, col_ptr, val_ptr}, {first pair (low 32 bits),
     // pairs, flags, first pair (high 32 bits)} with flags bit 0: small
@@ -86,14 +99,18 @@ struct FactorArgs {
     int32_t* store_list = nullptr;        // positions stored by one wave each
     int32_t* store_cnt = nullptr;         // one counter per level
     int32_t num_levels = 0;
-    // two sets of {pool, out_ix, out_val, 0}; level l reads set l & 1 and
-    // writes set (l + 1) & 1
+    // two sets of {pool, index entries, value entries stored, 0}; level l
+    // reads the pool of set l & 1 and writes set (l + 1) & 1
     int32_t* carry = nullptr;
     VT threshold = 0;
 };
 
-// positions per chunk of the level scans (256 threads x 8)
-constexpr int SCAN_CHUNK = 2048;
+constexpr int LIST_C = 4;
+// A row group is one workgroup's share of a level's dropping step: block
+// rows that follow each other, at most GROUP_ROWS fine rows, and at most
+// GROUP_BLOCKS off-diagonal blocks unless one block row has more.
+constexpr int GROUP_ROWS = 32;
+constexpr int GROUP_BLOCKS = 256;
 
 struct LevelRange {
     int32_t lo;        // offset of the level in the level block list
@@ -101,6 +118,10 @@ struct LevelRange {
     int32_t size;      // blocks in the level
     int32_t row_lo;    // offset of the level in lvl_rows
     int32_t level;     // level index
+    int32_t grp_lo;    // first row group
+    int32_t ngrp;      // row groups
+    int32_t end_ix;    // store sizes after the level when every block keeps
+    int32_t end_val;   // its capacity
 };
 
 // threads of a k_offdiag_tiny_scale workgroup (one per one-lane block)
@@ -125,14 +146,6 @@ __host__ __device__ inline int32_t fl_grid_tasks(int32_t count, int32_t cap)
 {
     return count > 0 ? (count < cap ? count : cap) : 0;
 }
-__host__ __device__ inline int32_t fl_grid_level_scan(const LevelRange& r)
-{
-    return (r.size + SCAN_CHUNK - 1) / SCAN_CHUNK;
-}
-__host__ __device__ inline int32_t fl_grid_store_tiny(const LevelRange& r)
-{
-    return (r.size + 255) / 256;
-}
 
 // One system of a batched refactor (device table entry).
 template<typename VT>
@@ -156,9 +169,7 @@ struct FactorBatchLevel {
     FactorItems pp;    // k_pivots_pairs
     FactorItems ts;    // k_offdiag_tiny_scale
     FactorItems off;   // k_offdiag and k_offdiag_general (BATCH_TASK_GRID per system)
-    FactorItems rn;    // k_rownorm
-    FactorItems sc;    // k_level_scan
-    FactorItems stt;   // k_store_tiny
+    FactorItems dr;    // k_drop
     FactorItems st;    // k_store (BATCH_TASK_GRID per system)
 };
 
@@ -173,7 +184,7 @@ void factor_batch_level(const FactorSys<VT>* fs, const FactorBatchLevel& L, int3
     hipStream_t st);
 // chunks of 256 entries factor_batch_begin needs for a system
 int64_t factor_batch_chunks(int32_t n, int64_t nnz, int64_t val_space, int32_t num_levels,
-    int32_t scan_maxch);
+    int32_t state_words);
 template<typename VT>
 void factor_begin(const FactorArgs<VT>& a, void* stream);
 template<typename VT>

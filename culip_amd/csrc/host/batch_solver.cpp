@@ -415,15 +415,8 @@ void BatchSolver::build_factor()
         for(int32_t b = 0; b < y.nb; ++b)
             max_h_ = std::max(max_h_, y.block_starts[b + 1] - y.block_starts[b]);
         lr_off[s] = lrs.size();
-        for(int32_t l = 0; l < y.num_levels; ++l) {
-            LevelRange r;
-            r.lo = y.lvlb_off[l];
-            r.size = y.lvlb_off[l + 1] - r.lo;
-            r.npiv = y.lvl_off[l + 1] - y.lvl_off[l];
-            r.row_lo = y.lvl_off[l];
-            r.level = l;
-            lrs.push_back(r);
-        }
+        const std::vector<LevelRange>& lv = sys_[s]->f->pat->levels;
+        lrs.insert(lrs.end(), lv.begin(), lv.end());
         max_levels = std::max(max_levels, y.num_levels);
     }
     // the solve layout's LDS tile of a pivot-block inverse is max_h_ squared
@@ -451,7 +444,7 @@ void BatchSolver::build_factor()
         p.totals = f.d_totals.as<int32_t>();
         p.scan_tmp = f.d_scan_tmp.as<int32_t>();
         const int64_t nch = factor_batch_chunks(f.n(), q.nnz, q.val_space, f.sym.num_levels,
-            q.a.scan_maxch);
+            q.a.state_words);
         for(int64_t c = 0; c < nch; ++c) chunks.push_back(make_int2(s, (int) c));
         for(int32_t r = 0; r < p.t.nb; ++r) blk.push_back(make_int2(s, r));
         for(int32_t c = 0; c < scan_chunks(f.n()); ++c) scan.push_back(make_int2(s, c));
@@ -473,29 +466,29 @@ void BatchSolver::build_factor()
     scan_ = put(d_scan_, scan);
     task_ = put(d_task_, task);
     // per level and launch: the workgroups of every system that has the level
-    std::vector<int2> it[7];
-    std::vector<std::array<size_t, 7>> off(max_levels + 1);
+    std::vector<int2> it[5];
+    std::vector<std::array<size_t, 5>> off(max_levels + 1);
     for(int32_t l = 0; l < max_levels; ++l) {
-        for(int k = 0; k < 7; ++k) off[l][k] = it[k].size();
+        for(int k = 0; k < 5; ++k) off[l][k] = it[k].size();
         for(int32_t s = 0; s < S; ++s) {
             if(l >= sys_[s]->f->sym.num_levels) continue;
             const LevelRange& r = lrs[lr_off[s] + l];
             const int32_t noff = r.size - r.npiv;
-            const int32_t cnt[7] = {fl_grid_pivots_pairs(r), fl_tiny_blocks(r),
-                fl_grid_tasks(noff, BATCH_TASK_GRID), r.npiv, fl_grid_level_scan(r),
-                fl_grid_store_tiny(r), fl_grid_tasks(r.size, BATCH_TASK_GRID)};
-            for(int k = 0; k < 7; ++k)
+            const int32_t cnt[5] = {fl_grid_pivots_pairs(r), fl_tiny_blocks(r),
+                fl_grid_tasks(noff, BATCH_TASK_GRID), r.ngrp,
+                fl_grid_tasks(noff, BATCH_TASK_GRID)};
+            for(int k = 0; k < 5; ++k)
                 for(int32_t q = 0; q < cnt[k]; ++q) it[k].push_back(make_int2(s, q));
         }
     }
-    for(int k = 0; k < 7; ++k) off[max_levels][k] = it[k].size();
-    FactorItems all[7];
-    for(int k = 0; k < 7; ++k) all[k] = put(d_fit_[k], it[k]);
+    for(int k = 0; k < 5; ++k) off[max_levels][k] = it[k].size();
+    FactorItems all[5];
+    for(int k = 0; k < 5; ++k) all[k] = put(d_fit_[k], it[k]);
     flevels_.assign(max_levels, FactorBatchLevel{});
     for(int32_t l = 0; l < max_levels; ++l) {
-        FactorItems* dst[7] = {&flevels_[l].pp, &flevels_[l].ts, &flevels_[l].off,
-            &flevels_[l].rn, &flevels_[l].sc, &flevels_[l].stt, &flevels_[l].st};
-        for(int k = 0; k < 7; ++k) {
+        FactorItems* dst[5] = {&flevels_[l].pp, &flevels_[l].ts, &flevels_[l].off,
+            &flevels_[l].dr, &flevels_[l].st};
+        for(int k = 0; k < 5; ++k) {
             dst[k]->items = all[k].items + off[l][k];
             dst[k]->count = (int32_t) (off[l + 1][k] - off[l][k]);
         }

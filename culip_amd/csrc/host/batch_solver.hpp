@@ -118,7 +118,7 @@ private:
     int32_t* h_flags_ = nullptr;
     BatchSys* h_sys_pinned_ = nullptr;
     // batched refactor: system tables, level ranges, work items
-    DevBuf d_fsys_, d_psys_, d_lr_, d_fit_[7], d_chunks_, d_blk_, d_scan_, d_task_;
+    DevBuf d_fsys_, d_psys_, d_lr_, d_fit_[5], d_chunks_, d_blk_, d_scan_, d_task_;
     std::vector<FactorBatchLevel> flevels_;
     int32_t max_h_ = 1;   // largest block height of the batch
     FactorItems chunks_, blk_, scan_, task_;

@@ -43,7 +43,7 @@ int64_t BildltPattern::device_bytes() const
     int64_t b = 0;
     for(const DevBuf* d : {&d_bs, &d_is_piv, &d_bin, &d_csr_off, &d_csc_off, &d_csc_idx, &d_upd_off,
             &d_upd_ki, &d_upd_kj, &d_lvlb_idx, &d_block_in_lvl, &d_lvl_rows, &d_ix_in,
-            &d_value_slot, &d_rfo, &d_lq_cap, &d_lq_fr, &d_off_task, &d_upd4})
+            &d_value_slot, &d_lq, &d_lq_val, &d_groups, &d_off_task, &d_upd4})
         b += (int64_t) d->bytes;
     return b;
 }
@@ -63,25 +63,11 @@ void BildltPattern::upload_static()
     upload(d_lvlb_idx, s.lvlb_idx);
     upload(d_block_in_lvl, s.block_in_lvl);
     upload(d_lvl_rows, s.lvl_rows);
-    upload(d_rfo, s.row_first_block_offset);
     upload(d_ix_in, s.ix_store);
     upload(d_value_slot, s.value_slot);
 
     const int32_t K = s.coarse_nnz;
-    // per level-list position: sparse capacity or -1 - rows * cols (dense),
-    // and the first fine row of the block row
-    {
-        std::vector<int32_t> cap(K), fr(K);
-        for(int32_t p = 0; p < K; ++p) {
-            const BlockMeta& m = s.blocks[s.lvlb_idx[p]];
-            const int32_t h = s.block_starts[m.block_row + 1] - s.block_starts[m.block_row];
-            const int32_t w = s.block_starts[m.block_col + 1] - s.block_starts[m.block_col];
-            cap[p] = (m.format == FMT_SPARSE) ? m.max_nnz : -1 - h * w;
-            fr[p] = s.block_starts[m.block_row];
-        }
-        upload(d_lq_cap, cap);
-        upload(d_lq_fr, fr);
-    }
+    build_levels();
     // off-diagonal task descriptors (12 int32 per level-list position) and
     // Schur pairs with the rows of their block k
     {
@@ -92,6 +78,16 @@ void BildltPattern::upload_static()
         for(int32_t l = 0; l < s.num_levels; ++l) {
             const int32_t lo = s.lvlb_off[l], hi = s.lvlb_off[l + 1];
             const int32_t npiv = s.lvl_off[l + 1] - s.lvl_off[l];
+            for(int32_t p = lo; p < lo + npiv; ++p) {
+                const int32_t b = s.lvlb_idx[p];
+                const BlockMeta& m = s.blocks[b];
+                const int32_t i = m.block_row;
+                int32_t* t = &task[(size_t) 12 * p];
+                t[0] = b; t[1] = s.block_starts[i];
+                t[2] = s.block_starts[i + 1] - s.block_starts[i]; t[3] = i;
+                t[4] = m.format; t[5] = m.nnz; t[6] = m.col_ptr; t[7] = m.val_ptr;
+                t[8] = s.csc_off[i]; t[9] = s.csc_off[i + 1] - 1 - s.csc_off[i];
+            }
             const int32_t lim = (hi - lo - npiv >= TINY_WIDE_LEVEL) ? TINY_PAIRS_WIDE : TINY_PAIRS;
             for(int32_t p = lo + npiv; p < hi; ++p) {
                 const int32_t b = s.lvlb_idx[p];
@@ -134,6 +130,69 @@ void BildltPattern::upload_static()
     uploaded = true;
 }
 
+// The level ranges and the row groups of the dropping step; per level-list
+// position its capacity, place in its row group, width and the offsets its
+// storage has when every block keeps its capacity (the input offsets: both
+// stores are laid out in level-list order).
+void BildltPattern::build_levels()
+{
+    const Symbolic& s = sym;
+    const int32_t K = s.coarse_nnz;
+    std::vector<int32_t> lq((size_t) 4 * K), lv(K), groups;
+    levels.assign(s.num_levels, LevelRange{});
+    auto height = [&](int32_t i) { return s.block_starts[i + 1] - s.block_starts[i]; };
+    auto end_of = [&](int32_t p, int32_t& ix, int32_t& val) {
+        ix = p < K ? s.blocks[s.lvlb_idx[p]].col_ptr : (int32_t) s.ix_space;
+        val = p < K ? s.blocks[s.lvlb_idx[p]].val_ptr : (int32_t) s.val_space;
+    };
+    for(int32_t l = 0; l < s.num_levels; ++l) {
+        LevelRange& r = levels[l];
+        r.lo = s.lvlb_off[l];
+        r.size = s.lvlb_off[l + 1] - r.lo;
+        r.npiv = s.lvl_off[l + 1] - s.lvl_off[l];
+        r.row_lo = s.lvl_off[l];
+        r.level = l;
+        r.grp_lo = (int32_t) (groups.size() / 4);
+        end_of(r.lo + r.size, r.end_ix, r.end_val);
+        // pivot blocks and the off-diagonal blocks of their block rows both
+        // follow in ascending block rows
+        int32_t q = r.npiv, rows = 0, first_q = r.npiv, first_p = 0;
+        auto close = [&](int32_t p) {
+            if(p > first_p)
+                for(int32_t v : {first_p, p - first_p, first_q, q - first_q}) groups.push_back(v);
+            first_p = p;
+            first_q = q;
+            rows = 0;
+        };
+        for(int32_t p = 0; p < r.npiv; ++p) {
+            const int32_t i = s.blocks[s.lvlb_idx[r.lo + p]].block_row;
+            const int32_t cnt = s.csr_off[i + 1] - s.csr_off[i] - 1;
+            if(rows + height(i) > GROUP_ROWS || (q - first_q) + cnt > GROUP_BLOCKS) close(p);
+            auto put = [&](int32_t at) {
+                const BlockMeta& m = s.blocks[s.lvlb_idx[at]];
+                CULIP_REQUIRE(m.block_row == i, "factor: level list not in block row order");
+                const int32_t w = height(m.block_col);
+                lq[4 * (size_t) at] = (m.format == FMT_SPARSE) ? m.max_nnz : -1 - height(i) * w;
+                lq[4 * (size_t) at + 1] = rows;
+                lq[4 * (size_t) at + 2] = w;
+                lq[4 * (size_t) at + 3] = m.col_ptr;
+                lv[at] = m.val_ptr;
+            };
+            put(r.lo + p);
+            for(int32_t k = 0; k < cnt; ++k) put(r.lo + q + k);
+            q += cnt;
+            rows += height(i);
+        }
+        close(r.npiv);
+        r.ngrp = (int32_t) (groups.size() / 4) - r.grp_lo;
+        CULIP_REQUIRE(q == r.size, "factor: level list does not end with its last block row");
+    }
+    num_groups = (int32_t) (groups.size() / 4);
+    upload(d_lq, lq);
+    upload(d_lq_val, lv);
+    upload(d_groups, groups);
+}
+
 void Bildlt::upload_pattern(hipStream_t st)
 {
     release_graphs();
@@ -141,8 +200,6 @@ void Bildlt::upload_pattern(hipStream_t st)
     const Symbolic& s = sym;
     const int32_t n = s.n, K = s.coarse_nnz;
     const int64_t mlb = std::max<int64_t>(1, s.max_level_blocks);
-    d_keep.ensure(sizeof(int32_t) * mlb);
-    d_granted.ensure(sizeof(int32_t) * mlb);
     // 32 row masks per pivot position, then one "any" word per position
     d_piv_umask.ensure(sizeof(uint32_t) * 33 * mlb);
     d_defer_list.ensure(sizeof(int32_t) * mlb);
@@ -151,13 +208,12 @@ void Bildlt::upload_pattern(hipStream_t st)
     d_wave_cnt.ensure(sizeof(int32_t) * std::max(1, s.num_levels));
     d_store_list.ensure(sizeof(int32_t) * mlb);
     d_store_cnt.ensure(sizeof(int32_t) * std::max(1, s.num_levels));
-    // per scan chunk 4 int64, then per level 2 int32 flags per chunk and
-    // a chunk ticket counter
-    {
-        const size_t maxch = (size_t) ((mlb + SCAN_CHUNK - 1) / SCAN_CHUNK);
-        d_chunk.ensure(sizeof(int64_t) * 4 * maxch +
-            sizeof(int32_t) * (2 * maxch + 1) * (size_t) std::max(1, s.num_levels));
-    }
+    // 3 int64 per row group, a ticket counter per level
+    d_grp_state.ensure(24 * (size_t) pat->num_groups + 4 * (size_t) std::max(1, s.num_levels));
+    d_c_val.ensure(vt() * LIST_C * mlb);
+    d_c_idx.ensure(sizeof(uint16_t) * LIST_C * mlb);
+    d_part_mask.ensure(sizeof(uint32_t) * mlb);
+    d_rn_first.ensure(vt() * mlb);
     d_vals.ensure(sizeof(double) * std::max<int64_t>(1, A.nnz()));
     d_val_in.ensure(vt() * std::max<int64_t>(1, s.val_space));
     d_bout.ensure(sizeof(BlockMeta) * std::max(1, K));
@@ -202,6 +258,10 @@ void Bildlt::upload_pattern(hipStream_t st)
     d_perm.ensure(sizeof(int32_t) * (size_t) std::max(1, n));
     d_perm_tmp.ensure(sizeof(double) * (size_t) std::max(1, n));
     d_chain_pub.ensure(sizeof(double) * 2 * (size_t) std::max(1, n));
+    // a refactor rewrites only the fields that its values decide
+    if(K > 0)
+        HIP_CHECK(hipMemcpyAsync(d_bout.p, d_bin.p, sizeof(BlockMeta) * (size_t) K,
+            hipMemcpyDeviceToDevice, st));
     h_trsv_err.ensure();
     // the presets on the caller's stream: no device-wide synchronisation,
     // which would break graph captures other threads run meanwhile
@@ -235,7 +295,6 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.lvlb_idx = d_lvlb_idx.as<int32_t>();
     a.block_in_lvl = d_block_in_lvl.as<int32_t>();
     a.lvl_rows = d_lvl_rows.as<int32_t>();
-    a.rfo = d_rfo.as<int32_t>();
     a.ix_in = d_ix_in.as<int32_t>();
     a.val_in = d_val_in.as<VT>();
     a.ix_out = d_ix_out.as<int32_t>();
@@ -247,20 +306,20 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.if_cnt = d_if_cnt.as<int32_t>();
     a.rn_part = d_rn_part.as<VT>();
     a.drop_cnt = d_drop_cnt.as<int32_t>();
-    a.keep = d_keep.as<int32_t>();
-    a.granted = d_granted.as<int32_t>();
+    a.c_val = d_c_val.as<VT>();
+    a.c_idx = d_c_idx.as<uint16_t>();
+    a.part_mask = d_part_mask.as<uint32_t>();
+    a.rn_first = d_rn_first.as<VT>();
     a.overflow = d_overflow.as<uint8_t>();
     a.piv_loc = d_piv_loc.as<int32_t>();
     a.row_mask = d_row_mask.as<uint32_t>();
     a.row_flag = d_row_flag.as<int32_t>();
-    a.lq_cap = d_lq_cap.as<int32_t>();
-    a.lq_fr = d_lq_fr.as<int32_t>();
-    a.chunk = d_chunk.as<int64_t>();
-    {
-        const int64_t mlb = std::max<int64_t>(1, sym.max_level_blocks);
-        a.scan_maxch = (int32_t) ((mlb + SCAN_CHUNK - 1) / SCAN_CHUNK);
-        a.scan_flags = (int32_t*) (a.chunk + 4 * (int64_t) a.scan_maxch);
-    }
+    a.lq = d_lq.as<int4>();
+    a.lq_val = d_lq_val.as<int32_t>();
+    a.groups = d_groups.as<int4>();
+    a.grp_state = d_grp_state.as<int64_t>();
+    a.grp_ticket = (int32_t*) (a.grp_state + 3 * (int64_t) pat->num_groups);
+    a.state_words = 6 * pat->num_groups + sym.num_levels;
     a.err = h_trsv_err.p;
     a.off_task = d_off_task.as<int32_t>();
     a.upd4 = d_upd4.as<int32_t>();
@@ -332,15 +391,7 @@ void Bildlt::factor_impl(hipStream_t st)
     gather_values<VT>(d_vals.as<double>(), d_value_slot.as<int64_t>(), A.nnz(), d_val_in.as<VT>(),
         s.val_space, st);
     factor_begin<VT>(a, st);
-    for(int32_t l = 0; l < s.num_levels; ++l) {
-        LevelRange r;
-        r.lo = s.lvlb_off[l];
-        r.size = s.lvlb_off[l + 1] - r.lo;
-        r.npiv = s.lvl_off[l + 1] - s.lvl_off[l];
-        r.row_lo = s.lvl_off[l];
-        r.level = l;
-        factor_level<VT>(a, r, st);
-    }
+    for(const LevelRange& r : pat->levels) factor_level<VT>(a, r, st);
     HIP_CHECK(hipGetLastError());
 
     // solve layout: count, scan, size, fill
@@ -654,7 +705,8 @@ int64_t Bildlt::numeric_bytes() const
     int64_t b = 0;
     for(const DevBuf* d : {&d_vals, &d_val_in, &d_bout, &d_ix_out, &d_val_out, &d_tri, &d_rn,
             &d_if_val, &d_if_idx, &d_if_cnt, &d_rn_part, &d_drop_cnt, &d_overflow, &d_piv_loc,
-            &d_carry, &d_totals, &d_task[0], &d_task[1], &d_keep, &d_granted, &d_chunk,
+            &d_carry, &d_totals, &d_task[0], &d_task[1], &d_grp_state, &d_c_val, &d_c_idx,
+            &d_part_mask, &d_rn_first,
             &d_scan_tmp, &d_piv_umask, &d_defer_list, &d_defer_cnt, &d_wave_list, &d_wave_cnt,
             &d_store_list, &d_store_cnt, &d_row_mask, &d_row_flag,
             &d_chain_pub, &d_jac[0], &d_jac[1], &d_jac[2]})
@@ -673,8 +725,9 @@ int64_t Bildlt::numeric_bytes_estimate(bool with_layout) const
     const int64_t mlb = std::max<int64_t>(1, s.max_level_blocks);
     auto r16 = [](int64_t b) { return std::max<int64_t>(16, b); };
     int64_t b = 0;
-    b += r16(4 * mlb) * 2 + r16(128 * mlb) + r16(4 * mlb) + r16(4 * std::max(1, s.num_levels));
-    b += r16(32 * ((mlb + SCAN_CHUNK - 1) / SCAN_CHUNK));
+    b += r16(132 * mlb) + r16(4 * mlb) + r16(4 * std::max(1, s.num_levels));
+    b += r16(24 * nb + 4 * std::max(1, s.num_levels));   // row groups (at most nb), tickets
+    b += r16(LIST_C * (v + 2) * mlb) + r16((4 + v) * mlb);   // short lists, row sums
     b += r16(8 * (int64_t) s.value_slot.size()) + 2 * r16(v * s.val_space) + r16(36 * K);
     b += r16(4 * s.ix_space) + 24 * n + v * n;
     b += v * 1024 * mlb + 2048 * mlb + 4 * mlb + v * 32 * mlb + 4 * mlb + mlb;

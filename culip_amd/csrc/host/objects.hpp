@@ -127,8 +127,11 @@ struct BildltPattern {
     bool uploaded = false;
     culip_prec prec = CULIP_PREC_F64;
     DevBuf d_bs, d_is_piv, d_bin, d_csr_off, d_csc_off, d_csc_idx, d_upd_off, d_upd_ki, d_upd_kj,
-        d_lvlb_idx, d_block_in_lvl, d_lvl_rows, d_ix_in, d_value_slot, d_rfo;
-    DevBuf d_lq_cap, d_lq_fr, d_off_task, d_upd4;
+        d_lvlb_idx, d_block_in_lvl, d_lvl_rows, d_ix_in, d_value_slot;
+    DevBuf d_lq, d_lq_val, d_groups, d_off_task, d_upd4;
+    std::vector<LevelRange> levels;
+    int32_t num_groups = 0;
+    void build_levels();
     void upload_static();
     int64_t device_bytes() const;
 };
@@ -142,8 +145,8 @@ struct Bildlt final : Precond {
     Symbolic& sym;
     bool& have_sym;
     DevBuf &d_bs, &d_is_piv, &d_bin, &d_csr_off, &d_csc_off, &d_csc_idx, &d_upd_off, &d_upd_ki,
-        &d_upd_kj, &d_lvlb_idx, &d_block_in_lvl, &d_lvl_rows, &d_ix_in, &d_value_slot, &d_rfo;
-    DevBuf &d_lq_cap, &d_lq_fr, &d_off_task, &d_upd4;
+        &d_upd_kj, &d_lvlb_idx, &d_block_in_lvl, &d_lvl_rows, &d_ix_in, &d_value_slot;
+    DevBuf &d_lq, &d_lq_val, &d_groups, &d_off_task, &d_upd4;
 
     culip_prec prec = CULIP_PREC_F64;
     bool uploaded = false;   // this instance's numeric buffers exist
@@ -160,7 +163,7 @@ struct Bildlt final : Precond {
     // numeric (per instance)
     DevBuf d_vals, d_val_in, d_bout, d_ix_out, d_val_out, d_tri, d_rn;
     DevBuf d_if_val, d_if_idx, d_if_cnt, d_rn_part, d_drop_cnt, d_overflow, d_piv_loc, d_carry;
-    DevBuf d_keep, d_granted, d_chunk;
+    DevBuf d_grp_state, d_c_val, d_c_idx, d_part_mask, d_rn_first;
     DevBuf d_piv_umask, d_defer_list, d_defer_cnt, d_wave_list, d_wave_cnt, d_store_list,
         d_store_cnt;
     DevBuf d_row_mask, d_row_flag;
@@ -200,8 +203,8 @@ struct Bildlt final : Precond {
           d_csr_off(p->d_csr_off), d_csc_off(p->d_csc_off), d_csc_idx(p->d_csc_idx),
           d_upd_off(p->d_upd_off), d_upd_ki(p->d_upd_ki), d_upd_kj(p->d_upd_kj),
           d_lvlb_idx(p->d_lvlb_idx), d_block_in_lvl(p->d_block_in_lvl), d_lvl_rows(p->d_lvl_rows),
-          d_ix_in(p->d_ix_in), d_value_slot(p->d_value_slot), d_rfo(p->d_rfo),
-          d_lq_cap(p->d_lq_cap), d_lq_fr(p->d_lq_fr), d_off_task(p->d_off_task),
+          d_ix_in(p->d_ix_in), d_value_slot(p->d_value_slot),
+          d_lq(p->d_lq), d_lq_val(p->d_lq_val), d_groups(p->d_groups), d_off_task(p->d_off_task),
           d_upd4(p->d_upd4), prec(p->prec)
     {
     }
