@@ -404,151 +404,10 @@ __device__ VT row_ssq(const VT* T, int r, int w)
     return s;
 }
 
-// dependency blocks staged per round of the pivot update; the first tile
-// holds the pivot tile for the factorization afterwards. Two keep the pivot
-// blocks' LDS (17.8 KB in FP64) below that of the one-lane off-diagonal
-// form they share launches with, so eight workgroups fit a CU.
-constexpr int PIV_ROUND = 2;
-
-template<typename VT>
-struct alignas(16) PivLds {
-    VT X[PIV_ROUND][1024];
-    VT cs[PIV_ROUND][32], cd[PIV_ROUND][32], cb[PIV_ROUND][32];
-    uint32_t mask[PIV_ROUND][32];
-};
-
-// T (registers, rows c0 + 2t of column j) -= A' D A for a staged tile A
-// whose nonzero rows per column are in mask; the arithmetic and order of
-// product() with R = A, one output row at a time
-template<typename VT>
-__device__ void product_regs(VT (&T)[16], const VT* A, const uint32_t* mask, const VT* cs,
-    const VT* cd, const VT* cb, int len)
-{
-    const int lane = lane_id();
-    const int j = lane & 31;
-    const int c0 = lane >> 5;
-    const uint32_t mk = (j < len) ? mask[j] : 0u;
-    if(mk) {
-        // one pass over the nonzero rows with sixteen independent
-        // accumulators (the loads of a row feed all of them)
-        VT acc[16];
-#pragma unroll
-        for(int t = 0; t < 16; ++t) acc[t] = 0;
-        for(uint32_t bits = mk; bits; bits &= bits - 1) {
-            const int l = __ffs(bits) - 1;
-            const VT r = A[32 * l + j];
-            const VT sup = cs[l], dia = cd[l], sub = cb[l];
-#pragma unroll
-            for(int t = 0; t < 16; ++t) {
-                const int c = c0 + 2 * t;
-                const VT left = (l == 0) ? (VT) 0 : A[32 * (l - 1) + c];
-                const VT mid = A[32 * l + c];
-                const VT right = (l == 31) ? (VT) 0 : A[32 * (l + 1) + c];
-                const VT lt = fma(sub, right, fma(dia, mid, sup * left));
-                acc[t] = fma(r, lt, acc[t]);
-            }
-        }
-#pragma unroll
-        for(int t = 0; t < 16; ++t)
-            if(c0 + 2 * t < len) T[t] -= acc[t];
-    }
-}
-
-// the tile element T[c][c] held by this lane (rows cq + 2t of column j)
-template<typename VT>
-__device__ __forceinline__ VT diag_get(const VT (&T)[16], bool own, int t0)
-{
-    VT v = (VT) 0;
-#pragma unroll
-    for(int t = 0; t < 16; ++t)
-        if(own && t == t0) v = T[t];
-    return v;
-}
-
-template<typename VT>
-__device__ __forceinline__ void diag_put(VT (&T)[16], bool own, int t0, VT v)
-{
-#pragma unroll
-    for(int t = 0; t < 16; ++t)
-        if(own && t == t0) T[t] = v;
-}
-
-__device__ __forceinline__ double lane_value(double v, int src)
-{
-    const unsigned long long b = (unsigned long long) __double_as_longlong(v);
-    const unsigned lo = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) b, src);
-    const unsigned hi = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) (b >> 32), src);
-    return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
-}
-
-__device__ __forceinline__ float lane_value(float v, int src)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-}
-
-// nonzero entries of a dependency block taken by the one-column form
-constexpr int COL_E = 4;
-
-// A dependency block of width w whose nonzero entries all lie in one column
-// c updates only T[c][c] in product_regs; this forms that update in one
-// lane with the same operations in the same order (rows ascending, the
-// three-term D product, fma accumulation). Returns false for any other
-// block; c = -1 when the block has no nonzero entry.
-template<typename VT>
-__device__ __forceinline__ bool column_update(const Dep& d, int w, const int32_t* ixs,
-    const VT* vals, const double* tri, int& c_out, VT& v_out)
-{
-    c_out = -1;
-    v_out = (VT) 0;
-    if(d.fmt != FMT_SPARSE || d.nnz > COL_E) return false;
-    constexpr int NONE = 1 << 20;
-    int r[COL_E];
-    VT v[COL_E];
-    int col = -1;
-    bool one_col = true;
-#pragma unroll
-    for(int e = 0; e < COL_E; ++e) {
-        r[e] = NONE;
-        v[e] = (VT) 0;
-        if(e < d.nnz) {
-            const int ix = ixs[(int64_t) d.cp + e];
-            const VT x = vals[(int64_t) d.vp + e];
-            if(x != (VT) 0) {
-                const int rr = ix / w, cc = ix - rr * w;
-                one_col = one_col && (col < 0 || cc == col);
-                col = cc;
-                r[e] = rr;
-                v[e] = x;
-            }
-        }
-    }
-    if(!one_col) return false;
-    if(col < 0) return true;
-    // rows ascending (sorting network on four)
-    auto cswap = [&](int p, int q) {
-        if(r[q] < r[p]) {
-            const int tr = r[p]; r[p] = r[q]; r[q] = tr;
-            const VT tv = v[p]; v[p] = v[q]; v[q] = tv;
-        }
-    };
-    cswap(0, 1); cswap(2, 3); cswap(0, 2); cswap(1, 3); cswap(1, 2);
-    VT acc = (VT) 0;
-#pragma unroll
-    for(int k = 0; k < COL_E; ++k) {
-        if(r[k] != NONE) {
-            const int l = r[k];
-            const double* t = tri + 3 * (int64_t) (d.rb + l);
-            const VT sup = (VT) t[0], dia = (VT) t[1], sub = (VT) t[2];
-            const VT left = (k > 0 && l > 0 && r[k - 1] == l - 1) ? v[k - 1] : (VT) 0;
-            const VT right = (k + 1 < COL_E && l < 31 && r[k + 1] == l + 1) ? v[k + 1] : (VT) 0;
-            const VT lt = fma(sub, right, fma(dia, v[k], sup * left));
-            acc = fma(v[k], lt, acc);
-        }
-    }
-    c_out = col;
-    v_out = acc;
-    return true;
-}
+// entries of a block taken by the one-lane forms, and updates beside the
+// diagonal one such block may make in a pivot tile
+constexpr int LIGHT_E = 8;
+constexpr int LIGHT_OFF = 4;
 
 template<typename VT>
 struct alignas(16) OffLds {
@@ -695,13 +554,273 @@ __device__ __forceinline__ bool pair_matches(uint32_t mi, uint32_t mj)
     return (mi & mj) != 0u || mi == ALL_ROWS || mj == ALL_ROWS;
 }
 
-// k_factor_pivot_blocks (kernels :1146-1283) for the pivot block at level
-// position q, one wave
+// LDS of a pivot block: the tile, and either the one-lane updates of a round
+// of blocks or one staged block
+template<typename VT, int NW>
+struct alignas(16) PivLds {
+    VT T[1024];
+    union {
+        struct {
+            VT val[NW][64 * LIGHT_E];                          // in block order
+            uint32_t cols[NW][32][64 * LIGHT_E / 32 + 1];      // per column: which are its own
+        } d;
+        struct {
+            VT X[1024];
+            VT cs[32], cd[32], cb[32];
+            uint32_t mask[32];
+        } h;
+    } u;
+    VT dia[32];
+    uint64_t heavy[NW];
+    Dep dep;
+    int32_t runs[NW];
+    uint32_t plain, tiny;  // rows scaled together last, of them with a replaced pivot
+};
+
+// What a dependency block U_ki with at most LIGHT_E entries subtracts from the
+// pivot tile, formed by one lane with product()'s operations in its order: per
+// column c of the block the update of T[c][c], and for two entries in one row
+// the update of T[c1][c2], c1 < c2 (the lower triangle is never read). False
+// for a block outside the form: more entries, a 2x2 pivot or a non-finite D
+// among its rows, or more than LIGHT_OFF updates beside the diagonal.
 template<typename VT>
-__device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
-    PivLds<VT>& s)
+struct LightUpd {
+    uint32_t cols;             // columns with entries
+    VT acc[LIGHT_E];           // update of the diagonal for the columns head[e]
+    int head[LIGHT_E];         // column of entry e when it is its first, else -1
+    int noff;
+    int oe[LIGHT_OFF];         // 32 c1 + c2
+    VT ov[LIGHT_OFF];
+};
+
+template<typename VT>
+__device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t* ixs,
+    const VT* vals, const double* tri, LightUpd<VT>& o)
 {
-    const int lane = lane_id();
+    o.cols = 0;
+    o.noff = 0;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) { o.acc[e] = (VT) 0; o.head[e] = -1; }
+#pragma unroll
+    for(int k = 0; k < LIGHT_OFF; ++k) { o.oe[k] = 0; o.ov[k] = (VT) 0; }
+    if(d.fmt != FMT_SPARSE || d.nnz > LIGHT_E) return false;
+    if(d.nnz == 0) return true;
+    constexpr int NONE = 1 << 20;
+    int key[LIGHT_E];          // 32 row + column, ascending
+    VT v[LIGHT_E];
+    bool sorted = true;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) {
+        const int at = min(e, d.nnz - 1);
+        const int ix = ixs[(int64_t) d.cp + at];
+        v[e] = vals[(int64_t) d.vp + at];
+        const int r = ix / w;
+        key[e] = (e < d.nnz && v[e] != (VT) 0) ? 32 * r + (ix - r * w) : NONE;
+    }
+#pragma unroll
+    for(int e = 1; e < LIGHT_E; ++e) sorted = sorted && key[e - 1] <= key[e];
+    if(!sorted) {
+        // odd-even transposition (entries over capacity are stored by size)
+#pragma unroll
+        for(int p = 0; p < LIGHT_E; ++p)
+#pragma unroll
+            for(int e = p & 1; e + 1 < LIGHT_E; e += 2)
+                if(key[e + 1] < key[e]) {
+                    const int tk = key[e]; key[e] = key[e + 1]; key[e + 1] = tk;
+                    const VT tv = v[e]; v[e] = v[e + 1]; v[e + 1] = tv;
+                }
+    }
+    VT lt[LIGHT_E];
+    bool ok = true;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) {
+        const double* t = tri + 3 * (int64_t) (d.rb + ((key[e] != NONE) ? key[e] >> 5 : 0));
+        const double sup = t[0], dia = t[1], sub = t[2];
+        ok = ok && (key[e] == NONE ||
+            (sup == 0.0 && sub == 0.0 && fabs(dia) < (double) INFINITY && finite_value(v[e])));
+        lt[e] = (VT) dia * v[e];
+    }
+    if(!ok) return false;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) {
+        if(key[e] == NONE) continue;
+        const int c = key[e] & 31;
+        bool first = true;
+#pragma unroll
+        for(int f = 0; f < e; ++f) first = first && (key[f] & 31) != c;
+        if(first) {
+            VT acc = fma(v[e], lt[e], (VT) 0);
+#pragma unroll
+            for(int f = e + 1; f < LIGHT_E; ++f)
+                if(key[f] != NONE && (key[f] & 31) == c) acc = fma(v[f], lt[f], acc);
+            o.acc[e] = acc;
+            o.head[e] = c;
+            o.cols |= 1u << c;
+        }
+#pragma unroll
+        for(int f = e + 1; f < LIGHT_E; ++f)
+            if(key[f] != NONE && (key[f] >> 5) == (key[e] >> 5)) {
+                const int el = 32 * c + (key[f] & 31);
+                const VT acc = fma(v[f], lt[e], (VT) 0);
+#pragma unroll
+                for(int k = 0; k < LIGHT_OFF; ++k) {
+                    ok = ok && !(k < o.noff && o.oe[k] == el);
+                    if(k == o.noff) { o.oe[k] = el; o.ov[k] = acc; }
+                }
+                ++o.noff;
+            }
+    }
+    return ok && o.noff <= LIGHT_OFF;
+}
+
+// T -= A' D A for the block staged in h.X by all NW waves: the arithmetic and
+// order of product() with R = A
+template<typename VT, int NW>
+__device__ void product_staged(PivLds<VT, NW>& s, int len)
+{
+    const int j = (int) threadIdx.x & 31;
+    const int c0 = (int) threadIdx.x >> 5;
+    constexpr int NR = 16 / NW, ST = 2 * NW;
+    const VT* A = s.u.h.X;
+    const uint32_t mk = (j < len) ? s.u.h.mask[j] : 0u;
+    if(mk) {
+        VT acc[NR];
+#pragma unroll
+        for(int t = 0; t < NR; ++t) acc[t] = 0;
+        for(uint32_t bits = mk; bits; bits &= bits - 1) {
+            const int l = __ffs(bits) - 1;
+            const VT r = A[32 * l + j];
+            const VT sup = s.u.h.cs[l], dia = s.u.h.cd[l], sub = s.u.h.cb[l];
+#pragma unroll
+            for(int t = 0; t < NR; ++t) {
+                const int c = c0 + ST * t;
+                const VT left = (l == 0) ? (VT) 0 : A[32 * (l - 1) + c];
+                const VT mid = A[32 * l + c];
+                const VT right = (l == 31) ? (VT) 0 : A[32 * (l + 1) + c];
+                const VT lt = fma(sub, right, fma(dia, mid, sup * left));
+                acc[t] = fma(r, lt, acc[t]);
+            }
+        }
+#pragma unroll
+        for(int t = 0; t < NR; ++t) {
+            const int c = c0 + ST * t;
+            if(c < len) s.T[32 * c + j] -= acc[t];
+        }
+    }
+}
+
+// one dependency block of any form, by all NW waves
+template<typename VT, int NW>
+__device__ void heavy_update(const FactorArgs<VT>& a, PivLds<VT, NW>& s, const Dep& d, int len)
+{
+    constexpr int TPB = 64 * NW;
+    const int t = (int) threadIdx.x;
+    for(int e = t; e < 1024; e += TPB) s.u.h.X[e] = (VT) 0;
+    if(t < 32) {
+        s.u.h.mask[t] = 0;
+        VT sup = 0, dia = 0, sub = 0;
+        if(t < d.rk) {
+            const double* td = a.tri + 3 * (int64_t) (d.rb + t);
+            sup = (VT) td[0];
+            dia = (VT) td[1];
+            sub = (VT) td[2];
+        }
+        s.u.h.cs[t] = sup;
+        s.u.h.cd[t] = dia;
+        s.u.h.cb[t] = sub;
+    }
+    __syncthreads();
+    auto put = [&](int r, int c, VT v) {
+        s.u.h.X[32 * r + c] = v;
+        if(v != (VT) 0) atomicOr(&s.u.h.mask[c], 1u << r);
+    };
+    if(d.fmt == FMT_DENSE) {
+        for(int e = t; e < d.rk * len; e += TPB) {
+            const int r = e / len;
+            put(r, e - r * len, a.val_out[(int64_t) d.vp + e]);
+        }
+    } else {
+        for(int e = t; e < d.nnz; e += TPB) {
+            const int ix = a.ix_out[(int64_t) d.cp + e];
+            const int r = ix / len;
+            put(r, ix - r * len, a.val_out[(int64_t) d.vp + e]);
+        }
+    }
+    __syncthreads();
+    product_staged<VT, NW>(s, len);
+    __syncthreads();
+}
+
+// the one-lane updates of the lanes with `mine` set, in block order
+template<typename VT, int NW>
+__device__ void apply_light(PivLds<VT, NW>& s, const LightUpd<VT>& o, bool mine)
+{
+    const int t = (int) threadIdx.x, lane = lane_id(), wv = t / WAVE;
+    const int n = mine ? __popc(o.cols) : 0;
+    int off = n;
+#pragma unroll
+    for(int k = 1; k < WAVE; k <<= 1) {
+        const int u = __shfl_up(off, k, WAVE);
+        if(lane >= k) off += u;
+    }
+    const int total = __shfl(off, WAVE - 1, WAVE);
+    off -= n;
+    const int words = (total + 31) / 32;
+    for(int k = lane; k < 32 * words; k += WAVE) s.u.d.cols[wv][k & 31][k >> 5] = 0u;
+    if(lane == 0) s.runs[wv] = words;
+    wave_sync();
+    if(n) {
+#pragma unroll
+        for(int e = 0; e < LIGHT_E; ++e)
+            if(o.head[e] >= 0) {
+                const int c = o.head[e];
+                const int at = off + __popc(o.cols & ((1u << c) - 1));
+                s.u.d.val[wv][at] = o.acc[e];
+                atomicOr(&s.u.d.cols[wv][c][at >> 5], 1u << (at & 31));
+            }
+    }
+    __syncthreads();
+    if(t < 32) {
+        VT d = s.T[33 * t];
+        for(int u = 0; u < NW; ++u)
+            for(int wd = 0; wd < s.runs[u]; ++wd)
+                for(uint32_t bits = s.u.d.cols[u][t][wd]; bits; bits &= bits - 1)
+                    d -= s.u.d.val[u][32 * wd + __ffs(bits) - 1];
+        s.T[33 * t] = d;
+    }
+    // updates beside the diagonal (few), one block after the other
+    const bool off_any = mine && o.noff > 0;
+    if(__syncthreads_or(off_any))
+        for(int u = 0; u < NW; ++u) {
+            if(u == wv)
+                for(uint64_t b = wave_ballot(off_any); b; b &= b - 1) {
+                    if(lane == __ffsll((long long) b) - 1) {
+#pragma unroll
+                        for(int k = 0; k < LIGHT_OFF; ++k)
+                            if(k < o.noff) s.T[o.oe[k]] -= o.ov[k];
+                    }
+                    wave_sync();
+                }
+            __syncthreads();
+        }
+}
+
+// k_factor_pivot_blocks (kernels :1146-1283) for the pivot block at level
+// position q, NW waves.
+// Bound by latency: the level's pivot blocks are far fewer than the chip has
+// CUs, and each waits for its tile, the ids of the blocks above it, their
+// metadata, their entries and D, five dependent round trips. All blocks above
+// it take these trips together, one per lane, and the updates are then added
+// per element in block order from LDS; blocks outside the one-lane form are
+// staged one by one in their place in that order. Of the pivot steps only
+// rows with an entry right of the diagonal (or a 2x2 pivot) are steps; the
+// others scale a row and change nothing else, so they are done together last.
+template<typename VT, int NW>
+__device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
+    PivLds<VT, NW>& s)
+{
+    constexpr int TPB = 64 * NW;
+    const int t = (int) threadIdx.x, lane = lane_id(), wv = t / WAVE;
     const int4 t0 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q)];
     const int4 t1 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q) + 1];
     const int4 t2 = ((const int4*) a.off_task)[3 * ((int64_t) lr.lo + q) + 2];
@@ -712,169 +831,222 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     const int len = t0.z;
     const int cb0 = t2.x;
     const int nd = t2.y;
-    const int j = lane & 31, cq = lane >> 5;
-    // metadata of the first 64 dependency blocks, in flight during the tile
-    // load; later chunks are fetched while the previous one is walked
-    Dep nxt{};
-    if(lane < nd) nxt = load_dep(a.bout, a.bs, a.csc_idx[cb0 + lane]);
-    // the pivot tile in registers (rows cq + 2t of column j)
-    VT* T0 = s.X[0];
-    tile_load(T0, t1, len, len, a.ix_in, a.val_in);
-    VT T[16];
-#pragma unroll
-    for(int t = 0; t < 16; ++t) T[t] = T0[32 * (cq + 2 * t) + j];
-    wave_sync();
-#pragma unroll
-    for(int u = 0; u < PIV_ROUND; ++u) tile_zero(s.X[u]);
-    if(lane < 32) {
-#pragma unroll
-        for(int u = 0; u < PIV_ROUND; ++u) s.mask[u][lane] = 0;
+    // the tile: dense input values (the factor's blocks on the diagonal are)
+    int blk = (t < nd) ? a.csc_idx[cb0 + t] : -1;
+    int piv = 1;
+    if(t < 32 && t < len) piv = a.is_piv[fr + t];
+    for(int e = t; e < 1024; e += TPB) {
+        const int r = e >> 5, c = e & 31;
+        VT v = (VT) 0;
+        if(t1.x == FMT_DENSE && r < len && c < len) v = a.val_in[(int64_t) t1.w + r * len + c];
+        s.T[e] = v;
     }
-    wave_sync();
-    // updates from the blocks (k, i) above the diagonal, in CSC order, 64
-    // blocks per chunk. A block whose nonzero entries lie in one column c
-    // (nearly all of them on sparse KKT patterns) changes only T[c][c]; its
-    // lane forms that value and the walk subtracts it from the diagonal
-    // register of the owning lane. Runs of other blocks are staged as tiles,
-    // PIV_ROUND per round, and go through product_regs.
-    const bool owns_diag = ((j & 1) == cq) && j < len;
-    const int tdiag = (j - cq) >> 1;
-    for(int c0 = 0; c0 < nd; c0 += 64) {
-        const Dep mine = nxt;
-        const int cnt = min(64, nd - c0);
-        int uc = -1;
-        VT uv = (VT) 0;
-        const bool simple = lane < cnt && column_update(mine, len, a.ix_out, a.val_out, a.tri,
-            uc, uv);
-        const uint64_t smask = wave_ballot(simple);
-        nxt = Dep{};
-        if(c0 + 64 + lane < nd) nxt = load_dep(a.bout, a.bs, a.csc_idx[cb0 + c0 + 64 + lane]);
-        VT dg = diag_get(T, owns_diag, tdiag);
-        int d = 0;
-        while(d < cnt) {
-            if((smask >> d) & 1ull) {
-                const int c = __builtin_amdgcn_readlane(uc, d);
-                if(c >= 0) {
-                    const VT v = lane_value(uv, d);
-                    if(owns_diag && j == c) dg -= v;
-                }
-                ++d;
-                continue;
-            }
-            // a run of staged blocks [d, d1)
-            const uint64_t later = smask >> d;
-            const int d1 = later ? min(cnt, d + __ffsll((long long) later) - 1) : cnt;
-            diag_put(T, owns_diag, tdiag, dg);
-            for(int r0 = d; r0 < d1; r0 += PIV_ROUND) {
-                const int nr = min(PIV_ROUND, d1 - r0);
-                Dep cur[PIV_ROUND];
-                Pre<VT> pc[PIV_ROUND];
-#pragma unroll
-                for(int u = 0; u < PIV_ROUND; ++u) {
-                    cur[u] = bcast(mine, u < nr ? r0 + u : r0);
-                    if(u < nr) pc[u] = prefetch(cur[u], a.ix_out, a.val_out, a.tri, true);
-                }
-#pragma unroll
-                for(int u = 0; u < PIV_ROUND; ++u) {
-                    if(u < nr) {
-                        stage(s.X[u], s.mask[u], cur[u], pc[u], len, a.ix_out, a.val_out);
-                        stage_d(s.cs[u], s.cd[u], s.cb[u], pc[u]);
-                    }
-                }
-                wave_sync();
-#pragma unroll
-                for(int u = 0; u < PIV_ROUND; ++u)
-                    if(u < nr) product_regs(T, s.X[u], s.mask[u], s.cs[u], s.cd[u], s.cb[u], len);
-                wave_sync();
-#pragma unroll
-                for(int u = 0; u < PIV_ROUND; ++u)
-                    if(u < nr) unstage(s.X[u], s.mask[u], cur[u], pc[u], len);
-                wave_sync();
-            }
-            dg = diag_get(T, owns_diag, tdiag);
-            d = d1;
+    if(t1.x != FMT_DENSE) {
+        __syncthreads();
+        for(int e = t; e < t1.y; e += TPB) {
+            const int ix = a.ix_in[(int64_t) t1.z + e];
+            const int r = ix / len;
+            s.T[32 * r + (ix - r * len)] = a.val_in[(int64_t) t1.w + e];
         }
-        diag_put(T, owns_diag, tdiag, dg);
     }
-    // the updated tile back to LDS (tile 0 is zero again after unstaging)
-#pragma unroll
-    for(int t = 0; t < 16; ++t) T0[32 * (cq + 2 * t) + j] = T[t];
-    wave_sync();
+    __syncthreads();
+    // updates from the blocks (k, i) above the diagonal, in CSC order
+    for(int c0 = 0; c0 < nd; c0 += TPB) {
+        if(c0) blk = (c0 + t < nd) ? a.csc_idx[cb0 + c0 + t] : -1;
+        Dep d{};
+        LightUpd<VT> up;
+        up.cols = 0;
+        up.noff = 0;
+        bool light = false;
+        if(blk >= 0) {
+            d = load_dep(a.bout, a.bs, blk);
+            light = light_update(d, len, a.ix_out, a.val_out, a.tri, up);
+        }
+        const uint64_t hm = wave_ballot(blk >= 0 && !light);
+        if(lane == 0) s.heavy[wv] = hm;
+        __syncthreads();
+        for(int start = 0, w = 0;;) {
+            // the next block outside the form
+            int h = -1;
+            for(; w < NW; ++w) {
+                uint64_t m = s.heavy[w];
+                if(start > 64 * w) m &= (start - 64 * w >= 64) ? 0ull : ~0ull << (start - 64 * w);
+                if(m) { h = 64 * w + __ffsll((long long) m) - 1; break; }
+            }
+            apply_light<VT, NW>(s, up, light && t >= start && (h < 0 || t < h));
+            __syncthreads();
+            if(h < 0) break;
+            if(t == h) s.dep = d;
+            __syncthreads();
+            const Dep hd = s.dep;
+            heavy_update<VT, NW>(a, s, hd, len);
+            start = h + 1;
+        }
+    }
     // d_factor_pivot_factorize (kernels :956-1083): static pivots, or a
     // numeric choice per step with symmetric interchanges (the pivot starts
     // and the block's rows in perm are rewritten as pivots are chosen)
     double* tri = a.tri + 3 * (int64_t) fr;
-    int32_t* fpiv = a.is_piv + fr;
-    int32_t* bperm = a.perm + fr;
-    int32_t rflag = 0;
-    int p = 0;
-    while(p < len) {
-        int order, p0 = p, p1 = p + 1;
-        if(a.pivoting == 1 && p < len - 1) select_bk(T0, len, p, order, p0, p1);
-        else if(a.pivoting == 2 && p < len - 1) select_rook(T0, len, p, order, p0, p1);
-        else order = (p < len - 1 && !fpiv[p + 1]) ? 2 : 1;
-        if(order == 1) {
-            if(a.pivoting && p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
-            if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
-            if(a.pivoting && lane == 0) fpiv[p] = 1;
+    VT* T0 = s.T;
+    const uint32_t live = len == 32 ? ~0u : (1u << len) - 1;
+    uint32_t M = 0;   // wave 0: columns right of the diagonal of row `lane`
+    if(wv == 0) {
+        int32_t rflag = 0;
+        uint32_t plain = 0, tiny = 0;
+        if(a.pivoting) {
+            int32_t* fpiv = a.is_piv + fr;
+            int32_t* bperm = a.perm + fr;
+            int p = 0;
+            while(p < len) {
+                int order = 1, p0 = p, p1 = p + 1;
+                if(p < len - 1) {
+                    if(a.pivoting == 1) select_bk(T0, len, p, order, p0, p1);
+                    else select_rook(T0, len, p, order, p0, p1);
+                }
+                if(order == 1) {
+                    if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
+                    if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
+                    if(lane == 0) fpiv[p] = 1;
+                } else {
+                    if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
+                    dense_pivot_op(T0, bperm, len, p + 1, p1);
+                    const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
+                                             : step_2x2<VT, VT>(T0, tri, p, len);
+                    rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
+                    if(lane == 0) {
+                        fpiv[p] = 1;
+                        fpiv[p + 1] = 0;
+                    }
+                }
+                wave_sync();
+                p += order;
+            }
+            if(lane < 32) M = (lane < 31) ? ~0u << (lane + 1) : 0u;
         } else {
-            if(a.pivoting) {
-                if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
-                dense_pivot_op(T0, bperm, len, p + 1, p1);
+            // columns right of the diagonal per row (a superset while steps
+            // fill rows in)
+#pragma unroll
+            for(int k = 0; k < 16; ++k) {
+                const int r = 2 * k + (lane >> 5), c = lane & 31;
+                const uint64_t b = wave_ballot(c > r && c < len && T0[64 * k + lane] != (VT) 0);
+                if(lane == 2 * k) M = (uint32_t) b;
+                if(lane == 2 * k + 1) M = (uint32_t) (b >> 32);
             }
-            const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
-                                     : step_2x2<VT, VT>(T0, tri, p, len);
-            rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
-            if(a.pivoting && lane == 0) {
-                fpiv[p] = 1;
-                fpiv[p + 1] = 0;
+            const uint32_t starts = (uint32_t) wave_ballot(lane < 32 && lane < len && piv != 0);
+            const uint32_t two = (~starts & live) >> 1;    // rows where a 2x2 pivot starts
+            uint32_t done = 0;
+            for(int p = 0; p < len;) {
+                const uint32_t cand = ((uint32_t) wave_ballot(lane < len && M != 0u) | two) &
+                    (~0u << p);
+                if(!cand) break;
+                p = __ffs(cand) - 1;
+                if((two >> p) & 1u) {
+                    const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
+                                             : step_2x2<VT, VT>(T0, tri, p, len);
+                    rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
+                    const uint32_t mm = (uint32_t) (__builtin_amdgcn_readlane((int) M, p) |
+                        __builtin_amdgcn_readlane((int) M, p + 1));
+                    if(lane > p + 1 && lane < 32 && ((mm >> lane) & 1u)) M |= mm & (~1u << lane);
+                    if(lane == p || lane == p + 1) M |= mm & (~1u << lane);
+                    done |= 3u << p;
+                    p += 2;
+                } else {
+                    if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
+                    const uint32_t mm = (uint32_t) __builtin_amdgcn_readlane((int) M, p);
+                    if(lane > p && lane < 32 && ((mm >> lane) & 1u)) M |= mm & (~1u << lane);
+                    done |= 1u << p;
+                    p += 1;
+                }
+                wave_sync();
             }
+            plain = live & ~done;
+            const bool own = lane < 32 && ((plain >> lane) & 1u);
+            VT d = T0[33 * (lane & 31)];
+            const bool rep = fabs((double) d) < 1e-8;
+            if(rep) d = (VT) 1e-6;
+            if(lane < 32) s.dia[lane] = d;
+            tiny = plain & (uint32_t) wave_ballot(own && rep);
+            if(own) {
+                tri[3 * lane] = 0.0;
+                tri[3 * lane + 1] = (double) d;
+                tri[3 * lane + 2] = 0.0;
+            }
+            if(wave_ballot(own && !finite_value(d))) rflag |= ROW_NONFINITE;
         }
-        wave_sync();
-        p += order;
+        if(lane == 0) {
+            s.plain = plain;
+            s.tiny = tiny;
+            a.row_flag[i] = rflag;
+        }
     }
-    uint32_t um = 0;
-    if(lane < len) {
-        a.rn[fr + lane] = row_ssq(T0, lane, len);
-        // nonzero columns right of the diagonal, for the U_ii' solves
-        for(int c = lane + 1; c < len; ++c)
-            if(T0[32 * lane + c] != (VT) 0) um |= 1u << c;
-        a.piv_umask[(int64_t) q * 32 + lane] = um;
-    } else if(lane < 32) {
-        a.piv_umask[(int64_t) q * 32 + lane] = 0u;   // all 32 words defined
+    __syncthreads();
+    // the remaining rows' steps: step_1x1 without its trailing update
+    if(s.plain) {
+        for(int e = t; e < 1024; e += TPB) {
+            const int r = e >> 5, c = e & 31;
+            if(!((s.plain >> r) & 1u)) continue;
+            const VT u = ((c < r) ? (VT) 0 : T0[e]) / s.dia[r];
+            T0[e] = (c == r && ((s.tiny >> r) & 1u)) ? (VT) 1 : u;
+        }
+        __syncthreads();
     }
-    // and whether there is any such column at all (one word per tile)
-    const bool um_some = wave_ballot(um != 0u) != 0ull;
-    if(lane == 0) a.piv_any[q] = um_some ? 1u : 0u;
+    if(wv == 0) {
+        // row sums of squares, and the nonzero columns right of the diagonal
+        // for the U_ii' solves (every other entry of a row is zero)
+        uint32_t um = 0;
+        if(lane < len) {
+            VT v = T0[33 * lane];
+            VT ssq = fma(v, v, (VT) 0);
+            for(uint32_t bits = M & live; bits; bits &= bits - 1) {
+                v = T0[32 * lane + __ffs(bits) - 1];
+                ssq = fma(v, v, ssq);
+                if(v != (VT) 0) um |= bits & (0u - bits);
+            }
+            a.rn[fr + lane] = ssq;
+        }
+        if(lane < 32) a.piv_umask[(int64_t) q * 32 + lane] = um;   // all 32 words defined
+        // and whether there is any such column at all (one word per tile)
+        const bool some = wave_ballot(um != 0u) != 0ull;
+        if(lane == 0) {
+            a.piv_any[q] = some ? 1u : 0u;
+            a.piv_loc[i] = q;
+        }
+    }
     // the tile for the level's off-diagonal blocks, and its final storage:
     // dense blocks keep their size, so the offset follows from the pool alone
     // (k_drop)
     VT* out = a.if_val + (int64_t) q * 1024;
     VT* fin = a.val_out + ((int64_t) t1.w - pool);
-    for(int e = lane; e < len * len; e += 64) {
+    for(int e = t; e < len * len; e += TPB) {
         const int r = e / len, c = e - r * len;
         const VT v = T0[32 * r + c];
         out[e] = v;
         fin[e] = v;
     }
-    if(lane == 0) {
-        a.piv_loc[i] = q;
-        a.row_flag[i] = rflag;
-    }
 }
 
-// the entry list of position q holding cnt entries
+// the entry list of position q: its first LIST_C entries in the compact
+// store, the others in the large one
 template<typename VT>
 struct EntryList {
+    VT* cv;
+    uint16_t* ci;
     VT* v;
     uint16_t* ix;
+    __device__ __forceinline__ VT val(int e) const { return e < LIST_C ? cv[e] : v[e]; }
+    __device__ __forceinline__ int idx(int e) const { return e < LIST_C ? ci[e] : ix[e]; }
+    __device__ __forceinline__ void set(int e, int i, VT x) const
+    {
+        (e < LIST_C ? ci : ix)[e] = (uint16_t) i;
+        (e < LIST_C ? cv : v)[e] = x;
+    }
 };
 
 template<typename VT>
-__device__ __forceinline__ EntryList<VT> entry_list(const FactorArgs<VT>& a, int q, int cnt)
+__device__ __forceinline__ EntryList<VT> entry_list(const FactorArgs<VT>& a, int q)
 {
-    if(cnt <= LIST_C) return {a.c_val + (int64_t) q * LIST_C, a.c_idx + (int64_t) q * LIST_C};
-    return {a.if_val + (int64_t) q * 1024, a.if_idx + (int64_t) q * 1024};
+    return {a.c_val + (int64_t) q * LIST_C, a.c_idx + (int64_t) q * LIST_C,
+        a.if_val + (int64_t) q * 1024, a.if_idx + (int64_t) q * 1024};
 }
 
 // a scaled off-diagonal tile X (one wave, stride 32) as position q leaves
@@ -905,23 +1077,16 @@ __device__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int 
         const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
         return r < hgt && c < wid && fabs((double) X[idx]) > NZ_EPS;
     };
-    int cnt = 0;
-#pragma unroll
-    for(int t = 0; t < 16; ++t) cnt += __popcll(wave_ballot(live(t)));
-    const EntryList<VT> o = entry_list(a, q, cnt);
+    const EntryList<VT> o = entry_list(a, q);
     int base = 0;
 #pragma unroll
     for(int t = 0; t < 16; ++t) {
         const bool pred = live(t);
         const uint64_t msk = wave_ballot(pred);
-        if(pred) {
-            const int pos = base + lanes_below(msk);
-            o.ix[pos] = (uint16_t) (64 * t + lane);
-            o.v[pos] = X[64 * t + lane];
-        }
+        if(pred) o.set(base + lanes_below(msk), 64 * t + lane, X[64 * t + lane]);
         base += __popcll(msk);
     }
-    if(lane == 0) a.if_cnt[q] = cnt;
+    if(lane == 0) a.if_cnt[q] = base;
 }
 
 // k_update_scale_offdiagonal_blocks (kernels :1628-1803) with
@@ -1315,14 +1480,15 @@ __device__ __forceinline__ void offdiag_body(const FactorArgs<VT>& a, const Leve
 // one column of the list arrays per lane; every value is formed by the same
 // operations in the same order as in the wave form (terms that are exact
 // zeros in the wave form are skipped).
-constexpr int TINY_E = 8;
+constexpr int TINY_E = LIGHT_E;
 constexpr int TINY_T = 32;
+constexpr int TINY_P = 12;  // the same while its Schur updates are added up
 constexpr int TINY_F = 4;   // pairs whose row masks are fetched together
 
-template<typename VT>
+template<typename VT, int CAP, int TPB>
 struct TinyLds {
-    VT v[TINY_T][TINY_TPB];
-    int16_t ix[TINY_T][TINY_TPB];
+    VT v[CAP][TPB];
+    int16_t ix[CAP][TPB];
 };
 
 template<typename VT>
@@ -1383,9 +1549,9 @@ __device__ __forceinline__ void tiny_raw(const int32_t* ix_out, const VT* val_ou
 // earlier levels and so run beside the level's pivot blocks. The tile list
 // is parked in the position's compact store (if_idx / if_val, count in
 // if_cnt); if_cnt[q] = -1 marks a position left to the other kernels.
-template<typename VT>
+template<typename VT, int TPB>
 __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
-    const int tid, TinyLds<VT>& s)
+    const int tid, TinyLds<VT, TINY_P, TPB>& s)
 {
     if(q >= lr.size) return;
     a.if_cnt[q] = -1;
@@ -1404,8 +1570,8 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
     const int4* pairs = (const int4*) a.upd4 + pair_first(t2);
     VT* tv = &s.v[0][tid];
     int16_t* ti = &s.ix[0][tid];
-    auto V = [&](int k) -> VT& { return tv[k * TINY_TPB]; };
-    auto I = [&](int k) -> int16_t& { return ti[k * TINY_TPB]; };
+    auto V = [&](int k) -> VT& { return tv[k * TPB]; };
+    auto I = [&](int k) -> int16_t& { return ti[k * TPB]; };
     int n = 0;
     auto find = [&](int idx) {
         for(int k = 0; k < n; ++k)
@@ -1499,7 +1665,7 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
                     int k = find(idx);
                     if(k < 0) {
                         if(acc == (VT) 0) continue;
-                        if(n == TINY_T) { to_wave_form(a, lr, q); return; }
+                        if(n == TINY_P) { to_wave_form(a, lr, q); return; }
                         k = n++;
                         I(k) = (int16_t) idx;
                         V(k) = 0;
@@ -1546,7 +1712,7 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
                         int k = find(idx);
                         if(k < 0) {
                             if(acc[f] == (VT) 0) continue;
-                            if(n == TINY_T) { to_wave_form(a, lr, q); return; }
+                            if(n == TINY_P) { to_wave_form(a, lr, q); return; }
                             k = n++;
                             I(k) = (int16_t) idx;
                             V(k) = 0;
@@ -1583,11 +1749,8 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
         }
     }
     // the tile list for the second phase
-    const EntryList<VT> o = entry_list(a, q, n);
-    for(int k = 0; k < n; ++k) {
-        o.ix[k] = (uint16_t) I(k);
-        o.v[k] = V(k);
-    }
+    const EntryList<VT> o = entry_list(a, q);
+    for(int k = 0; k < n; ++k) o.set(k, I(k), V(k));
     a.if_cnt[q] = n;
 }
 
@@ -1598,7 +1761,7 @@ template<typename VT>
 __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a, const LevelRange& lr,
     int bid_, int nblk_)
 {
-    __shared__ TinyLds<VT> s;
+    __shared__ TinyLds<VT, TINY_T, TINY_TPB> s;
     const int tid = threadIdx.x;
     const int q = lr.npiv + bid_ * TINY_TPB + tid;
     if(q >= lr.size) return;
@@ -1624,10 +1787,10 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
         return -1;
     };
     {
-        const EntryList<VT> o = entry_list(a, q, n);
+        const EntryList<VT> o = entry_list(a, q);
         for(int k = 0; k < n; ++k) {
-            I(k) = (int16_t) o.ix[k];
-            V(k) = o.v[k];
+            I(k) = (int16_t) o.idx(k);
+            V(k) = o.val(k);
         }
     }
     // U_ii' forward substitution over the rows in ascending order
@@ -1684,13 +1847,12 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
     }
     // row sums of squares (columns ascending) and the compact list
     uint32_t rows = 0;
-    int nr = 0, cnt = 0;
+    int nr = 0;
     for(int k = 0; k < n;) {
         const int r = I(k) >> 5;
         VT ssq = 0;
         while(k < n && (I(k) >> 5) == r) {
             ssq = fma(V(k), V(k), ssq);
-            cnt += fabs((double) V(k)) > NZ_EPS;
             ++k;
         }
         if(!(ssq == (VT) 0)) {
@@ -1701,39 +1863,33 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
         }
     }
     a.part_mask[q] = rows;
-    const EntryList<VT> o = entry_list(a, q, cnt);
+    const EntryList<VT> o = entry_list(a, q);
     int pos = 0;
-    for(int m = 0; m < n; ++m) {
-        const VT v = V(m);
-        if(fabs((double) v) > NZ_EPS) {
-            o.ix[pos] = (uint16_t) I(m);
-            o.v[pos] = v;
-            ++pos;
-        }
-    }
-    a.if_cnt[q] = cnt;
+    for(int m = 0; m < n; ++m)
+        if(fabs((double) V(m)) > NZ_EPS) o.set(pos++, I(m), V(m));
+    a.if_cnt[q] = pos;
 }
 // The level's pivot blocks (workgroups 0 .. npiv - 1) and the first phase
-// of the one-lane off-diagonal form (the rest, 64 positions each) in one
+// of the one-lane off-diagonal form (the rest, 64 NW positions each) in one
 // launch: the two read disjoint data and never wait for each other.
-template<typename VT>
+template<typename VT, int NW>
 union PivPairsLds {
-    PivLds<VT> piv;
-    TinyLds<VT> tiny;
+    PivLds<VT, NW> piv;
+    TinyLds<VT, TINY_P, 64 * NW> tiny;
 };
 
-template<typename VT>
+template<typename VT, int NW>
 __device__ __forceinline__ void pivots_pairs_body(const FactorArgs<VT>& a, const LevelRange& lr,
-    int bid_, int nblk_)
+    int bid_)
 {
-    __shared__ PivPairsLds<VT> u;
+    __shared__ PivPairsLds<VT, NW> u;
     const int w = bid_;
     if(w < lr.npiv) {
-        pivots_one<VT>(a, lr, w, u.piv);
+        pivots_one<VT, NW>(a, lr, w, u.piv);
         return;
     }
-    const int q0 = lr.npiv + (w - lr.npiv) * TINY_TPB;
-    tiny_pairs_one<VT>(a, lr, q0 + (int) threadIdx.x, (int) threadIdx.x, u.tiny);
+    const int q0 = lr.npiv + (w - lr.npiv) * 64 * NW;
+    tiny_pairs_one<VT, 64 * NW>(a, lr, q0 + (int) threadIdx.x, (int) threadIdx.x, u.tiny);
 }
 
 
@@ -1772,7 +1928,7 @@ constexpr int DR_TPB = GROUP_BLOCKS;
 constexpr int DR_NW = DR_TPB / WAVE;
 constexpr int DR_RUNS = 512;        // row sums a wave lays out at once
 constexpr int32_t CAP_NONE = -0x7fffffff;
-constexpr int STORE_TINY = 16;      // entries of a block stored by one lane
+constexpr int LIST_GROUP = 16;      // entries of a block taken by sixteen lanes
 constexpr int GROUP_SPIN_LIMIT = 1 << 22;
 
 template<typename VT>
@@ -1850,7 +2006,7 @@ __device__ int64_t pool_before(const int64_t* st, int g, int64_t pool0, int32_t*
     }
 }
 
-// the position a thread of k_drop works on
+// the position a thread of k_drop works on, with its first LIST_C entries
 template<typename VT>
 struct DropPos {
     int cap, row0, w, col, val, blk, cnt;
@@ -1862,108 +2018,150 @@ template<typename VT>
 __device__ __forceinline__ void drop_load(const FactorArgs<VT>& a, const LevelRange& lr, int q,
     bool in, DropPos<VT>& p)
 {
-    p.cap = CAP_NONE;
-    p.row0 = p.w = p.col = p.val = p.blk = p.cnt = 0;
+    const int qc = in ? q : 0;
+    const int4 l = a.lq[lr.lo + qc];
+    p.cap = in ? l.x : CAP_NONE;
+    p.row0 = l.y;
+    p.w = l.z;
+    p.col = l.w;
+    p.val = a.lq_val[lr.lo + qc];
+    p.blk = a.lvlb_idx[lr.lo + qc];
+    p.cnt = in ? a.if_cnt[qc] : 0;
 #pragma unroll
-    for(int e = 0; e < LIST_C; ++e) { p.v[e] = (VT) 0; p.ix[e] = 0; }
-    if(in) {
-        const int4 l = a.lq[lr.lo + q];
-        p.cap = l.x;
-        p.row0 = l.y;
-        p.w = l.z;
-        p.col = l.w;
-        p.val = a.lq_val[lr.lo + q];
-        p.blk = a.lvlb_idx[lr.lo + q];
-        p.cnt = a.if_cnt[q];
-        // beyond cnt (or for longer lists) these are not used
+    for(int e = 0; e < LIST_C; ++e) {
+        p.v[e] = a.c_val[(int64_t) qc * LIST_C + e];
+        p.ix[e] = a.c_idx[(int64_t) qc * LIST_C + e];
+    }
+}
+
+// Lists of LIST_C + 1 to LIST_GROUP entries (and any of at most LIST_GROUP
+// that overflow) are taken by sixteen lanes each, four at a time. visit(src,
+// e, on): this lane is entry e of lane src's list (src < 0: no list); on:
+// which four lists, as lanes of the wave.
+template<typename Visit>
+__device__ __forceinline__ void by_sixteen(uint64_t lanes, Visit visit)
+{
+    const int g = lane_id() >> 4;
+    while(lanes) {
+        int on[4];
+        int src = -1;
 #pragma unroll
-        for(int e = 0; e < LIST_C; ++e) {
-            p.v[e] = a.c_val[(int64_t) q * LIST_C + e];
-            p.ix[e] = a.c_idx[(int64_t) q * LIST_C + e];
+        for(int k = 0; k < 4; ++k) {
+            on[k] = lanes ? __ffsll((long long) lanes) - 1 : -1;
+            lanes &= lanes - 1;
+            if(g == k) src = on[k];
         }
+        visit(src, lane_id() & 15, on);
     }
 }
 
 // entries of a sparse position that survive |v| >= tau * sqrtf(norm)
-// (kernels :1919-1946); lists over STORE_TINY entries by the whole wave
+// (kernels :1919-1946); lists over LIST_GROUP entries by the whole wave
 template<typename VT>
 __device__ __forceinline__ int drop_count(const FactorArgs<VT>& a, int q, const DropPos<VT>& p,
     const VT* nrm)
 {
     auto keeps = [&](VT v, VT n) { return !(fabs(v) < a.threshold * n); };
     int keep = 0;
-    const bool big = p.cap >= 0 && p.cnt > STORE_TINY;
-    if(p.cap >= 0 && !big) {
-        if(p.cnt <= LIST_C) {
+    if(p.cap >= 0 && p.cnt <= LIST_C) {
 #pragma unroll
-            for(int e = 0; e < LIST_C; ++e)
-                if(e < p.cnt) keep += keeps(p.v[e], nrm[p.row0 + (p.ix[e] >> 5)]);
-        } else {
-            const EntryList<VT> l = entry_list(a, q, p.cnt);
-            for(int e = 0; e < p.cnt; ++e) keep += keeps(l.v[e], nrm[p.row0 + (l.ix[e] >> 5)]);
-        }
+        for(int e = 0; e < LIST_C; ++e)
+            if(e < p.cnt) keep += keeps(p.v[e], nrm[p.row0 + (p.ix[e] >> 5)]);
     }
-    for(uint64_t bm = wave_ballot(big); bm; bm &= bm - 1) {
+    by_sixteen(wave_ballot(p.cap >= 0 && p.cnt > LIST_C && p.cnt <= LIST_GROUP),
+        [&](int src, int e, const int (&on)[4]) {
+            const int from = max(src, 0);
+            const int bq = __shfl(q, from), bc = __shfl(p.cnt, from), br = __shfl(p.row0, from);
+            const EntryList<VT> l = entry_list(a, bq);
+            const bool in = src >= 0 && e < bc;
+            const bool k = in && keeps(l.val(in ? e : 0), nrm[br + ((in ? l.idx(e) : 0) >> 5)]);
+            const uint64_t kb = wave_ballot(k);
+#pragma unroll
+            for(int u = 0; u < 4; ++u)
+                if(lane_id() == on[u]) keep = __popc((uint32_t) (kb >> (16 * u)) & 0xffffu);
+        });
+    for(uint64_t bm = wave_ballot(p.cap >= 0 && p.cnt > LIST_GROUP); bm; bm &= bm - 1) {
         const int src = __ffsll((long long) bm) - 1;
         const int bq = __shfl(q, src), bc = __shfl(p.cnt, src), br = __shfl(p.row0, src);
-        const EntryList<VT> l = entry_list(a, bq, bc);
+        const EntryList<VT> l = entry_list(a, bq);
         int k = 0;
         for(int e0 = 0; e0 < bc; e0 += WAVE) {
-            const int e = e0 + lane_id();
-            const bool s = e < bc && keeps(l.v[min(e, bc - 1)], nrm[br + (l.ix[min(e, bc - 1)] >> 5)]);
-            k += __popcll(wave_ballot(s));
+            const int e = min(e0 + lane_id(), bc - 1);
+            const bool on = e0 + lane_id() < bc && keeps(l.val(e), nrm[br + (l.idx(e) >> 5)]);
+            k += __popcll(wave_ballot(on));
         }
         if(lane_id() == src) keep = k;
     }
     return keep;
 }
 
-// Final storage of a sparse block with at most STORE_TINY entries by one
-// lane (the selection and order of store_one), and its row mask
+// Final storage of the wave's sparse blocks with at most LIST_GROUP entries
+// (`mine`: this lane has one; the selection and order of store_one), and
+// their row masks. NaN entries are counted but never written.
 template<typename VT>
-__device__ void drop_store(const FactorArgs<VT>& a, int q, const DropPos<VT>& p, const VT* nrm,
-    int px, int pv, bool overflow, int max_nnz, int32_t rflag)
+__device__ __forceinline__ void drop_store(const FactorArgs<VT>& a, int q, const DropPos<VT>& p,
+    const VT* nrm, const int32_t* rflags, int px, int pv, bool mine, bool overflow, int max_nnz)
 {
-    VT* out_v = a.val_out + pv;
-    int32_t* out_i = a.ix_out + px;
-    uint32_t rows = 0;
-    bool bad = false;
-    auto kept = [&](VT v, int ix) { return !(fabs(v) < a.threshold * nrm[p.row0 + (ix >> 5)]); };
-    auto write = [&](int pos, VT v, int ix) {
-        out_i[pos] = (ix >> 5) * p.w + (ix & 31);
-        out_v[pos] = v;
-        rows |= 1u << (ix >> 5);
-    };
-    int pos = 0;
-    if(p.cnt <= LIST_C && !overflow) {
+    auto keeps = [&](VT v, VT n) { return !(fabs(v) < a.threshold * n); };
+    const bool shared = mine && (overflow || p.cnt > LIST_C);
+    if(mine && !shared) {
+        uint32_t rows = 0;
+        bool bad = false;
+        int pos = 0;
 #pragma unroll
         for(int e = 0; e < LIST_C; ++e) {
-            if(e < p.cnt && kept(p.v[e], p.ix[e])) {
+            const int r = p.ix[e] >> 5;
+            if(e < p.cnt && keeps(p.v[e], nrm[p.row0 + r])) {
                 bad = bad || !finite_value(p.v[e]);
-                if(fabs(p.v[e]) >= (VT) 0) write(pos++, p.v[e], p.ix[e]);
+                if(fabs(p.v[e]) >= (VT) 0) {
+                    a.ix_out[(int64_t) px + pos] = r * p.w + (p.ix[e] & 31);
+                    a.val_out[(int64_t) pv + pos] = p.v[e];
+                    rows |= 1u << r;
+                    ++pos;
+                }
             }
         }
-    } else {
-        const EntryList<VT> l = entry_list(a, q, p.cnt);
-        for(int e = 0; e < p.cnt; ++e) {
-            const VT v = l.v[e];
-            const int ix = l.ix[e];
-            if(!kept(v, ix)) continue;
-            bad = bad || !finite_value(v);
-            const VT key = fabs(v);
-            if(!(key >= (VT) 0)) continue;
-            if(!overflow) { write(pos++, v, ix); continue; }
+        a.row_mask[p.blk] = store_row_mask(rows, bad, rflags[p.row0]);
+    }
+    by_sixteen(wave_ballot(shared), [&](int src, int e, const int (&)[4]) {
+        const int from = max(src, 0), base = lane_id() & 48;
+        const int bq = __shfl(q, from), bc = __shfl(p.cnt, from), br = __shfl(p.row0, from);
+        const int bw = __shfl(p.w, from), bx = __shfl(px, from), bv = __shfl(pv, from);
+        const int bm = __shfl(max_nnz, from), bb = __shfl(p.blk, from);
+        const bool bo = __shfl((int) overflow, from) != 0;
+        const EntryList<VT> l = entry_list(a, bq);
+        const bool in = src >= 0 && e < bc;
+        const VT v = in ? l.val(e) : (VT) 0;
+        const int ix = in ? l.idx(e) : 0;
+        const bool k = in && keeps(v, nrm[br + (ix >> 5)]);
+        const bool bad = k && !finite_value(v);
+        // -1: no entry or a dropped one
+        const VT key = k ? (VT) fabs(v) : (VT) -1;
+        const bool w = key >= (VT) 0;
+        const uint32_t wg = (uint32_t) (wave_ballot(w) >> base) & 0xffffu;
+        int at = __popc(wg & ((1u << e) - 1));
+        if(wave_ballot(src >= 0 && bo)) {
             // over capacity: the max_nnz largest, ties to the lower index
             int rank = 0;
-            for(int f = 0; f < p.cnt; ++f) {
-                const VT u = l.v[f];
-                const int fx = l.ix[f];
-                rank += kept(u, fx) && ((VT) fabs(u) > key || ((VT) fabs(u) == key && fx < ix));
+#pragma unroll
+            for(int f = 0; f < LIST_GROUP; ++f) {
+                const VT kf = __shfl(key, base + f);
+                const int xf = __shfl(ix, base + f);
+                rank += kf > key || (kf == key && xf < ix);
             }
-            if(rank < max_nnz) write(rank, v, ix);
+            if(bo) at = rank;
         }
-    }
-    a.row_mask[p.blk] = store_row_mask(rows, bad, rflag);
+        uint32_t row = 0;
+        if(w && !(bo && at >= bm)) {
+            a.ix_out[(int64_t) bx + at] = (ix >> 5) * bw + (ix & 31);
+            a.val_out[(int64_t) bv + at] = v;
+            row = 1u << (ix >> 5);
+        }
+#pragma unroll
+        for(int o = 1; o < 16; o <<= 1) row |= (uint32_t) __shfl_xor((int) row, o);
+        const bool any_bad = ((wave_ballot(bad) >> base) & 0xffffull) != 0;
+        if(src >= 0 && e == 0) a.row_mask[bb] = store_row_mask(row, any_bad, rflags[br]);
+    });
 }
 
 // One launch per level, one workgroup per row group (its ticket's, so every
@@ -2108,32 +2306,31 @@ __device__ __forceinline__ void drop_body(const FactorArgs<VT>& a, const LevelRa
                 &ctot);
             tot = ctot;
         }
+        const int64_t pl = map_apply(ex, pool);
+        const int32_t px = (int32_t) (pos.col - pl), pv = (int32_t) (pos.val - pl);
+        bool overflow = false, mine = false;
+        int32_t room = 0;
         if(in) {
-            const int64_t pl = map_apply(ex, pool);
-            const int32_t px = (int32_t) (pos.col - pl), pv = (int32_t) (pos.val - pl);
             BlockMeta& o = a.bout[pos.blk];
             o.col_ptr = px;
             o.val_ptr = pv;
-            bool wave_form = true, overflow = false;
+            o.nnz = 0;
             if(pos.cap >= 0) {
                 const int64_t e = (int64_t) dcnt - pos.cap;
                 const int32_t gr = (int32_t) (e > 0 ? (e < pl ? e : pl) : 0);
-                const int32_t room = pos.cap + gr;
+                room = pos.cap + gr;
                 overflow = dcnt > room;
                 o.nnz = overflow ? room : dcnt;
                 o.max_nnz = room;
                 o.got_extra = gr;
-                wave_form = pos.cnt > STORE_TINY;
-                if(!wave_form)
-                    drop_store(a, q, pos, s.nrm, px, pv, overflow, room, s.rflag[pos.row0]);
-            } else {
-                o.nnz = 0;
+                mine = pos.cnt <= LIST_GROUP;
             }
-            if(wave_form) {
+            if(!mine) {
                 a.overflow[q] = overflow ? 1 : 0;
                 a.store_list[atomicAdd(a.store_cnt + lr.level, 1)] = q;
             }
         }
+        drop_store(a, q, pos, s.nrm, s.rflag, px, pv, mine, overflow, room);
         pool = map_apply(tot, pool);
     }
 }
@@ -2150,7 +2347,7 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
     const int fr = a.bs[mo.block_row];
     const int h = a.bs[mo.block_row + 1] - fr;
     const int w = a.bs[mo.block_col + 1] - a.bs[mo.block_col];
-    const VT* vals = a.if_val + (int64_t) q * 1024;   // more than LIST_C entries
+    const VT* vals = a.if_val + (int64_t) q * 1024;
     VT* out_v = a.val_out + mo.val_ptr;
     if(mo.format == FMT_DENSE) {
         for(int e = lane; e < h * w; e += 64) out_v[e] = vals[e];
@@ -2166,7 +2363,7 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
         const bool any_bad = wave_ballot(bad) != 0ull;
         if(lane == 0) a.row_mask[b] = store_row_mask(rows, any_bad, rflag);
     };
-    const uint16_t* ixs = a.if_idx + (int64_t) q * 1024;
+    const EntryList<VT> l = entry_list(a, q);
     int32_t* out_i = a.ix_out + mo.col_ptr;
     if(lane < h) nrm[lane] = drop_norm(a.rn[fr + lane]);
     wave_sync();
@@ -2179,8 +2376,8 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
             VT v = 0;
             int ix = 0;
             if(e < cnt) {
-                v = vals[e];
-                ix = ixs[e];
+                v = l.val(e);
+                ix = l.idx(e);
                 k = !(fabs(v) < a.threshold * nrm[ix >> 5]);
             }
             const uint64_t mask = wave_ballot(k);
@@ -2199,8 +2396,8 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
     // over capacity: keep the max_nnz largest |v|, ties to the lower tile
     // index, written in that order (CUB BlockRadixSort descending, stable)
     for(int e = lane; e < cnt; e += 64) {
-        const VT v = vals[e];
-        const int ix = ixs[e];
+        const VT v = l.val(e);
+        const int ix = l.idx(e);
         const bool k = !(fabs(v) < a.threshold * nrm[ix >> 5]);
         key[e] = k ? (VT) fabs(v) : (VT) -1;
         kix[e] = (uint16_t) ix;
@@ -2217,9 +2414,9 @@ __device__ void store_one(const FactorArgs<VT>& a, const LevelRange& lr, int q, 
         }
         if(rank < mo.max_nnz) {
             out_i[rank] = (ie >> 5) * w + (ie & 31);
-            out_v[rank] = vals[e];
+            out_v[rank] = l.val(e);
             rows |= 1u << (ie >> 5);
-            bad = bad || !finite_value(vals[e]);
+            bad = bad || !finite_value(l.val(e));
         }
     }
     keep_mask();
@@ -2264,10 +2461,10 @@ __global__ __launch_bounds__(TINY_TPB) void k_offdiag_tiny_scale(FactorArgs<VT> 
     offdiag_tiny_scale_body<VT>(a, lr, blockIdx.x, gridDim.x);
 }
 
-template<typename VT>
-__global__ __launch_bounds__(64) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
+template<typename VT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
 {
-    pivots_pairs_body<VT>(a, lr, blockIdx.x, gridDim.x);
+    pivots_pairs_body<VT, NW>(a, lr, blockIdx.x);
 }
 
 template<typename VT>
@@ -2379,7 +2576,7 @@ __global__ __launch_bounds__(64) void bk_pivots_pairs(const FactorSys<VT>* fs, c
     const int2 it = items[blockIdx.x];
     const FactorSys<VT>& F = fs[it.x];
     const LevelRange lr = F.lr[level];
-    pivots_pairs_body<VT>(F.a, lr, it.y, fl_grid_pivots_pairs(lr));
+    pivots_pairs_body<VT, 1>(F.a, lr, it.y);
 }
 
 template<typename VT>
@@ -2481,8 +2678,12 @@ void factor_level(const FactorArgs<VT>& a, const LevelRange& r, void* stream)
     hipStream_t st = (hipStream_t) stream;
     const int noff = r.size - r.npiv;
     const int tiny_blocks = fl_tiny_blocks(r);
-    if(fl_grid_pivots_pairs(r) > 0)
-        k_pivots_pairs<VT><<<fl_grid_pivots_pairs(r), 64, 0, st>>>(a, r);
+    if(r.size > 0) {
+        if(r.piv_waves == 4)
+            k_pivots_pairs<VT, 4><<<fl_grid_pivots_pairs(r, 4), 256, 0, st>>>(a, r);
+        else
+            k_pivots_pairs<VT, 1><<<fl_grid_pivots_pairs(r, 1), 64, 0, st>>>(a, r);
+    }
     if(noff > 0) {
         const int grid = fl_grid_tasks(noff, 2048);
         k_offdiag_tiny_scale<VT><<<tiny_blocks, TINY_TPB, 0, st>>>(a, r);

@@ -42,9 +42,9 @@ struct FactorArgs {
     double* tri = nullptr;                // 3n, tridiagonal D
     VT* rn = nullptr;                     // n, row sums of squares
     // per level position scratch
-    // the entries of a position before dropping: LIST_C or fewer in c_val /
+    // the entries of a position before dropping: the first LIST_C in c_val /
     // c_idx (contiguous over the positions, so that neighbouring positions
-    // share cache lines), more in if_val / if_idx; dense tiles in if_val
+    // share cache lines), the others in if_val / if_idx; dense tiles in if_val
     VT* if_val = nullptr;                 // 1024 per position
     uint16_t* if_idx = nullptr;           // 1024 per position
     VT* c_val = nullptr;                  // LIST_C per position
@@ -122,6 +122,7 @@ struct LevelRange {
     int32_t ngrp;      // row groups
     int32_t end_ix;    // store sizes after the level when every block keeps
     int32_t end_val;   // its capacity
+    int32_t piv_waves; // waves per pivot block when the system runs alone
 };
 
 // threads of a k_offdiag_tiny_scale workgroup (one per one-lane block)
@@ -138,9 +139,9 @@ __host__ __device__ inline int32_t fl_tiny_blocks(const LevelRange& r)
     const int32_t noff = r.size - r.npiv;
     return noff > 0 ? (noff + TINY_TPB - 1) / TINY_TPB : 0;
 }
-__host__ __device__ inline int32_t fl_grid_pivots_pairs(const LevelRange& r)
+__host__ __device__ inline int32_t fl_grid_pivots_pairs(const LevelRange& r, int32_t waves)
 {
-    return r.npiv + fl_tiny_blocks(r);
+    return r.npiv + (r.size - r.npiv + 64 * waves - 1) / (64 * waves);
 }
 __host__ __device__ inline int32_t fl_grid_tasks(int32_t count, int32_t cap)
 {

@@ -474,7 +474,7 @@ void BatchSolver::build_factor()
             if(l >= sys_[s]->f->sym.num_levels) continue;
             const LevelRange& r = lrs[lr_off[s] + l];
             const int32_t noff = r.size - r.npiv;
-            const int32_t cnt[5] = {fl_grid_pivots_pairs(r), fl_tiny_blocks(r),
+            const int32_t cnt[5] = {fl_grid_pivots_pairs(r, 1), fl_tiny_blocks(r),
                 fl_grid_tasks(noff, BATCH_TASK_GRID), r.ngrp,
                 fl_grid_tasks(noff, BATCH_TASK_GRID)};
             for(int k = 0; k < 5; ++k)

@@ -153,6 +153,13 @@ void BildltPattern::build_levels()
         r.row_lo = s.lvl_off[l];
         r.level = l;
         r.grp_lo = (int32_t) (groups.size() / 4);
+        // four waves per pivot block where one wave would take its blocks in
+        // several rounds; below that one wave takes them at once
+        r.piv_waves = 1;
+        for(int32_t p = 0; p < r.npiv; ++p) {
+            const int32_t i = s.blocks[s.lvlb_idx[r.lo + p]].block_row;
+            if(s.csc_off[i + 1] - s.csc_off[i] - 1 > 64) r.piv_waves = 4;
+        }
         end_of(r.lo + r.size, r.end_ix, r.end_val);
         // pivot blocks and the off-diagonal blocks of their block rows both
         // follow in ascending block rows
