@@ -396,14 +396,6 @@ __device__ bool step_2x2(VT* T, double* tri, int p, int len)
     return fabs(d11) + fabs(d12) + fabs(d22) < (AT) INFINITY;   // D is finite
 }
 
-template<typename VT>
-__device__ VT row_ssq(const VT* T, int r, int w)
-{
-    VT s = 0;
-    for(int j = 0; j < w; ++j) s = fma(T[32 * r + j], T[32 * r + j], s);
-    return s;
-}
-
 // entries of a block taken by the one-lane forms, and updates beside the
 // diagonal one such block may make in a pivot tile
 constexpr int LIGHT_E = 8;
@@ -575,6 +567,8 @@ struct alignas(16) PivLds {
     Dep dep;
     int32_t runs[NW];
     uint32_t plain, tiny;  // rows scaled together last, of them with a replaced pivot
+    int32_t rflag;
+    int32_t perm[32];      // old place of each row (numeric pivoting)
 };
 
 // What a dependency block U_ki with at most LIGHT_E entries subtracts from the
@@ -805,6 +799,10 @@ __device__ void apply_light(PivLds<VT, NW>& s, const LightUpd<VT>& o, bool mine)
         }
 }
 
+// piv_flag: an entry right of the diagonal, a 2x2 pivot, a non-finite D, rows
+// out of their order
+constexpr uint32_t PIV_ANY = 1, PIV_2X2 = 2, PIV_NONFINITE = 4, PIV_PERM = 8;
+
 // k_factor_pivot_blocks (kernels :1146-1283) for the pivot block at level
 // position q, NW waves.
 // Bound by latency: the level's pivot blocks are far fewer than the chip has
@@ -895,7 +893,9 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
         uint32_t plain = 0, tiny = 0;
         if(a.pivoting) {
             int32_t* fpiv = a.is_piv + fr;
-            int32_t* bperm = a.perm + fr;
+            int32_t* bperm = s.perm;
+            if(lane < 32) bperm[lane] = lane;
+            wave_sync();
             int p = 0;
             while(p < len) {
                 int order = 1, p0 = p, p1 = p + 1;
@@ -976,6 +976,7 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
         if(lane == 0) {
             s.plain = plain;
             s.tiny = tiny;
+            s.rflag = rflag;
             a.row_flag[i] = rflag;
         }
     }
@@ -1005,10 +1006,20 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
             a.rn[fr + lane] = ssq;
         }
         if(lane < 32) a.piv_umask[(int64_t) q * 32 + lane] = um;   // all 32 words defined
-        // and whether there is any such column at all (one word per tile)
-        const bool some = wave_ballot(um != 0u) != 0ull;
+        // what the off-diagonal blocks of the row ask first
+        uint32_t flags = wave_ballot(um != 0u) ? PIV_ANY : 0u;
+        if(s.rflag & ROW_2X2) flags |= PIV_2X2;
+        if(s.rflag & ROW_NONFINITE) flags |= PIV_NONFINITE;
+        if(a.pivoting) {
+            const int p = (lane < len) ? s.perm[lane] : lane;
+            if(wave_ballot(lane < len && p != lane)) flags |= PIV_PERM;
+            if(lane < len) {
+                a.perm[fr + lane] = fr + p;
+                a.piv_iperm[(int64_t) q * 32 + p] = (uint8_t) lane;
+            }
+        }
         if(lane == 0) {
-            a.piv_any[q] = some ? 1u : 0u;
+            a.piv_flag[q] = flags;
             a.piv_loc[i] = q;
         }
     }
@@ -1056,7 +1067,20 @@ __device__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int 
     int format)
 {
     const int lane = lane_id();
-    const VT ssq = (lane < hgt) ? row_ssq(X, lane, wid) : (VT) 0;
+    // nonzero entries per row; a row's sum skips exact zeros
+    uint32_t nz = 0;
+#pragma unroll
+    for(int t = 0; t < 16; ++t) {
+        const int r = 2 * t + (lane >> 5), c = lane & 31;
+        const uint64_t b = wave_ballot(r < hgt && c < wid && X[64 * t + lane] != (VT) 0);
+        if(lane == 2 * t) nz = (uint32_t) b;
+        if(lane == 2 * t + 1) nz = (uint32_t) (b >> 32);
+    }
+    VT ssq = (VT) 0;
+    for(uint32_t bits = nz; bits; bits &= bits - 1) {
+        const VT v = X[32 * lane + __ffs(bits) - 1];
+        ssq = fma(v, v, ssq);
+    }
     const uint64_t rows = wave_ballot(!(ssq == (VT) 0));
     if((rows >> lane) & 1ull) {
         const int j = lanes_below(rows);
@@ -1238,18 +1262,29 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
     offdiag_output(a, q, s.T, hgt, wid, m.format);
 }
 
+__device__ __forceinline__ double lane_value(double v, int src)
+{
+    const unsigned long long b = (unsigned long long) __double_as_longlong(v);
+    const unsigned lo = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) b, src);
+    const unsigned hi = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) (b >> 32), src);
+    return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+}
+
 // ---------------------------------------------------------------------------
-// Off-diagonal blocks whose right factors U_kj are sparse with at most 64
-// entries (every block at level-0 fill of the KKT workloads): the output
-// tile lives in registers (lane j + 32 c0 holds rows c0, c0 + 2, ... of
-// column j), U_ki is staged in the one LDS tile, and U_kj becomes a list of
-// its nonzero entries ordered by (column, row), so a wave needs about 10 KB
-// of LDS instead of 25 KB. Arithmetic and order are those of the general
-// form. A block with a larger right factor is handed to k_offdiag_general.
+// Off-diagonal blocks outside the one-lane form, one wave each, the output
+// tile in LDS. The matching pairs of a chunk of 64 are taken one per lane
+// where both blocks have at most LIGHT_E entries: each lane forms its pair's
+// few updates (entries that share a row), all lanes together going through
+// the chain of dependent loads once, and the updates are applied in pair
+// order. Other pairs are staged one at a time in their place in that order:
+// U_ki as a tile, U_kj (at most 64 entries, else the block is handed to
+// k_offdiag_general) as a list ordered by (column, row). Arithmetic and order
+// are those of the general form.
 
 template<typename VT>
 struct alignas(16) OffLdsSmall {
-    VT X[1024];
+    VT X[1024];   // the output tile
+    VT A[1024];   // a staged U_ki, the rows' old order, U_ii
     VT cs[32], cd[32], cb[32];
     VT rv[64];
     int32_t cst[33];
@@ -1291,7 +1326,7 @@ __device__ void list_build(VT* rv, uint8_t* rl, int32_t* cst, const Dep& d, cons
 // T[c][j] -= sum_l R[l][j] * Lt[c][l] over the listed rows l of column j,
 // ascending, Lt as in product()
 template<typename VT>
-__device__ void product_list(VT (&T)[16], const VT* A, const VT* rv, const uint8_t* rl,
+__device__ void product_list(VT* T, const VT* A, const VT* rv, const uint8_t* rl,
     const int32_t* cst, const VT* cs, const VT* cd, const VT* cb, int lh, int rh)
 {
     const int lane = lane_id();
@@ -1301,24 +1336,84 @@ __device__ void product_list(VT (&T)[16], const VT* A, const VT* rv, const uint8
     const int k1 = (j < rh) ? cst[j + 1] : 0;
     if(k0 < k1) {
         // one output row at a time keeps a single accumulator live
-#pragma unroll
-        for(int t = 0; t < 16; ++t) {
-            const int c = c0 + 2 * t;
-            if(c < lh) {
-                VT acc = 0;
-                for(int k = k0; k < k1; ++k) {
-                    const int l = rl[k];
-                    const VT r = rv[k];
-                    const VT left = (l == 0) ? (VT) 0 : A[32 * (l - 1) + c];
-                    const VT mid = A[32 * l + c];
-                    const VT right = (l == 31) ? (VT) 0 : A[32 * (l + 1) + c];
-                    const VT lt = fma(cb[l], right, fma(cd[l], mid, cs[l] * left));
-                    acc = fma(r, lt, acc);
-                }
-                T[t] -= acc;
+        for(int c = c0; c < lh; c += 2) {
+            VT acc = 0;
+            for(int k = k0; k < k1; ++k) {
+                const int l = rl[k];
+                const VT r = rv[k];
+                const VT left = (l == 0) ? (VT) 0 : A[32 * (l - 1) + c];
+                const VT mid = A[32 * l + c];
+                const VT right = (l == 31) ? (VT) 0 : A[32 * (l + 1) + c];
+                const VT lt = fma(cb[l], right, fma(cd[l], mid, cs[l] * left));
+                acc = fma(r, lt, acc);
             }
+            T[32 * c + j] -= acc;
         }
     }
+}
+
+// What a Schur pair of blocks with at most LIGHT_E entries each subtracts,
+// formed by one lane with product()'s operations: one update per pair of
+// entries in a common row. False outside the form: more entries, a 2x2 pivot
+// or a non-finite value among the rows, more than LIGHT_OFF updates or two of
+// one element.
+template<typename VT>
+struct PairUpd {
+    int n;
+    int el[LIGHT_OFF];   // 32 row + column of the tile
+    VT v[LIGHT_OFF];
+};
+
+template<typename VT>
+__device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, int hgt, int wid,
+    const int32_t* ixs, const VT* vals, const double* tri, PairUpd<VT>& o)
+{
+    o.n = 0;
+#pragma unroll
+    for(int k = 0; k < LIGHT_OFF; ++k) { o.el[k] = -1; o.v[k] = (VT) 0; }
+    if(di.fmt != FMT_SPARSE || di.nnz > LIGHT_E || di.nnz == 0 || dj.fmt != FMT_SPARSE ||
+        dj.nnz > LIGHT_E || dj.nnz == 0)
+        return false;
+    int ki[LIGHT_E], kj[LIGHT_E];   // 32 row + column, -1 for no entry
+    VT vi[LIGHT_E], vj[LIGHT_E], dd[LIGHT_E];
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) {
+        const int ai = min(e, di.nnz - 1), aj = min(e, dj.nnz - 1);
+        ki[e] = ixs[(int64_t) di.cp + ai];
+        vi[e] = vals[(int64_t) di.vp + ai];
+        kj[e] = ixs[(int64_t) dj.cp + aj];
+        vj[e] = vals[(int64_t) dj.vp + aj];
+    }
+    bool ok = true;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) {
+        const int ri = ki[e] / hgt, rj = kj[e] / wid;
+        ki[e] = 32 * ri + (ki[e] - ri * hgt);
+        kj[e] = 32 * rj + (kj[e] - rj * wid);
+        const double* t = tri + 3 * (int64_t) (dj.rb + rj);
+        const double sup = t[0], dia = t[1], sub = t[2];
+        ok = ok && sup == 0.0 && sub == 0.0 && fabs(dia) < (double) INFINITY &&
+            finite_value(vi[e]) && finite_value(vj[e]);
+        dd[e] = (VT) dia;
+        if(e >= di.nnz) ki[e] = -1;
+        if(e >= dj.nnz || vj[e] == (VT) 0) kj[e] = -1;
+    }
+#pragma unroll
+    for(int f = 0; f < LIGHT_E; ++f)
+#pragma unroll
+        for(int e = 0; e < LIGHT_E; ++e)
+            if(kj[f] >= 0 && (ki[e] >> 5) == (kj[f] >> 5)) {
+                const int el = 32 * (ki[e] & 31) + (kj[f] & 31);
+                const VT lt = dd[f] * vi[e];
+                const VT acc = fma(vj[f], lt, (VT) 0);
+#pragma unroll
+                for(int k = 0; k < LIGHT_OFF; ++k) {
+                    ok = ok && !(k < o.n && o.el[k] == el);
+                    if(k == o.n) { o.el[k] = el; o.v[k] = acc; }
+                }
+                ++o.n;
+            }
+    return ok && o.n <= LIGHT_OFF;
 }
 
 template<typename VT>
@@ -1332,123 +1427,133 @@ __device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr,
     const int4 t2 = ((const int4*) a.off_task)[3 * p + 2];
     const int fr = t0.y;
     const int hgt = t0.z & 255, wid = (t0.z >> 8) & 255;
-    const bool all1x1 = ((t0.z >> 16) & 1) != 0;
     const int pq = t0.w;
     const int np = t2.y;
     const int4* pairs = (const int4*) a.upd4 + pair_first(t2);
-    const int j = lane & 31, c0 = lane >> 5;
-
-    // input block A_ij into the register tile
-    tile_zero(s.X);
-    wave_sync();
-    if(t1.x == FMT_DENSE) {
-#pragma unroll
-        for(int t = 0; t < 16; ++t) {
-            const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
-            if(r < hgt && c < wid) s.X[idx] = a.val_in[(int64_t) t1.w + r * wid + c];
-        }
-    } else {
-        for(int e = lane; e < t1.y; e += 64) {
-            const int ix = a.ix_in[(int64_t) t1.z + e];
-            const int r = ix / wid, c = ix - r * wid;
-            s.X[32 * r + c] = a.val_in[(int64_t) t1.w + e];
-        }
-    }
-    wave_sync();
-    VT T[16];
-#pragma unroll
-    for(int t = 0; t < 16; ++t) T[t] = s.X[32 * (c0 + 2 * t) + j];
-    wave_sync();
-    tile_zero(s.X);
-    wave_sync();
+    // what the end needs, in flight meanwhile
+    const uint32_t flags = a.piv_flag[pq];
+    const uint32_t um_row = (lane < hgt) ? a.piv_umask[(int64_t) pq * 32 + lane] : 0u;
+    const double d_row = a.tri[3 * (int64_t) (fr + min(lane, hgt - 1)) + 1];
+    tile_load(s.X, t1, hgt, wid, a.ix_in, a.val_in);
+    bool staging = false;   // s.A is zero
 
     // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order
     for(int e0 = 0; e0 < np; e0 += 64) {
         Dep mi{}, mj{};
-        bool hit = false;
+        PairUpd<VT> up;
+        up.n = 0;
+        bool hit = false, light = false;
         if(e0 + lane < np) {
             const int4 pr = pairs[e0 + lane];
             hit = pair_matches(a.row_mask[pr.x], a.row_mask[pr.y]);
             if(hit) {
                 mi = dep_meta(a.bout, pr.x, pr.z, pr.w);
                 mj = dep_meta(a.bout, pr.y, pr.z, pr.w);
+                light = light_pair(mi, mj, hgt, wid, a.ix_out, a.val_out, a.tri, up);
             }
         }
-        uint64_t hits = wave_ballot(hit);
-        if(!hits) continue;
-        if(wave_ballot(hit && !small_sparse<VT>(mj))) {
+        if(wave_ballot(hit && !light && !small_sparse<VT>(mj))) {
             if(lane == 0) a.defer_list[atomicAdd(a.defer_cnt + lr.level, 1)] = q;
             return;
         }
-        int d = __ffsll((long long) hits) - 1;
-        Dep ci = bcast(mi, d), cj = bcast(mj, d);
-        Pre<VT> pi = prefetch(ci, a.ix_out, a.val_out, a.tri, true);
-        Pre<VT> pj = prefetch(cj, a.ix_out, a.val_out, a.tri, false);
-        while(hits) {
-            hits &= hits - 1;
-            Dep ni = ci, nj = cj;
-            Pre<VT> qi = pi, qj = pj;
-            if(hits) {
-                d = __ffsll((long long) hits) - 1;
-                ni = bcast(mi, d);
-                nj = bcast(mj, d);
-                qi = prefetch(ni, a.ix_out, a.val_out, a.tri, true);
-                qj = prefetch(nj, a.ix_out, a.val_out, a.tri, false);
+        const uint64_t heavy = wave_ballot(hit && !light);
+        for(uint64_t m = wave_ballot(hit && (!light || up.n > 0)); m; m &= m - 1) {
+            const int d = __ffsll((long long) m) - 1;
+            if(!((heavy >> d) & 1ull)) {
+                if(lane == d) {
+#pragma unroll
+                    for(int k = 0; k < LIGHT_OFF; ++k)
+                        if(k < up.n) s.X[up.el[k]] -= up.v[k];
+                }
+                wave_sync();
+                continue;
             }
-            stage(s.X, (uint32_t*) nullptr, ci, pi, hgt, a.ix_out, a.val_out);
+            if(!staging) {
+                tile_zero(s.A);
+                wave_sync();
+                staging = true;
+            }
+            const Dep ci = bcast(mi, d), cj = bcast(mj, d);
+            const Pre<VT> pi = prefetch(ci, a.ix_out, a.val_out, a.tri, true);
+            const Pre<VT> pj = prefetch(cj, a.ix_out, a.val_out, a.tri, false);
+            stage(s.A, (uint32_t*) nullptr, ci, pi, hgt, a.ix_out, a.val_out);
             list_build(s.rv, s.rl, s.cst, cj, pj, wid);
             stage_d(s.cs, s.cd, s.cb, pi);
             wave_sync();
-            product_list(T, s.X, s.rv, s.rl, s.cst, s.cs, s.cd, s.cb, hgt, wid);
+            product_list(s.X, s.A, s.rv, s.rl, s.cst, s.cs, s.cd, s.cb, hgt, wid);
             wave_sync();
-            unstage(s.X, (uint32_t*) nullptr, ci, pi, hgt);
+            unstage(s.A, (uint32_t*) nullptr, ci, pi, hgt);
             wave_sync();
-            ci = ni; cj = nj; pi = qi; pj = qj;
         }
     }
-
-    // the updated tile back to LDS, row c, column j
-#pragma unroll
-    for(int t = 0; t < 16; ++t) s.X[32 * (c0 + 2 * t) + j] = T[t];
-    wave_sync();
-
-    // U_ii' forward substitution in place, column jc per lane (lanes >= 32
-    // idle), over the nonzero columns of the pivot rows (exact no-ops skipped)
-    const VT* piv = a.if_val + (int64_t) pq * 1024;
-    const uint32_t um_row = (lane < hgt) ? a.piv_umask[(int64_t) pq * 32 + lane] : 0u;
+    // rows in the block row's pivoting order (kernels :1733-1751)
+    if(flags & PIV_PERM) {
+        tile_copy(s.A, s.X);
+        wave_sync();
+        for(int e = lane; e < hgt * 32; e += 64) {
+            const int r = e >> 5, c = e & 31;
+            s.X[e] = s.A[32 * (a.perm[fr + r] - fr) + c];
+        }
+        wave_sync();
+    }
     const int jc = lane;
     VT* col = s.X + jc;
-    for(int ii = 0; ii < hgt; ++ii) {
-        const uint32_t um = (uint32_t) __builtin_amdgcn_readlane((int) um_row, ii);
-        if(um && jc < wid) {
-            const VT rv = col[32 * ii];
-            if(rv != (VT) 0) {
-                const VT pv = rv / piv[ii * hgt + ii];
-                for(uint32_t bits = um; bits; bits &= bits - 1) {
-                    const int l = __ffs(bits) - 1;
-                    col[32 * l] = fma(-piv[ii * hgt + l], pv, col[32 * l]);
-                }
+    // U_ii' forward substitution, column jc per lane (lanes >= 32 idle), over
+    // the nonzero columns of the pivot rows (exact no-ops skipped), the
+    // column in registers and U_ii in LDS
+    if(flags & PIV_ANY) {
+        const VT* piv = a.if_val + (int64_t) pq * 1024;
+        for(int e = lane; e < hgt * hgt; e += 64) {
+            const int r = e / hgt;
+            s.A[32 * r + (e - r * hgt)] = piv[e];
+        }
+        wave_sync();
+        VT x[32];
+#pragma unroll
+        for(int l = 0; l < 32; ++l) x[l] = (l < hgt && jc < wid) ? col[32 * l] : (VT) 0;
+#pragma unroll
+        for(int ii = 0; ii < 32; ++ii) {
+            const uint32_t um = (uint32_t) __builtin_amdgcn_readlane((int) um_row, ii);
+            if(um && wave_ballot(x[ii] != (VT) 0)) {
+                const bool on = x[ii] != (VT) 0;
+                const VT pv = x[ii] / s.A[33 * ii];
+#pragma unroll
+                for(int l = ii + 1; l < 32; ++l)
+                    if((um >> l) & 1u) {
+                        const VT y = fma(-s.A[32 * ii + l], pv, x[l]);
+                        x[l] = on ? y : x[l];
+                    }
             }
         }
+        if(jc < wid) {
+#pragma unroll
+            for(int l = 0; l < 32; ++l)
+                if(l < hgt) col[32 * l] = x[l];
+        }
+        wave_sync();
     }
     // D solve in place (d_left_solve_with_D_Ut, kernels :1533-1566); a row
     // is written only after both rows it reads have been read
-    const double* D = a.tri + 3 * (int64_t) fr;
-    const int32_t* ip = a.is_piv + fr;
-    if(jc < wid) {
-        if(all1x1) {
-            for(int l = 0; l < hgt; ++l) col[32 * l] = (VT) ((double) col[32 * l] / D[3 * l + 1]);
-        } else {
-            for(int l = 0; l < hgt; ++l) {
-                const bool p1 = ip[l] != 0;
-                const bool p2 = (l + 1 < hgt) && !ip[l + 1];
-                const VT rl = col[32 * l];
-                const VT right = (l < 31) ? col[32 * (l + 1)] : rl;
-                VT x1, x2;
-                givens_d_solve(a.piv64 != 0, D + 3 * l, l, hgt, rl, right, p2, x1, x2);
-                if(p1) col[32 * l] = x1;
-                if(p2) col[32 * (l + 1)] = x2;
-            }
+    if(!(flags & PIV_2X2)) {
+        for(int l = 0; l < hgt; ++l) {
+            const VT x = (jc < wid) ? col[32 * l] : (VT) 0;
+            // a finite D leaves a row of zeros as it is
+            if(wave_ballot(x != (VT) 0) == 0ull && !(flags & PIV_NONFINITE)) continue;
+            const double dl = lane_value(d_row, l);
+            if(jc < wid) col[32 * l] = (VT) ((double) x / dl);
+        }
+    } else if(jc < wid) {
+        const double* D = a.tri + 3 * (int64_t) fr;
+        const int32_t* ip = a.is_piv + fr;
+        for(int l = 0; l < hgt; ++l) {
+            const bool p1 = ip[l] != 0;
+            const bool p2 = (l + 1 < hgt) && !ip[l + 1];
+            const VT rl = col[32 * l];
+            const VT right = (l < 31) ? col[32 * (l + 1)] : rl;
+            VT x1, x2;
+            givens_d_solve(a.piv64 != 0, D + 3 * l, l, hgt, rl, right, p2, x1, x2);
+            if(p1) col[32 * l] = x1;
+            if(p2) col[32 * (l + 1)] = x2;
         }
     }
     wave_sync();
@@ -1481,7 +1586,7 @@ __device__ __forceinline__ void offdiag_body(const FactorArgs<VT>& a, const Leve
 // operations in the same order as in the wave form (terms that are exact
 // zeros in the wave form are skipped).
 constexpr int TINY_E = LIGHT_E;
-constexpr int TINY_T = 32;
+constexpr int TINY_T = 16;
 constexpr int TINY_P = 12;  // the same while its Schur updates are added up
 constexpr int TINY_F = 4;   // pairs whose row masks are fetched together
 
@@ -1559,11 +1664,6 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
     const int4 t0 = ((const int4*) a.off_task)[3 * p];
     const int4 t1 = ((const int4*) a.off_task)[3 * p + 1];
     const int4 t2 = ((const int4*) a.off_task)[3 * p + 2];
-    if(a.pivoting) {
-        // rows in pivoting order: every block takes the general form
-        a.defer_list[atomicAdd(a.defer_cnt + lr.level, 1)] = q;
-        return;
-    }
     if(!(t2.z & 1)) { to_wave_form(a, lr, q); return; }
     const int hgt = t0.z & 255, wid = (t0.z >> 8) & 255;
     const int np = t2.y;
@@ -1755,28 +1855,103 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
 }
 
 // One-lane form, second phase (after the level's pivot blocks): the tile
-// list of the first phase through U_ii' and D, then the row partial sums and
-// the compact entries.
+// list of the first phase in the block row's pivoting order, through U_ii'
+// and D, then the row sums of squares and the compact entries. Lists of at
+// most LIST_C entries whose rows have nothing right of the diagonal of U_ii
+// (nearly all at level-0 fill) stay in registers; the others go through LDS.
 template<typename VT>
 __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a, const LevelRange& lr,
-    int bid_, int nblk_)
+    int bid_)
 {
     __shared__ TinyLds<VT, TINY_T, TINY_TPB> s;
     const int tid = threadIdx.x;
     const int q = lr.npiv + bid_ * TINY_TPB + tid;
     if(q >= lr.size) return;
-    // the parked count and the task record together (neither waits for
-    // the other)
+    // the parked count, the first entries and the task record together
+    // (none waits for the others)
     const int64_t p = (int64_t) lr.lo + q;
     const int4 t0 = ((const int4*) a.off_task)[3 * p];
     int n = a.if_cnt[q];
+    VT v[LIST_C];
+    int ix[LIST_C];
+#pragma unroll
+    for(int e = 0; e < LIST_C; ++e) {
+        v[e] = a.c_val[(int64_t) q * LIST_C + e];
+        ix[e] = a.c_idx[(int64_t) q * LIST_C + e];
+    }
     if(n < 0) return;
     const int fr = t0.y;
     const int hgt = t0.z & 255;
     const int pq = t0.w;
-    // a pivot block without entries right of its diagonal (nearly all at
-    // level-0 fill) leaves the forward substitution with nothing to do
-    const uint32_t um_any = a.piv_any[pq];
+    const uint32_t flags = a.piv_flag[pq];
+    if(flags & PIV_2X2) {
+        // numeric pivoting chose a 2x2 pivot
+        to_wave_form(a, lr, q);
+        return;
+    }
+    const uint8_t* iperm = a.piv_iperm + (int64_t) pq * 32;
+    const uint32_t* umask = a.piv_umask + (int64_t) pq * 32;
+    const double* D = a.tri + 3 * (int64_t) fr;
+    const EntryList<VT> o = entry_list(a, q);
+    bool plain = n <= LIST_C;
+    if(plain) {
+        if(flags & PIV_PERM) {
+#pragma unroll
+            for(int e = 0; e < LIST_C; ++e)
+                if(e < n) ix[e] = 32 * iperm[ix[e] >> 5] + (ix[e] & 31);
+        }
+        if(flags & PIV_ANY) {
+#pragma unroll
+            for(int e = 0; e < LIST_C; ++e)
+                if(e < n) plain = plain && (umask[ix[e] >> 5] == 0u || v[e] == (VT) 0);
+        }
+    }
+    if(plain) {
+        constexpr int NONE = 1 << 20;
+        double dv[LIST_C];
+#pragma unroll
+        for(int e = 0; e < LIST_C; ++e) dv[e] = (e < n) ? D[3 * (ix[e] >> 5) + 1] : 1.0;
+#pragma unroll
+        for(int e = 0; e < LIST_C; ++e) {
+            if(e < n) v[e] = (VT) ((double) v[e] / dv[e]);
+            else ix[e] = NONE;
+        }
+        // tile order (row-major)
+        auto order = [&](int x, int y) {
+            if(ix[y] < ix[x]) {
+                const int ti = ix[x]; ix[x] = ix[y]; ix[y] = ti;
+                const VT tv = v[x]; v[x] = v[y]; v[y] = tv;
+            }
+        };
+        static_assert(LIST_C == 4, "sorting network on four");
+        order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+        uint32_t rows = 0;
+        int nr = 0, cnt = 0;
+        VT ssq = 0;
+#pragma unroll
+        for(int e = 0; e < LIST_C; ++e) {
+            if(ix[e] == NONE) continue;
+            ssq = fma(v[e], v[e], ssq);
+            // the row ends here
+            if(e == LIST_C - 1 || (ix[min(e + 1, LIST_C - 1)] >> 5) != (ix[e] >> 5)) {
+                if(!(ssq == (VT) 0)) {
+                    if(nr == 0) a.rn_first[q] = ssq;
+                    else a.rn_part[(int64_t) q * 32 + nr] = ssq;
+                    rows |= 1u << (ix[e] >> 5);
+                    ++nr;
+                }
+                ssq = 0;
+            }
+            if(fabs((double) v[e]) > NZ_EPS) {
+                o.cv[cnt] = v[e];
+                o.ci[cnt] = (uint16_t) ix[e];
+                ++cnt;
+            }
+        }
+        a.part_mask[q] = rows;
+        a.if_cnt[q] = cnt;
+        return;
+    }
     VT* tv = &s.v[0][tid];
     int16_t* ti = &s.ix[0][tid];
     auto V = [&](int k) -> VT& { return tv[k * TINY_TPB]; };
@@ -1786,20 +1961,24 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
             if(I(k) == idx) return k;
         return -1;
     };
-    {
-        const EntryList<VT> o = entry_list(a, q);
-        for(int k = 0; k < n; ++k) {
-            I(k) = (int16_t) o.idx(k);
-            V(k) = o.val(k);
-        }
+    for(int k = 0; k < n; ++k) {
+        int at = o.idx(k);
+        if(flags & PIV_PERM) at = 32 * iperm[at >> 5] + (at & 31);
+        I(k) = (int16_t) at;
+        V(k) = o.val(k);
     }
-    // U_ii' forward substitution over the rows in ascending order
+    // U_ii' forward substitution over the rows in ascending order: the next
+    // row with an entry and something right of its diagonal
     const VT* piv = a.if_val + (int64_t) pq * 1024;
-    for(int ii = 0; ii < hgt && um_any != 0; ++ii) {
-        bool any = false;
-        for(int k = 0; k < n; ++k) any = any || ((I(k) >> 5) == ii && V(k) != (VT) 0);
-        if(!any) continue;
-        const uint32_t um = a.piv_umask[(int64_t) pq * 32 + ii];
+    for(int ii = -1; flags & PIV_ANY;) {
+        int nxt = 32;
+        for(int k = 0; k < n; ++k) {
+            const int r = I(k) >> 5;
+            if(r > ii && r < nxt && V(k) != (VT) 0) nxt = r;
+        }
+        if(nxt >= hgt) break;
+        ii = nxt;
+        const uint32_t um = umask[ii];
         if(!um) continue;
         const VT d = piv[ii * hgt + ii];
         const int n0 = n;
@@ -1823,7 +2002,6 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
     }
     // D solve (1x1 pivots): the Givens-form solve reduces to a division;
     // the divisors of eight entries are loaded together
-    const double* D = a.tri + 3 * (int64_t) fr;
     for(int k0 = 0; k0 < n; k0 += 8) {
         double dv[8];
 #pragma unroll
@@ -1863,7 +2041,6 @@ __device__ __forceinline__ void offdiag_tiny_scale_body(const FactorArgs<VT>& a,
         }
     }
     a.part_mask[q] = rows;
-    const EntryList<VT> o = entry_list(a, q);
     int pos = 0;
     for(int m = 0; m < n; ++m)
         if(fabs((double) V(m)) > NZ_EPS) o.set(pos++, I(m), V(m));
@@ -2458,11 +2635,16 @@ __global__ __launch_bounds__(64, 3) void k_offdiag(FactorArgs<VT> a, LevelRange 
 template<typename VT>
 __global__ __launch_bounds__(TINY_TPB) void k_offdiag_tiny_scale(FactorArgs<VT> a, LevelRange lr)
 {
-    offdiag_tiny_scale_body<VT>(a, lr, blockIdx.x, gridDim.x);
+    offdiag_tiny_scale_body<VT>(a, lr, blockIdx.x);
 }
 
+// waves per SIMD the pivot and pair launch is compiled for: as many as its
+// registers allow without spills
+template<typename VT>
+constexpr int PP_WAVES = sizeof(VT) == 4 ? 3 : 2;
+
 template<typename VT, int NW>
-__global__ __launch_bounds__(64 * NW) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
+__global__ __launch_bounds__(64 * NW, PP_WAVES<VT>) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
 {
     pivots_pairs_body<VT, NW>(a, lr, blockIdx.x);
 }
@@ -2570,7 +2752,7 @@ __global__ void bk_gather(const FactorSys<VT>* fs, const int2* items)
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64) void bk_pivots_pairs(const FactorSys<VT>* fs, const int2* items,
+__global__ __launch_bounds__(64, PP_WAVES<VT>) void bk_pivots_pairs(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
     const int2 it = items[blockIdx.x];
@@ -2586,7 +2768,7 @@ __global__ __launch_bounds__(TINY_TPB) void bk_offdiag_tiny_scale(const FactorSy
     const int2 it = items[blockIdx.x];
     const FactorSys<VT>& F = fs[it.x];
     const LevelRange lr = F.lr[level];
-    offdiag_tiny_scale_body<VT>(F.a, lr, it.y, fl_tiny_blocks(lr));
+    offdiag_tiny_scale_body<VT>(F.a, lr, it.y);
 }
 
 template<typename VT>

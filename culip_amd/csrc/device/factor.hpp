@@ -91,7 +91,8 @@ struct FactorArgs {
     // static, per Schur pair: {block (k, i), block (k, j), first row of k, rows of k}
     const int32_t* upd4 = nullptr;
     uint32_t* piv_umask = nullptr;        // 32 per pivot position: nonzero columns > row
-    uint32_t* piv_any = nullptr;          // per pivot position: any such column
+    uint32_t* piv_flag = nullptr;         // per pivot position: PIV_ANY, ...
+    uint8_t* piv_iperm = nullptr;         // 32 per pivot position: new place of a row
     int32_t* defer_list = nullptr;        // positions left to the general kernel
     int32_t* defer_cnt = nullptr;         // one counter per level
     int32_t* wave_list = nullptr;         // positions left to the one-wave kernel

@@ -207,8 +207,8 @@ void Bildlt::upload_pattern(hipStream_t st)
     const Symbolic& s = sym;
     const int32_t n = s.n, K = s.coarse_nnz;
     const int64_t mlb = std::max<int64_t>(1, s.max_level_blocks);
-    // 32 row masks per pivot position, then one "any" word per position
-    d_piv_umask.ensure(sizeof(uint32_t) * 33 * mlb);
+    // per pivot position 32 row masks, one word of flags, 32 bytes of order
+    d_piv_umask.ensure(sizeof(uint32_t) * (33 + 8) * mlb);
     d_defer_list.ensure(sizeof(int32_t) * mlb);
     d_defer_cnt.ensure(sizeof(int32_t) * std::max(1, s.num_levels));
     d_wave_list.ensure(sizeof(int32_t) * mlb);
@@ -331,7 +331,8 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.off_task = d_off_task.as<int32_t>();
     a.upd4 = d_upd4.as<int32_t>();
     a.piv_umask = d_piv_umask.as<uint32_t>();
-    a.piv_any = a.piv_umask + 32 * std::max<int64_t>(1, sym.max_level_blocks);
+    a.piv_flag = a.piv_umask + 32 * std::max<int64_t>(1, sym.max_level_blocks);
+    a.piv_iperm = (uint8_t*) (a.piv_flag + std::max<int64_t>(1, sym.max_level_blocks));
     a.defer_list = d_defer_list.as<int32_t>();
     a.defer_cnt = d_defer_cnt.as<int32_t>();
     a.wave_list = d_wave_list.as<int32_t>();
@@ -732,7 +733,7 @@ int64_t Bildlt::numeric_bytes_estimate(bool with_layout) const
     const int64_t mlb = std::max<int64_t>(1, s.max_level_blocks);
     auto r16 = [](int64_t b) { return std::max<int64_t>(16, b); };
     int64_t b = 0;
-    b += r16(132 * mlb) + r16(4 * mlb) + r16(4 * std::max(1, s.num_levels));
+    b += r16(164 * mlb) + r16(4 * mlb) + r16(4 * std::max(1, s.num_levels));
     b += r16(24 * nb + 4 * std::max(1, s.num_levels));   // row groups (at most nb), tickets
     b += r16(LIST_C * (v + 2) * mlb) + r16((4 + v) * mlb);   // short lists, row sums
     b += r16(8 * (int64_t) s.value_slot.size()) + 2 * r16(v * s.val_space) + r16(36 * K);
