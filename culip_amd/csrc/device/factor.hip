@@ -396,6 +396,22 @@ __device__ bool step_2x2(VT* T, double* tri, int p, int len)
     return fabs(d11) + fabs(d12) + fabs(d22) < (AT) INFINITY;   // D is finite
 }
 
+// ix / w for an entry index ix < 1024 and a width 1 <= w <= 32 as
+// (ix * m) >> 20, m = ceil(2^20 / w): the excess ix (m w - 2^20) / (2^20 w) is
+// below 1023 * 31 / 2^20 / w < 1 / w
+struct RowOf {
+    uint32_t m;
+    int w;
+    __device__ __forceinline__ explicit RowOf(int w_) : m(((1u << 20) + w_ - 1) / w_), w(w_) {}
+    __device__ __forceinline__ int row(int ix) const { return (int) (((uint32_t) ix * m) >> 20); }
+    // 32 row + column
+    __device__ __forceinline__ int at(int ix) const
+    {
+        const int r = row(ix);
+        return 32 * r + (ix - r * w);
+    }
+};
+
 // entries of a block taken by the one-lane forms, and updates beside the
 // diagonal one such block may make in a pivot tile
 constexpr int LIGHT_E = 8;
@@ -587,8 +603,8 @@ struct LightUpd {
     VT ov[LIGHT_OFF];
 };
 
-template<typename VT>
-__device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t* ixs,
+template<typename VT, int E>
+__device__ __forceinline__ bool light_update(const Dep& d, const RowOf& w, const int32_t* ixs,
     const VT* vals, const double* tri, LightUpd<VT>& o)
 {
     o.cols = 0;
@@ -597,37 +613,36 @@ __device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t*
     for(int e = 0; e < LIGHT_E; ++e) { o.acc[e] = (VT) 0; o.head[e] = -1; }
 #pragma unroll
     for(int k = 0; k < LIGHT_OFF; ++k) { o.oe[k] = 0; o.ov[k] = (VT) 0; }
-    if(d.fmt != FMT_SPARSE || d.nnz > LIGHT_E) return false;
+    if(d.fmt != FMT_SPARSE || d.nnz > E) return false;
     if(d.nnz == 0) return true;
     constexpr int NONE = 1 << 20;
-    int key[LIGHT_E];          // 32 row + column, ascending
-    VT v[LIGHT_E];
+    int key[E];          // 32 row + column, ascending
+    VT v[E];
     bool sorted = true;
 #pragma unroll
-    for(int e = 0; e < LIGHT_E; ++e) {
+    for(int e = 0; e < E; ++e) {
         const int at = min(e, d.nnz - 1);
         const int ix = ixs[(int64_t) d.cp + at];
         v[e] = vals[(int64_t) d.vp + at];
-        const int r = ix / w;
-        key[e] = (e < d.nnz && v[e] != (VT) 0) ? 32 * r + (ix - r * w) : NONE;
+        key[e] = (e < d.nnz && v[e] != (VT) 0) ? w.at(ix) : NONE;
     }
 #pragma unroll
-    for(int e = 1; e < LIGHT_E; ++e) sorted = sorted && key[e - 1] <= key[e];
+    for(int e = 1; e < E; ++e) sorted = sorted && key[e - 1] <= key[e];
     if(!sorted) {
         // odd-even transposition (entries over capacity are stored by size)
 #pragma unroll
-        for(int p = 0; p < LIGHT_E; ++p)
+        for(int p = 0; p < E; ++p)
 #pragma unroll
-            for(int e = p & 1; e + 1 < LIGHT_E; e += 2)
+            for(int e = p & 1; e + 1 < E; e += 2)
                 if(key[e + 1] < key[e]) {
                     const int tk = key[e]; key[e] = key[e + 1]; key[e + 1] = tk;
                     const VT tv = v[e]; v[e] = v[e + 1]; v[e + 1] = tv;
                 }
     }
-    VT lt[LIGHT_E];
+    VT lt[E];
     bool ok = true;
 #pragma unroll
-    for(int e = 0; e < LIGHT_E; ++e) {
+    for(int e = 0; e < E; ++e) {
         const double* t = tri + 3 * (int64_t) (d.rb + ((key[e] != NONE) ? key[e] >> 5 : 0));
         const double sup = t[0], dia = t[1], sub = t[2];
         ok = ok && (key[e] == NONE ||
@@ -636,7 +651,7 @@ __device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t*
     }
     if(!ok) return false;
 #pragma unroll
-    for(int e = 0; e < LIGHT_E; ++e) {
+    for(int e = 0; e < E; ++e) {
         if(key[e] == NONE) continue;
         const int c = key[e] & 31;
         bool first = true;
@@ -645,14 +660,14 @@ __device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t*
         if(first) {
             VT acc = fma(v[e], lt[e], (VT) 0);
 #pragma unroll
-            for(int f = e + 1; f < LIGHT_E; ++f)
+            for(int f = e + 1; f < E; ++f)
                 if(key[f] != NONE && (key[f] & 31) == c) acc = fma(v[f], lt[f], acc);
             o.acc[e] = acc;
             o.head[e] = c;
             o.cols |= 1u << c;
         }
 #pragma unroll
-        for(int f = e + 1; f < LIGHT_E; ++f)
+        for(int f = e + 1; f < E; ++f)
             if(key[f] != NONE && (key[f] >> 5) == (key[e] >> 5)) {
                 const int el = 32 * c + (key[f] & 31);
                 const VT acc = fma(v[f], lt[e], (VT) 0);
@@ -670,7 +685,7 @@ __device__ __forceinline__ bool light_update(const Dep& d, int w, const int32_t*
 // T -= A' D A for the block staged in h.X by all NW waves: the arithmetic and
 // order of product() with R = A
 template<typename VT, int NW>
-__device__ void product_staged(PivLds<VT, NW>& s, int len)
+__device__ __forceinline__ void product_staged(PivLds<VT, NW>& s, int len)
 {
     const int j = (int) threadIdx.x & 31;
     const int c0 = (int) threadIdx.x >> 5;
@@ -705,7 +720,7 @@ __device__ void product_staged(PivLds<VT, NW>& s, int len)
 
 // one dependency block of any form, by all NW waves
 template<typename VT, int NW>
-__device__ void heavy_update(const FactorArgs<VT>& a, PivLds<VT, NW>& s, const Dep& d, int len)
+__device__ __forceinline__ void heavy_update(const FactorArgs<VT>& a, PivLds<VT, NW>& s, const Dep& d, int len)
 {
     constexpr int TPB = 64 * NW;
     const int t = (int) threadIdx.x;
@@ -747,7 +762,7 @@ __device__ void heavy_update(const FactorArgs<VT>& a, PivLds<VT, NW>& s, const D
 
 // the one-lane updates of the lanes with `mine` set, in block order
 template<typename VT, int NW>
-__device__ void apply_light(PivLds<VT, NW>& s, const LightUpd<VT>& o, bool mine)
+__device__ __forceinline__ void apply_light(PivLds<VT, NW>& s, const LightUpd<VT>& o, bool mine)
 {
     const int t = (int) threadIdx.x, lane = lane_id(), wv = t / WAVE;
     const int n = mine ? __popc(o.cols) : 0;
@@ -814,7 +829,7 @@ constexpr uint32_t PIV_ANY = 1, PIV_2X2 = 2, PIV_NONFINITE = 4, PIV_PERM = 8;
 // rows with an entry right of the diagonal (or a 2x2 pivot) are steps; the
 // others scale a row and change nothing else, so they are done together last.
 template<typename VT, int NW>
-__device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
+__device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
     PivLds<VT, NW>& s)
 {
     constexpr int TPB = 64 * NW;
@@ -849,6 +864,7 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
     }
     __syncthreads();
     // updates from the blocks (k, i) above the diagonal, in CSC order
+    const RowOf width(len);
     for(int c0 = 0; c0 < nd; c0 += TPB) {
         if(c0) blk = (c0 + t < nd) ? a.csc_idx[cb0 + c0 + t] : -1;
         Dep d{};
@@ -858,8 +874,13 @@ __device__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const 
         bool light = false;
         if(blk >= 0) {
             d = load_dep(a.bout, a.bs, blk);
-            light = light_update(d, len, a.ix_out, a.val_out, a.tri, up);
         }
+        // blocks of one or two entries (nearly all on large sparse patterns)
+        // without the eight-entry form's work
+        if(wave_ballot(blk >= 0 && !(d.fmt == FMT_SPARSE && d.nnz <= 2)) == 0ull)
+            light = blk >= 0 && light_update<VT, 2>(d, width, a.ix_out, a.val_out, a.tri, up);
+        else
+            light = blk >= 0 && light_update<VT, LIGHT_E>(d, width, a.ix_out, a.val_out, a.tri, up);
         const uint64_t hm = wave_ballot(blk >= 0 && !light);
         if(lane == 0) s.heavy[wv] = hm;
         __syncthreads();
@@ -1063,7 +1084,7 @@ __device__ __forceinline__ EntryList<VT> entry_list(const FactorArgs<VT>& a, int
 // a scaled off-diagonal tile X (one wave, stride 32) as position q leaves
 // it: row sums of squares, and the dense tile or the entries above NZ_EPS
 template<typename VT>
-__device__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int hgt, int wid,
+__device__ __forceinline__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int hgt, int wid,
     int format)
 {
     const int lane = lane_id();
@@ -1364,20 +1385,21 @@ struct PairUpd {
     VT v[LIGHT_OFF];
 };
 
-template<typename VT>
-__device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, int hgt, int wid,
+template<typename VT, int E>
+__device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, const RowOf& hgt,
+    const RowOf& wid,
     const int32_t* ixs, const VT* vals, const double* tri, PairUpd<VT>& o)
 {
     o.n = 0;
 #pragma unroll
     for(int k = 0; k < LIGHT_OFF; ++k) { o.el[k] = -1; o.v[k] = (VT) 0; }
-    if(di.fmt != FMT_SPARSE || di.nnz > LIGHT_E || di.nnz == 0 || dj.fmt != FMT_SPARSE ||
-        dj.nnz > LIGHT_E || dj.nnz == 0)
+    if(di.fmt != FMT_SPARSE || di.nnz > E || di.nnz == 0 || dj.fmt != FMT_SPARSE ||
+        dj.nnz > E || dj.nnz == 0)
         return false;
-    int ki[LIGHT_E], kj[LIGHT_E];   // 32 row + column, -1 for no entry
-    VT vi[LIGHT_E], vj[LIGHT_E], dd[LIGHT_E];
+    int ki[E], kj[E];   // 32 row + column, -1 for no entry
+    VT vi[E], vj[E], dd[E];
 #pragma unroll
-    for(int e = 0; e < LIGHT_E; ++e) {
+    for(int e = 0; e < E; ++e) {
         const int ai = min(e, di.nnz - 1), aj = min(e, dj.nnz - 1);
         ki[e] = ixs[(int64_t) di.cp + ai];
         vi[e] = vals[(int64_t) di.vp + ai];
@@ -1386,11 +1408,10 @@ __device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, int hgt
     }
     bool ok = true;
 #pragma unroll
-    for(int e = 0; e < LIGHT_E; ++e) {
-        const int ri = ki[e] / hgt, rj = kj[e] / wid;
-        ki[e] = 32 * ri + (ki[e] - ri * hgt);
-        kj[e] = 32 * rj + (kj[e] - rj * wid);
-        const double* t = tri + 3 * (int64_t) (dj.rb + rj);
+    for(int e = 0; e < E; ++e) {
+        ki[e] = hgt.at(ki[e]);
+        kj[e] = wid.at(kj[e]);
+        const double* t = tri + 3 * (int64_t) (dj.rb + (kj[e] >> 5));
         const double sup = t[0], dia = t[1], sub = t[2];
         ok = ok && sup == 0.0 && sub == 0.0 && fabs(dia) < (double) INFINITY &&
             finite_value(vi[e]) && finite_value(vj[e]);
@@ -1399,9 +1420,9 @@ __device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, int hgt
         if(e >= dj.nnz || vj[e] == (VT) 0) kj[e] = -1;
     }
 #pragma unroll
-    for(int f = 0; f < LIGHT_E; ++f)
+    for(int f = 0; f < E; ++f)
 #pragma unroll
-        for(int e = 0; e < LIGHT_E; ++e)
+        for(int e = 0; e < E; ++e)
             if(kj[f] >= 0 && (ki[e] >> 5) == (kj[f] >> 5)) {
                 const int el = 32 * (ki[e] & 31) + (kj[f] & 31);
                 const VT lt = dd[f] * vi[e];
@@ -1417,7 +1438,7 @@ __device__ __forceinline__ bool light_pair(const Dep& di, const Dep& dj, int hgt
 }
 
 template<typename VT>
-__device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr, int q,
+__device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr, int q,
     OffLdsSmall<VT>& s)
 {
     const int lane = lane_id();
@@ -1436,6 +1457,7 @@ __device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr,
     const double d_row = a.tri[3 * (int64_t) (fr + min(lane, hgt - 1)) + 1];
     tile_load(s.X, t1, hgt, wid, a.ix_in, a.val_in);
     bool staging = false;   // s.A is zero
+    const RowOf height(hgt), width(wid);
 
     // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order
     for(int e0 = 0; e0 < np; e0 += 64) {
@@ -1449,7 +1471,8 @@ __device__ void offdiag_small_one(const FactorArgs<VT>& a, const LevelRange& lr,
             if(hit) {
                 mi = dep_meta(a.bout, pr.x, pr.z, pr.w);
                 mj = dep_meta(a.bout, pr.y, pr.z, pr.w);
-                light = light_pair(mi, mj, hgt, wid, a.ix_out, a.val_out, a.tri, up);
+                light = light_pair<VT, LIGHT_E>(mi, mj, height, width, a.ix_out, a.val_out, a.tri,
+                    up);
             }
         }
         if(wave_ballot(hit && !light && !small_sparse<VT>(mj))) {
@@ -1577,18 +1600,18 @@ __device__ __forceinline__ void offdiag_body(const FactorArgs<VT>& a, const Leve
 // One lane per off-diagonal block for small blocks (at level-0 fill of the
 // KKT workloads: 1-2 entries each; a wave then works on 64 blocks instead of
 // one). Static eligibility (task bit, set by the host): sparse input with at
-// most TINY_E entries, at most 8 Schur pairs (16 at a level with 8192 or
+// most LIGHT_E entries, at most 8 Schur pairs (16 at a level with 8192 or
 // more off-diagonal blocks), 1x1 pivots in the block row.
-// At run time every dependency must be sparse with at most TINY_E entries
-// and the tile must stay within TINY_T nonzeros; otherwise the position goes
-// to the wave form before anything is written. The tile is a list of (row * 32 + col, value) in LDS,
-// one column of the list arrays per lane; every value is formed by the same
-// operations in the same order as in the wave form (terms that are exact
-// zeros in the wave form are skipped).
-constexpr int TINY_E = LIGHT_E;
+// At run time every matching pair must be within light_pair's form and the
+// tile must stay within TINY_P nonzeros (TINY_T while it is scaled);
+// otherwise the position goes to the wave form before anything is written.
+// The tile is a list of (row * 32 + col, value) in LDS, one column of the
+// list arrays per lane; every value is formed by the same operations in the
+// same order as in the wave form (terms that are exact zeros there are
+// skipped).
 constexpr int TINY_T = 16;
 constexpr int TINY_P = 12;  // the same while its Schur updates are added up
-constexpr int TINY_F = 4;   // pairs whose row masks are fetched together
+constexpr int TINY_F = 6;   // pairs whose row masks are fetched together
 
 template<typename VT, int CAP, int TPB>
 struct TinyLds {
@@ -1602,60 +1625,13 @@ __device__ __forceinline__ void to_wave_form(const FactorArgs<VT>& a, const Leve
     a.wave_list[atomicAdd(a.wave_cnt + lr.level, 1)] = q;
 }
 
-// metadata of the two factored blocks of one Schur pair, as far as the
-// one-lane form needs it; ok = both are sparse with at most TINY_E entries
-struct TinyMeta {
-    bool ok;
-    int nnz_i, cp_i, vp_i, nnz_j, cp_j, vp_j;
-};
-
-__device__ __forceinline__ TinyMeta tiny_meta(const BlockMeta* bout, int4 pp)
-{
-    TinyMeta t;
-    const BlockMeta mi = bout[pp.x], mj = bout[pp.y];
-    t.ok = mi.format == FMT_SPARSE && mi.nnz <= TINY_E && mj.format == FMT_SPARSE &&
-        mj.nnz <= TINY_E;
-    t.nnz_i = mi.nnz;
-    t.cp_i = mi.col_ptr;
-    t.vp_i = mi.val_ptr;
-    t.nnz_j = mj.nnz;
-    t.cp_j = mj.col_ptr;
-    t.vp_j = mj.val_ptr;
-    return t;
-}
-
-// the stored entries of both blocks (nothing for a pair outside the form)
-template<typename VT>
-struct TinyRaw {
-    int ixi[TINY_E], ixj[TINY_E];
-    VT vi[TINY_E], vj[TINY_E];
-};
-
-template<typename VT>
-__device__ __forceinline__ void tiny_raw(const int32_t* ix_out, const VT* val_out,
-    const TinyMeta& m, TinyRaw<VT>& r)
-{
-#pragma unroll
-    for(int e = 0; e < TINY_E; ++e) {
-        r.ixi[e] = 0; r.vi[e] = 0; r.ixj[e] = 0; r.vj[e] = 0;
-        if(m.ok && e < m.nnz_i) {
-            r.ixi[e] = ix_out[(int64_t) m.cp_i + e];
-            r.vi[e] = val_out[(int64_t) m.vp_i + e];
-        }
-        if(m.ok && e < m.nnz_j) {
-            r.ixj[e] = ix_out[(int64_t) m.cp_j + e];
-            r.vj[e] = val_out[(int64_t) m.vp_j + e];
-        }
-    }
-}
-
 // One-lane form, first phase: the Schur updates of the off-diagonal block at
 // level position q (thread tid of its workgroup), which read only blocks of
 // earlier levels and so run beside the level's pivot blocks. The tile list
 // is parked in the position's compact store (if_idx / if_val, count in
 // if_cnt); if_cnt[q] = -1 marks a position left to the other kernels.
 template<typename VT, int TPB>
-__device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
+__device__ __forceinline__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
     const int tid, TinyLds<VT, TINY_P, TPB>& s)
 {
     if(q >= lr.size) return;
@@ -1678,173 +1654,80 @@ __device__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, co
             if(I(k) == idx) return k;
         return -1;
     };
-    // input entries
-    for(int e = 0; e < t1.y; ++e) {
-        const int ix = a.ix_in[(int64_t) t1.z + e];
-        const int r = ix / wid, c = ix - r * wid;
-        I(n) = (int16_t) (32 * r + c);
-        V(n) = a.val_in[(int64_t) t1.w + e];
-        ++n;
+    const RowOf height(hgt), width(wid);
+    // the first pairs' records beside the input entries
+    int4 rec[TINY_F];
+    auto records = [&](int p0) {
+#pragma unroll
+        for(int u = 0; u < TINY_F; ++u) rec[u] = pairs[min(p0 + u, np - 1)];
+    };
+    if(np > 0) records(0);
+    n = t1.y;
+    for(int e0 = 0; e0 < n; e0 += 4) {
+        int ix[4];
+        VT v[4];
+#pragma unroll
+        for(int u = 0; u < 4; ++u) {
+            const int e = min(e0 + u, n - 1);
+            ix[u] = a.ix_in[(int64_t) t1.z + e];
+            v[u] = a.val_in[(int64_t) t1.w + e];
+        }
+#pragma unroll
+        for(int u = 0; u < 4; ++u)
+            if(e0 + u < n) {
+                I(e0 + u) = (int16_t) width.at(ix[u]);
+                V(e0 + u) = v[u];
+            }
     }
     // A_ij -= U_ki' D_k U_kj over the Schur pairs, in order: the row masks
     // of TINY_F pairs are fetched together, and of the pairs that match (few)
-    // the metadata, entries and D are read one pair after the other
+    // the metadata, entries and D are read one pair after the other. A pair
+    // outside light_pair's form leaves the block to the one-wave form.
     for(int p0 = 0; p0 < np; p0 += TINY_F) {
+        if(p0) records(p0);
         uint32_t hits = 0;
         {
-            int2 pr[TINY_F];
             uint32_t mi[TINY_F], mj[TINY_F];
 #pragma unroll
             for(int u = 0; u < TINY_F; ++u) {
-                const int4 r = pairs[min(p0 + u, np - 1)];
-                pr[u] = make_int2(r.x, r.y);
-            }
-#pragma unroll
-            for(int u = 0; u < TINY_F; ++u) {
-                mi[u] = a.row_mask[pr[u].x];
-                mj[u] = a.row_mask[pr[u].y];
+                mi[u] = a.row_mask[rec[u].x];
+                mj[u] = a.row_mask[rec[u].y];
             }
 #pragma unroll
             for(int u = 0; u < TINY_F; ++u)
                 if(p0 + u < np && pair_matches(mi[u], mj[u])) hits |= 1u << u;
         }
         for(; hits; hits &= hits - 1) {
-            const int4 pc = pairs[p0 + __ffs(hits) - 1];
-            const TinyMeta mc = tiny_meta(a.bout, pc);
-            if(!mc.ok) {
+            const int at = __ffs(hits) - 1;
+            int4 pc = rec[0];
+#pragma unroll
+            for(int u = 1; u < TINY_F; ++u)
+                if(u == at) pc = rec[u];
+            const Dep mi = dep_meta(a.bout, pc.x, pc.z, pc.w);
+            const Dep mj = dep_meta(a.bout, pc.y, pc.z, pc.w);
+            PairUpd<VT> up;
+            const bool ok = wave_ballot(mi.nnz > 2 || mj.nnz > 2) == 0ull
+                ? light_pair<VT, 2>(mi, mj, height, width, a.ix_out, a.val_out, a.tri, up)
+                : light_pair<VT, LIGHT_E>(mi, mj, height, width, a.ix_out, a.val_out, a.tri, up);
+            if(!ok) {
                 to_wave_form(a, lr, q);
                 return;
             }
-            TinyRaw<VT> rc;
-            tiny_raw(a.ix_out, a.val_out, mc, rc);
-            const int rb = pc.z;
-            // U_ki: rows l of block k, columns c (rows of block i), width hgt
-            int al[TINY_E], ac[TINY_E];
-            VT av[TINY_E];
-    #pragma unroll
-            for(int e = 0; e < TINY_E; ++e) {
-                al[e] = -4; ac[e] = -1; av[e] = 0;
-                if(e < mc.nnz_i) {
-                    const int ix = rc.ixi[e];
-                    al[e] = ix / hgt;
-                    ac[e] = ix - al[e] * hgt;
-                    av[e] = rc.vi[e];
-                }
-            }
-            // U_kj: rows l, columns j, width wid; nonzero entries by (column, row)
-            int rl[TINY_E], rj[TINY_E];
-            VT rv[TINY_E];
-    #pragma unroll
-            for(int e = 0; e < TINY_E; ++e) {
-                rl[e] = 0; rj[e] = 64; rv[e] = 0;
-                if(e < mc.nnz_j) {
-                    const int ix = rc.ixj[e];
-                    const VT v = rc.vj[e];
-                    if(v != (VT) 0) {
-                        rl[e] = ix / wid;
-                        rj[e] = ix - rl[e] * wid;
-                        rv[e] = v;
+#pragma unroll
+            for(int u = 0; u < LIGHT_OFF; ++u) {
+                if(u >= up.n) continue;
+                int k = find(up.el[u]);
+                if(k < 0) {
+                    if(up.v[u] == (VT) 0) continue;
+                    if(n == TINY_P) {
+                        to_wave_form(a, lr, q);
+                        return;
                     }
+                    k = n++;
+                    I(k) = (int16_t) up.el[u];
+                    V(k) = 0;
                 }
-            }
-            if(mc.nnz_i == 1 && mc.nnz_j == 1) {
-                // one entry on each side (nearly every pair at level-0 fill):
-                // the general form below reduces to one product for the single
-                // element (column of U_ki's entry, column of U_kj's entry), with
-                // the same operations
-                if(rj[0] < 64) {
-                    const int l = rl[0];
-                    const double* td = a.tri + 3 * (int64_t) (rb + l);
-                    const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
-                    const VT left = (al[0] == l - 1) ? av[0] : (VT) 0;
-                    const VT mid = (al[0] == l) ? av[0] : (VT) 0;
-                    const VT right = (al[0] == l + 1) ? av[0] : (VT) 0;
-                    const VT lt = fma(sub, right, fma(dia, mid, sup * left));
-                    const VT acc = fma(rv[0], lt, (VT) 0);
-                    const int idx = 32 * ac[0] + rj[0];
-                    int k = find(idx);
-                    if(k < 0) {
-                        if(acc == (VT) 0) continue;
-                        if(n == TINY_P) { to_wave_form(a, lr, q); return; }
-                        k = n++;
-                        I(k) = (int16_t) idx;
-                        V(k) = 0;
-                    }
-                    V(k) -= acc;
-                }
-                continue;
-            }
-            int key[TINY_E], rank[TINY_E];
-    #pragma unroll
-            for(int e = 0; e < TINY_E; ++e) key[e] = rj[e] * 32 + rl[e];
-    #pragma unroll
-            for(int e = 0; e < TINY_E; ++e) {
-                int rk = 0;
-    #pragma unroll
-                for(int f = 0; f < TINY_E; ++f) rk += (key[f] < key[e]) || (key[f] == key[e] && f < e);
-                rank[e] = rk;
-            }
-            // distinct columns of U_ki
-            int dc[TINY_E];
-    #pragma unroll
-            for(int e = 0; e < TINY_E; ++e) {
-                bool seen = ac[e] < 0;
-    #pragma unroll
-                for(int f = 0; f < e; ++f) seen = seen || (ac[f] == ac[e]);
-                dc[e] = -1;
-                if(!seen) dc[e] = ac[e];
-            }
-            // columns j in ascending order; within a column, rows ascending
-            VT acc[TINY_E];
-            int curj = -1;
-            for(int rk = 0; rk <= TINY_E; ++rk) {
-                int e = -1;
-    #pragma unroll
-                for(int f = 0; f < TINY_E; ++f)
-                    if(rank[f] == rk) e = f;
-                const int j = (rk < TINY_E && e >= 0) ? rj[e] : 64;
-                if(j != curj && curj >= 0 && curj < 64) {
-                    // column curj done: T[c][curj] -= acc[c]
-    #pragma unroll
-                    for(int f = 0; f < TINY_E; ++f) {
-                        if(dc[f] < 0) continue;
-                        const int idx = 32 * dc[f] + curj;
-                        int k = find(idx);
-                        if(k < 0) {
-                            if(acc[f] == (VT) 0) continue;
-                            if(n == TINY_P) { to_wave_form(a, lr, q); return; }
-                            k = n++;
-                            I(k) = (int16_t) idx;
-                            V(k) = 0;
-                        }
-                        V(k) -= acc[f];
-                    }
-                }
-                if(j >= 64) break;
-                if(j != curj) {
-                    curj = j;
-    #pragma unroll
-                    for(int f = 0; f < TINY_E; ++f) acc[f] = 0;
-                }
-                const int l = rl[e];
-                const VT r = rv[e];
-                const double* td = a.tri + 3 * (int64_t) (rb + l);
-                const VT sup = (VT) td[0], dia = (VT) td[1], sub = (VT) td[2];
-    #pragma unroll
-                for(int f = 0; f < TINY_E; ++f) {
-                    if(dc[f] < 0) continue;
-                    const int c = dc[f];
-                    VT left = 0, mid = 0, right = 0;
-    #pragma unroll
-                    for(int g = 0; g < TINY_E; ++g) {
-                        if(ac[g] != c) continue;
-                        if(al[g] == l - 1) left = av[g];
-                        if(al[g] == l) mid = av[g];
-                        if(al[g] == l + 1) right = av[g];
-                    }
-                    const VT lt = fma(sub, right, fma(dia, mid, sup * left));
-                    acc[f] = fma(r, lt, acc[f]);
-                }
+                V(k) -= up.v[u];
             }
         }
     }
@@ -2619,6 +2502,11 @@ __device__ __forceinline__ void store_body(const FactorArgs<VT>& a, const LevelR
 // its pivot block (earlier levels, final storage) take its pivoting order in
 // their columns: sparse entries get new column indices in place, dense rows
 // are gathered column by column.
+// waves per SIMD the pivot, pair and one-wave off-diagonal kernels are compiled
+// for: as many as their registers allow with few spills
+template<typename VT>
+constexpr int PP_WAVES = sizeof(VT) == 4 ? 3 : 2;
+
 // the single-system kernels: the bodies at their own grid position
 template<typename VT>
 __global__ __launch_bounds__(64) void k_offdiag_general(FactorArgs<VT> a, LevelRange lr)
@@ -2627,7 +2515,7 @@ __global__ __launch_bounds__(64) void k_offdiag_general(FactorArgs<VT> a, LevelR
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64, 3) void k_offdiag(FactorArgs<VT> a, LevelRange lr)
+__global__ __launch_bounds__(64, PP_WAVES<VT>) void k_offdiag(FactorArgs<VT> a, LevelRange lr)
 {
     offdiag_body<VT>(a, lr, blockIdx.x, gridDim.x);
 }
@@ -2637,11 +2525,6 @@ __global__ __launch_bounds__(TINY_TPB) void k_offdiag_tiny_scale(FactorArgs<VT> 
 {
     offdiag_tiny_scale_body<VT>(a, lr, blockIdx.x);
 }
-
-// waves per SIMD the pivot and pair launch is compiled for: as many as its
-// registers allow without spills
-template<typename VT>
-constexpr int PP_WAVES = sizeof(VT) == 4 ? 3 : 2;
 
 template<typename VT, int NW>
 __global__ __launch_bounds__(64 * NW, PP_WAVES<VT>) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
@@ -2772,7 +2655,7 @@ __global__ __launch_bounds__(TINY_TPB) void bk_offdiag_tiny_scale(const FactorSy
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64, 3) void bk_offdiag(const FactorSys<VT>* fs, const int2* items,
+__global__ __launch_bounds__(64, PP_WAVES<VT>) void bk_offdiag(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
     const int2 it = items[blockIdx.x];
