@@ -571,44 +571,156 @@ __device__ __forceinline__ bool published(double v)
     return (unsigned long long) __double_as_longlong(v) != CHAIN_EMPTY;
 }
 
-// waits until every lane's value xv[k] (column c[k]) is published; rdy[k]
-// on entry: xv[k] already usable
-__device__ void wait_published(const double* pub, const int (&c)[TRSV_PF], double (&xv)[TRSV_PF],
-    bool (&rdy)[TRSV_PF], int32_t* err, int& spins)
-{
-    bool all = true;
-#pragma unroll
-    for(int k = 0; k < TRSV_PF; ++k) all = all && rdy[k];
-    while(wave_ballot(!all)) {
-        __builtin_amdgcn_s_sleep(1);
-        if(++spins > SPIN_LIMIT) {
-            // err is pinned host memory: the host reads it without a copy
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            return;
-        }
-        all = true;
-#pragma unroll
-        for(int k = 0; k < TRSV_PF; ++k) {
-            if(!rdy[k]) {
-                xv[k] = pub_load(pub + c[k]);
-                rdy[k] = published(xv[k]);
-            }
-            all = all && rdy[k];
-        }
-    }
-}
-
-// what a block row loads before it can wait: its first TRSV_PF chunks of
-// off-diagonal entries (clamped in range), its own right-hand side and the
-// first 64 entries of U_ii^-1
+// One group of up to TRSV_PF 64-entry chunks of a block row's off-diagonal
+// entries: columns, values and local rows (64: no entry).
 template<typename VT>
-struct ChainHead {
+struct ChainGroup {
     int c[TRSV_PF], sg[TRSV_PF];
     VT v[TRSV_PF];
+};
+
+// what a block row loads before it can wait: its first group (clamped in
+// range), its own right-hand side and the first 64 entries of U_ii^-1
+template<typename VT>
+struct ChainHead {
+    ChainGroup<VT> g;
     double bo;
     int ic, il;
     VT iv;
 };
+
+// The segmented sums over a chunk as far as they follow from its local rows
+// alone, formed while the x values are on their way: how many lanes of this
+// lane's 16-lane row before it belong to its segment, whether the segment
+// reaches into the rows before (scan steps over lanes 15 and 31), and on lane
+// r < 32 the lane that ends row r's segment (-1: no entry of the row).
+struct ScanPlan {
+    int dist;
+    bool cross15, cross31;
+    int end;
+};
+
+__device__ __forceinline__ ScanPlan scan_plan(int sg, int8_t* ends)
+{
+    const int lane = lane_id();
+    ScanPlan p;
+    const int before = dpp_move<0x138, 0xf>(-1, sg);   // every lane active
+    const uint64_t heads = wave_ballot(before != sg) | 1ull;
+    // the first lane of this lane's segment
+    const int start = 63 - __clzll((long long) (heads & (~0ull >> (63 - lane))));
+    p.dist = min(lane - start, lane & 15);
+    p.cross15 = (lane & 16) != 0 && start < (lane & ~15);
+    p.cross31 = lane >= 32 && start < 32;
+    const int nsg = next_lane(sg, -1);
+    wave_sync();
+    if(lane < 32) ends[lane] = -1;
+    wave_sync();
+    if(sg < 64 && (lane == 63 || nsg != sg)) ends[sg] = (int8_t) lane;
+    wave_sync();
+    p.end = ends[lane & 31];
+    return p;
+}
+
+// a lane move whose result is used only where the lane has a source
+template<int CTRL, int ROW_MASK>
+__device__ __forceinline__ double dpp_take(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, CTRL, ROW_MASK, 0xf, false),
+        __builtin_amdgcn_mov_dpp(lo, CTRL, ROW_MASK, 0xf, false));
+}
+
+// seg_scan_runs_fma(a, x, .) with the plan of its local rows: the same tree
+// and roundings
+__device__ __forceinline__ double planned_scan(double a, double x, const ScanPlan& p)
+{
+    double v = a * x;
+    const double f = fma(a, x, dpp_take<0x111, 0xf>(v));
+    v = p.dist >= 1 ? f : v;
+    double s = v + dpp_take<0x112, 0xf>(v);
+    v = p.dist >= 2 ? s : v;
+    s = v + dpp_take<0x114, 0xf>(v);
+    v = p.dist >= 4 ? s : v;
+    s = v + dpp_take<0x118, 0xf>(v);
+    v = p.dist >= 8 ? s : v;
+    s = v + dpp_take<0x142, 0xa>(v);
+    v = p.cross15 ? s : v;
+    s = v + dpp_take<0x143, 0xc>(v);
+    return p.cross31 ? s : v;
+}
+
+// Reloads the x values of the lanes set in m[k], all in one round trip. One
+// block with its own wait: written as loads under conditions, the compiler
+// waits for each before it issues the next.
+__device__ __forceinline__ void reload_missing(const double* pub, const int (&c)[TRSV_PF],
+    const uint64_t (&m)[TRSV_PF], double (&xv)[TRSV_PF])
+{
+    static_assert(TRSV_PF == 4, "four chunks");
+    const double* p0 = pub + c[0];
+    const double* p1 = pub + c[1];
+    const double* p2 = pub + c[2];
+    const double* p3 = pub + c[3];
+    uint64_t saved;
+    asm volatile("s_mov_b64 %[sv], exec\n\t"
+                 "s_mov_b64 exec, %[m0]\n\t"
+                 "global_load_dwordx2 %[x0], %[p0], off sc1\n\t"
+                 "s_mov_b64 exec, %[m1]\n\t"
+                 "global_load_dwordx2 %[x1], %[p1], off sc1\n\t"
+                 "s_mov_b64 exec, %[m2]\n\t"
+                 "global_load_dwordx2 %[x2], %[p2], off sc1\n\t"
+                 "s_mov_b64 exec, %[m3]\n\t"
+                 "global_load_dwordx2 %[x3], %[p3], off sc1\n\t"
+                 "s_mov_b64 exec, %[sv]\n\t"
+                 "s_waitcnt vmcnt(0)"
+                 : [x0] "+&v"(xv[0]), [x1] "+&v"(xv[1]), [x2] "+&v"(xv[2]), [x3] "+&v"(xv[3]),
+                 [sv] "=&s"(saved)
+                 : [m0] "s"(m[0]), [m1] "s"(m[1]), [m2] "s"(m[2]), [m3] "s"(m[3]), [p0] "v"(p0),
+                 [p1] "v"(p1), [p2] "v"(p2), [p3] "v"(p3)
+                 : "memory");
+}
+
+// y (lane r: row r) minus the row sums of a group, chunk after chunk. A
+// chunk is scanned as soon as its values are there, while the others are
+// still on their way: the latest values of a block row all belong to the
+// levels next to its own, so they sit in one chunk (the last for U', the first
+// for U) and only that chunk's scan follows the last arrival. chunks: how many
+// of the group have entries; their values past the row's end are cleared.
+template<typename VT>
+__device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup<VT>& g,
+    double (&xv)[TRSV_PF], const ScanPlan (&p)[TRSV_PF], int chunks, double y, int32_t* err,
+    int& spins)
+{
+    double sum[TRSV_PF];
+    uint32_t open = chunks >= TRSV_PF ? (1u << TRSV_PF) - 1 : (1u << chunks) - 1;
+    for(;;) {
+        uint64_t m[TRSV_PF];
+#pragma unroll
+        for(int k = 0; k < TRSV_PF; ++k) {
+            m[k] = 0;
+            if((open >> k) & 1u) {
+                m[k] = wave_ballot(g.sg[k] < 64 && !published(xv[k]));
+                if(m[k] == 0) {
+                    const double v = planned_scan((double) g.v[k], g.sg[k] < 64 ? xv[k] : 0.0,
+                        p[k]);
+                    sum[k] = __shfl(v, max(p[k].end, 0), WAVE);
+                    open &= ~(1u << k);
+                }
+            }
+        }
+        if(open == 0) break;
+        if(++spins > SPIN_LIMIT) {
+            // err is pinned host memory: the host reads it without a copy
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            return y;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        reload_missing(pub, g.c, m, xv);
+    }
+#pragma unroll
+    for(int k = 0; k < TRSV_PF; ++k)
+        if(k < chunks) y = p[k].end >= 0 ? y - sum[k] : y;
+    return y;
+}
 
 // The right-hand side of one block row as K src (rows fr .. fr + h - 1 of a
 // CSR matrix), formed exactly as k_csr_spmv forms those rows: eight lanes
@@ -678,19 +790,26 @@ __device__ double block_rhs(const CsrRhs& k, int fr, int h)
 }
 
 template<typename VT>
+__device__ __forceinline__ void chain_group(int e0, int oe, const int32_t* o_col, const VT* o_val,
+    const uint8_t* o_lr, ChainGroup<VT>& g)
+{
+#pragma unroll
+    for(int k = 0; k < TRSV_PF; ++k) {
+        const int e = max(min(e0 + 64 * k + lane_id(), oe - 1), 0);
+        g.c[k] = o_col[e];
+        g.v[k] = o_val[e];
+        g.sg[k] = o_lr[e];
+    }
+}
+
+template<typename VT>
 __device__ __forceinline__ void chain_fetch(int4 t0, int4 t1, const int32_t* o_col, const VT* o_val,
     const uint8_t* o_lr, const int32_t* i_col, const VT* i_val, const uint8_t* i_lr,
     const double* x, bool rhs_fused, ChainHead<VT>& f)
 {
     const int lane = lane_id();
-    const int fr = t0.x, h = t0.y, ob = t0.z, oe = t0.w, ib = t1.x, ie = t1.y;
-#pragma unroll
-    for(int k = 0; k < TRSV_PF; ++k) {
-        const int e = max(min(ob + 64 * k + lane, oe - 1), 0);
-        f.c[k] = o_col[e];
-        f.v[k] = o_val[e];
-        f.sg[k] = o_lr[e];
-    }
+    const int fr = t0.x, h = t0.y, ib = t1.x, ie = t1.y;
+    chain_group<VT>(t0.z, t0.w, o_col, o_val, o_lr, f.g);
     // this block row's own right-hand side: no other wave writes x (with a
     // fused product it is formed after the current block row instead)
     f.bo = rhs_fused ? 0.0 : x[fr + min(lane, h - 1)];
@@ -700,14 +819,25 @@ __device__ __forceinline__ void chain_fetch(int4 t0, int4 t1, const int32_t* o_c
     f.il = i_lr[ei];
 }
 
+// Between the arrival of a block row's last x value and the store of its
+// results lies the part of every level that no other wave hides. All that
+// does not depend on x is done before (ScanPlan), the chunks that are complete
+// are summed while the last one is awaited, rows are summed by lane reads
+// instead of LDS updates, and U_ii^-1 of up to 64 entries stays in registers.
+// Measured (publish to arrival / arrival to publish, per level, n = 400,000):
+// 0.9-1.1 us / 0.5-0.6 us; a lone pair of waves on two XCDs exchanges a value
+// in 0.4-0.5 us. U, D and U' solve together 251 -> 219 us at n = 400,000,
+// 124 -> 112 us at n = 2,000. Reading values from block rows over 2,048 rows
+// back through the caches instead was slower (257 us).
 template<typename VT, bool FUSED>
-__global__ __launch_bounds__(64) void k_trsv_chain(const int4* task, int32_t nb, int32_t reverse,
+__global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t nb, int32_t reverse,
     const int32_t* o_col, const VT* o_val, const uint8_t* o_lr, const int32_t* i_col,
     const VT* i_val, const uint8_t* i_lr, double* pub, double* next_pub, int32_t* err, double* x,
     CsrRhs rhs)
 {
-    __shared__ double y[33];     // FP64 accumulation for both factor precisions
+    __shared__ double y_lds[33];     // general U_ii^-1 only
     __shared__ double res[33];
+    __shared__ int8_t ends[32];
     const int lane = lane_id();
     const int G = gridDim.x;
     constexpr bool fused = FUSED;
@@ -728,57 +858,69 @@ __global__ __launch_bounds__(64) void k_trsv_chain(const int4* task, int32_t nb,
     for(;;) {
         int4 n0, n1;
         task_at(w + G, n0, n1);
-        ChainHead<VT> nxt;
-        bool fetched = false;
+        ChainHead<VT> nxt = cur;
         const int fr = t0.x, h = t0.y, ob = t0.z, oe = t0.w, ib = t1.x, ie = t1.y;
         if(lane < h) next_pub[fr + lane] = empty;
-        wave_sync();
-        if(lane < h) { y[lane] = cur.bo; res[lane] = 0; }
-        for(int e0 = ob; e0 < oe; e0 += 64 * TRSV_PF) {
-            int c[TRSV_PF], sg[TRSV_PF];
-            VT v[TRSV_PF];
-            if(e0 == ob) {
+        // U_ii^-1: diagonal (one entry per row, on the diagonal), or up to 64
+        // entries taken by one planned scan, or in chunks of 64
+        const bool diagonal = ie - ib == h &&
+            wave_ballot(lane < h && (cur.il != lane || cur.ic != fr + lane)) == 0;
+        const bool one_chunk = ie - ib <= 64;
+        const bool last = w + G >= nb;
+        double y = cur.bo;
+        ScanPlan ip;
+        if(!diagonal && one_chunk) ip = scan_plan(ib + lane < ie ? cur.il : 64, ends);
+        if(ob < oe) {
+            ChainGroup<VT> g = cur.g;
+            for(int e0 = ob;;) {
+                double xv[TRSV_PF];
+                ScanPlan plan[TRSV_PF];
 #pragma unroll
-                for(int k = 0; k < TRSV_PF; ++k) { c[k] = cur.c[k]; v[k] = cur.v[k]; sg[k] = cur.sg[k]; }
-            } else {
+                for(int k = 0; k < TRSV_PF; ++k) xv[k] = pub_load(pub + g.c[k]);
 #pragma unroll
                 for(int k = 0; k < TRSV_PF; ++k) {
-                    const int e = min(e0 + 64 * k + lane, oe - 1);
-                    c[k] = o_col[e];
-                    v[k] = o_val[e];
-                    sg[k] = o_lr[e];
+                    const bool in = e0 + 64 * k + lane < oe;
+                    g.v[k] = in ? g.v[k] : (VT) 0;
+                    g.sg[k] = in ? g.sg[k] : 64;
                 }
+                // the next loads go out here: they are younger than the reads
+                // above, so a row whose values are all there does not wait
+                // for them
+                ChainGroup<VT> gn;
+                const bool more = e0 + 64 * TRSV_PF < oe;
+                if(more)
+                    chain_group<VT>(e0 + 64 * TRSV_PF, oe, o_col, o_val, o_lr, gn);
+                else if(!last)
+                    chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
+                const int chunks = (oe - e0 + 63) / 64;
+                plan[0] = scan_plan(g.sg[0], ends);
+                if(chunks > 1) plan[1] = scan_plan(g.sg[1], ends);
+                if(chunks > 2) plan[2] = scan_plan(g.sg[2], ends);
+                if(chunks > 3) plan[3] = scan_plan(g.sg[3], ends);
+                y = chain_sums<VT>(pub, g, xv, plan, chunks, y, err, spins);
+                if(!more) break;
+                e0 += 64 * TRSV_PF;
+                g = gn;
             }
-            double xv[TRSV_PF];
-            bool rdy[TRSV_PF];
-#pragma unroll
-            for(int k = 0; k < TRSV_PF; ++k) xv[k] = pub_load(pub + c[k]);
-#pragma unroll
-            for(int k = 0; k < TRSV_PF; ++k) {
-                const bool in = e0 + 64 * k + lane < oe;
-                v[k] = in ? v[k] : (VT) 0;
-                sg[k] = in ? sg[k] : 64;
-                rdy[k] = !in || published(xv[k]);
-            }
-            wait_published(pub, c, xv, rdy, err, spins);
-            if(!fetched) {
-                chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
-                fetched = true;
-            }
-            wave_sync();
-#pragma unroll
-            for(int k = 0; k < TRSV_PF; ++k) {
-                if(e0 + 64 * k >= oe) break;
-                double p = seg_scan_runs_fma((double) v[k], sg[k] < 64 ? xv[k] : 0.0, sg[k]);
-                const int nsg = next_lane(sg[k], -1);
-                if(sg[k] < 64 && (lane == 63 || nsg != sg[k])) y[sg[k]] -= p;
-                wave_sync();
-            }
+        } else if(!last) {
+            chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
         }
-        if(!fetched) chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
-        wave_sync();
-        const double r = apply_inverse<VT>(fr, h, ib, ie, cur.ic, cur.iv, cur.il, i_col, i_val, i_lr, y,
-            res);
+        double r;
+        if(diagonal) {
+            r = fma((double) cur.iv, y, 0.0);
+        } else if(one_chunk) {
+            const bool in = ib + lane < ie;
+            const double yy = __shfl(y, in ? cur.ic - fr : 0, WAVE);
+            const double v = planned_scan(in ? (double) cur.iv : 0.0, yy, ip);
+            r = 0.0 + __shfl(v, max(ip.end, 0), WAVE);
+            r = ip.end >= 0 ? r : 0.0;
+        } else {
+            wave_sync();
+            if(lane < h) { y_lds[lane] = y; res[lane] = 0; }
+            wave_sync();
+            r = apply_inverse<VT>(fr, h, ib, ie, cur.ic, cur.iv, cur.il, i_col, i_val, i_lr, y_lds,
+                res);
+        }
         if(lane < h) {
             __hip_atomic_store(pub + fr + lane, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             x[fr + lane] = r;
@@ -1131,9 +1273,11 @@ template void solve_plan_count<float>(const SolveTopo&, const float*, float*, So
 template void solve_plan_fill<double>(const SolveTopo&, const double*, const double*, SolvePlan<double>&, void*);
 template void solve_plan_fill<float>(const SolveTopo&, const float*, const float*, SolvePlan<float>&, void*);
 // Waves of k_trsv_chain per CU. A solve needs all of its waves resident.
-// The kernel's registers let a CU hold 16 of its waves, so with 4 per CU
-// TRSV_SINGLE_MAX_CONCURRENT = 4 such solves fit on the GPU at the same
-// time; other kernels end on their own.
+// TRSV_SINGLE_MAX_CONCURRENT = 4 such solves have to fit on the GPU at the
+// same time (other kernels end on their own), so at most a quarter of what a
+// CU holds: its registers let a CU hold 12 of this kernel's waves, three per
+// solve. (Compiled for 16 per CU, it spills 18-25 registers inside the rows'
+// critical path: 430 us instead of 236 for both solves at n = 400,000.)
 constexpr int CHAIN_WAVES_PER_CU = 4;
 
 // grid of k_trsv_chain: CHAIN_WAVES_PER_CU waves per CU, fewer when the
