@@ -140,9 +140,13 @@ __device__ inline double* batch_vec(const BatchSys& s, int32_t id)
 void batch_expand(const int4* ent, int32_t count, int2* items, int32_t interleaved_total,
     hipStream_t st);
 
-// the steps of the recurrence (sqmr.hip)
+// the steps of the recurrence (sqmr.hip), a: iterations launched since the
+// systems' counters last moved (BS_SCALARS moves them past its own)
 enum BatchStep : int32_t {
     BS_ALPHA, BS_VNEXT, BS_VSCALE, BS_BETA, BS_PUPDATE, BS_SCALARS,
+    BS_DOTS,          // beta, and alpha of the next iteration
+    BS_PV,            // pupdate, and vnext of the next iteration
+    BS_SV,            // scalars, and vscale of the next iteration
     BS_INIT_FILL,     // the run's vectors to zero
     BS_SUMSQ,         // part slot 6 = ||a||^2
     BS_INIT_V, BS_INIT_W,

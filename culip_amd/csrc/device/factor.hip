@@ -543,7 +543,6 @@ __device__ void dense_pivot_op(VT* T, int32_t* perm, int len, int pa, int pb)
 // is widened by one row each way), and a non-finite entry or D makes the
 // products of unmatched rows NaN (the mask ALL_ROWS matches every block).
 constexpr uint32_t ALL_ROWS = 0xffffffffu;
-constexpr int32_t ROW_2X2 = 1, ROW_NONFINITE = 2;
 
 template<typename T>
 __device__ __forceinline__ bool finite_value(T v) { return fabs(v) < (T) INFINITY; }
@@ -998,7 +997,6 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
             s.plain = plain;
             s.tiny = tiny;
             s.rflag = rflag;
-            a.row_flag[i] = rflag;
         }
     }
     __syncthreads();
@@ -1041,6 +1039,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
         }
         if(lane == 0) {
             a.piv_flag[q] = flags;
+            a.row_flag[i] = s.rflag | ((flags & PIV_ANY) ? ROW_COUPLED : 0);
             a.piv_loc[i] = q;
         }
     }

@@ -59,8 +59,7 @@ struct FactorArgs {
     uint8_t* overflow = nullptr;
     int32_t* piv_loc = nullptr;           // nb
     // rows of each factored off-diagonal block that can contribute to a
-    // Schur product (store_row_mask), and per block row what its pivots add
-    // to that (ROW_2X2, ROW_NONFINITE)
+    // Schur product (store_row_mask), and per block row ROW_2X2, ...
     uint32_t* row_mask = nullptr;         // per coarse block
     int32_t* row_flag = nullptr;          // nb
     // static, in level-list order: {capacity of a sparse block (max_nnz >= 0)
@@ -107,6 +106,10 @@ struct FactorArgs {
 };
 
 constexpr int LIST_C = 4;
+// row_flag: what a block row's pivot block left (a 2x2 pivot, a non-finite D,
+// an entry of U_ii right of its diagonal; with none of them U_ii is the
+// identity)
+constexpr int32_t ROW_2X2 = 1, ROW_NONFINITE = 2, ROW_COUPLED = 4;
 // A row group is one workgroup's share of a level's dropping step: block
 // rows that follow each other, at most GROUP_ROWS fine rows, and at most
 // GROUP_BLOCKS off-diagonal blocks unless one block row has more.

@@ -25,41 +25,34 @@ namespace culip {
 namespace {
 
 // columns of U_ii^-1 by back substitution, in double; X[r][c] at X[hm r + c]
-// (hm x hm LDS, hm >= h: the largest block height of the launch)
+// (hm x hm LDS, hm >= h: the largest block height of the launch). Lane c forms
+// column c. U's rows come in with one round of loads, and only their nonzero
+// entries are visited, ascending (the others would add exact zeros).
 template<typename VT>
 __device__ void diag_inverse(const VT* U, int h, double* X, int hm)
 {
     const int c = lane_id();
-    // a tile with no entry right of its diagonal (most pivot blocks of a
-    // sparse pattern) has the diagonal inverse: the back substitution below
-    // would only add exact zeros to it
-    bool offd = false;
-    if(c < h)
-        for(int k = c + 1; k < h; ++k) offd = offd || (U[c * h + k] != (VT) 0);
-    if(wave_ballot(offd) == 0) {
-        for(int e = c; e < hm * hm; e += 64) {
-            const int r = e / hm, q = e - r * hm;
-            X[e] = (r == q && r < h) ? 1.0 / (double) U[r * h + r] : 0.0;
-        }
-        wave_sync();
-        return;
-    }
-    for(int r = hm - 1; r >= 0; --r) {
-        if(c < hm) {
-            double v = 0.0;
-            if(c < h && r < h && r <= c) {
-                if(r == c) {
-                    v = 1.0 / (double) U[r * h + r];
-                } else {
-                    double s = 0.0;
-                    for(int k = r + 1; k <= c; ++k) s = fma((double) U[r * h + k], X[hm * k + c], s);
-                    v = -s / (double) U[r * h + r];
-                }
+    VT u[32];   // U's column c
+#pragma unroll
+    for(int r = 0; r < 32; ++r) u[r] = (r < h && c < h) ? U[r * h + c] : (VT) 0;
+#pragma unroll
+    for(int r = 31; r >= 0; --r) {
+        if(r < hm) {
+            const double d = (double) wave_bcast(u[r], r);
+            double s = 0.0;
+            for(uint64_t m = wave_ballot(c > r && u[r] != (VT) 0); m; m &= m - 1) {
+                const int k = __ffsll((long long) m) - 1;
+                const double uk = (double) wave_bcast(u[r], k);
+                if(k <= c && c < hm) s = fma(uk, X[hm * k + c], s);
             }
-            X[hm * r + c] = v;
+            if(c < hm) {
+                double v = 0.0;
+                if(c < h && r < h && r <= c) v = (r == c) ? 1.0 / d : -s / d;
+                X[hm * r + c] = v;
+            }
+            wave_sync();
         }
     }
-    wave_sync();
 }
 
 // up to 64 factored blocks staged one per lane: metadata, and the entries
@@ -128,41 +121,64 @@ __device__ __forceinline__ void plan_rank(const PlanStage<VT>& sg, int nblk, int
     }
 }
 
-// X: hm x hm doubles of LDS (the launch's dynamic LDS), hm >= every block
-// height of the launch
+// LDS of a plan_rows workgroup: the pivot block's inverse (hm x hm doubles, hm
+// >= every block height of the launch), then the staged blocks in its place
+template<typename VT>
+inline size_t plan_rows_lds(int hm)
+{
+    const size_t x = sizeof(double) * (size_t) hm * (size_t) hm;
+    return x > sizeof(PlanStage<VT>) ? x : sizeof(PlanStage<VT>);
+}
+
 template<typename VT, bool FILL>
 __device__ __forceinline__ void plan_rows_body(const SolveTopo& t, const VT* val_out,
-    const SolvePlan<VT>& p, int bid_, double* X, int hm)
+    const SolvePlan<VT>& p, int bid_, void* lds, int hm)
 {
     const int lane = lane_id();
     const int i = bid_;
     const int fr = t.bs[i];
     const int h = t.bs[i + 1] - fr;
     // pivot block inverse rows (ui) and columns (ti)
-    const BlockMeta dm = t.bout[t.csr_off[i]];
-    diag_inverse(val_out + dm.val_ptr, h, X, hm);
-    if(lane < h) {
-        int cr = 0, cc = 0;
-        int32_t wr = 0, wc = 0;
-        if(FILL) { wr = p.ui_ptr[fr + lane]; wc = p.ti_ptr[fr + lane]; }
-        for(int c = 0; c < h; ++c) {
-            const double v = X[hm * lane + c];  // row lane of U^-1
-            if(v != 0.0) {
-                if(FILL) { p.ui_col[wr + cr] = fr + c; p.ui_val[wr + cr] = (VT) v; p.ui_lr[wr + cr] = (uint8_t) lane; }
-                ++cr;
-            }
-            const double u = X[hm * c + lane];  // column lane of U^-1
-            if(u != 0.0) {
-                if(FILL) { p.ti_col[wc + cc] = fr + c; p.ti_val[wc + cc] = (VT) u; p.ti_lr[wc + cc] = (uint8_t) lane; }
-                ++cc;
+    if(t.row_flag[i] == 0) {
+        // U_ii is the identity (most pivot blocks of a sparse pattern): its
+        // tile is not read
+        if(lane < h) {
+            if(FILL) {
+                const int32_t wr = p.ui_ptr[fr + lane], wc = p.ti_ptr[fr + lane];
+                p.ui_col[wr] = fr + lane; p.ui_val[wr] = (VT) 1; p.ui_lr[wr] = (uint8_t) lane;
+                p.ti_col[wc] = fr + lane; p.ti_val[wc] = (VT) 1; p.ti_lr[wc] = (uint8_t) lane;
+            } else {
+                p.ui_ptr[fr + lane + 1] = 1;
+                p.ti_ptr[fr + lane + 1] = 1;
             }
         }
-        if(!FILL) { p.ui_ptr[fr + lane + 1] = cr; p.ti_ptr[fr + lane + 1] = cc; }
+    } else {
+        double* X = (double*) lds;
+        const BlockMeta dm = t.bout[t.csr_off[i]];
+        diag_inverse(val_out + dm.val_ptr, h, X, hm);
+        if(lane < h) {
+            int cr = 0, cc = 0;
+            int32_t wr = 0, wc = 0;
+            if(FILL) { wr = p.ui_ptr[fr + lane]; wc = p.ti_ptr[fr + lane]; }
+            for(int c = 0; c < h; ++c) {
+                const double v = X[hm * lane + c];  // row lane of U^-1
+                if(v != 0.0) {
+                    if(FILL) { p.ui_col[wr + cr] = fr + c; p.ui_val[wr + cr] = (VT) v; p.ui_lr[wr + cr] = (uint8_t) lane; }
+                    ++cr;
+                }
+                const double u = X[hm * c + lane];  // column lane of U^-1
+                if(u != 0.0) {
+                    if(FILL) { p.ti_col[wc + cc] = fr + c; p.ti_val[wc + cc] = (VT) u; p.ti_lr[wc + cc] = (uint8_t) lane; }
+                    ++cc;
+                }
+            }
+            if(!FILL) { p.ui_ptr[fr + lane + 1] = cr; p.ti_ptr[fr + lane + 1] = cc; }
+        }
     }
     // off-diagonal blocks of block row i (uo), by block id; 64 blocks at a
     // time are staged (metadata and small entry lists) one per lane, then
     // walked in order by the lanes of the fine rows
-    __shared__ PlanStage<VT> sg;
+    PlanStage<VT>& sg = *(PlanStage<VT>*) lds;
     int cnt = 0;
     const int32_t base = (FILL && lane < h) ? p.uo_ptr[fr + lane] : 0;
     const int b0 = t.csr_off[i] + 1, b1 = t.csr_off[i + 1];
@@ -1186,7 +1202,7 @@ template<typename VT>
 void solve_plan_count(const SolveTopo& t, const VT* val_out, VT*, SolvePlan<VT>& p, void* stream)
 {
     hipStream_t st = (hipStream_t) stream;
-    k_plan_rows<VT, false><<<t.nb, 64, sizeof(double) * 1024, st>>>(t, val_out, p);
+    k_plan_rows<VT, false><<<t.nb, 64, plan_rows_lds<VT>(32), st>>>(t, val_out, p);
     k_plan_cols<VT, false><<<t.nb, 64, 0, st>>>(t, val_out, p);
 }
 
@@ -1195,7 +1211,7 @@ void solve_plan_fill(const SolveTopo& t, const VT* val_out, const VT*, SolvePlan
     void* stream)
 {
     hipStream_t st = (hipStream_t) stream;
-    k_plan_rows<VT, true><<<t.nb, 64, sizeof(double) * 1024, st>>>(t, val_out, p);
+    k_plan_rows<VT, true><<<t.nb, 64, plan_rows_lds<VT>(32), st>>>(t, val_out, p);
     k_plan_cols<VT, true><<<t.nb, 64, 0, st>>>(t, val_out, p);
     const unsigned g = (unsigned) ((t.nb + 255) / 256);
     k_plan_tasks<<<g, 256, 0, st>>>(t.nb, t.lvl_rows, t.bs, p.uo_ptr, p.ui_ptr, p.task_u);
@@ -1441,7 +1457,7 @@ void plan_batch(const PlanSys<VT>* ps, FactorItems blk, FactorItems scan, Factor
 {
     if(blk.count <= 0) return;
     const unsigned nb = (unsigned) blk.count;
-    const size_t lds = sizeof(double) * (size_t) hm * (size_t) hm;
+    const size_t lds = plan_rows_lds<VT>(hm);
     bk_plan_rows<VT, false><<<nb, 64, lds, st>>>(ps, blk.items, hm);
     bk_plan_cols<VT, false><<<nb, 64, 0, st>>>(ps, blk.items);
     for(int32_t q = 0; q < 4; ++q) {

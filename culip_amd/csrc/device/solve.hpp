@@ -35,6 +35,7 @@ struct SolveTopo {
     const int32_t* csc_off;     // coarse CSC offsets
     const int32_t* csc_idx;     // block ids of a column by row
     const BlockMeta* bout;      // factored metadata
+    const int32_t* row_flag;    // per block row ROW_2X2, ... (factor.hpp)
     const int32_t* ix_out;
     const double* tri;
     const int32_t* is_piv;

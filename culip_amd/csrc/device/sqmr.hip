@@ -11,6 +11,16 @@
 //   k_beta    beta's two dots
 //   k_pupdate w_{k+1} /= beta, p_k, x += tau p_k, ||x||^2
 //   k_scalars the scalar recurrence, quasi-residual and the stopping test
+// Between two true-residual checks the vector work of neighbouring iterations
+// is merged, three kernels instead of six, since beta(k) and alpha(k + 1) read
+// the same Av, and x, p and the scalars of iteration k do not enter v_{k+2}
+// other than through beta(k) and eta, which every workgroup forms itself:
+//   k_dots    beta's two dots and alpha's of iteration k + 1
+//   k_pv      k_pupdate of iteration k and k_vnext of k + 1
+//   k_sv      k_vscale of iteration k + 1 and, on one more workgroup,
+//             k_scalars of iteration k
+// with alpha's and delta's partial sums in two sets of slots used in turn. Every
+// value is formed by the same operations as in the six kernels (same bits).
 // D \ v_k is reused from the previous iteration (the reference recomputes the
 // same vector). Every workgroup reduces the per-workgroup partial sums in the
 // same fixed order, so all scalars are identical everywhere and run to run.
@@ -25,6 +35,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace culip {
 
@@ -36,7 +47,9 @@ constexpr int TPB = 256;
 enum {
     S_ALPHA = 0, S_BETA = 1, S_DELTA = 4, S_NORMA = 7, S_EPS = 8, S_BROT = 9, S_BRR = 10,
     S_AROT = 11, S_C = 12, S_S = 15, S_TAU = 18, S_RHO = 19, S_GAMMA = 20, S_NORMPB = 21,
-    S_NORMX = 22, S_ETA = 26, S_ITER = 27, NSCAL = 32
+    S_NORMX = 22, S_ETA = 26, S_ITER = 27, NSCAL = 32,
+    // beside the state: eta between k_pv and k_sv
+    SCAL_ETA = 44
 };
 static_assert(S_GAMMA == SQMR_S_GAMMA && S_NORMPB == SQMR_S_NORMPB, "scalar slots");
 
@@ -112,6 +125,31 @@ __device__ void reduce_parts(const double* part, int G, const int (&slot)[K], do
     __syncthreads();
 }
 
+// block_sum of K values at once (each summed exactly as block_sum sums it); sh
+// holds K * (waves + 1) doubles
+template<int K>
+__device__ __forceinline__ void block_sums(double (&v)[K], double* sh)
+{
+    const int tid = threadIdx.x, nw = (int) (blockDim.x >> 6);
+#pragma unroll
+    for(int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
+    __syncthreads();
+    if((tid & 63) == 0) {
+#pragma unroll
+        for(int k = 0; k < K; ++k) sh[k * nw + (tid >> 6)] = v[k];
+    }
+    __syncthreads();
+    if(tid < K) {
+        double t = 0.0;
+        for(int q = 0; q < nw; ++q) t += sh[tid * nw + q];
+        sh[K * nw + tid] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for(int k = 0; k < K; ++k) v[k] = sh[K * nw + k];
+    __syncthreads();
+}
+
 // block_sum of two values at once (each summed exactly as block_sum sums it)
 __device__ void block_sum2(double& a, double& b, double* sh)
 {
@@ -131,6 +169,9 @@ __device__ void block_sum2(double& a, double& b, double* sh)
     b = sh[2 * nw + 1];
     __syncthreads();
 }
+
+// alpha's two partial-sum slots and delta's (alpha_slot + 2) of iteration k
+__host__ __device__ __forceinline__ int alpha_slot(int k) { return (k & 1) ? 6 : 0; }
 
 __device__ __forceinline__ double& part_at(double* part, int slot, int q, int G)
 {
@@ -233,10 +274,23 @@ __device__ __forceinline__ DRow dload(int64_t g, int32_t n, const double* tri, c
     return d;
 }
 
-// dsolve on loaded inputs (the same operations)
+// dsolve on loaded inputs (the same operations). Where every lane has a 1x1
+// pivot the rotation is exactly +-1 and 0 and the solve is one division: sqrt
+// of the rounded square is |p11| (no over- or underflow in the range tested),
+// and the products with zero vanish for finite right-hand sides.
 __device__ __forceinline__ DP dsolve_loaded(const DRow& d, double r1, double r2)
 {
     DP o;
+    const double ap = fabs(d.p11);
+    const bool plain = d.this_piv && d.next_piv && d.p12 == 0.0 && ap > 1e-140 && ap < 1e140 &&
+        fabs(r1) < 1e140 && fabs(r2) < 1e140;
+    if(wave_ballot(!plain) == 0ull) {
+        o.g1 = r1 / d.p11;
+        o.g2 = 0.0;
+        o.w1 = true;
+        o.w2 = false;
+        return o;
+    }
     const double p22 = !d.next_piv ? d.p22n : 1.0;
     const double gr = sqrt(fma(d.p11, d.p11, d.p12 * d.p12));
     const double c = d.p11 / gr, s = d.p12 / gr;
@@ -252,7 +306,7 @@ __device__ __forceinline__ DP dsolve_loaded(const DRow& d, double r1, double r2)
 
 template<int R = VR>
 __device__ __forceinline__ void alpha_body(int q_, int G_, int32_t n, const double* Av, const double* v,
-    const double* z, const double* tri, const int32_t* ip, double* part)
+    const double* z, const double* tri, const int32_t* ip, double* part, int k)
 {
     __shared__ double sh[16];
     double num = 0.0, den = 0.0;
@@ -284,7 +338,10 @@ __device__ __forceinline__ void alpha_body(int q_, int G_, int32_t n, const doub
         }
     }
     block_sum2(num, den, sh);
-    if(threadIdx.x == 0) { part_at(part, 0, q_, G_) = num; part_at(part, 1, q_, G_) = den; }
+    if(threadIdx.x == 0) {
+        part_at(part, alpha_slot(k), q_, G_) = num;
+        part_at(part, alpha_slot(k) + 1, q_, G_) = den;
+    }
 }
 
 // The kernels that start with a reduction of the previous kernel's partial
@@ -310,7 +367,8 @@ __device__ __forceinline__ void vnext_body(int q_, int G_, int32_t n, int k, con
     int64_t g0 = (int64_t) q_ * TPB + threadIdx.x;
     if(g0 < n) load(g0);
     double rp[2];
-    reduce_parts<2>(part, G, {0, 1}, rp, sh);
+    const int s0 = alpha_slot(k);
+    reduce_parts<2>(part, G, {s0, s0 + 1}, rp, sh);
     const double alpha = rp[0] / rp[1];
     const double beta = scal[S_BETA + k % 3];
     double ss = 0.0;
@@ -326,13 +384,14 @@ __device__ __forceinline__ void vnext_body(int q_, int G_, int32_t n, int k, con
         if(g0 + S * R < n) load(g0 + S * R);
     }
     ss = block_sum(ss, sh);
-    if(threadIdx.x == 0) part_at(part, 2, q_, G_) = ss;
+    if(threadIdx.x == 0) part_at(part, s0 + 2, q_, G_) = ss;
 }
 
+// eta: S_ETA of the iteration before (scal[S_ETA], or where k_pv left it)
 template<int R = VR>
-__device__ __forceinline__ void vscale_body(int q_, int G_, int32_t n, const double* tv, double* v1,
-    double* z, double* w1, double* ev, const double* tri, const int32_t* ip, const double* scal,
-    const double* part)
+__device__ __forceinline__ void vscale_body(int q_, int G_, int32_t n, int k, const double* tv,
+    double* v1, double* z, double* w1, double* ev, const double* tri, const int32_t* ip,
+    const double* eta, const double* part)
 {
     __shared__ double sh[16];
     const int G = G_;
@@ -350,9 +409,9 @@ __device__ __forceinline__ void vscale_body(int q_, int G_, int32_t n, const dou
     };
     int64_t g0 = (int64_t) q_ * TPB + threadIdx.x;
     if(g0 < n) load(g0);
-    const double delta = sqrt(reduce_part(part, G, 2, sh));
+    const double delta = sqrt(reduce_part(part, G, alpha_slot(k) + 2, sh));
     const double t = 1.0 / delta;
-    const double we = scal[S_ETA] * delta;
+    const double we = *eta * delta;
     for(; g0 < n; g0 += S * R) {
 #pragma unroll
         for(int r = 0; r < R; ++r) {
@@ -410,15 +469,17 @@ __device__ __forceinline__ void iteration_scalars(double* S, const double* scal,
     scalar_step<K0>(S, alpha, delta, beta);
 }
 
-template<int K0, int R>
-__device__ __forceinline__ void pupdate(int q_, int G_, int32_t n, double* w1, const double* vk, double* pk,
-    const double* pkm1, const double* pkm2, double* x, const double* scal, double* part,
-    const int32_t* flags)
+// NEXT: with vnext of iteration k + 1 (K0 = k mod 3), whose v_{k+1} is vn and
+// whose Av is av; both read v_k
+template<int K0, int R, bool NEXT>
+__device__ __forceinline__ void pupdate(int q_, int G_, int32_t n, int k, double* w1,
+    const double* vk, double* pk, const double* pkm1, const double* pkm2, double* x, double* scal,
+    double* part, const int32_t* flags, const double* av, const double* vn, double* tv)
 {
     __shared__ double sh[64];
     const int G = G_;
     const int64_t SG = (int64_t) G * TPB;
-    double ww[R], a[R], b[R], c[R], xx[R];
+    double ww[R], a[R], b[R], c[R], xx[R], an[R], bn[R];
     auto load = [&](int64_t g0) {
 #pragma unroll
         for(int r = 0; r < R; ++r) {
@@ -428,31 +489,50 @@ __device__ __forceinline__ void pupdate(int q_, int G_, int32_t n, double* w1, c
             b[r] = pkm1[g];
             c[r] = pkm2[g];
             xx[r] = x[g];
+            if(NEXT) {
+                an[r] = av[g];
+                bn[r] = vn[g];
+            }
         }
     };
     int64_t g0 = (int64_t) q_ * TPB + threadIdx.x;
     if(g0 < n) load(g0);
-    double rp[5];
-    reduce_parts<5>(part, G, {0, 1, 2, 3, 4}, rp, sh);
-    // one thread runs the scalar step and shares the five factors the
-    // update needs (the step's 32 scalars held by every thread would cost
-    // the registers of two more waves per SIMD)
+    constexpr int NS = NEXT ? 7 : 5;
+    const int s0 = alpha_slot(k), s1 = alpha_slot(k + 1);
+    double rp[NS];
+    {
+        int slot[NS];
+        const int all[7] = {s0, s0 + 1, s0 + 2, 3, 4, s1, s1 + 1};
+#pragma unroll
+        for(int q = 0; q < NS; ++q) slot[q] = all[q];
+        reduce_parts<NS>(part, G, slot, rp, sh);
+    }
+    // one thread runs the scalar step and shares the factors the update needs
+    // (the step's 32 scalars held by every thread would cost the registers of
+    // two more waves per SIMD)
     if(threadIdx.x == 0) {
+        const double r5[5] = {rp[0], rp[1], rp[2], rp[3], rp[4]};
         double S[NSCAL];
-        iteration_scalars<K0>(S, scal, rp);
-        sh[32] = 1.0 / S[S_BETA + (K0 + 1) % 3];
-        sh[33] = -S[S_BRR];
-        sh[34] = -S[S_EPS];
-        sh[35] = 1.0 / S[S_RHO];
-        sh[36] = S[S_TAU];
+        iteration_scalars<K0>(S, scal, r5);
+        sh[40] = 1.0 / S[S_BETA + (K0 + 1) % 3];
+        sh[41] = -S[S_BRR];
+        sh[42] = -S[S_EPS];
+        sh[43] = 1.0 / S[S_RHO];
+        sh[44] = S[S_TAU];
+        if(NEXT) {
+            sh[45] = S[S_BETA + (K0 + 1) % 3];
+            // for k_sv, whose scalars of this iteration run beside it
+            if(q_ == 0) scal[SCAL_ETA] = S[S_ETA];
+        }
     }
     __syncthreads();
-    const double ib = sh[32], nbrr = sh[33], neps = sh[34], ir = sh[35], tau = sh[36];
+    const double ib = sh[40], nbrr = sh[41], neps = sh[42], ir = sh[43], tau = sh[44];
+    const double alpha = NEXT ? rp[NS - 2] / rp[NS - 1] : 0.0, beta = NEXT ? sh[45] : 0.0;
     // after a Lanczos breakdown (flagged by the previous iteration) the
     // recurrence divides by a vanishing delta: x keeps the value it had when
     // the breakdown was detected
     const bool frozen = flags[0] != 0;
-    double ss = 0.0;
+    double ss[2] = {0.0, 0.0};
     for(; g0 < n; g0 += SG * R) {
 #pragma unroll
         for(int r = 0; r < R; ++r) {
@@ -466,23 +546,88 @@ __device__ __forceinline__ void pupdate(int q_, int G_, int32_t n, double* w1, c
             pk[g] = p;
             const double xv = frozen ? xx[r] : fma(tau, p, xx[r]);
             if(!frozen) x[g] = xv;
-            ss = fma(xv, xv, ss);
+            ss[0] = fma(xv, xv, ss[0]);
+            if(NEXT) {
+                const double t = fma(-beta, a[r], fma(-alpha, bn[r], an[r]));
+                tv[g] = t;
+                ss[1] = fma(t, t, ss[1]);
+            }
         }
         if(g0 + SG * R < n) load(g0 + SG * R);
     }
-    ss = block_sum(ss, sh);
-    if(threadIdx.x == 0) part_at(part, 5, q_, G_) = ss;
+    if(NEXT) block_sums<2>(ss, sh);
+    else ss[0] = block_sum(ss[0], sh);
+    if(threadIdx.x == 0) {
+        part_at(part, 5, q_, G_) = ss[0];
+        if(NEXT) part_at(part, s1 + 2, q_, G_) = ss[1];
+    }
 }
 
-template<int R = VR>
-__device__ __forceinline__ void pupdate_body(int q_, int G_, int32_t n, int k, double* w1, const double* vk,
-    double* pk, const double* pkm1, const double* pkm2, double* x, const double* scal,
-    double* part, const int32_t* flags)
+template<int R, bool NEXT>
+__device__ __forceinline__ void pupdate_body(int q_, int G_, int32_t n, int k, double* w1,
+    const double* vk, double* pk, const double* pkm1, const double* pkm2, double* x, double* scal,
+    double* part, const int32_t* flags, const double* av, const double* vn, double* tv)
 {
     switch(k % 3) {
-    case 0: pupdate<0, R>(q_, G_, n, w1, vk, pk, pkm1, pkm2, x, scal, part, flags); break;
-    case 1: pupdate<1, R>(q_, G_, n, w1, vk, pk, pkm1, pkm2, x, scal, part, flags); break;
-    default: pupdate<2, R>(q_, G_, n, w1, vk, pk, pkm1, pkm2, x, scal, part, flags); break;
+    case 0:
+        pupdate<0, R, NEXT>(q_, G_, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part, flags, av, vn, tv);
+        break;
+    case 1:
+        pupdate<1, R, NEXT>(q_, G_, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part, flags, av, vn, tv);
+        break;
+    default:
+        pupdate<2, R, NEXT>(q_, G_, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part, flags, av, vn, tv);
+        break;
+    }
+}
+
+// beta's dots of iteration k (w_k, Av, v_k) and alpha's of iteration k + 1
+// (v_{k+1}, Av, z): each summed as beta_body and alpha_body sum them
+template<int R>
+__device__ __forceinline__ void dots_body(int q_, int G_, int32_t n, int k, const double* wk,
+    const double* Av, const double* vk, const double* vn, const double* z, const double* tri,
+    const int32_t* ip, double* part)
+{
+    __shared__ double sh[32];
+    double d[4] = {0.0, 0.0, 0.0, 0.0};   // beta, alpha: numerator, denominator
+    const int64_t S = (int64_t) G_ * TPB;
+    for(int64_t g0 = (int64_t) q_ * TPB + threadIdx.x; g0 < n; g0 += S * R) {
+        double av[R], av1[R], ww[R], vv[R], v1[R], v11[R], zz[R];
+        DRow dr[R];
+#pragma unroll
+        for(int r = 0; r < R; ++r) {
+            const int64_t g = min(g0 + r * S, (int64_t) n - 1);
+            const int64_t g1 = min(g + 1, (int64_t) n - 1);
+            av[r] = Av[g];
+            av1[r] = Av[g1];
+            ww[r] = wk[g];
+            vv[r] = vk[g];
+            v1[r] = vn[g];
+            v11[r] = vn[g1];
+            zz[r] = z[g];
+            if(tri) dr[r] = dload(g, n, tri, ip);
+        }
+#pragma unroll
+        for(int r = 0; r < R; ++r) {
+            const int64_t g = g0 + r * S;
+            if(g >= n) break;
+            d[0] = fma(ww[r], av[r], d[0]);
+            d[1] = fma(ww[r], vv[r], d[1]);
+            DP o;
+            if(tri) o = dsolve_loaded(dr[r], av[r], (g < n - 1) ? av1[r] : 0.0);
+            else { o.g1 = av[r]; o.g2 = 0; o.w1 = true; o.w2 = false; }
+            if(o.w1) d[2] = fma(v1[r], o.g1, d[2]);
+            if(o.w2) d[2] = fma(v11[r], o.g2, d[2]);
+            d[3] = fma(v1[r], zz[r], d[3]);
+        }
+    }
+    block_sums<4>(d, sh);
+    if(threadIdx.x == 0) {
+        const int s1 = alpha_slot(k + 1);
+        part_at(part, 3, q_, G_) = d[0];
+        part_at(part, 4, q_, G_) = d[1];
+        part_at(part, s1, q_, G_) = d[2];
+        part_at(part, s1 + 1, q_, G_) = d[3];
     }
 }
 
@@ -497,7 +642,8 @@ __device__ __forceinline__ void scalars(int k, int G, double* scal, const double
     __shared__ double sh[64];
     double S[NSCAL];
     double r6[6];
-    reduce_parts<6>(part, G, {0, 1, 2, 3, 4, 5}, r6, sh);
+    const int s0 = alpha_slot(k);
+    reduce_parts<6>(part, G, {s0, s0 + 1, s0 + 2, 3, 4, 5}, r6, sh);
     const double r[5] = {r6[0], r6[1], r6[2], r6[3], r6[4]};
     iteration_scalars<K0>(S, scal, r);
     const double nx = sqrt(r6[5]);
@@ -514,7 +660,7 @@ __device__ __forceinline__ void scalars(int k, int G, double* scal, const double
     }
 }
 
-__global__ __launch_bounds__(TPB) void k_scalars(int k, int G, double* scal, const double* part,
+__device__ __forceinline__ void scalars_body(int k, int G, double* scal, const double* part,
     int32_t* flags, double tol, double brel)
 {
     switch(k % 3) {
@@ -522,6 +668,12 @@ __global__ __launch_bounds__(TPB) void k_scalars(int k, int G, double* scal, con
     case 1: scalars<1>(k, G, scal, part, flags, tol, brel); break;
     default: scalars<2>(k, G, scal, part, flags, tol, brel); break;
     }
+}
+
+__global__ __launch_bounds__(TPB) void k_scalars(int k, int G, double* scal, const double* part,
+    int32_t* flags, double tol, double brel)
+{
+    scalars_body(k, G, scal, part, flags, tol, brel);
 }
 
 // start: tv = Pl \ b (done by the caller); v0 = tv / ||tv||, z = D \ v0
@@ -636,9 +788,9 @@ __device__ __forceinline__ void norm2_pair_body(int q_, int G_, int32_t n, const
 // arithmetic), else VR
 template<int R>
 __global__ __launch_bounds__(TPB) void k_alpha(int32_t n, const double* Av, const double* v,
-    const double* z, const double* tri, const int32_t* ip, double* part)
+    const double* z, const double* tri, const int32_t* ip, double* part, int k)
 {
-    alpha_body<R>(blockIdx.x, gridDim.x, n, Av, v, z, tri, ip, part);
+    alpha_body<R>(blockIdx.x, gridDim.x, n, Av, v, z, tri, ip, part, k);
 }
 
 template<int R>
@@ -649,11 +801,11 @@ __global__ __launch_bounds__(TPB) void k_vnext(int32_t n, int k, const double* A
 }
 
 template<int R>
-__global__ __launch_bounds__(TPB) void k_vscale(int32_t n, const double* tv, double* v1,
+__global__ __launch_bounds__(TPB) void k_vscale(int32_t n, int k, const double* tv, double* v1,
     double* z, double* w1, double* ev, const double* tri, const int32_t* ip, const double* scal,
     const double* part)
 {
-    vscale_body<R>(blockIdx.x, gridDim.x, n, tv, v1, z, w1, ev, tri, ip, scal, part);
+    vscale_body<R>(blockIdx.x, gridDim.x, n, k, tv, v1, z, w1, ev, tri, ip, scal + S_ETA, part);
 }
 
 template<int R>
@@ -665,10 +817,44 @@ __global__ __launch_bounds__(TPB) void k_beta(int32_t n, const double* wk, const
 
 template<int R>
 __global__ __launch_bounds__(TPB) void k_pupdate(int32_t n, int k, double* w1, const double* vk,
-    double* pk, const double* pkm1, const double* pkm2, double* x, const double* scal,
+    double* pk, const double* pkm1, const double* pkm2, double* x, double* scal,
     double* part, const int32_t* flags)
 {
-    pupdate_body<R>(blockIdx.x, gridDim.x, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part, flags);
+    pupdate_body<R, false>(blockIdx.x, gridDim.x, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part,
+        flags, nullptr, nullptr, nullptr);
+}
+
+// the merged kernels of iterations k and k + 1 (top of the file)
+template<int R>
+__global__ __launch_bounds__(TPB) void k_dots(int32_t n, int k, const double* wk, const double* Av,
+    const double* vk, const double* vn, const double* z, const double* tri, const int32_t* ip,
+    double* part)
+{
+    dots_body<R>(blockIdx.x, gridDim.x, n, k, wk, Av, vk, vn, z, tri, ip, part);
+}
+
+template<int R>
+__global__ __launch_bounds__(TPB) void k_pv(int32_t n, int k, double* w1, const double* vk,
+    double* pk, const double* pkm1, const double* pkm2, double* x, double* scal, double* part,
+    const int32_t* flags, const double* av, const double* vn, double* tv)
+{
+    pupdate_body<R, true>(blockIdx.x, gridDim.x, n, k, w1, vk, pk, pkm1, pkm2, x, scal, part, flags,
+        av, vn, tv);
+}
+
+// vscale of iteration k + 1 on all workgroups but the last, which runs the
+// scalars of iteration k
+template<int R>
+__global__ __launch_bounds__(TPB) void k_sv(int32_t n, int k, const double* tv, double* v1,
+    double* z, double* w1, double* ev, const double* tri, const int32_t* ip, double* scal,
+    const double* part, int32_t* flags, double tol, double brel)
+{
+    const int G = (int) gridDim.x - 1;
+    if((int) blockIdx.x == G) {
+        scalars_body(k, G, scal, part, flags, tol, brel);
+        return;
+    }
+    vscale_body<R>(blockIdx.x, G, n, k + 1, tv, v1, z, w1, ev, tri, ip, scal + SCAL_ETA, part);
 }
 
 __global__ __launch_bounds__(TPB) void k_sumsq(int32_t n, const double* a, double* part, int slot)
@@ -752,67 +938,94 @@ __global__ void k_batch_holes(int2* items, int32_t total)
     if(i < total) items[i] = make_int2(-1, 0);
 }
 
+// j: how many iterations of the launch sequence precede this one (the
+// systems' counters move on at the sequence's end, bk_scalars)
 template<int R>
-__global__ __launch_bounds__(TPB) void bk_alpha(const int2* items, const BatchSys* sys)
+__global__ __launch_bounds__(TPB) void bk_alpha(const int2* items, const BatchSys* sys, int32_t j)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k = *S.iter;
-    alpha_body<R>(it.y, S.G, S.n, S.av[k & 1], S.v[k % 3], S.z, S.tri, S.ip, S.part);
+    const int k = *S.iter + j;
+    alpha_body<R>(it.y, S.G, S.n, S.av[k & 1], S.v[k % 3], S.z, S.tri, S.ip, S.part, k);
 }
 
 template<int R>
-__global__ __launch_bounds__(TPB) void bk_vnext(const int2* items, const BatchSys* sys)
+__global__ __launch_bounds__(TPB) void bk_vnext(const int2* items, const BatchSys* sys, int32_t j)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k = *S.iter;
+    const int k = *S.iter + j;
     vnext_body<R>(it.y, S.G, S.n, k, S.av[k & 1], S.v[k % 3], S.v[(k + 2) % 3], S.tv, S.scal,
         S.part);
 }
 
 template<int R>
-__global__ __launch_bounds__(TPB) void bk_vscale(const int2* items, const BatchSys* sys)
+__global__ __launch_bounds__(TPB) void bk_vscale(const int2* items, const BatchSys* sys, int32_t j)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k1 = (*S.iter + 1) % 3;
-    vscale_body<R>(it.y, S.G, S.n, S.tv, S.v[k1], S.z, S.w[k1], S.ev, S.tri, S.ip, S.scal, S.part);
+    const int k = *S.iter + j, k1 = (k + 1) % 3;
+    vscale_body<R>(it.y, S.G, S.n, k, S.tv, S.v[k1], S.z, S.w[k1], S.ev, S.tri, S.ip,
+        S.scal + S_ETA, S.part);
 }
 
 template<int R>
-__global__ __launch_bounds__(TPB) void bk_beta(const int2* items, const BatchSys* sys)
+__global__ __launch_bounds__(TPB) void bk_beta(const int2* items, const BatchSys* sys, int32_t j)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k = *S.iter;
+    const int k = *S.iter + j;
     beta_body<R>(it.y, S.G, S.n, S.w[k % 3], S.av[(k & 1) ^ 1], S.v[k % 3], S.part);
 }
 
 template<int R>
-__global__ __launch_bounds__(TPB) void bk_pupdate(const int2* items, const BatchSys* sys)
+__global__ __launch_bounds__(TPB) void bk_dots(const int2* items, const BatchSys* sys, int32_t j)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k = *S.iter;
+    const int k = *S.iter + j;
+    dots_body<R>(it.y, S.G, S.n, k, S.w[k % 3], S.av[(k & 1) ^ 1], S.v[k % 3], S.v[(k + 1) % 3],
+        S.z, S.tri, S.ip, S.part);
+}
+
+template<int R, bool NEXT>
+__global__ __launch_bounds__(TPB) void bk_pupdate(const int2* items, const BatchSys* sys, int32_t j)
+{
+    const int2 it = items[blockIdx.x];
+    const BatchSys& S = sys[it.x];
+    const int k = *S.iter + j;
     const int k0 = k % 3, k1 = (k + 1) % 3, km1 = (k + 2) % 3;
-    pupdate_body<R>(it.y, S.G, S.n, k, S.w[k1], S.v[k0], S.p[k0], S.p[km1], S.p[k1], S.xt, S.scal,
-        S.part, S.flags);
+    pupdate_body<R, NEXT>(it.y, S.G, S.n, k, S.w[k1], S.v[k0], S.p[k0], S.p[km1], S.p[k1], S.xt,
+        S.scal, S.part, S.flags, S.av[(k & 1) ^ 1], S.v[k1], S.tv);
+}
+
+// k_sv: the vector items, then one item per system for the scalars
+template<int R>
+__global__ __launch_bounds__(TPB) void bk_sv(const int2* items, const int2* one, int32_t nvec,
+    const BatchSys* sys, int32_t j, double tol, double brel)
+{
+    const bool sc = (int) blockIdx.x >= nvec;
+    const int2 it = sc ? one[(int) blockIdx.x - nvec] : items[blockIdx.x];
+    const BatchSys& S = sys[it.x];
+    const int k = *S.iter + j;
+    if(sc) {
+        scalars_body(k, S.G, S.scal, S.part, S.flags, tol, brel);
+        return;
+    }
+    const int k2 = (k + 2) % 3;
+    vscale_body<R>(it.y, S.G, S.n, k + 1, S.tv, S.v[k2], S.z, S.w[k2], S.ev, S.tri, S.ip,
+        S.scal + SCAL_ETA, S.part);
 }
 
 // the scalar recurrence of every listed system, then its iteration counter
 // moves on (every thread has read it before the first barrier in scalars)
 __global__ __launch_bounds__(TPB) void bk_scalars(const int2* items, const BatchSys* sys,
-    double tol, double brel)
+    int32_t j, double tol, double brel)
 {
     const int2 it = items[blockIdx.x];
     const BatchSys& S = sys[it.x];
-    const int k = *S.iter;
-    switch(k % 3) {
-    case 0: scalars<0>(k, S.G, S.scal, S.part, S.flags, tol, brel); break;
-    case 1: scalars<1>(k, S.G, S.scal, S.part, S.flags, tol, brel); break;
-    default: scalars<2>(k, S.G, S.scal, S.part, S.flags, tol, brel); break;
-    }
+    const int k = *S.iter + j;
+    scalars_body(k, S.G, S.scal, S.part, S.flags, tol, brel);
     if(threadIdx.x == 0) *S.iter = k + 1;
 }
 
@@ -891,12 +1104,16 @@ int32_t sqmr_grid(int32_t n)
     return g;
 }
 
+// partial-sum slots: two sets of alpha's and delta's, beta's, ||x||^2
+constexpr int PART_SLOTS = 9;
+
 static size_t align_up(size_t v) { return (v + 255) & ~(size_t) 255; }
 
 size_t sqmr_work_bytes(int32_t n)
 {
     const size_t vec = align_up(sizeof(double) * (size_t) (n > 0 ? n : 1));
-    return 19 * vec + align_up(sizeof(double) * 8 * sqmr_grid(n)) + align_up(sizeof(double) * 64) +
+    return 19 * vec + align_up(sizeof(double) * PART_SLOTS * sqmr_grid(n)) +
+        align_up(sizeof(double) * 64) +
         align_up(sizeof(int32_t) * 8);
 }
 
@@ -911,7 +1128,7 @@ void sqmr_work_bind(SqmrWork& w, int32_t n, char* base, int32_t* host_flags, dou
     for(int q = 0; q < 18; ++q) { *vecs[q] = (double*) (base + off); off += vec; }
     off += vec;  // spare
     w.part = (double*) (base + off);
-    off += align_up(sizeof(double) * 8 * w.grid);
+    off += align_up(sizeof(double) * PART_SLOTS * w.grid);
     w.scal = (double*) (base + off);
     off += align_up(sizeof(double) * 64);
     w.flags = (int32_t*) (base + off);
@@ -985,35 +1202,47 @@ static void sqmr_run(const SqmrOps& ops, SqmrWork& w, const double* b, double* x
     // (the 3-cyclic vectors) and the parity of `cur` (the two A ev vectors),
     // so iterations i and i + 6 launch the same work
     const bool one_round = (int64_t) n <= (int64_t) G * TPB;
-    auto launch_iteration = [&](int i) {
+    // first / last: nothing of the iteration was launched with the one before
+    // it / nothing of the next one goes with it
+    const double brel = period > 0 ? SQMR_BREAKDOWN_REL : -1.0;
+    auto vectors = [&](auto rounds, int i, bool before, bool first, bool last) {
+        constexpr int R = decltype(rounds)::value;
         const int k0 = i % 3, k1 = (i + 1) % 3, km1 = (i + 2) % 3, km2 = (i + 1) % 3;
-        const int nxt = cur ^ 1;
-        if(one_round) {
-            k_alpha<1><<<G, TPB, 0, st>>>(n, w.av[cur], w.v[k0], w.z, ops.tri, ops.is_piv, w.part);
-            k_vnext<1><<<G, TPB, 0, st>>>(n, i, w.av[cur], w.v[k0], w.v[km1], w.tv, w.scal, w.part);
-            k_vscale<1><<<G, TPB, 0, st>>>(n, w.tv, w.v[k1], w.z, w.w[k1], w.ev, ops.tri,
-                ops.is_piv, w.scal, w.part);
-        } else {
-            k_alpha<VR><<<G, TPB, 0, st>>>(n, w.av[cur], w.v[k0], w.z, ops.tri, ops.is_piv, w.part);
-            k_vnext<VR><<<G, TPB, 0, st>>>(n, i, w.av[cur], w.v[k0], w.v[km1], w.tv, w.scal,
-                w.part);
-            k_vscale<VR><<<G, TPB, 0, st>>>(n, w.tv, w.v[k1], w.z, w.w[k1], w.ev, ops.tri,
-                ops.is_piv, w.scal, w.part);
+        const double* tri = ops.tri;
+        const int32_t* ip = ops.is_piv;
+        if(before) {
+            if(!first) return;
+            k_alpha<R><<<G, TPB, 0, st>>>(n, w.av[cur], w.v[k0], w.z, tri, ip, w.part, i);
+            k_vnext<R><<<G, TPB, 0, st>>>(n, i, w.av[cur], w.v[k0], w.v[km1], w.tv, w.scal, w.part);
+            k_vscale<R><<<G, TPB, 0, st>>>(n, i, w.tv, w.v[k1], w.z, w.w[k1], w.ev, tri, ip,
+                w.scal, w.part);
+            return;
         }
+        const double* av = w.av[cur ^ 1];
+        if(last) {
+            k_beta<R><<<G, TPB, 0, st>>>(n, w.w[k0], av, w.v[k0], w.part);
+            k_pupdate<R><<<G, TPB, 0, st>>>(n, i, w.w[k1], w.v[k0], w.p[k0], w.p[km1], w.p[km2],
+                w.xt, w.scal, w.part, w.flags);
+            k_scalars<<<1, TPB, 0, st>>>(i, G, w.scal, w.part, w.flags, opt.tol, brel);
+        } else {
+            const int k2 = (i + 2) % 3;
+            k_dots<R><<<G, TPB, 0, st>>>(n, i, w.w[k0], av, w.v[k0], w.v[k1], w.z, tri, ip, w.part);
+            k_pv<R><<<G, TPB, 0, st>>>(n, i, w.w[k1], w.v[k0], w.p[k0], w.p[km1], w.p[km2], w.xt,
+                w.scal, w.part, w.flags, av, w.v[k1], w.tv);
+            k_sv<R><<<G + 1, TPB, 0, st>>>(n, i, w.tv, w.v[k2], w.z, w.w[k2], w.ev, tri, ip, w.scal,
+                w.part, w.flags, opt.tol, brel);
+        }
+    };
+    auto launch_vectors = [&](int i, bool before, bool first, bool last) {
+        if(one_round) vectors(std::integral_constant<int, 1>(), i, before, first, last);
+        else vectors(std::integral_constant<int, VR>(), i, before, first, last);
+    };
+    auto launch_iteration = [&](int i, bool first, bool last) {
+        launch_vectors(i, true, first, last);
         if(ops.right) ops.right(w.ev, st);
-        apply_left_op(w.ev, w.av[nxt]);
-        if(one_round) {
-            k_beta<1><<<G, TPB, 0, st>>>(n, w.w[k0], w.av[nxt], w.v[k0], w.part);
-            k_pupdate<1><<<G, TPB, 0, st>>>(n, i, w.w[k1], w.v[k0], w.p[k0], w.p[km1], w.p[km2],
-                w.xt, w.scal, w.part, w.flags);
-        } else {
-            k_beta<VR><<<G, TPB, 0, st>>>(n, w.w[k0], w.av[nxt], w.v[k0], w.part);
-            k_pupdate<VR><<<G, TPB, 0, st>>>(n, i, w.w[k1], w.v[k0], w.p[k0], w.p[km1], w.p[km2],
-                w.xt, w.scal, w.part, w.flags);
-        }
-        k_scalars<<<1, TPB, 0, st>>>(i, G, w.scal, w.part, w.flags, opt.tol,
-            period > 0 ? SQMR_BREAKDOWN_REL : -1.0);
-        cur = nxt;
+        apply_left_op(w.ev, w.av[cur ^ 1]);
+        launch_vectors(i, false, first, last);
+        cur ^= 1;
         HIPCHK(hipGetLastError());
     };
     // with the true-residual gate, the `period` iterations between two
@@ -1034,7 +1263,8 @@ static void sqmr_run(const SqmrOps& ops, SqmrWork& w, const double* b, double* x
             if(!ex) {
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                 try {
-                    for(int j = 0; j < period; ++j) launch_iteration(it + j);
+                    for(int j = 0; j < period; ++j)
+                        launch_iteration(it + j, j == 0, j == period - 1);
                 } catch(...) {
                     // leave the stream usable: end the broken capture
                     hipGraph_t bad = nullptr;
@@ -1051,8 +1281,10 @@ static void sqmr_run(const SqmrOps& ops, SqmrWork& w, const double* b, double* x
             HIPCHK(hipGraphLaunch(ex, st));
             cur = cur0 ^ (period & 1);
             it += period - 1;
+        } else if(period > 0) {
+            launch_iteration(it, it % period == 0, (it + 1) % period == 0 || it + 1 == opt.max_it);
         } else {
-            launch_iteration(it);
+            launch_iteration(it, true, true);
         }
 
         if(period > 0) {
@@ -1208,37 +1440,51 @@ void batch_step(BatchStep s, const BatchLists& L, const BatchSys* sys, int32_t a
     auto grid = [](const BatchList& l) { return (unsigned) l.count; };
     switch(s) {
     case BS_ALPHA:
-        if(L.vec.count) {
-            if(L.one_round) bk_alpha<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-            else bk_alpha<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-        }
+        if(!L.vec.count) break;
+        if(L.one_round) bk_alpha<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_alpha<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
         break;
     case BS_VNEXT:
-        if(L.vec.count) {
-            if(L.one_round) bk_vnext<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-            else bk_vnext<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-        }
+        if(!L.vec.count) break;
+        if(L.one_round) bk_vnext<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_vnext<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
         break;
     case BS_VSCALE:
-        if(L.vec.count) {
-            if(L.one_round) bk_vscale<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-            else bk_vscale<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-        }
+        if(!L.vec.count) break;
+        if(L.one_round) bk_vscale<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_vscale<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
         break;
     case BS_BETA:
-        if(L.vec.count) {
-            if(L.one_round) bk_beta<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-            else bk_beta<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-        }
+        if(!L.vec.count) break;
+        if(L.one_round) bk_beta<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_beta<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        break;
+    case BS_DOTS:
+        if(!L.vec.count) break;
+        if(L.one_round) bk_dots<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_dots<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
         break;
     case BS_PUPDATE:
-        if(L.vec.count) {
-            if(L.one_round) bk_pupdate<1><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-            else bk_pupdate<VR><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys);
-        }
+        if(!L.vec.count) break;
+        if(L.one_round) bk_pupdate<1, false><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_pupdate<VR, false><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
         break;
+    case BS_PV:
+        if(!L.vec.count) break;
+        if(L.one_round) bk_pupdate<1, true><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        else bk_pupdate<VR, true><<<grid(L.vec), TPB, 0, st>>>(L.vec.items, sys, a);
+        break;
+    case BS_SV: {
+        if(!L.vec.count) break;
+        const unsigned g = grid(L.vec) + grid(L.sys);
+        if(L.one_round)
+            bk_sv<1><<<g, TPB, 0, st>>>(L.vec.items, L.sys.items, L.vec.count, sys, a, tol, brel);
+        else
+            bk_sv<VR><<<g, TPB, 0, st>>>(L.vec.items, L.sys.items, L.vec.count, sys, a, tol, brel);
+        break;
+    }
     case BS_SCALARS:
-        if(L.sys.count) bk_scalars<<<grid(L.sys), TPB, 0, st>>>(L.sys.items, sys, tol, brel);
+        if(L.sys.count) bk_scalars<<<grid(L.sys), TPB, 0, st>>>(L.sys.items, sys, a, tol, brel);
         break;
     case BS_INIT_FILL:
         if(L.row.count) bk_init_fill<<<grid(L.row), 256, 0, st>>>(L.row.items, sys);

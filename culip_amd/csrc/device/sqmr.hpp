@@ -39,7 +39,7 @@ struct SqmrWork {
     double* rt = nullptr;
     double* xacc = nullptr;     // refinement: accumulated solution
     double* rhs = nullptr;      // refinement: current residual
-    double* part = nullptr;     // 8 * grid partial sums
+    double* part = nullptr;     // PART_SLOTS * grid partial sums
     double* scal = nullptr;     // 32 scalars
     int32_t* flags = nullptr;   // 4 ints: test[0], test[1]
     int32_t* host_flags = nullptr;  // pinned

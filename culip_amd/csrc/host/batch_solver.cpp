@@ -370,18 +370,31 @@ void BatchSolver::start_runs(const BatchLists& L, hipStream_t st)
     jacobi(L, true, BV_AVCUR, BV_EV, st);
 }
 
-// launch_iteration of sqmr_run for every listed system
-void BatchSolver::iteration(const BatchLists& L, hipStream_t st)
+// `steps` iterations of every listed system (launch_iteration of sqmr_run,
+// the vector work of neighbouring iterations merged as there)
+void BatchSolver::iterations(const BatchLists& L, int32_t steps, hipStream_t st)
 {
     const BatchSys* d = d_sys_.as<BatchSys>();
-    batch_step(BS_ALPHA, L, d, 0, 0, 0, 0, st);
-    batch_step(BS_VNEXT, L, d, 0, 0, 0, 0, st);
-    batch_step(BS_VSCALE, L, d, 0, 0, 0, 0, st);
-    jacobi(L, false, BV_EV, BV_NONE, st);
-    jacobi(L, true, BV_AVNXT, BV_EV, st);
-    batch_step(BS_BETA, L, d, 0, 0, 0, 0, st);
-    batch_step(BS_PUPDATE, L, d, 0, 0, 0, 0, st);
-    batch_step(BS_SCALARS, L, d, 0, 0, o_.sqmr.tol, SQMR_BREAKDOWN_REL, st);
+    const double tol = o_.sqmr.tol;
+    for(int32_t j = 0; j < steps; ++j) {
+        if(j == 0) {
+            batch_step(BS_ALPHA, L, d, j, 0, 0, 0, st);
+            batch_step(BS_VNEXT, L, d, j, 0, 0, 0, st);
+            batch_step(BS_VSCALE, L, d, j, 0, 0, 0, st);
+        }
+        jacobi(L, false, BV_EV, BV_NONE, st);
+        // the systems' counters stay where they are until the last step
+        jacobi(L, true, (j & 1) ? BV_AVCUR : BV_AVNXT, BV_EV, st);
+        if(j == steps - 1) {
+            batch_step(BS_BETA, L, d, j, 0, 0, 0, st);
+            batch_step(BS_PUPDATE, L, d, j, 0, 0, 0, st);
+            batch_step(BS_SCALARS, L, d, j, 0, tol, SQMR_BREAKDOWN_REL, st);
+        } else {
+            batch_step(BS_DOTS, L, d, j, 0, 0, 0, st);
+            batch_step(BS_PV, L, d, j, 0, 0, 0, st);
+            batch_step(BS_SV, L, d, j, 0, tol, SQMR_BREAKDOWN_REL, st);
+        }
+    }
 }
 
 void BatchSolver::run_solution(const BatchLists& L, hipStream_t st)
@@ -518,7 +531,7 @@ void BatchSolver::capture_segment(const BatchLists& L, int32_t period,
     seg_ids_.clear();
     HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     try {
-        for(int32_t j = 0; j < period; ++j) iteration(L, st);
+        iterations(L, period, st);
     } catch(...) {
         hipGraph_t bad = nullptr;
         (void) hipStreamEndCapture(st, &bad);
@@ -614,13 +627,12 @@ void BatchSolver::solve(const double* const* vals, const double* const* rhs, dou
                     aligned = false;
                     break;
                 }
-            int32_t steps = 1;
+            const int32_t steps = aligned ? period : 1;
             if(aligned && act == seg_prev_) {
                 if(!seg_exec_ || seg_ids_ != act) capture_segment(L, period, act, st);
                 HIP_CHECK(hipGraphLaunch(seg_exec_, st));
-                steps = period;
             } else {
-                iteration(L, st);
+                iterations(L, steps, st);
             }
             if(aligned) seg_prev_ = act;
             for(int32_t s : act) st_[s].it += steps - 1;

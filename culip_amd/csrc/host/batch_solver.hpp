@@ -92,7 +92,7 @@ private:
     template<typename VT> void factor_batched(hipStream_t st);
     const BatchLists& lists(ListSlot& slot, const std::vector<int32_t>& ids, hipStream_t st);
     void start_runs(const BatchLists& L, hipStream_t st);
-    void iteration(const BatchLists& L, hipStream_t st);
+    void iterations(const BatchLists& L, int32_t steps, hipStream_t st);
     void jacobi(const BatchLists& L, bool transpose, int32_t target, int32_t product_src,
         hipStream_t st);
     // x of each listed system = right(D \ xt); then its residual against

@@ -382,6 +382,7 @@ SolveTopo Bildlt::topo() const
     t.csc_off = d_csc_off.as<int32_t>();
     t.csc_idx = d_csc_idx.as<int32_t>();
     t.bout = d_bout.as<BlockMeta>();
+    t.row_flag = d_row_flag.as<int32_t>();
     t.ix_out = d_ix_out.as<int32_t>();
     t.tri = d_tri.as<double>();
     t.is_piv = d_fis_piv.as<int32_t>();
