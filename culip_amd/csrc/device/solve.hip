@@ -994,12 +994,137 @@ struct JacobiHead {
     VT iv;
 };
 
+// The item's block rows two at a time, lanes 0-31 one and lanes 32-63 the
+// next, for block rows of at most 64 entries (one chunk). A chunk's first 32
+// entries are scanned by the half's lanes, where the steps within 16 lanes and
+// over lane 15 are the same as in a chunk of its own; where some block row of
+// the item has more (wide), the other 32 are scanned the same way, and the
+// step over lane 31 is the sum of the first half's last lane, added where the
+// segment goes on: the chunk's tree. A sweep over small blocks is bound by
+// instructions, not by bytes (about 300 per block row; 28 of a chunk's 64 lanes
+// are in use at a block height of 8). All loads of the item (two passes) go
+// out together. 256 systems of 1,000-10,000 rows: 91.2 us per sweep one block
+// row at a time, 67.5 us so. offdiag: the item has an off-diagonal entry, so
+// o_col may be read at the clamped places. y64, res64: 64 doubles of LDS each.
+template<typename VT>
+__device__ __forceinline__ void jacobi_pairs(int4 tk, int cnt, bool offdiag, bool wide,
+    const int32_t* o_col,
+    const VT* o_val, const uint8_t* o_lr, const int32_t* i_col, const VT* i_val,
+    const uint8_t* i_lr, const double* b, const double* xsrc, double* xout, double* y64,
+    double* res64)
+{
+    constexpr int PASSES = JACOBI_BATCH_ROWS / 2;
+    const int lane = lane_id(), l = lane & 31, half = lane & 32;
+    int fr[PASSES], h[PASSES], sg[PASSES], ic[PASSES], il[PASSES], ni[PASSES], c[PASSES];
+    int sg2[PASSES], c2[PASSES];
+    VT v[PASSES], v2[PASSES], iv[PASSES];
+    double bo[PASSES], xv[PASSES], xv2[PASSES];
+#pragma unroll
+    for(int q = 0; q < PASSES; ++q) {
+        const int j = 2 * q + (lane >> 5);
+        const int jc = min(j, cnt - 1);
+        fr[q] = __shfl(tk.x, 2 * jc);
+        h[q] = j < cnt ? __shfl(tk.y, 2 * jc) : 0;
+        const int hc = max(__shfl(tk.y, 2 * jc), 1);
+        const int ob = __shfl(tk.z, 2 * jc), ow = __shfl(tk.w, 2 * jc);
+        const int oe = offdiag && j < cnt ? ow : ob;
+        const int ib = __shfl(tk.x, 2 * jc + 1), ie = __shfl(tk.y, 2 * jc + 1);
+        ni[q] = j < cnt ? ie - ib : 0;
+        bo[q] = b[fr[q] + min(l, hc - 1)];
+        const int ei = ib + min(l, max(ie - ib - 1, 0));
+        ic[q] = i_col[ei];
+        iv[q] = i_val[ei];
+        il[q] = i_lr[ei];
+        c[q] = 0;
+        v[q] = (VT) 0;
+        sg[q] = 64;
+        if(offdiag) {
+            const int e = max(min(ob + l, oe - 1), 0);
+            c[q] = o_col[e];
+            const VT vr = o_val[e];
+            const int sr = o_lr[e];
+            if(ob + l < oe) {
+                v[q] = vr;
+                sg[q] = sr;
+            }
+        }
+        c2[q] = 0;
+        v2[q] = (VT) 0;
+        sg2[q] = 64;
+        if(wide) {
+            const int e = max(min(ob + 32 + l, oe - 1), 0);
+            c2[q] = o_col[e];
+            const VT vr = o_val[e];
+            const int sr = o_lr[e];
+            if(ob + 32 + l < oe) {
+                v2[q] = vr;
+                sg2[q] = sr;
+            }
+        }
+    }
+#pragma unroll
+    for(int q = 0; q < PASSES; ++q) {
+        xv[q] = offdiag && sg[q] < 64 ? xsrc[c[q]] : 0.0;
+        xv2[q] = wide && sg2[q] < 64 ? xsrc[c2[q]] : 0.0;
+    }
+#pragma unroll
+    for(int q = 0; q < PASSES; ++q) {
+        if(2 * q >= cnt) break;
+        double y = l < h[q] ? bo[q] : 0.0;
+        y64[lane] = y;
+        wave_sync();
+        if(offdiag) {
+            // distinct segments in the two halves
+            const int seg = sg[q] < 64 ? sg[q] + half : 64;
+            const double p = seg_scan_runs_fma((double) v[q], xv[q], half ? seg + 64 : seg);
+            int nsg = next_lane(seg, -1);
+            if(wide) {
+                const int seg2 = sg2[q] < 64 ? sg2[q] + half : 64;
+                double p2 = seg_scan_runs_fma((double) v2[q], xv2[q], half ? seg2 + 64 : seg2);
+                const double last = __shfl(p, half + 31);
+                const int seg31 = __shfl(seg, half + 31);
+                if(seg2 < 64 && seg31 == seg2) p2 = p2 + last;
+                const int first2 = __shfl(seg2, half);
+                if(l == 31) nsg = first2;
+                if(seg < 64 && nsg != seg) y64[seg] -= p;
+                const int nsg2 = next_lane(seg2, -1);
+                wave_sync();
+                if(seg2 < 64 && (l == 31 || nsg2 != seg2)) y64[seg2] -= p2;
+            } else if(seg < 64 && (l == 31 || nsg != seg)) {
+                y64[seg] -= p;
+            }
+            wave_sync();
+            y = y64[lane];
+        }
+        // U_ii^-1: one entry per row on the diagonal in both block rows, or
+        // one scan over the entries of both
+        double r;
+        if(wave_ballot(l < h[q] && (ni[q] != h[q] || il[q] != l || ic[q] != fr[q] + l)) == 0ull) {
+            r = fma((double) iv[q], y, 0.0);
+        } else {
+            const bool in = l < ni[q];
+            const int seg = in ? il[q] + half : 64;
+            res64[lane] = 0.0;
+            const double yv = y64[in ? half + ic[q] - fr[q] : lane];
+            const double p = seg_scan_runs_fma(in ? (double) iv[q] : 0.0, yv, half ? seg + 64 : seg);
+            const int nsg = next_lane(seg, -1);
+            wave_sync();
+            if(seg < 64 && (l == 31 || nsg != seg)) res64[seg] += p;
+            wave_sync();
+            r = res64[lane];
+        }
+        if(l < h[q]) xout[fr[q] + l] = r;
+        wave_sync();
+    }
+}
+
 template<typename VT>
 __global__ __launch_bounds__(64) void bk_jacobi_sweep(const int2* items, const BatchSys* sys,
     int32_t tr, int32_t b_id, int32_t in, int32_t out)
 {
-    __shared__ double y[33];
-    __shared__ double res[33];
+    __shared__ double y64[64], res64[64];
+    double* y = y64;
+    double* res = res64;
     const int lane = lane_id();
     const int2 it = items[blockIdx.x];
     if(it.x < 0) return;   // a hole of an XCD-aware list
@@ -1096,6 +1221,17 @@ __global__ __launch_bounds__(64) void bk_jacobi_sweep(const int2* items, const B
         if(lane < h) xout[fr + lane] = r;
         wave_sync();
     };
+    // two block rows per pass where every block row of the item has at most
+    // 64 entries off the diagonal and 32 in U_ii^-1
+    const int off_cnt = offdiag ? tk.w - tk.z : 0, inv_cnt = __shfl(tk.y - tk.x, lane | 1);
+    const bool mine = lane < 2 * cnt && (lane & 1) == 0;
+    if(wave_ballot(mine && (off_cnt > 64 || inv_cnt > 32)) == 0ull) {
+        const bool some = wave_ballot(mine && off_cnt > 0) != 0ull;
+        const bool wide = wave_ballot(mine && off_cnt > 32) != 0ull;
+        jacobi_pairs<VT>(tk, cnt, some, wide, o_col, o_val, o_lr, i_col, i_val, i_lr, b, xsrc,
+            xout, y64, res64);
+        return;
+    }
     JacobiHead<VT> A, B;
     head(0, A);
     gather(0, A);
