@@ -49,6 +49,35 @@ __device__ __forceinline__ int64_t pair_first(int4 t2)
     return (int64_t) (((uint64_t) (uint32_t) t2.w << 32) | (uint32_t) t2.x);
 }
 
+__device__ __forceinline__ double lane_value(double v, int src)
+{
+    const unsigned long long b = (unsigned long long) __double_as_longlong(v);
+    const unsigned lo = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) b, src);
+    const unsigned hi = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) (b >> 32), src);
+    return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+}
+
+__device__ __forceinline__ float lane_value(float v, int src)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+
+// ix / w for an entry index ix < 1024 and a width 1 <= w <= 32 as
+// (ix * m) >> 20, m = ceil(2^20 / w): the excess ix (m w - 2^20) / (2^20 w) is
+// below 1023 * 31 / 2^20 / w < 1 / w
+struct RowOf {
+    uint32_t m;
+    int w;
+    __device__ __forceinline__ explicit RowOf(int w_) : m(((1u << 20) + w_ - 1) / w_), w(w_) {}
+    __device__ __forceinline__ int row(int ix) const { return (int) (((uint32_t) ix * m) >> 20); }
+    // 32 row + column
+    __device__ __forceinline__ int at(int ix) const
+    {
+        const int r = row(ix);
+        return 32 * r + (ix - r * w);
+    }
+};
+
 template<typename VT>
 __device__ __forceinline__ void tile_zero(VT* T)
 {
@@ -71,6 +100,7 @@ template<typename VT>
 __device__ void tile_load(VT* T, int4 m, int h, int w, const int32_t* ixs, const VT* vals)
 {
     const int lane = lane_id();
+    const RowOf width(w);
     tile_zero(T);
     wave_sync();
     if(m.x == FMT_DENSE) {
@@ -81,9 +111,7 @@ __device__ void tile_load(VT* T, int4 m, int h, int w, const int32_t* ixs, const
         }
     } else {
         for(int e = lane; e < m.y; e += 64) {
-            const int ix = ixs[(int64_t) m.z + e];
-            const int r = ix / w, c = ix - r * w;
-            T[32 * r + c] = vals[(int64_t) m.w + e];
+            T[width.at(ixs[(int64_t) m.z + e])] = vals[(int64_t) m.w + e];
         }
     }
     wave_sync();
@@ -161,15 +189,15 @@ __device__ __forceinline__ Pre<VT> prefetch(const Dep& d, const int32_t* ixs, co
 // Writes a dependency block (width w) into tile X and, when mask is set,
 // the nonzero rows of each column into mask[c] (LDS, integer atomics).
 template<typename VT>
-__device__ void stage(VT* X, uint32_t* mask, const Dep& d, const Pre<VT>& p, int w,
+__device__ void stage(VT* X, uint32_t* mask, const Dep& d, const Pre<VT>& p, const RowOf& wd,
     const int32_t* ixs, const VT* vals)
 {
-    const int lane = lane_id();
+    const int lane = lane_id(), w = wd.w;
     if(small_sparse<VT>(d)) {
         if(lane < d.nnz) {
-            const int r = p.ix / w, c = p.ix - r * w;
-            X[32 * r + c] = p.v;
-            if(mask && p.v != (VT) 0) atomicOr(&mask[c], 1u << r);
+            const int k = wd.at(p.ix);
+            X[k] = p.v;
+            if(mask && p.v != (VT) 0) atomicOr(&mask[k & 31], 1u << (k >> 5));
         }
     } else if(d.fmt == FMT_DENSE) {
 #pragma unroll
@@ -185,22 +213,19 @@ __device__ void stage(VT* X, uint32_t* mask, const Dep& d, const Pre<VT>& p, int
         for(int e = lane; e < d.nnz; e += 64) {
             const int ix = ixs[(int64_t) d.cp + e];
             const VT v = vals[(int64_t) d.vp + e];
-            const int r = ix / w, c = ix - r * w;
-            X[32 * r + c] = v;
-            if(mask && v != (VT) 0) atomicOr(&mask[c], 1u << r);
+            const int k = wd.at(ix);
+            X[k] = v;
+            if(mask && v != (VT) 0) atomicOr(&mask[k & 31], 1u << (k >> 5));
         }
     }
 }
 
 template<typename VT>
-__device__ void unstage(VT* X, uint32_t* mask, const Dep& d, const Pre<VT>& p, int w)
+__device__ void unstage(VT* X, uint32_t* mask, const Dep& d, const Pre<VT>& p, const RowOf& wd)
 {
     const int lane = lane_id();
     if(small_sparse<VT>(d)) {
-        if(lane < d.nnz) {
-            const int r = p.ix / w, c = p.ix - r * w;
-            X[32 * r + c] = (VT) 0;
-        }
+        if(lane < d.nnz) X[wd.at(p.ix)] = (VT) 0;
     } else {
         tile_zero(X);
     }
@@ -395,22 +420,6 @@ __device__ bool step_2x2(VT* T, double* tri, int p, int len)
     wave_sync();
     return fabs(d11) + fabs(d12) + fabs(d22) < (AT) INFINITY;   // D is finite
 }
-
-// ix / w for an entry index ix < 1024 and a width 1 <= w <= 32 as
-// (ix * m) >> 20, m = ceil(2^20 / w): the excess ix (m w - 2^20) / (2^20 w) is
-// below 1023 * 31 / 2^20 / w < 1 / w
-struct RowOf {
-    uint32_t m;
-    int w;
-    __device__ __forceinline__ explicit RowOf(int w_) : m(((1u << 20) + w_ - 1) / w_), w(w_) {}
-    __device__ __forceinline__ int row(int ix) const { return (int) (((uint32_t) ix * m) >> 20); }
-    // 32 row + column
-    __device__ __forceinline__ int at(int ix) const
-    {
-        const int r = row(ix);
-        return 32 * r + (ix - r * w);
-    }
-};
 
 // entries of a block taken by the one-lane forms, and updates beside the
 // diagonal one such block may make in a pivot tile
@@ -1080,23 +1089,54 @@ __device__ __forceinline__ EntryList<VT> entry_list(const FactorArgs<VT>& a, int
         a.if_val + (int64_t) q * 1024, a.if_idx + (int64_t) q * 1024};
 }
 
-// a scaled off-diagonal tile X (one wave, stride 32) as position q leaves
-// it: row sums of squares, and the dense tile or the entries above NZ_EPS
+// An off-diagonal tile X (one wave, stride 32, zero outside hgt x wid) as
+// position q leaves it: divided by D where that is left to do (by_d; d_row
+// holds row l's 1x1 pivot in lane l; a finite D leaves a row of zeros as it
+// is), then the row sums of squares and the dense tile or the entries above
+// NZ_EPS. The tile is mostly zeros: the loop takes the pairs of rows that have
+// an entry.
 template<typename VT>
-__device__ __forceinline__ void offdiag_output(const FactorArgs<VT>& a, int q, const VT* X, int hgt, int wid,
-    int format)
+__device__ __forceinline__ void offdiag_output(const FactorArgs<VT>& a, int q, VT* X, bool by_d,
+    bool nonfinite, double d_row, int hgt, int wid, int format)
 {
     const int lane = lane_id();
+    const EntryList<VT> o = entry_list(a, q);
+    uint32_t act = 0;
+#pragma unroll
+    for(int t = 0; t < 16; ++t)
+        if(wave_ballot(X[64 * t + lane] != (VT) 0)) act |= 1u << t;
+    if(by_d && nonfinite) act = (uint32_t) ((1ull << ((hgt + 1) / 2)) - 1ull);
     // nonzero entries per row; a row's sum skips exact zeros
     uint32_t nz = 0;
-#pragma unroll
-    for(int t = 0; t < 16; ++t) {
-        const int r = 2 * t + (lane >> 5), c = lane & 31;
-        const uint64_t b = wave_ballot(r < hgt && c < wid && X[64 * t + lane] != (VT) 0);
+    int base = 0;
+#pragma unroll 1
+    for(; act; act &= act - 1) {
+        const int t = __ffs(act) - 1;
+        VT x = X[64 * t + lane];
+        if(by_d) {
+            const uint64_t b = wave_ballot(x != (VT) 0);
+            const double lo = lane_value(d_row, 2 * t), hi = lane_value(d_row, 2 * t + 1);
+            const bool some = (lane < 32 ? (uint32_t) b : (uint32_t) (b >> 32)) != 0u;
+            const bool in = (lane & 31) < wid && 2 * t + (lane >> 5) < hgt;
+            const VT y = (VT) ((double) x / (lane < 32 ? lo : hi));
+            if(in && (some || nonfinite)) {
+                x = y;
+                X[64 * t + lane] = y;
+            }
+        }
+        const uint64_t b = wave_ballot(x != (VT) 0);
         if(lane == 2 * t) nz = (uint32_t) b;
         if(lane == 2 * t + 1) nz = (uint32_t) (b >> 32);
+        if(format != FMT_DENSE) {
+            const bool live = fabs((double) x) > NZ_EPS;
+            const uint64_t msk = wave_ballot(live);
+            if(live) o.set(base + lanes_below(msk), 64 * t + lane, x);
+            base += __popcll(msk);
+        }
     }
+    wave_sync();
     VT ssq = (VT) 0;
+#pragma unroll 1
     for(uint32_t bits = nz; bits; bits &= bits - 1) {
         const VT v = X[32 * lane + __ffs(bits) - 1];
         ssq = fma(v, v, ssq);
@@ -1107,30 +1147,19 @@ __device__ __forceinline__ void offdiag_output(const FactorArgs<VT>& a, int q, c
         if(j == 0) a.rn_first[q] = ssq;
         else a.rn_part[(int64_t) q * 32 + j] = ssq;
     }
-    if(lane == 0) a.part_mask[q] = (uint32_t) rows;
     if(format == FMT_DENSE) {
         VT* oval = a.if_val + (int64_t) q * 1024;
-        for(int e = lane; e < hgt * wid; e += 64) {
-            const int r = e / wid, c = e - r * wid;
-            oval[e] = X[32 * r + c];
+#pragma unroll 4
+        for(int t = 0; t < 16; ++t) {
+            const int r = 2 * t + (lane >> 5), c = lane & 31;
+            if(r < hgt && c < wid) oval[r * wid + c] = X[64 * t + lane];
         }
-        if(lane == 0) a.if_cnt[q] = hgt * wid;
-        return;
+        base = hgt * wid;
     }
-    auto live = [&](int t) {
-        const int idx = 64 * t + lane, r = idx >> 5, c = idx & 31;
-        return r < hgt && c < wid && fabs((double) X[idx]) > NZ_EPS;
-    };
-    const EntryList<VT> o = entry_list(a, q);
-    int base = 0;
-#pragma unroll
-    for(int t = 0; t < 16; ++t) {
-        const bool pred = live(t);
-        const uint64_t msk = wave_ballot(pred);
-        if(pred) o.set(base + lanes_below(msk), 64 * t + lane, X[64 * t + lane]);
-        base += __popcll(msk);
+    if(lane == 0) {
+        a.part_mask[q] = (uint32_t) rows;
+        a.if_cnt[q] = base;
     }
-    if(lane == 0) a.if_cnt[q] = base;
 }
 
 // k_update_scale_offdiagonal_blocks (kernels :1628-1803) with
@@ -1167,6 +1196,7 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
     const int np = (int) (a.upd_off[b + 1] - p0);
     const int pq = a.piv_loc[i];
     const bool all1x1 = (wave_ballot(lane < hgt && !a.is_piv[fr + (lane & 31)]) == 0);
+    const RowOf height(hgt), width(wid);
     tile_zero(s.A);
     if(lane < 32) { s.mask[lane] = 0; s.umask[lane] = 0; }
     if(np > 0) tile_zero(s.R);
@@ -1199,14 +1229,14 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
                 qi = prefetch(ni, a.ix_out, a.val_out, a.tri, true);
                 qj = prefetch(nj, a.ix_out, a.val_out, a.tri, false);
             }
-            stage(s.A, (uint32_t*) nullptr, ci, pi, hgt, a.ix_out, a.val_out);
-            stage(s.R, s.mask, cj, pj, wid, a.ix_out, a.val_out);
+            stage(s.A, (uint32_t*) nullptr, ci, pi, height, a.ix_out, a.val_out);
+            stage(s.R, s.mask, cj, pj, width, a.ix_out, a.val_out);
             stage_d(s.cs, s.cd, s.cb, pi);
             wave_sync();
             product(s.T, s.A, s.R, s.mask, s.cs, s.cd, s.cb, hgt, wid);
             wave_sync();
-            unstage(s.A, (uint32_t*) nullptr, ci, pi, hgt);
-            unstage(s.R, s.mask, cj, pj, wid);
+            unstage(s.A, (uint32_t*) nullptr, ci, pi, height);
+            unstage(s.R, s.mask, cj, pj, width);
             wave_sync();
             ci = ni; cj = nj; pi = qi; pj = qj;
         }
@@ -1279,15 +1309,7 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
         }
     }
     wave_sync();
-    offdiag_output(a, q, s.T, hgt, wid, m.format);
-}
-
-__device__ __forceinline__ double lane_value(double v, int src)
-{
-    const unsigned long long b = (unsigned long long) __double_as_longlong(v);
-    const unsigned lo = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) b, src);
-    const unsigned hi = (unsigned) __builtin_amdgcn_readlane((int) (unsigned) (b >> 32), src);
-    return __longlong_as_double((long long) (((unsigned long long) hi << 32) | lo));
+    offdiag_output(a, q, s.T, false, false, 0.0, hgt, wid, m.format);
 }
 
 // ---------------------------------------------------------------------------
@@ -1355,19 +1377,32 @@ __device__ void product_list(VT* T, const VT* A, const VT* rv, const uint8_t* rl
     const int k0 = (j < rh) ? cst[j] : 0;
     const int k1 = (j < rh) ? cst[j + 1] : 0;
     if(k0 < k1) {
-        // one output row at a time keeps a single accumulator live
-        for(int c = c0; c < lh; c += 2) {
-            VT acc = 0;
+        // four output rows of a lane together: their LDS reads are in flight at
+        // once (one row at a time waits for them 16 times: 5.8 us a pair)
+#pragma unroll 1
+        for(int c4 = c0; c4 < lh; c4 += 8) {
+            VT acc[4];
+#pragma unroll
+            for(int t = 0; t < 4; ++t) acc[t] = 0;
+#pragma unroll 1
             for(int k = k0; k < k1; ++k) {
                 const int l = rl[k];
                 const VT r = rv[k];
-                const VT left = (l == 0) ? (VT) 0 : A[32 * (l - 1) + c];
-                const VT mid = A[32 * l + c];
-                const VT right = (l == 31) ? (VT) 0 : A[32 * (l + 1) + c];
-                const VT lt = fma(cb[l], right, fma(cd[l], mid, cs[l] * left));
-                acc = fma(r, lt, acc);
+                const VT sup = cs[l], dia = cd[l], sub = cb[l];
+                const VT* Al = A + 32 * l + c4;
+                const VT* Ap = l == 0 ? Al : Al - 32;
+                const VT* An = l == 31 ? Al : Al + 32;
+#pragma unroll
+                for(int t = 0; t < 4; ++t) {
+                    const VT left = (l == 0) ? (VT) 0 : Ap[2 * t];
+                    const VT right = (l == 31) ? (VT) 0 : An[2 * t];
+                    const VT lt = fma(sub, right, fma(dia, Al[2 * t], sup * left));
+                    acc[t] = fma(r, lt, acc[t]);
+                }
             }
-            T[32 * c + j] -= acc;
+#pragma unroll
+            for(int t = 0; t < 4; ++t)
+                if(c4 + 2 * t < lh) T[32 * (c4 + 2 * t) + j] -= acc[t];
         }
     }
 }
@@ -1455,6 +1490,17 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
     const uint32_t um_row = (lane < hgt) ? a.piv_umask[(int64_t) pq * 32 + lane] : 0u;
     const double d_row = a.tri[3 * (int64_t) (fr + min(lane, hgt - 1)) + 1];
     tile_load(s.X, t1, hgt, wid, a.ix_in, a.val_in);
+    // U_ii for the end, rows 2 t and 2 t + 1 in register t (what lies beyond
+    // its hgt x hgt elements is not used)
+    VT u[16];
+#pragma unroll
+    for(int t = 0; t < 16; ++t) u[t] = (VT) 0;
+    if(flags & PIV_ANY) {
+        const VT* piv = a.if_val + (int64_t) pq * 1024;
+        const int u0 = (lane >> 5) * hgt + (lane & 31);
+#pragma unroll
+        for(int t = 0; t < 16; ++t) u[t] = piv[min(u0 + 2 * t * hgt, 1023)];
+    }
     bool staging = false;   // s.A is zero
     const RowOf height(hgt), width(wid);
 
@@ -1470,10 +1516,18 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
             if(hit) {
                 mi = dep_meta(a.bout, pr.x, pr.z, pr.w);
                 mj = dep_meta(a.bout, pr.y, pr.z, pr.w);
-                light = light_pair<VT, LIGHT_E>(mi, mj, height, width, a.ix_out, a.val_out, a.tri,
-                    up);
             }
         }
+        if(!wave_ballot(hit)) continue;
+        // the form costs the square of its entries: the short one where no
+        // pair in it would need more
+        const bool in_form = hit && mi.fmt == FMT_SPARSE && mi.nnz <= LIGHT_E &&
+            mj.fmt == FMT_SPARSE && mj.nnz <= LIGHT_E;
+        const bool longer = wave_ballot(in_form && max(mi.nnz, mj.nnz) > LIGHT_E / 2) != 0ull;
+        if(in_form)
+            light = longer ?
+                light_pair<VT, LIGHT_E>(mi, mj, height, width, a.ix_out, a.val_out, a.tri, up) :
+                light_pair<VT, LIGHT_E / 2>(mi, mj, height, width, a.ix_out, a.val_out, a.tri, up);
         if(wave_ballot(hit && !light && !small_sparse<VT>(mj))) {
             if(lane == 0) a.defer_list[atomicAdd(a.defer_cnt + lr.level, 1)] = q;
             return;
@@ -1498,13 +1552,13 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
             const Dep ci = bcast(mi, d), cj = bcast(mj, d);
             const Pre<VT> pi = prefetch(ci, a.ix_out, a.val_out, a.tri, true);
             const Pre<VT> pj = prefetch(cj, a.ix_out, a.val_out, a.tri, false);
-            stage(s.A, (uint32_t*) nullptr, ci, pi, hgt, a.ix_out, a.val_out);
+            stage(s.A, (uint32_t*) nullptr, ci, pi, height, a.ix_out, a.val_out);
             list_build(s.rv, s.rl, s.cst, cj, pj, wid);
             stage_d(s.cs, s.cd, s.cb, pi);
             wave_sync();
             product_list(s.X, s.A, s.rv, s.rl, s.cst, s.cs, s.cd, s.cb, hgt, wid);
             wave_sync();
-            unstage(s.A, (uint32_t*) nullptr, ci, pi, hgt);
+            unstage(s.A, (uint32_t*) nullptr, ci, pi, height);
             wave_sync();
         }
     }
@@ -1518,53 +1572,45 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
         }
         wave_sync();
     }
+    // U_ii' forward substitution over the pivot rows with an element beyond the
+    // diagonal and a nonzero in the tile (exact no-ops are skipped): the lanes
+    // of both halves hold the row, lane l updates elements 64 t + l of the
+    // tile. Short loops: with all 32 x 32 steps written out the code did not
+    // fit beside the rest in the instruction cache, and a CU's first block of a
+    // launch took 11-24 us here, where later ones took 0.7
+    if(flags & PIV_ANY) {
+#pragma unroll
+        for(int t = 0; t < 16; ++t) s.A[64 * t + lane] = u[t];
+        wave_sync();
+#pragma unroll 1
+        for(uint64_t m = wave_ballot(um_row != 0u); m; m &= m - 1) {
+            const int ii = __ffsll((long long) m) - 1;
+            const uint32_t um = (uint32_t) __builtin_amdgcn_readlane((int) um_row, ii);
+            const VT x = s.X[32 * ii + (lane & 31)];
+            const bool on = x != (VT) 0;
+            if(wave_ballot(on) == 0ull) continue;
+            const VT pv = x / s.A[33 * ii];
+#pragma unroll 1
+            for(int g = 0; g < 4; ++g) {
+                const uint32_t bits = (um >> (8 * g)) & 255u;
+                if(bits == 0u) continue;
+                VT* X = s.X + 256 * g + lane;
+                const VT* U = s.A + 32 * ii + 8 * g + (lane >> 5);
+                VT y[4];
+#pragma unroll
+                for(int t = 0; t < 4; ++t) y[t] = fma(-U[2 * t], pv, X[64 * t]);
+#pragma unroll
+                for(int t = 0; t < 4; ++t)
+                    if(on && ((bits >> (2 * t + (lane >> 5))) & 1u)) X[64 * t] = y[t];
+            }
+            wave_sync();
+        }
+    }
     const int jc = lane;
     VT* col = s.X + jc;
-    // U_ii' forward substitution, column jc per lane (lanes >= 32 idle), over
-    // the nonzero columns of the pivot rows (exact no-ops skipped), the
-    // column in registers and U_ii in LDS
-    if(flags & PIV_ANY) {
-        const VT* piv = a.if_val + (int64_t) pq * 1024;
-        for(int e = lane; e < hgt * hgt; e += 64) {
-            const int r = e / hgt;
-            s.A[32 * r + (e - r * hgt)] = piv[e];
-        }
-        wave_sync();
-        VT x[32];
-#pragma unroll
-        for(int l = 0; l < 32; ++l) x[l] = (l < hgt && jc < wid) ? col[32 * l] : (VT) 0;
-#pragma unroll
-        for(int ii = 0; ii < 32; ++ii) {
-            const uint32_t um = (uint32_t) __builtin_amdgcn_readlane((int) um_row, ii);
-            if(um && wave_ballot(x[ii] != (VT) 0)) {
-                const bool on = x[ii] != (VT) 0;
-                const VT pv = x[ii] / s.A[33 * ii];
-#pragma unroll
-                for(int l = ii + 1; l < 32; ++l)
-                    if((um >> l) & 1u) {
-                        const VT y = fma(-s.A[32 * ii + l], pv, x[l]);
-                        x[l] = on ? y : x[l];
-                    }
-            }
-        }
-        if(jc < wid) {
-#pragma unroll
-            for(int l = 0; l < 32; ++l)
-                if(l < hgt) col[32 * l] = x[l];
-        }
-        wave_sync();
-    }
     // D solve in place (d_left_solve_with_D_Ut, kernels :1533-1566); a row
     // is written only after both rows it reads have been read
-    if(!(flags & PIV_2X2)) {
-        for(int l = 0; l < hgt; ++l) {
-            const VT x = (jc < wid) ? col[32 * l] : (VT) 0;
-            // a finite D leaves a row of zeros as it is
-            if(wave_ballot(x != (VT) 0) == 0ull && !(flags & PIV_NONFINITE)) continue;
-            const double dl = lane_value(d_row, l);
-            if(jc < wid) col[32 * l] = (VT) ((double) x / dl);
-        }
-    } else if(jc < wid) {
+    if((flags & PIV_2X2) && jc < wid) {
         const double* D = a.tri + 3 * (int64_t) fr;
         const int32_t* ip = a.is_piv + fr;
         for(int l = 0; l < hgt; ++l) {
@@ -1579,7 +1625,7 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
         }
     }
     wave_sync();
-    offdiag_output(a, q, s.X, hgt, wid, t1.x);
+    offdiag_output(a, q, s.X, !(flags & PIV_2X2), flags & PIV_NONFINITE, d_row, hgt, wid, t1.x);
 }
 
 // the positions k_offdiag_tiny leaves to the wave form, grid-stride
