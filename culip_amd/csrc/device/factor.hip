@@ -856,23 +856,29 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
     int blk = (t < nd) ? a.csc_idx[cb0 + t] : -1;
     int piv = 1;
     if(t < 32 && t < len) piv = a.is_piv[fr + t];
-    for(int e = t; e < 1024; e += TPB) {
-        const int r = e >> 5, c = e & 31;
-        VT v = (VT) 0;
-        if(t1.x == FMT_DENSE && r < len && c < len) v = a.val_in[(int64_t) t1.w + r * len + c];
-        s.T[e] = v;
-    }
-    if(t1.x != FMT_DENSE) {
-        __syncthreads();
-        for(int e = t; e < t1.y; e += TPB) {
-            const int ix = a.ix_in[(int64_t) t1.z + e];
-            const int r = ix / len;
-            s.T[32 * r + (ix - r * len)] = a.val_in[(int64_t) t1.w + e];
+    const RowOf width(len);
+    if(t1.x == FMT_DENSE) {
+        // all of a thread's loads in flight at once, at places within the block
+        // (one by one under their own conditions: 5 us of a one-wave block's 25)
+        VT v[1024 / TPB];
+#pragma unroll
+        for(int k = 0; k < 1024 / TPB; ++k) {
+            const int e = t + TPB * k, r = min(e >> 5, len - 1), c = min(e & 31, len - 1);
+            v[k] = a.val_in[(int64_t) t1.w + r * len + c];
         }
+#pragma unroll
+        for(int k = 0; k < 1024 / TPB; ++k) {
+            const int e = t + TPB * k;
+            s.T[e] = ((e >> 5) < len && (e & 31) < len) ? v[k] : (VT) 0;
+        }
+    } else {
+        for(int e = t; e < 1024; e += TPB) s.T[e] = (VT) 0;
+        __syncthreads();
+        for(int e = t; e < t1.y; e += TPB)
+            s.T[width.at(a.ix_in[(int64_t) t1.z + e])] = a.val_in[(int64_t) t1.w + e];
     }
     __syncthreads();
     // updates from the blocks (k, i) above the diagonal, in CSC order
-    const RowOf width(len);
     for(int c0 = 0; c0 < nd; c0 += TPB) {
         if(c0) blk = (c0 + t < nd) ? a.csc_idx[cb0 + c0 + t] : -1;
         Dep d{};
@@ -1011,11 +1017,12 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
     __syncthreads();
     // the remaining rows' steps: step_1x1 without its trailing update
     if(s.plain) {
+        const uint32_t rows = s.plain, ones = s.tiny;
+#pragma unroll 4
         for(int e = t; e < 1024; e += TPB) {
             const int r = e >> 5, c = e & 31;
-            if(!((s.plain >> r) & 1u)) continue;
             const VT u = ((c < r) ? (VT) 0 : T0[e]) / s.dia[r];
-            T0[e] = (c == r && ((s.tiny >> r) & 1u)) ? (VT) 1 : u;
+            if((rows >> r) & 1u) T0[e] = (c == r && ((ones >> r) & 1u)) ? (VT) 1 : u;
         }
         __syncthreads();
     }
@@ -1057,9 +1064,9 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
     // (k_drop)
     VT* out = a.if_val + (int64_t) q * 1024;
     VT* fin = a.val_out + ((int64_t) t1.w - pool);
+#pragma unroll 4
     for(int e = t; e < len * len; e += TPB) {
-        const int r = e / len, c = e - r * len;
-        const VT v = T0[32 * r + c];
+        const VT v = T0[width.at(e)];
         out[e] = v;
         fin[e] = v;
     }

@@ -1429,7 +1429,7 @@ template void solve_plan_fill<float>(const SolveTopo&, const float*, const float
 // same time (other kernels end on their own), so at most a quarter of what a
 // CU holds: its registers let a CU hold 12 of this kernel's waves, three per
 // solve. (Compiled for 16 per CU, it spills 18-25 registers inside the rows'
-// critical path: 430 us instead of 236 for both solves at n = 400,000.)
+// critical path: 403 us instead of 236 for both solves at n = 400,000.)
 constexpr int CHAIN_WAVES_PER_CU = 4;
 
 // grid of k_trsv_chain: CHAIN_WAVES_PER_CU waves per CU, fewer when the
