@@ -3,7 +3,7 @@
 // Reference: libs/la/preconditioner/block_ildlt.impl.cuh:1519-1671 (schedule)
 // and block_ildlt_kernels.impl.cuh:1146-2074 (kernels). Per level:
 //   k_pivots_pairs
-//               one wave per pivot block: A_ii -= sum_k U_ki' D_k U_ki over
+//               one or four waves per pivot block: A_ii -= sum_k U_ki' D_k U_ki over
 //               the block column, 1x1/2x2 LDL' of the tile (static or
 //               numeric pivots), row sums; in the same launch, one lane per
 //               small off-diagonal block: its Schur updates
@@ -22,11 +22,9 @@
 //   k_store     one wave per remaining block: compacted final storage
 //
 // The dependency blocks of a tile are walked with their metadata fetched
-// lane-parallel up front. In the pivot blocks a block whose nonzero entries share
-// one column (one entry, on sparse KKT patterns) has its whole update -- one
-// diagonal element -- formed by its own lane, so the serial walk over the
-// block column costs a few scalar instructions per block; other blocks are
-// staged as tiles. The update U' D U is applied over the nonzero rows
+// lane-parallel up front. A block (or pair of blocks) of few entries has its
+// whole update formed by its own lane, and the updates are applied in block
+// order; other blocks are staged as tiles. The update U' D U is applied over the nonzero rows
 // of the right factor only, with D applied on the fly: every term the
 // reference adds is added, in the same order with the same fused
 // multiply-adds as the CPU oracle's restatement; the skipped terms are exact
@@ -565,6 +563,9 @@ __device__ __forceinline__ uint32_t store_row_mask(uint32_t m, bool any_bad, int
     return m;
 }
 
+// Most Schur pairs share no row. Leaving those out by two 4-byte masks instead
+// of the blocks' metadata and entries: refactor 10.3 -> 7.7 ms at n = 2,000,
+// 11.9 -> 10.6 ms at n = 400,000.
 __device__ __forceinline__ bool pair_matches(uint32_t mi, uint32_t mj)
 {
     return (mi & mj) != 0u || mi == ALL_ROWS || mj == ALL_ROWS;
@@ -836,6 +837,8 @@ constexpr uint32_t PIV_ANY = 1, PIV_2X2 = 2, PIV_NONFINITE = 4, PIV_PERM = 8;
 // staged one by one in their place in that order. Of the pivot steps only
 // rows with an entry right of the diagonal (or a 2x2 pivot) are steps; the
 // others scale a row and change nothing else, so they are done together last.
+// FP64 refactor, blocks above taken by rounds of one wave -> at once: 7.1 ->
+// 5.2 ms at n = 2,000, 8.3 -> 6.4 ms at n = 400,000.
 template<typename VT, int NW>
 __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
     PivLds<VT, NW>& s)
@@ -1328,7 +1331,11 @@ __device__ void offdiag_general_one(const FactorArgs<VT>& a, const LevelRange& l
 // order. Other pairs are staged one at a time in their place in that order:
 // U_ki as a tile, U_kj (at most 64 entries, else the block is handed to
 // k_offdiag_general) as a list ordered by (column, row). Arithmetic and order
-// are those of the general form.
+// are those of the general form. Bound by latency, at small sizes by the few
+// blocks with staged pairs: FP64, a level at n = 2,000 took 36.9 us with every
+// step of substitution, scaling and output written out, 24.8 with loops over
+// what is there (refactor 3.73 -> 3.27 ms; 4.23 -> 3.65 at n = 33,333 with
+// Bunch-Kaufman pivots).
 
 template<typename VT>
 struct alignas(16) OffLdsSmall {
@@ -2285,7 +2292,8 @@ __device__ __forceinline__ void drop_store(const FactorArgs<VT>& a, int q, const
 // and each thread writes its block's metadata and entries.
 // Bound by latency: about eight dependent memory round trips. It replaced a
 // row-norm launch, a chunked scan with two waits and a store launch (11.6 +
-// 36 + 8 us per level at n = 400,000, 5 + 44 + 18 us at n = 2,000).
+// 36 + 8 us per level at n = 400,000, 5 + 44 + 18 us at n = 2,000); itself 21
+// and 29 us.
 template<typename VT>
 __device__ __forceinline__ void drop_body(const FactorArgs<VT>& a, const LevelRange& lr)
 {

@@ -1003,7 +1003,7 @@ struct JacobiHead {
 // segment goes on: the chunk's tree. A sweep over small blocks is bound by
 // instructions, not by bytes (about 300 per block row; 28 of a chunk's 64 lanes
 // are in use at a block height of 8). All loads of the item (two passes) go
-// out together. 256 systems of 1,000-10,000 rows: 91.2 us per sweep one block
+// out together. 256 systems of 1,000-40,000 primal rows: 91.2 us per sweep one block
 // row at a time, 67.5 us so. offdiag: the item has an off-diagonal entry, so
 // o_col may be read at the clamped places. y64, res64: 64 doubles of LDS each.
 template<typename VT>
