@@ -300,6 +300,10 @@ class BlockiLDLt(_Handle):
         """Testing hook: records a timed-out single-launch solve from the host."""
         check(lib().culip_bildlt_inject_solve_error(self._h))
 
+    def _set_spin_limit(self, polls):
+        """Testing hook: polls after which single-launch waits give up."""
+        check(lib().culip_bildlt_set_spin_limit(self._h, polls))
+
     def _release(self):
         if getattr(self, "_h", None):
             lib().culip_bildlt_destroy(self._h)

@@ -112,6 +112,7 @@ _SIGS = [
                                         C.POINTER(C.POINTER(C.c_double)), C.POINTER(C.c_int64)]),
     ("culip_bildlt_device_bytes", C.c_int64, [C.c_void_p]),
     ("culip_bildlt_inject_solve_error", C.c_int, [C.c_void_p]),
+    ("culip_bildlt_set_spin_limit", C.c_int, [C.c_void_p, C.c_int32]),
     ("culip_bildlt_set_graphs", C.c_int, [C.c_void_p, C.c_int32]),
     ("culip_bildlt_set_pivoting", C.c_int, [C.c_void_p, C.c_int]),
     ("culip_bildlt_set_pivot_precision", C.c_int, [C.c_void_p, C.c_int]),

@@ -573,8 +573,8 @@ __global__ __launch_bounds__(64) void k_jacobi_sweep(const int4* task, const int
 // block row waits and computes, the wave already loads the task and first
 // entries of its next one. Each wave also presets its rows of next_pub, the
 // buffer of the next single-launch solve. Every wait is bounded: past
-// SPIN_LIMIT polls the wave records an error in *err and goes on.
-constexpr int SPIN_LIMIT = 1 << 22;
+// spin_limit polls the wave records an error in *err, and the block row and
+// all that depend on it become NaN.
 constexpr unsigned long long CHAIN_EMPTY = 0x7ff4c0de5eed1234ull;
 
 __device__ __forceinline__ double pub_load(const double* p)
@@ -700,11 +700,12 @@ __device__ __forceinline__ void reload_missing(const double* pub, const int (&c)
 // still on their way: the latest values of a block row all belong to the
 // levels next to its own, so they sit in one chunk (the last for U', the first
 // for U) and only that chunk's scan follows the last arrival. chunks: how many
-// of the group have entries; their values past the row's end are cleared.
+// of the group have entries; their values past the row's end are cleared. NaN
+// when the wait gives up, so that no partial sum is taken for a solution.
 template<typename VT>
 __device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup<VT>& g,
     double (&xv)[TRSV_PF], const ScanPlan (&p)[TRSV_PF], int chunks, double y, int32_t* err,
-    int& spins)
+    int32_t spin_limit, int& spins)
 {
     double sum[TRSV_PF];
     uint32_t open = chunks >= TRSV_PF ? (1u << TRSV_PF) - 1 : (1u << chunks) - 1;
@@ -724,10 +725,11 @@ __device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup
             }
         }
         if(open == 0) break;
-        if(++spins > SPIN_LIMIT) {
+        if(++spins > spin_limit) {
             // err is pinned host memory: the host reads it without a copy
             __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            return y;
+            // a quiet NaN, which readers of the row take as published
+            return __longlong_as_double(0x7ff8000000000000ll);
         }
         __builtin_amdgcn_s_sleep(1);
         reload_missing(pub, g.c, m, xv);
@@ -848,8 +850,8 @@ __device__ __forceinline__ void chain_fetch(int4 t0, int4 t1, const int32_t* o_c
 template<typename VT, bool FUSED>
 __global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t nb, int32_t reverse,
     const int32_t* o_col, const VT* o_val, const uint8_t* o_lr, const int32_t* i_col,
-    const VT* i_val, const uint8_t* i_lr, double* pub, double* next_pub, int32_t* err, double* x,
-    CsrRhs rhs)
+    const VT* i_val, const uint8_t* i_lr, double* pub, double* next_pub, int32_t* err,
+    int32_t spin_limit, double* x, CsrRhs rhs)
 {
     __shared__ double y_lds[33];     // general U_ii^-1 only
     __shared__ double res[33];
@@ -913,7 +915,7 @@ __global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t 
                 if(chunks > 1) plan[1] = scan_plan(g.sg[1], ends);
                 if(chunks > 2) plan[2] = scan_plan(g.sg[2], ends);
                 if(chunks > 3) plan[3] = scan_plan(g.sg[3], ends);
-                y = chain_sums<VT>(pub, g, xv, plan, chunks, y, err, spins);
+                y = chain_sums<VT>(pub, g, xv, plan, chunks, y, err, spin_limit, spins);
                 if(!more) break;
                 e0 += 64 * TRSV_PF;
                 g = gn;
@@ -1458,17 +1460,17 @@ int chain_grid(int32_t nb)
 template<typename VT>
 hipError_t trsv_chain(const int4* task, int32_t nb, int32_t reverse, const int32_t* o_col,
     const VT* o_val, const uint8_t* o_lr, const int32_t* i_col, const VT* i_val,
-    const uint8_t* i_lr, double* pub, double* next_pub, int32_t* err, double* x, CsrRhs rhs,
+    const uint8_t* i_lr, double* pub, double* next_pub, const SolveTopo& t, double* x, CsrRhs rhs,
     hipStream_t st)
 {
     const int g = chain_grid<VT>(nb);
     if(g <= 0) return hipErrorInvalidConfiguration;
     if(rhs.rp)
         k_trsv_chain<VT, true><<<g, 64, 0, st>>>(task, nb, reverse, o_col, o_val, o_lr, i_col, i_val,
-            i_lr, pub, next_pub, err, x, rhs);
+            i_lr, pub, next_pub, t.err, t.spin_limit, x, rhs);
     else
         k_trsv_chain<VT, false><<<g, 64, 0, st>>>(task, nb, reverse, o_col, o_val, o_lr, i_col,
-            i_val, i_lr, pub, next_pub, err, x, rhs);
+            i_val, i_lr, pub, next_pub, t.err, t.spin_limit, x, rhs);
     return hipGetLastError();
 }
 
@@ -1480,7 +1482,7 @@ int trsv_upper_single(const SolveTopo& t, const SolvePlan<VT>& p, double* x, int
     double* pub = t.chain_pub + (parity ? t.n : 0);
     double* next = t.chain_pub + (parity ? 0 : t.n);
     return (int) trsv_chain<VT>(p.task_u, t.nb, 1, p.uo_col, p.uo_val, p.uo_lr, p.ui_col, p.ui_val,
-        p.ui_lr, pub, next, t.err, x, CsrRhs{nullptr, nullptr, nullptr, nullptr},
+        p.ui_lr, pub, next, t, x, CsrRhs{nullptr, nullptr, nullptr, nullptr},
         (hipStream_t) stream);
 }
 
@@ -1501,7 +1503,7 @@ int trsv_upper_t_single_product(const SolveTopo& t, const SolvePlan<VT>& p, cons
     const CsrRhs rhs = K ? CsrRhs{K->row_ptr, K->col, K->val, src}
                          : CsrRhs{nullptr, nullptr, nullptr, nullptr};
     return (int) trsv_chain<VT>(p.task_t, t.nb, 0, p.to_col, p.to_val, p.to_lr, p.ti_col, p.ti_val,
-        p.ti_lr, pub, next, t.err, x, rhs, (hipStream_t) stream);
+        p.ti_lr, pub, next, t, x, rhs, (hipStream_t) stream);
 }
 
 void chain_reset(double* pub, int64_t count, void* stream)

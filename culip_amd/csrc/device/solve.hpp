@@ -42,7 +42,12 @@ struct SolveTopo {
     // single-launch solves
     double* chain_pub;          // 2n published values, two halves used in turn
     int32_t* err;               // set when a dependency wait gave up
+    int32_t spin_limit;         // polls after which a wave's waits give up
 };
+
+// polls of a single-launch solve's wave before its waits give up (seconds; a
+// wait takes a few)
+constexpr int32_t CHAIN_SPIN_LIMIT = 1 << 22;
 
 // Counting pass of the layout: fills the four count arrays (n entries each,
 // stored in the *_ptr arrays shifted by one) and the pivot-block inverses.

@@ -388,6 +388,7 @@ SolveTopo Bildlt::topo() const
     t.is_piv = d_fis_piv.as<int32_t>();
     t.chain_pub = d_chain_pub.as<double>();
     t.err = h_trsv_err.p;
+    t.spin_limit = spin_limit;
     return t;
 }
 

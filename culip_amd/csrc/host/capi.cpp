@@ -635,6 +635,14 @@ culip_status culip_bildlt_inject_solve_error(culip_bildlt* h)
     });
 }
 
+culip_status culip_bildlt_set_spin_limit(culip_bildlt* h, int32_t polls)
+{
+    return guarded([&] {
+        CULIP_REQUIRE(h, "bildlt: null argument");
+        h->b.spin_limit = polls < 0 ? CHAIN_SPIN_LIMIT : std::min(polls, CHAIN_SPIN_LIMIT);
+    });
+}
+
 void culip_bildlt_destroy(culip_bildlt* h) { delete h; }
 
 // ---- SPMV -----------------------------------------------------------------

@@ -190,6 +190,7 @@ struct Bildlt final : Precond {
     culip_solve_algorithm solve_algo = CULIP_TRSV_SINGLE;
     int32_t jacobi_sweeps = 0;
     mutable int32_t chain_parity = 0;
+    int32_t spin_limit = CHAIN_SPIN_LIMIT;   // less only by the testing hook
     DevBuf d_jac[3];          // block-Jacobi right-hand side and iterates
 
     // host copies for inspection

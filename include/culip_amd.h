@@ -290,6 +290,10 @@ culip_status culip_bildlt_set_graphs(culip_bildlt * h, int32_t enable);
  * single-launch solve whose dependency wait gave up, as the kernel would
  * (after upload; CULIP_ERR_STATE before). */
 culip_status culip_bildlt_inject_solve_error(culip_bildlt * h);
+/* Testing hook, no counterpart in the reference: the polls after which the
+ * dependency waits of the object's single-launch solves give up, at most the
+ * library's own limit (polls < 0: that limit again). */
+culip_status culip_bildlt_set_spin_limit(culip_bildlt * h, int32_t polls);
 void culip_bildlt_destroy(culip_bildlt * h);
 
 /* ------------------------------------------------------------------------ */

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import culip_amd as ca
+from conftest import sym_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +125,44 @@ def test_solve_error_reported_once(hip_device):
     x.zero_()
     q.solve(b, x)
     assert q.result["true_rel_residual"] <= 1e-8
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind", ["kkt", "dense_pivots"])
+def test_solve_that_gives_up_waiting_leaves_nan(hip_device, kind, prec):
+    """A single-launch solve whose waits give up at once (the testing hook's
+    limit of no polls; every wave still runs to its end): each row is either
+    the solution bit for bit or NaN, never a partial sum; the next call says
+    so once, and the solve after it is whole again."""
+    import torch
+    if kind == "kkt":
+        _, p = _system(2000, 801, B=32)
+        csr, piv, blocks = (p.row_ptr, p.col, p.val), p.piv_starts, p.block_starts
+    else:   # inverses of more than 64 entries, 2x2 pivots
+        csr, piv, blocks, _ = sym_problem(n_blocks=15, bmax=32, density=0.1, seed=15)
+    g = ca.BlockiLDLt(*csr, piv, blocks, prec)
+    g.compute(0, 1.0, 1e-4)
+    A = ca.CSRMatrixSPMV(*csr)
+    b = torch.tensor(np.random.default_rng(4).normal(size=csr[0].size - 1), device=hip_device)
+
+    def solve(side):
+        x = torch.zeros_like(b)
+        if side == "product":
+            assert g.left_product(A, b, x)
+        else:
+            getattr(g, f"solve_{side}")(b, x)
+        torch.cuda.synchronize()
+        return x.cpu().numpy()
+
+    for side in ("left", "right", "product"):
+        ref = solve(side)
+        assert np.isfinite(ref).all()
+        g._set_spin_limit(0)
+        x = solve(side)
+        gone = np.isnan(x)
+        assert gone.any() and np.array_equal(x[~gone], ref[~gone]), side
+        g._set_spin_limit(-1)
+        with pytest.raises(ca.CulipError) as e:
+            solve(side)
+        assert "timed out" in str(e.value)
+        assert np.array_equal(solve(side), ref), side
