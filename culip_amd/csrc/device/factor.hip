@@ -443,7 +443,7 @@ struct alignas(16) OffLds {
 
 // largest value over the wave and the lowest lane holding it among the
 // lanes with `in` set (the reference's shuffle reduction keeps the lower
-// lane on ties)
+// lane on ties); NaN is never the largest
 template<typename VT>
 __device__ __forceinline__ int wave_argmax_first(VT v, bool in, VT& best)
 {
@@ -482,7 +482,9 @@ __device__ void select_bk(const VT* T, int len, int p, int& order, int& p0, int&
     p1 = r;
 }
 
-// d_select_pivot_rook (kernels :838-948)
+// d_select_pivot_rook (kernels :838-948). The search ends: wi is the
+// magnitude of an entry of row r, so the largest of row r is at least wi, and
+// the loop goes on only while it grows.
 template<typename VT>
 __device__ void select_rook(const VT* T, int len, int p, int& order, int& p0, int& p1)
 {

@@ -40,11 +40,14 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+// largest value that is not NaN: the same on every lane (a comparison would
+// keep one operand or the other of a NaN, by its place, and the lanes would
+// part)
 template<typename T>
 __device__ __forceinline__ T wave_max(T v)
 {
 #pragma unroll
-    for(int o = WAVE / 2; o > 0; o >>= 1) { T u = __shfl_xor(v, o, WAVE); v = v > u ? v : u; }
+    for(int o = WAVE / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, WAVE));
     return v;
 }
 

@@ -174,3 +174,57 @@ def test_pivoting_edge_cases(hip_device, case, mode):
             ref = o.solve(side, b)
             err = np.linalg.norm(x.cpu().numpy() - ref) / max(np.linalg.norm(ref), 1e-300)
             assert err < 1e-12, (algo, side, err)
+
+
+def _nan_diagonal(csr, rows):
+    rp, ci, cv = csr
+    cv = cv.copy()
+    for r in rows:
+        at = np.arange(rp[r], rp[r + 1])
+        cv[at[ci[at] == r]] = np.nan
+    return rp, ci, cv
+
+
+def _block_diagonal(seed):
+    """Blocks of 1 to 32 rows without blocks beside the diagonal, few entries
+    in each, and in every other block one row whose diagonal is NaN."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    hs = np.concatenate([np.arange(1, 33), rng.integers(2, 33, size=30)])
+    bs = np.concatenate([[0], np.cumsum(hs)[:-1]]).astype(np.int32)
+    blocks = []
+    for h in hs:
+        a = np.triu(rng.normal(size=(h, h)) * (rng.random((h, h)) < 1.5 / h), 1)
+        blocks.append(a + a.T + np.diag(rng.normal(size=h) + 3.0))
+    A = sp.block_diag(blocks).tocsr()
+    A.sort_indices()
+    n = A.shape[0]
+    csr = (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    rows = [b + rng.integers(h) for b, h in zip(bs[::2], hs[::2])]
+    return _nan_diagonal(csr, rows), np.arange(n, dtype=np.int32), bs
+
+
+@pytest.mark.parametrize("t", ["d", "f"])
+@pytest.mark.parametrize("mode", ["bk", "rook"])
+@pytest.mark.parametrize("kind", ["block_diagonal", "color", "natural"])
+def test_nan_diagonal_equals_oracle(hip_device, kind, mode, t):
+    """NaN on K's diagonal: the pivot searches pass over it as the oracle's
+    comparisons do, with every lane of one mind about the largest entry, and
+    it reaches the same entries of U and D and the same norms. (Beside the
+    diagonal only in a block row that is NaN from its first row on: of a row
+    before a NaN row the oracle's 2x2 form makes NaN, the division does not.)"""
+    if kind == "block_diagonal":
+        csr, piv, bs = _block_diagonal(3)
+    else:
+        k = ca.KKT(1300, 520, 4, 3, seed=7)
+        p = ca.Prep(k.row_ptr, k.col, k.val, 1300, 16,
+                    ca.ORDER_BLOCK_COLOR if kind == "color" else ca.ORDER_NATURAL)
+        piv, bs = p.piv_starts, p.block_starts
+        csr = _nan_diagonal((p.row_ptr, p.col, p.val),
+                            [bs[bs.size // 5], bs[bs.size // 3], bs[bs.size // 2]])
+    g, o = _pair(csr, piv, bs, mode, t=t, prec="f64")
+    assert np.isnan(o.get("tri")).any() and np.isfinite(o.get("tri")).any()
+    for nm in ("fblocks", "fix_store", "perm", "fis_piv"):
+        assert np.array_equal(g.get_int(nm), o.get(nm)), nm
+    for nm in ("fval_store", "tri", "row_norms"):
+        assert np.array_equal(g.get_real(nm), o.get(nm), equal_nan=True), nm
