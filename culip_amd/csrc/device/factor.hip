@@ -40,6 +40,9 @@ namespace {
 
 constexpr double NZ_EPS = 1e-10;
 
+template<typename T>
+__device__ __forceinline__ bool finite_value(T v) { return fabs(v) < (T) INFINITY; }
+
 // first Schur pair of an off-diagonal task: low and high 32 bits in the
 // third int4's x and w
 __device__ __forceinline__ int64_t pair_first(int4 t2)
@@ -315,9 +318,14 @@ __device__ __forceinline__ void givens_d_solve(bool f64, const double* D, int l,
     else givens_d_solve<VT, VT>(D, l, hgt, rl, right, p2, x1, x2);
 }
 
+// What a pivot step came upon: a D that is not finite; a multiplier that is
+// not, after which rows and columns beyond the pivot row's nonzero ones have
+// changed (0 inf and 0 NaN are NaN).
+constexpr uint32_t STEP_BAD_D = 1, STEP_BAD_ROW = 2;
+
 // d_ldlt_1x1_step (kernels :538-585)
 template<typename VT>
-__device__ bool step_1x1(VT* T, double* tri, int p, int len)
+__device__ uint32_t step_1x1(VT* T, double* tri, int p, int len)
 {
     const int lane = lane_id();
     const int j = lane & 31, half = lane >> 5;
@@ -349,7 +357,8 @@ __device__ bool step_1x1(VT* T, double* tri, int p, int len)
     if(mod && lane == 0) T[32 * p + p] = 1;
     if(lane < 3) tri[3 * p + lane] = (lane == 1) ? (double) d : 0.0;
     wave_sync();
-    return fabs(d) < (VT) INFINITY;   // D is finite
+    return (finite_value(d) ? 0u : STEP_BAD_D) |
+        (wave_ballot(!finite_value(u) || !finite_value(ru)) ? STEP_BAD_ROW : 0u);
 }
 
 // d_ldlt_2x2_step (kernels :589-675): Givens rotation of the 2x2 pivot.
@@ -358,7 +367,7 @@ __device__ bool step_1x1(VT* T, double* tri, int p, int len)
 // products with the FP64-exact row factors r1, r2. A replaced near-singular
 // pivot is (VT) 1e-6 on the diagonal in both forms.
 template<typename VT, typename AT>
-__device__ bool step_2x2(VT* T, double* tri, int p, int len)
+__device__ uint32_t step_2x2(VT* T, double* tri, int p, int len)
 {
     const int lane = lane_id();
     const int j = lane & 31, half = lane >> 5;
@@ -416,7 +425,13 @@ __device__ bool step_2x2(VT* T, double* tri, int p, int len)
         tri[3 * (p + 1) + lane] = (lane == 0) ? (double) d12 : ((lane == 1) ? (double) d22 : 0.0);
     }
     wave_sync();
-    return fabs(d11) + fabs(d12) + fabs(d22) < (AT) INFINITY;   // D is finite
+    // two products of finite factors may also overflow and meet as NaN, first
+    // of all on the diagonal
+    const VT dj = T[33 * j];
+    const bool bad = !finite_value(u1) || !finite_value(u2) || !finite_value(r1) ||
+        !finite_value(r2) || dj != dj;
+    return (finite_value(fabs(d11) + fabs(d12) + fabs(d22)) ? 0u : STEP_BAD_D) |
+        (wave_ballot(bad) ? STEP_BAD_ROW : 0u);
 }
 
 // entries of a block taken by the one-lane forms, and updates beside the
@@ -552,9 +567,6 @@ __device__ void dense_pivot_op(VT* T, int32_t* perm, int len, int pa, int pb)
 // is widened by one row each way), and a non-finite entry or D makes the
 // products of unmatched rows NaN (the mask ALL_ROWS matches every block).
 constexpr uint32_t ALL_ROWS = 0xffffffffu;
-
-template<typename T>
-__device__ __forceinline__ bool finite_value(T v) { return fabs(v) < (T) INFINITY; }
 
 // the mask of a stored block with entries in the rows m (dense blocks:
 // ALL_ROWS), any_bad: one of them is not finite; flag: its row's row_flag
@@ -837,8 +849,9 @@ constexpr uint32_t PIV_ANY = 1, PIV_2X2 = 2, PIV_NONFINITE = 4, PIV_PERM = 8;
 // it take these trips together, one per lane, and the updates are then added
 // per element in block order from LDS; blocks outside the one-lane form are
 // staged one by one in their place in that order. Of the pivot steps only
-// rows with an entry right of the diagonal (or a 2x2 pivot) are steps; the
-// others scale a row and change nothing else, so they are done together last.
+// rows with an entry right of the diagonal (or a 2x2 pivot, or a NaN on the
+// diagonal, which reaches all rows below) are steps; the others scale a row and
+// change nothing else, so they are done together last.
 // FP64 refactor, blocks above taken by rounds of one wave -> at once: 7.1 ->
 // 5.2 ms at n = 2,000, 8.3 -> 6.4 ms at n = 400,000.
 template<typename VT, int NW>
@@ -945,14 +958,14 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
                 }
                 if(order == 1) {
                     if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
-                    if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
+                    if(step_1x1(T0, tri, p, len) & STEP_BAD_D) rflag |= ROW_NONFINITE;
                     if(lane == 0) fpiv[p] = 1;
                 } else {
                     if(p0 != p) dense_pivot_op(T0, bperm, len, p, p0);
                     dense_pivot_op(T0, bperm, len, p + 1, p1);
-                    const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
-                                             : step_2x2<VT, VT>(T0, tri, p, len);
-                    rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
+                    const uint32_t bad = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
+                                                 : step_2x2<VT, VT>(T0, tri, p, len);
+                    rflag |= (bad & STEP_BAD_D) ? (ROW_2X2 | ROW_NONFINITE) : ROW_2X2;
                     if(lane == 0) {
                         fpiv[p] = 1;
                         fpiv[p + 1] = 0;
@@ -963,8 +976,8 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
             }
             if(lane < 32) M = (lane < 31) ? ~0u << (lane + 1) : 0u;
         } else {
-            // columns right of the diagonal per row (a superset while steps
-            // fill rows in)
+            // columns right of the diagonal per row: a superset while steps fill
+            // rows in (all of them after a multiplier that is not finite)
 #pragma unroll
             for(int k = 0; k < 16; ++k) {
                 const int r = 2 * k + (lane >> 5), c = lane & 31;
@@ -972,6 +985,9 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
                 if(lane == 2 * k) M = (uint32_t) b;
                 if(lane == 2 * k + 1) M = (uint32_t) (b >> 32);
             }
+            const uint32_t right = lane < len ? live & (~1u << lane) : 0u;
+            const VT d0 = T0[33 * (lane & 31)];
+            if(d0 != d0) M = right;
             const uint32_t starts = (uint32_t) wave_ballot(lane < 32 && lane < len && piv != 0);
             const uint32_t two = (~starts & live) >> 1;    // rows where a 2x2 pivot starts
             uint32_t done = 0;
@@ -980,10 +996,11 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
                     (~0u << p);
                 if(!cand) break;
                 p = __ffs(cand) - 1;
+                uint32_t bad;
                 if((two >> p) & 1u) {
-                    const bool fin = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
-                                             : step_2x2<VT, VT>(T0, tri, p, len);
-                    rflag |= fin ? ROW_2X2 : (ROW_2X2 | ROW_NONFINITE);
+                    bad = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
+                                  : step_2x2<VT, VT>(T0, tri, p, len);
+                    rflag |= ROW_2X2;
                     const uint32_t mm = (uint32_t) (__builtin_amdgcn_readlane((int) M, p) |
                         __builtin_amdgcn_readlane((int) M, p + 1));
                     if(lane > p + 1 && lane < 32 && ((mm >> lane) & 1u)) M |= mm & (~1u << lane);
@@ -991,12 +1008,14 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
                     done |= 3u << p;
                     p += 2;
                 } else {
-                    if(!step_1x1(T0, tri, p, len)) rflag |= ROW_NONFINITE;
+                    bad = step_1x1(T0, tri, p, len);
                     const uint32_t mm = (uint32_t) __builtin_amdgcn_readlane((int) M, p);
                     if(lane > p && lane < 32 && ((mm >> lane) & 1u)) M |= mm & (~1u << lane);
                     done |= 1u << p;
                     p += 1;
                 }
+                if(bad & STEP_BAD_D) rflag |= ROW_NONFINITE;
+                if(bad & STEP_BAD_ROW) M = right;
                 wave_sync();
             }
             plain = live & ~done;

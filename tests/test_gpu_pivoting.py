@@ -185,9 +185,10 @@ def _nan_diagonal(csr, rows):
     return rp, ci, cv
 
 
-def _block_diagonal(seed):
+def _block_diagonal(seed, two_by_two=False):
     """Blocks of 1 to 32 rows without blocks beside the diagonal, few entries
-    in each, and in every other block one row whose diagonal is NaN."""
+    in each, and in every other block one row whose diagonal is NaN; 1x1
+    static pivots, or every fourth pair of rows of a block a 2x2 one."""
     import scipy.sparse as sp
     rng = np.random.default_rng(seed)
     hs = np.concatenate([np.arange(1, 33), rng.integers(2, 33, size=30)])
@@ -201,20 +202,25 @@ def _block_diagonal(seed):
     n = A.shape[0]
     csr = (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
     rows = [b + rng.integers(h) for b, h in zip(bs[::2], hs[::2])]
-    return _nan_diagonal(csr, rows), np.arange(n, dtype=np.int32), bs
+    piv = np.ones(n, dtype=bool)
+    if two_by_two:
+        for b, h in zip(bs, hs):
+            piv[b + 1:b + h:4] = False
+    return _nan_diagonal(csr, rows), np.flatnonzero(piv).astype(np.int32), bs
 
 
 @pytest.mark.parametrize("t", ["d", "f"])
-@pytest.mark.parametrize("mode", ["bk", "rook"])
-@pytest.mark.parametrize("kind", ["block_diagonal", "color", "natural"])
+@pytest.mark.parametrize("mode", ["static", "bk", "rook"])
+@pytest.mark.parametrize("kind", ["block_diagonal", "two_by_two", "color", "natural"])
 def test_nan_diagonal_equals_oracle(hip_device, kind, mode, t):
     """NaN on K's diagonal: the pivot searches pass over it as the oracle's
     comparisons do, with every lane of one mind about the largest entry, and
-    it reaches the same entries of U and D and the same norms. (Beside the
+    it reaches the same entries of U and D and the same norms, also from a row
+    without an entry right of the diagonal. (Beside the
     diagonal only in a block row that is NaN from its first row on: of a row
     before a NaN row the oracle's 2x2 form makes NaN, the division does not.)"""
-    if kind == "block_diagonal":
-        csr, piv, bs = _block_diagonal(3)
+    if kind in ("block_diagonal", "two_by_two"):
+        csr, piv, bs = _block_diagonal(3, kind == "two_by_two")
     else:
         k = ca.KKT(1300, 520, 4, 3, seed=7)
         p = ca.Prep(k.row_ptr, k.col, k.val, 1300, 16,
