@@ -1054,13 +1054,16 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
         // row sums of squares, and the nonzero columns right of the diagonal
         // for the U_ii' solves (every other entry of a row is zero)
         uint32_t um = 0;
+        bool bounded = true;
         if(lane < len) {
             VT v = T0[33 * lane];
             VT ssq = fma(v, v, (VT) 0);
+            bounded = fabs(v) > (VT) 0.5 && fabs(v) < (VT) 0x1p30;
             for(uint32_t bits = M & live; bits; bits &= bits - 1) {
                 v = T0[32 * lane + __ffs(bits) - 1];
                 ssq = fma(v, v, ssq);
                 if(v != (VT) 0) um |= bits & (0u - bits);
+                bounded = bounded && fabs(v) < (VT) 0x1p30;
             }
             a.rn[fr + lane] = ssq;
         }
@@ -1069,6 +1072,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
         uint32_t flags = wave_ballot(um != 0u) ? PIV_ANY : 0u;
         if(s.rflag & ROW_2X2) flags |= PIV_2X2;
         if(s.rflag & ROW_NONFINITE) flags |= PIV_NONFINITE;
+        const bool unbounded = wave_ballot(!bounded) != 0ull;
         if(a.pivoting) {
             const int p = (lane < len) ? s.perm[lane] : lane;
             if(wave_ballot(lane < len && p != lane)) flags |= PIV_PERM;
@@ -1079,7 +1083,8 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
         }
         if(lane == 0) {
             a.piv_flag[q] = flags;
-            a.row_flag[i] = s.rflag | ((flags & PIV_ANY) ? ROW_COUPLED : 0);
+            a.row_flag[i] = s.rflag | ((flags & PIV_ANY) ? ROW_COUPLED : 0) |
+                (unbounded ? ROW_UNBOUNDED : 0);
             a.piv_loc[i] = q;
         }
     }

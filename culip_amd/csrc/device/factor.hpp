@@ -108,8 +108,9 @@ struct FactorArgs {
 constexpr int LIST_C = 4;
 // row_flag: what a block row's pivot block left (a 2x2 pivot, a non-finite D,
 // an entry of U_ii right of its diagonal; with none of them U_ii is the
-// identity)
-constexpr int32_t ROW_2X2 = 1, ROW_NONFINITE = 2, ROW_COUPLED = 4;
+// identity; an entry of 2^30 or more, a diagonal of 1/2 or less or NaN: without
+// them no value of U_ii^-1 exceeds 2 (1 + 2^31)^31 < 2^1024)
+constexpr int32_t ROW_2X2 = 1, ROW_NONFINITE = 2, ROW_COUPLED = 4, ROW_UNBOUNDED = 8;
 // A row group is one workgroup's share of a level's dropping step: block
 // rows that follow each other, at most GROUP_ROWS fine rows, and at most
 // GROUP_BLOCKS off-diagonal blocks unless one block row has more.

@@ -24,10 +24,38 @@ namespace culip {
 
 namespace {
 
+// diag_inverse with every term added, also those with a zero of U (0 inf and
+// 0 NaN are NaN); a tile without an entry beside its diagonal has none in X.
+// For the tiles whose inverse may not be finite (ROW_UNBOUNDED).
+template<typename VT>
+__device__ __forceinline__ void diag_inverse_all_terms(const VT* U, int h, double* X, int hm)
+{
+    const int c = lane_id();
+    bool beside = false;
+    if(c < h)
+#pragma unroll 1
+        for(int k = c + 1; k < h; ++k) beside = beside || (U[c * h + k] != (VT) 0);
+    const bool coupled = wave_ballot(beside) != 0ull;
+#pragma unroll 1
+    for(int r = hm - 1; r >= 0; --r) {
+        double v = 0.0;
+        if(r <= c && c < h) {
+            const double d = (double) U[r * h + r];
+            double s = 0.0;
+#pragma unroll 1
+            for(int k = r + 1; k <= c; ++k) s = fma((double) U[r * h + k], X[hm * k + c], s);
+            v = (r == c) ? 1.0 / d : (coupled ? -s / d : 0.0);
+        }
+        if(c < hm) X[hm * r + c] = v;
+    }
+    wave_sync();
+}
+
 // columns of U_ii^-1 by back substitution, in double; X[r][c] at X[hm r + c]
 // (hm x hm LDS, hm >= h: the largest block height of the launch). Lane c forms
 // column c. U's rows come in with one round of loads, and only their nonzero
-// entries are visited, ascending (the others would add exact zeros).
+// entries are visited, ascending (the others would add exact zeros to a finite
+// X).
 template<typename VT>
 __device__ void diag_inverse(const VT* U, int h, double* X, int hm)
 {
@@ -139,7 +167,8 @@ __device__ __forceinline__ void plan_rows_body(const SolveTopo& t, const VT* val
     const int fr = t.bs[i];
     const int h = t.bs[i + 1] - fr;
     // pivot block inverse rows (ui) and columns (ti)
-    if(t.row_flag[i] == 0) {
+    const int32_t flag = t.row_flag[i];
+    if(flag == 0) {
         // U_ii is the identity (most pivot blocks of a sparse pattern): its
         // tile is not read
         if(lane < h) {
@@ -155,7 +184,8 @@ __device__ __forceinline__ void plan_rows_body(const SolveTopo& t, const VT* val
     } else {
         double* X = (double*) lds;
         const BlockMeta dm = t.bout[t.csr_off[i]];
-        diag_inverse(val_out + dm.val_ptr, h, X, hm);
+        if(flag & ROW_UNBOUNDED) diag_inverse_all_terms(val_out + dm.val_ptr, h, X, hm);
+        else diag_inverse(val_out + dm.val_ptr, h, X, hm);
         if(lane < h) {
             int cr = 0, cc = 0;
             int32_t wr = 0, wc = 0;

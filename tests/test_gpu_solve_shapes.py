@@ -109,3 +109,58 @@ def test_iterates_do_not_depend_on_check_period(hip_device, algo, sweeps):
             out.append(x.cpu().numpy())
         for x in out[1:]:
             assert np.array_equal(out[0], x), (max_it, algo)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_nan_reaches_the_rows_of_the_substitution(hip_device, prec):
+    """A NaN in a pivot block's U_ii reaches the solution's rows that back and
+    forward substitution with U_ii give NaN (zeros beside it included) and no
+    others, in every schedule; blocks beside the diagonal there are none."""
+    import scipy.sparse as sp
+    import torch
+    rng = np.random.default_rng(11)
+    hs = np.concatenate([np.arange(1, 33), [32, 17, 8]])
+    bs = np.concatenate([[0], np.cumsum(hs)[:-1]]).astype(np.int32)
+    blocks, bad = [], []
+    for b, h in zip(bs, hs):
+        a = np.triu(rng.normal(size=(h, h)) * (rng.random((h, h)) < 1.5 / h), 1)
+        blocks.append(a + a.T + np.diag(rng.normal(size=h) + 3.0))
+        bad.append(b + rng.integers(h))
+    A = sp.block_diag(blocks).tocsr()
+    A.sort_indices()
+    n = A.shape[0]
+    val = A.data.copy()
+    rows = np.repeat(np.arange(n), np.diff(A.indptr))
+    val[(rows == A.indices) & np.isin(rows, bad)] = np.nan
+    csr = (A.indptr.astype(np.int32), A.indices.astype(np.int32), val)
+    args = (*csr, np.arange(n, dtype=np.int32), bs)
+    g = ca.BlockiLDLt(*args, prec)
+    g.compute(0, 1.0, 1e-4)
+    # U_ii as stored (dense, block after block)
+    U = g.get_real("fval_store")
+    b = rng.normal(size=n)
+    ref = {"left": b.copy(), "right": b.copy()}
+    for k, (f, h) in enumerate(zip(bs, hs)):
+        u = U[(hs[:k] ** 2).sum():][:h * h].reshape(h, h).astype(np.float64)
+        assert np.isnan(u[bad[k] - f]).all()
+        inv = np.zeros((h, h))     # columns of the inverse by back substitution
+        beside = (np.triu(u, 1) != 0).any()
+        for c in range(h):
+            for r in range(c, -1, -1):
+                s = sum((u[r, j] * inv[j, c] for j in range(r + 1, c + 1)), 0.0)
+                inv[r, c] = 1.0 / u[r, r] if r == c else -s / u[r, r] if beside else 0.0
+        for side, m in (("left", inv.T), ("right", inv)):
+            ref[side][f:f + h] = [sum(m[r, c] * b[f + c] for c in range(h) if m[r, c] != 0)
+                                  for r in range(h)]
+    db = torch.tensor(b, device=hip_device)
+    for algo, sweeps in (("levels", 0), ("single", 0), ("jacobi", 1)):
+        g.set_solve_algorithm(algo, sweeps)
+        for side, want in ref.items():
+            x = torch.zeros_like(db)
+            getattr(g, f"solve_{side}")(db, x)
+            x = x.cpu().numpy()
+            assert np.array_equal(np.isnan(x), np.isnan(want)), (algo, side)
+            ok = ~np.isnan(want)
+            assert ok.any()
+            assert np.linalg.norm((x - want)[ok]) <= \
+                (1e-12 if prec == "f64" else 1e-5) * np.linalg.norm(want[ok]), (algo, side)
