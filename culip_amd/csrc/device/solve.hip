@@ -1459,14 +1459,15 @@ template void solve_plan_fill<float>(const SolveTopo&, const float*, const float
 // Waves of k_trsv_chain per CU. A solve needs all of its waves resident.
 // TRSV_SINGLE_MAX_CONCURRENT = 4 such solves have to fit on the GPU at the
 // same time (other kernels end on their own), so at most a quarter of what a
-// CU holds: its registers let a CU hold 12 of this kernel's waves, three per
-// solve. (Compiled for 16 per CU, it spills 18-25 registers inside the rows'
-// critical path: 403 us instead of 236 for both solves at n = 400,000.)
-constexpr int CHAIN_WAVES_PER_CU = 4;
+// CU holds: its registers (147-161) let a CU hold 12 of this kernel's waves,
+// three per solve. (Compiled for 16 per CU, it spills 18-25 registers inside
+// the rows' critical path: 403 us instead of 236 for both solves at n =
+// 400,000. As compiled, 59-75 scalar registers go to lanes of vector ones.)
+constexpr int CHAIN_WAVES_PER_CU = 3;
 
-// grid of k_trsv_chain: CHAIN_WAVES_PER_CU waves per CU, fewer when the
-// kernel's occupancy would not hold TRSV_SINGLE_MAX_CONCURRENT solves (CU
-// count and occupancy queried once per device)
+// grid of k_trsv_chain: CHAIN_WAVES_PER_CU waves per CU, fewer should either
+// instance's occupancy not hold TRSV_SINGLE_MAX_CONCURRENT solves (CU count
+// and occupancy queried once per device)
 template<typename VT>
 int chain_grid(int32_t nb)
 {
@@ -1475,11 +1476,14 @@ int chain_grid(int32_t nb)
     if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
     if(cus[dev] == 0) {
         hipDeviceProp_t pr;
-        int o = 0;
+        int fused = 0, plain = 0;
         if(hipGetDeviceProperties(&pr, dev) != hipSuccess) return 0;
-        if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_trsv_chain<VT, true>, 64, 0) != hipSuccess)
+        if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fused, k_trsv_chain<VT, true>, 64, 0) !=
+                hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&plain, k_trsv_chain<VT, false>, 64, 0) !=
+                hipSuccess)
             return 0;
-        occ[dev] = o;
+        occ[dev] = min(fused, plain);
         cus[dev] = pr.multiProcessorCount;
     }
     const int per = max(1, min(CHAIN_WAVES_PER_CU, occ[dev] / TRSV_SINGLE_MAX_CONCURRENT));
