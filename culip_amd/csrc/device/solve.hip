@@ -617,6 +617,34 @@ __device__ __forceinline__ bool published(double v)
     return (unsigned long long) __double_as_longlong(v) != CHAIN_EMPTY;
 }
 
+// waits until every lane's value xv[k] (column c[k]) is published; rdy[k]
+// on entry: xv[k] already usable. What is missing when it gives up stays
+// CHAIN_EMPTY, a NaN.
+__device__ void wait_published(const double* pub, const int (&c)[TRSV_PF], double (&xv)[TRSV_PF],
+    bool (&rdy)[TRSV_PF], int32_t* err, int32_t spin_limit, int& spins)
+{
+    bool all = true;
+#pragma unroll
+    for(int k = 0; k < TRSV_PF; ++k) all = all && rdy[k];
+    while(wave_ballot(!all)) {
+        __builtin_amdgcn_s_sleep(1);
+        if(++spins > spin_limit) {
+            // err is pinned host memory: the host reads it without a copy
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            return;
+        }
+        all = true;
+#pragma unroll
+        for(int k = 0; k < TRSV_PF; ++k) {
+            if(!rdy[k]) {
+                xv[k] = pub_load(pub + c[k]);
+                rdy[k] = published(xv[k]);
+            }
+            all = all && rdy[k];
+        }
+    }
+}
+
 // One group of up to TRSV_PF 64-entry chunks of a block row's off-diagonal
 // entries: columns, values and local rows (64: no entry).
 template<typename VT>
@@ -636,35 +664,37 @@ struct ChainHead {
 };
 
 // The segmented sums over a chunk as far as they follow from its local rows
-// alone, formed while the x values are on their way: how many lanes of this
-// lane's 16-lane row before it belong to its segment, whether the segment
-// reaches into the rows before (scan steps over lanes 15 and 31), and on lane
-// r < 32 the lane that ends row r's segment (-1: no entry of the row).
+// alone, formed while the x values are on their way, in one register: how many
+// lanes of this lane's 16-lane row before it belong to its segment, whether the
+// segment reaches into the rows before (scan steps over lanes 15 and 31), and
+// on lane r < 32 the lane that ends row r's segment (-1: no entry of the row).
 struct ScanPlan {
-    int dist;
-    bool cross15, cross31;
-    int end;
+    int bits;
+    __device__ __forceinline__ int dist() const { return bits & 15; }
+    __device__ __forceinline__ bool cross15() const { return (bits & 16) != 0; }
+    __device__ __forceinline__ bool cross31() const { return (bits & 32) != 0; }
+    __device__ __forceinline__ int end() const { return bits >> 8; }
 };
 
 __device__ __forceinline__ ScanPlan scan_plan(int sg, int8_t* ends)
 {
-    const int lane = lane_id();
-    ScanPlan p;
+    int lane = lane_id();
+    // what follows from the lane alone is formed here, not held over the loop
+    asm volatile("" : "+v"(lane));
     const int before = dpp_move<0x138, 0xf>(-1, sg);   // every lane active
     const uint64_t heads = wave_ballot(before != sg) | 1ull;
     // the first lane of this lane's segment
     const int start = 63 - __clzll((long long) (heads & (~0ull >> (63 - lane))));
-    p.dist = min(lane - start, lane & 15);
-    p.cross15 = (lane & 16) != 0 && start < (lane & ~15);
-    p.cross31 = lane >= 32 && start < 32;
+    int bits = min(lane - start, lane & 15);
+    if((lane & 16) != 0 && start < (lane & ~15)) bits |= 16;
+    if(lane >= 32 && start < 32) bits |= 32;
     const int nsg = next_lane(sg, -1);
     wave_sync();
     if(lane < 32) ends[lane] = -1;
     wave_sync();
     if(sg < 64 && (lane == 63 || nsg != sg)) ends[sg] = (int8_t) lane;
     wave_sync();
-    p.end = ends[lane & 31];
-    return p;
+    return ScanPlan{bits | (int) ends[lane & 31] * 256};
 }
 
 // a lane move whose result is used only where the lane has a source
@@ -682,62 +712,82 @@ __device__ __forceinline__ double planned_scan(double a, double x, const ScanPla
 {
     double v = a * x;
     const double f = fma(a, x, dpp_take<0x111, 0xf>(v));
-    v = p.dist >= 1 ? f : v;
+    const int dist = p.dist();
+    v = dist >= 1 ? f : v;
     double s = v + dpp_take<0x112, 0xf>(v);
-    v = p.dist >= 2 ? s : v;
+    v = dist >= 2 ? s : v;
     s = v + dpp_take<0x114, 0xf>(v);
-    v = p.dist >= 4 ? s : v;
+    v = dist >= 4 ? s : v;
     s = v + dpp_take<0x118, 0xf>(v);
-    v = p.dist >= 8 ? s : v;
+    v = dist >= 8 ? s : v;
     s = v + dpp_take<0x142, 0xa>(v);
-    v = p.cross15 ? s : v;
+    v = p.cross15() ? s : v;
     s = v + dpp_take<0x143, 0xc>(v);
-    return p.cross31 ? s : v;
+    return p.cross31() ? s : v;
 }
 
-// Reloads the x values of the lanes set in m[k], all in one round trip. One
-// block with its own wait: written as loads under conditions, the compiler
-// waits for each before it issues the next.
-__device__ __forceinline__ void reload_missing(const double* pub, const int (&c)[TRSV_PF],
+// Reloads the x values (byte offsets off[k]) of the lanes set in m[k], all in
+// one round trip. One block with its own wait: written as loads under
+// conditions, the compiler waits for each before it issues the next.
+__device__ __forceinline__ void reload_missing(const double* pub, const uint32_t (&off)[TRSV_PF],
     const uint64_t (&m)[TRSV_PF], double (&xv)[TRSV_PF])
 {
     static_assert(TRSV_PF == 4, "four chunks");
-    const double* p0 = pub + c[0];
-    const double* p1 = pub + c[1];
-    const double* p2 = pub + c[2];
-    const double* p3 = pub + c[3];
     uint64_t saved;
     asm volatile("s_mov_b64 %[sv], exec\n\t"
                  "s_mov_b64 exec, %[m0]\n\t"
-                 "global_load_dwordx2 %[x0], %[p0], off sc1\n\t"
+                 "global_load_dwordx2 %[x0], %[o0], %[pub] sc1\n\t"
                  "s_mov_b64 exec, %[m1]\n\t"
-                 "global_load_dwordx2 %[x1], %[p1], off sc1\n\t"
+                 "global_load_dwordx2 %[x1], %[o1], %[pub] sc1\n\t"
                  "s_mov_b64 exec, %[m2]\n\t"
-                 "global_load_dwordx2 %[x2], %[p2], off sc1\n\t"
+                 "global_load_dwordx2 %[x2], %[o2], %[pub] sc1\n\t"
                  "s_mov_b64 exec, %[m3]\n\t"
-                 "global_load_dwordx2 %[x3], %[p3], off sc1\n\t"
+                 "global_load_dwordx2 %[x3], %[o3], %[pub] sc1\n\t"
                  "s_mov_b64 exec, %[sv]\n\t"
                  "s_waitcnt vmcnt(0)"
                  : [x0] "+&v"(xv[0]), [x1] "+&v"(xv[1]), [x2] "+&v"(xv[2]), [x3] "+&v"(xv[3]),
                  [sv] "=&s"(saved)
-                 : [m0] "s"(m[0]), [m1] "s"(m[1]), [m2] "s"(m[2]), [m3] "s"(m[3]), [p0] "v"(p0),
-                 [p1] "v"(p1), [p2] "v"(p2), [p3] "v"(p3)
+                 : [m0] "s"(m[0]), [m1] "s"(m[1]), [m2] "s"(m[2]), [m3] "s"(m[3]), [o0] "v"(off[0]),
+                 [o1] "v"(off[1]), [o2] "v"(off[2]), [o3] "v"(off[3]), [pub] "s"(pub)
                  : "memory");
+}
+
+// waits until all x values of a group are there; what is missing when it gives
+// up stays CHAIN_EMPTY, a NaN
+__device__ __forceinline__ void wait_group(const double* pub, const uint32_t (&off)[TRSV_PF],
+    const int (&sg)[TRSV_PF], double (&xv)[TRSV_PF], int32_t* err, int32_t spin_limit, int& spins)
+{
+    for(;;) {
+        uint64_t m[TRSV_PF], any = 0;
+#pragma unroll
+        for(int k = 0; k < TRSV_PF; ++k) {
+            m[k] = wave_ballot(sg[k] < 64 && !published(xv[k]));
+            any |= m[k];
+        }
+        if(any == 0) return;
+        if(++spins > spin_limit) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        reload_missing(pub, off, m, xv);
+    }
 }
 
 // y (lane r: row r) minus the row sums of a group, chunk after chunk. A
 // chunk is scanned as soon as its values are there, while the others are
 // still on their way: the latest values of a block row all belong to the
 // levels next to its own, so they sit in one chunk (the last for U', the first
-// for U) and only that chunk's scan follows the last arrival. chunks: how many
-// of the group have entries; their values past the row's end are cleared. NaN
-// when the wait gives up, so that no partial sum is taken for a solution.
+// for U) and only that chunk's scan follows the last arrival. off: the byte
+// offsets of the values in pub; chunks: how many of the group have entries;
+// their values past the row's end are cleared. xv[k] becomes chunk k's sum.
+// NaN when the wait gives up, so that no partial sum is taken for a solution.
 template<typename VT>
-__device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup<VT>& g,
-    double (&xv)[TRSV_PF], const ScanPlan (&p)[TRSV_PF], int chunks, double y, int32_t* err,
-    int32_t spin_limit, int& spins)
+__device__ __forceinline__ double chain_sums(const double* pub, const uint32_t (&off)[TRSV_PF],
+    const VT (&a)[TRSV_PF], const int (&sg)[TRSV_PF], double (&xv)[TRSV_PF],
+    const ScanPlan (&p)[TRSV_PF], int chunks, double y, int32_t* err, int32_t spin_limit,
+    int& spins)
 {
-    double sum[TRSV_PF];
     uint32_t open = chunks >= TRSV_PF ? (1u << TRSV_PF) - 1 : (1u << chunks) - 1;
     for(;;) {
         uint64_t m[TRSV_PF];
@@ -745,11 +795,10 @@ __device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup
         for(int k = 0; k < TRSV_PF; ++k) {
             m[k] = 0;
             if((open >> k) & 1u) {
-                m[k] = wave_ballot(g.sg[k] < 64 && !published(xv[k]));
+                m[k] = wave_ballot(sg[k] < 64 && !published(xv[k]));
                 if(m[k] == 0) {
-                    const double v = planned_scan((double) g.v[k], g.sg[k] < 64 ? xv[k] : 0.0,
-                        p[k]);
-                    sum[k] = __shfl(v, max(p[k].end, 0), WAVE);
+                    const double v = planned_scan((double) a[k], sg[k] < 64 ? xv[k] : 0.0, p[k]);
+                    xv[k] = __shfl(v, max(p[k].end(), 0), WAVE);
                     open &= ~(1u << k);
                 }
             }
@@ -762,11 +811,11 @@ __device__ __forceinline__ double chain_sums(const double* pub, const ChainGroup
             return __longlong_as_double(0x7ff8000000000000ll);
         }
         __builtin_amdgcn_s_sleep(1);
-        reload_missing(pub, g.c, m, xv);
+        reload_missing(pub, off, m, xv);
     }
 #pragma unroll
     for(int k = 0; k < TRSV_PF; ++k)
-        if(k < chunks) y = p[k].end >= 0 ? y - sum[k] : y;
+        if(k < chunks) y = p[k].end() >= 0 ? y - xv[k] : y;
     return y;
 }
 
@@ -782,11 +831,12 @@ struct CsrRhs {
     const double* src;
 };
 
-constexpr int RHS_U = 3;   // entries per lane and row whose loads go together
-
+// RHS_U: entries per lane and row whose loads go together (the same sums for any)
+template<int RHS_U>
 __device__ double block_rhs(const CsrRhs& k, int fr, int h)
 {
-    const int lane = lane_id();
+    int lane = lane_id();
+    asm volatile("" : "+v"(lane));
     const int sub = lane & 7, g = lane >> 3;
     int s[4], e[4];
 #pragma unroll
@@ -867,23 +917,25 @@ __device__ __forceinline__ void chain_fetch(int4 t0, int4 t1, const int32_t* o_c
     f.il = i_lr[ei];
 }
 
-// Between the arrival of a block row's last x value and the store of its
-// results lies the part of every level that no other wave hides. All that
-// does not depend on x is done before (ScanPlan), the chunks that are complete
-// are summed while the last one is awaited, rows are summed by lane reads
-// instead of LDS updates, and U_ii^-1 of up to 64 entries stays in registers.
-// Measured (publish to arrival / arrival to publish, per level, n = 400,000):
-// 0.9-1.1 us / 0.5-0.6 us; a lone pair of waves on two XCDs exchanges a value
-// in 0.4-0.5 us. U, D and U' solve together 251 -> 219 us at n = 400,000,
-// 124 -> 112 us at n = 2,000. Reading values from block rows over 2,048 rows
-// back through the caches instead was slower (257 us).
-template<typename VT, bool FUSED>
-__global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t nb, int32_t reverse,
+// Two forms with the same values (chain_form). Walked: a row's groups one after
+// the other, each awaited as a whole, the chunks summed into LDS. Planned:
+// between the arrival of a block row's last x value and the store of its results
+// lies the part of every level that no other wave hides, so of a row of one
+// group all that does not depend on x is done before (ScanPlan), the chunks that
+// are complete are summed while the last one is awaited, and rows are summed by
+// lane reads instead of LDS updates; rows of more groups are summed as in the
+// walked form (their values are mostly there, and plans only cost: 13.4 ms
+// instead of 11.1 for a factor with fill of n = 10,000); U_ii^-1 of up to 64
+// entries stays in registers. Measured (publish to arrival / arrival to publish,
+// per level, n = 400,000): 0.9-1.1 us / 0.5-0.6 us; a lone pair of waves on two
+// XCDs exchanges a value in 0.4-0.5 us.
+template<typename VT, bool FUSED, bool PLANNED>
+__global__ __launch_bounds__(64, 4) void k_trsv_chain(const int4* task, int32_t nb, int32_t reverse,
     const int32_t* o_col, const VT* o_val, const uint8_t* o_lr, const int32_t* i_col,
     const VT* i_val, const uint8_t* i_lr, double* pub, double* next_pub, int32_t* err,
     int32_t spin_limit, double* x, CsrRhs rhs)
 {
-    __shared__ double y_lds[33];     // general U_ii^-1 only
+    __shared__ double y_lds[33];     // FP64 accumulation for both factor precisions
     __shared__ double res[33];
     __shared__ int8_t ends[32];
     const int lane = lane_id();
@@ -902,27 +954,110 @@ __global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t 
     task_at(w, t0, t1);
     ChainHead<VT> cur;
     chain_fetch<VT>(t0, t1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, cur);
-    if(fused) cur.bo = block_rhs(rhs, t0.x, t0.y);
+    if(fused) cur.bo = block_rhs<3>(rhs, t0.x, t0.y);
+    constexpr int RHS_U = PLANNED ? 2 : 3;   // beside the loop's registers
     for(;;) {
         int4 n0, n1;
         task_at(w + G, n0, n1);
-        ChainHead<VT> nxt = cur;
+        ChainHead<VT> nxt;
         const int fr = t0.x, h = t0.y, ob = t0.z, oe = t0.w, ib = t1.x, ie = t1.y;
         if(lane < h) next_pub[fr + lane] = empty;
-        // U_ii^-1: diagonal (one entry per row, on the diagonal), or up to 64
-        // entries taken by one planned scan, or in chunks of 64
-        const bool diagonal = ie - ib == h &&
-            wave_ballot(lane < h && (cur.il != lane || cur.ic != fr + lane)) == 0;
-        const bool one_chunk = ie - ib <= 64;
-        const bool last = w + G >= nb;
-        double y = cur.bo;
-        ScanPlan ip;
-        if(!diagonal && one_chunk) ip = scan_plan(ib + lane < ie ? cur.il : 64, ends);
-        if(ob < oe) {
-            ChainGroup<VT> g = cur.g;
-            for(int e0 = ob;;) {
-                double xv[TRSV_PF];
+        double r;
+        if(PLANNED) {
+            // U_ii^-1: diagonal (one entry per row, on the diagonal), or up to
+            // 64 entries taken by one planned scan, or in chunks of 64
+            const bool diagonal = ie - ib == h &&
+                wave_ballot(lane < h && (cur.il != lane || cur.ic != fr + lane)) == 0;
+            const bool one_chunk = ie - ib <= 64;
+            double y = cur.bo;
+            ScanPlan ip;
+            if(!diagonal && one_chunk) ip = scan_plan(ib + lane < ie ? cur.il : 64, ends);
+            double xv[TRSV_PF];
+            uint32_t off[TRSV_PF];
+            if(ob < oe)
+#pragma unroll
+                for(int k = 0; k < TRSV_PF; ++k) {
+                    off[k] = 8u * (uint32_t) cur.g.c[k];
+                    xv[k] = pub_load((const double*) ((const char*) pub + off[k]));
+                }
+#pragma unroll
+            for(int k = 0; k < TRSV_PF; ++k) {
+                const bool in = ob + 64 * k + lane < oe;
+                cur.g.v[k] = in ? cur.g.v[k] : (VT) 0;
+                cur.g.sg[k] = in ? cur.g.sg[k] : 64;
+            }
+            // the next loads go out here: they are younger than the reads
+            // above, so a row whose values are all there does not wait for them
+            if(w + G < nb)
+                chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
+            if(oe - ob > 64 * TRSV_PF) {
+                // several groups: awaited as a whole and summed into LDS
+                wave_sync();
+                if(lane < h) y_lds[lane] = y;
+                wave_sync();
+#pragma unroll 1
+                for(int e0 = ob;;) {
+                    wait_group(pub, off, cur.g.sg, xv, err, spin_limit, spins);
+#pragma unroll
+                    for(int k = 0; k < TRSV_PF; ++k) {
+                        if(e0 + 64 * k >= oe) break;
+                        const int sg = cur.g.sg[k];
+                        const double q = seg_scan_runs_fma((double) cur.g.v[k],
+                            sg < 64 ? xv[k] : 0.0, sg);
+                        const int nsg = next_lane(sg, -1);
+                        if(sg < 64 && (lane == 63 || nsg != sg)) y_lds[sg] -= q;
+                        wave_sync();
+                    }
+                    e0 += 64 * TRSV_PF;
+                    if(e0 >= oe) break;
+                    chain_group<VT>(e0, oe, o_col, o_val, o_lr, cur.g);
+#pragma unroll
+                    for(int k = 0; k < TRSV_PF; ++k) {
+                        off[k] = 8u * (uint32_t) cur.g.c[k];
+                        xv[k] = pub_load((const double*) ((const char*) pub + off[k]));
+                    }
+#pragma unroll
+                    for(int k = 0; k < TRSV_PF; ++k) {
+                        const bool in = e0 + 64 * k + lane < oe;
+                        cur.g.v[k] = in ? cur.g.v[k] : (VT) 0;
+                        cur.g.sg[k] = in ? cur.g.sg[k] : 64;
+                    }
+                }
+                y = y_lds[min(lane, 32)];
+            } else if(ob < oe) {
                 ScanPlan plan[TRSV_PF];
+                const int chunks = (oe - ob + 63) / 64;
+                plan[0] = scan_plan(cur.g.sg[0], ends);
+                if(chunks > 1) plan[1] = scan_plan(cur.g.sg[1], ends);
+                if(chunks > 2) plan[2] = scan_plan(cur.g.sg[2], ends);
+                if(chunks > 3) plan[3] = scan_plan(cur.g.sg[3], ends);
+                y = chain_sums<VT>(pub, off, cur.g.v, cur.g.sg, xv, plan, chunks, y, err, spin_limit,
+                    spins);
+            }
+            if(diagonal) {
+                r = fma((double) cur.iv, y, 0.0);
+            } else if(one_chunk) {
+                const bool in = ib + lane < ie;
+                const double yy = __shfl(y, in ? cur.ic - fr : 0, WAVE);
+                const double v = planned_scan(in ? (double) cur.iv : 0.0, yy, ip);
+                r = 0.0 + __shfl(v, max(ip.end(), 0), WAVE);
+                r = ip.end() >= 0 ? r : 0.0;
+            } else {
+                wave_sync();
+                if(lane < h) { y_lds[lane] = y; res[lane] = 0; }
+                wave_sync();
+                r = apply_inverse<VT>(fr, h, ib, ie, cur.ic, cur.iv, cur.il, i_col, i_val, i_lr,
+                    y_lds, res);
+            }
+        } else {
+            wave_sync();
+            if(lane < h) { y_lds[lane] = cur.bo; res[lane] = 0; }
+            ChainGroup<VT> g = cur.g;
+            bool fetched = false;
+            for(int e0 = ob; e0 < oe; e0 += 64 * TRSV_PF) {
+                if(e0 != ob) chain_group<VT>(e0, oe, o_col, o_val, o_lr, g);
+                double xv[TRSV_PF];
+                bool rdy[TRSV_PF];
 #pragma unroll
                 for(int k = 0; k < TRSV_PF; ++k) xv[k] = pub_load(pub + g.c[k]);
 #pragma unroll
@@ -930,41 +1065,26 @@ __global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t 
                     const bool in = e0 + 64 * k + lane < oe;
                     g.v[k] = in ? g.v[k] : (VT) 0;
                     g.sg[k] = in ? g.sg[k] : 64;
+                    rdy[k] = !in || published(xv[k]);
                 }
-                // the next loads go out here: they are younger than the reads
-                // above, so a row whose values are all there does not wait
-                // for them
-                ChainGroup<VT> gn;
-                const bool more = e0 + 64 * TRSV_PF < oe;
-                if(more)
-                    chain_group<VT>(e0 + 64 * TRSV_PF, oe, o_col, o_val, o_lr, gn);
-                else if(!last)
+                wait_published(pub, g.c, xv, rdy, err, spin_limit, spins);
+                if(!fetched) {
                     chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
-                const int chunks = (oe - e0 + 63) / 64;
-                plan[0] = scan_plan(g.sg[0], ends);
-                if(chunks > 1) plan[1] = scan_plan(g.sg[1], ends);
-                if(chunks > 2) plan[2] = scan_plan(g.sg[2], ends);
-                if(chunks > 3) plan[3] = scan_plan(g.sg[3], ends);
-                y = chain_sums<VT>(pub, g, xv, plan, chunks, y, err, spin_limit, spins);
-                if(!more) break;
-                e0 += 64 * TRSV_PF;
-                g = gn;
+                    fetched = true;
+                }
+                wave_sync();
+#pragma unroll
+                for(int k = 0; k < TRSV_PF; ++k) {
+                    if(e0 + 64 * k >= oe) break;
+                    const double p = seg_scan_runs_fma((double) g.v[k], g.sg[k] < 64 ? xv[k] : 0.0,
+                        g.sg[k]);
+                    const int nsg = next_lane(g.sg[k], -1);
+                    if(g.sg[k] < 64 && (lane == 63 || nsg != g.sg[k])) y_lds[g.sg[k]] -= p;
+                    wave_sync();
+                }
             }
-        } else if(!last) {
-            chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
-        }
-        double r;
-        if(diagonal) {
-            r = fma((double) cur.iv, y, 0.0);
-        } else if(one_chunk) {
-            const bool in = ib + lane < ie;
-            const double yy = __shfl(y, in ? cur.ic - fr : 0, WAVE);
-            const double v = planned_scan(in ? (double) cur.iv : 0.0, yy, ip);
-            r = 0.0 + __shfl(v, max(ip.end, 0), WAVE);
-            r = ip.end >= 0 ? r : 0.0;
-        } else {
-            wave_sync();
-            if(lane < h) { y_lds[lane] = y; res[lane] = 0; }
+            if(!fetched)
+                chain_fetch<VT>(n0, n1, o_col, o_val, o_lr, i_col, i_val, i_lr, x, fused, nxt);
             wave_sync();
             r = apply_inverse<VT>(fr, h, ib, ie, cur.ic, cur.iv, cur.il, i_col, i_val, i_lr, y_lds,
                 res);
@@ -977,7 +1097,7 @@ __global__ __launch_bounds__(64, 3) void k_trsv_chain(const int4* task, int32_t 
         if(w >= nb) break;
         // the next block row's K src: its loads overlap the wait for its
         // inputs, which rarely have all arrived by now
-        if(fused) nxt.bo = block_rhs(rhs, n0.x, n0.y);
+        if(fused) nxt.bo = block_rhs<RHS_U>(rhs, n0.x, n0.y);
         t0 = n0;
         t1 = n1;
         cur = nxt;
@@ -995,7 +1115,7 @@ __global__ __launch_bounds__(64) void k_jacobi_first_product(const int4* task,
     __shared__ double y[33];
     __shared__ double res[33];
     const int4 t0 = task[2 * blockIdx.x];
-    const double bo = block_rhs(rhs, t0.x, t0.y);
+    const double bo = block_rhs<3>(rhs, t0.x, t0.y);
     // each lane reads back only the row it wrote (lanes >= h are masked)
     if(lane_id() < t0.y) b[t0.x + lane_id()] = bo;
     block_row_solve<VT>(t0, task[2 * blockIdx.x + 1], false, o_col, o_val, o_lr, i_col, i_val,
@@ -1456,55 +1576,86 @@ template void solve_plan_count<double>(const SolveTopo&, const double*, double*,
 template void solve_plan_count<float>(const SolveTopo&, const float*, float*, SolvePlan<float>&, void*);
 template void solve_plan_fill<double>(const SolveTopo&, const double*, const double*, SolvePlan<double>&, void*);
 template void solve_plan_fill<float>(const SolveTopo&, const float*, const float*, SolvePlan<float>&, void*);
-// Waves of k_trsv_chain per CU. A solve needs all of its waves resident.
-// TRSV_SINGLE_MAX_CONCURRENT = 4 such solves have to fit on the GPU at the
-// same time (other kernels end on their own), so at most a quarter of what a
-// CU holds: its registers (147-161) let a CU hold 12 of this kernel's waves,
-// three per solve. (Compiled for 16 per CU, it spills 18-25 registers inside
-// the rows' critical path: 403 us instead of 236 for both solves at n =
-// 400,000. As compiled, 59-75 scalar registers go to lanes of vector ones.)
-constexpr int CHAIN_WAVES_PER_CU = 3;
+// Waves of k_trsv_chain per CU at most. A solve needs all of its waves resident.
+// TRSV_SINGLE_MAX_CONCURRENT = 4 such solves, of any instances, have to fit on
+// the GPU at the same time (other kernels end on their own): all are compiled
+// for 16 waves per CU (at most 128 registers), a quarter of them each.
+constexpr int CHAIN_WAVES_PER_CU = 4;
 
-// grid of k_trsv_chain: CHAIN_WAVES_PER_CU waves per CU, fewer should either
-// instance's occupancy not hold TRSV_SINGLE_MAX_CONCURRENT solves (CU count
-// and occupancy queried once per device)
 template<typename VT>
-int chain_grid(int32_t nb)
+using ChainKernel = void (*)(const int4*, int32_t, int32_t, const int32_t*, const VT*,
+    const uint8_t*, const int32_t*, const VT*, const uint8_t*, double*, double*, int32_t*, int32_t,
+    double*, CsrRhs);
+
+template<typename VT>
+ChainKernel<VT> chain_kernel(bool fused, bool planned)
 {
-    static int cus[64] = {0}, occ[64] = {0};
+    if(fused) return planned ? k_trsv_chain<VT, true, true> : k_trsv_chain<VT, true, false>;
+    return planned ? k_trsv_chain<VT, false, true> : k_trsv_chain<VT, false, false>;
+}
+
+// CUs of the current device and waves per CU a solve may have: as many as let
+// TRSV_SINGLE_MAX_CONCURRENT solves of any instance fit (queried once per device)
+struct ChainRoom {
+    int cus, per_cu;
+};
+
+template<typename VT>
+ChainRoom chain_room()
+{
+    static ChainRoom room[64] = {};
     int dev = 0;
-    if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    if(cus[dev] == 0) {
+    if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return {};
+    if(room[dev].cus == 0) {
         hipDeviceProp_t pr;
-        int fused = 0, plain = 0;
-        if(hipGetDeviceProperties(&pr, dev) != hipSuccess) return 0;
-        if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fused, k_trsv_chain<VT, true>, 64, 0) !=
-                hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&plain, k_trsv_chain<VT, false>, 64, 0) !=
-                hipSuccess)
-            return 0;
-        occ[dev] = min(fused, plain);
-        cus[dev] = pr.multiProcessorCount;
+        if(hipGetDeviceProperties(&pr, dev) != hipSuccess) return {};
+        int per = CHAIN_WAVES_PER_CU;
+        for(int k = 0; k < 4; ++k) {
+            int o = 0;
+            if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o,
+                    chain_kernel<VT>((k & 1) != 0, (k & 2) != 0), 64, 0) != hipSuccess)
+                return {};
+            per = min(per, o / TRSV_SINGLE_MAX_CONCURRENT);
+        }
+        room[dev] = {pr.multiProcessorCount, max(1, per)};
     }
-    const int per = max(1, min(CHAIN_WAVES_PER_CU, occ[dev] / TRSV_SINGLE_MAX_CONCURRENT));
-    const int g = cus[dev] * per;
-    return min(g, (int) nb);
+    return room[dev];
+}
+
+// The form of a solve by its block rows per level. Few (up to 3 in 2 CUs): the
+// levels' latency counts, the planned form, with three waves per CU up to one
+// row in 2 CUs, since more waves only poll. Many: the waves are busy with rows
+// whose values are there, and the walked form takes less time for each. us, U'
+// / U / U' with K src on 256 CUs, rows per level: planned 3, planned 4, walked
+//   36 (n = 40,000, blocks of 32)      82 /  96 /  80    86 /  98 /  84    91 / 111 /  91
+//   262 (n = 300,000, blocks of 32)    95 / 106 / 119    93 / 107 / 111   104 / 122 / 121
+//   365 (n = 100,000, blocks of 16)    45 /  44 /  54    44 /  43 /  48    44 /  45 /  48
+//   437 (n = 40,000, blocks of 8)      34 /  33 /  38    32 /  32 /  35    32 /  32 /  33
+//   3,090 (n = 300,000, blocks of 8)  131 / 122 / 249   106 /  99 / 196    89 /  82 / 187
+struct ChainForm {
+    bool planned;
+    int per_cu;
+};
+
+inline ChainForm chain_form(const SolveTopo& t, int cus)
+{
+    const int64_t rows2 = 2 * (int64_t) t.nb, levels = t.num_levels;
+    // the planned form reaches values by 32-bit byte offsets
+    if(rows2 > 3 * levels * cus || t.n >= (1 << 29)) return {false, CHAIN_WAVES_PER_CU};
+    return {true, rows2 <= levels * cus ? 3 : CHAIN_WAVES_PER_CU};
 }
 
 template<typename VT>
-hipError_t trsv_chain(const int4* task, int32_t nb, int32_t reverse, const int32_t* o_col,
-    const VT* o_val, const uint8_t* o_lr, const int32_t* i_col, const VT* i_val,
-    const uint8_t* i_lr, double* pub, double* next_pub, const SolveTopo& t, double* x, CsrRhs rhs,
-    hipStream_t st)
+hipError_t trsv_chain(const int4* task, int32_t reverse, const int32_t* o_col, const VT* o_val,
+    const uint8_t* o_lr, const int32_t* i_col, const VT* i_val, const uint8_t* i_lr, double* pub,
+    double* next_pub, const SolveTopo& t, double* x, CsrRhs rhs, hipStream_t st)
 {
-    const int g = chain_grid<VT>(nb);
-    if(g <= 0) return hipErrorInvalidConfiguration;
-    if(rhs.rp)
-        k_trsv_chain<VT, true><<<g, 64, 0, st>>>(task, nb, reverse, o_col, o_val, o_lr, i_col, i_val,
-            i_lr, pub, next_pub, t.err, t.spin_limit, x, rhs);
-    else
-        k_trsv_chain<VT, false><<<g, 64, 0, st>>>(task, nb, reverse, o_col, o_val, o_lr, i_col,
-            i_val, i_lr, pub, next_pub, t.err, t.spin_limit, x, rhs);
+    const ChainRoom room = chain_room<VT>();
+    if(room.cus <= 0) return hipErrorInvalidConfiguration;
+    const ChainForm form = chain_form(t, room.cus);
+    const int g = min(room.cus * min(form.per_cu, room.per_cu), (int) t.nb);
+    chain_kernel<VT>(rhs.rp != nullptr, form.planned)<<<g, 64, 0, st>>>(task, t.nb, reverse, o_col,
+        o_val, o_lr, i_col, i_val, i_lr, pub, next_pub, t.err, t.spin_limit, x, rhs);
     return hipGetLastError();
 }
 
@@ -1515,7 +1666,7 @@ int trsv_upper_single(const SolveTopo& t, const SolvePlan<VT>& p, double* x, int
     if(t.nb <= 0) return 0;
     double* pub = t.chain_pub + (parity ? t.n : 0);
     double* next = t.chain_pub + (parity ? 0 : t.n);
-    return (int) trsv_chain<VT>(p.task_u, t.nb, 1, p.uo_col, p.uo_val, p.uo_lr, p.ui_col, p.ui_val,
+    return (int) trsv_chain<VT>(p.task_u, 1, p.uo_col, p.uo_val, p.uo_lr, p.ui_col, p.ui_val,
         p.ui_lr, pub, next, t, x, CsrRhs{nullptr, nullptr, nullptr, nullptr},
         (hipStream_t) stream);
 }
@@ -1536,7 +1687,7 @@ int trsv_upper_t_single_product(const SolveTopo& t, const SolvePlan<VT>& p, cons
     double* next = t.chain_pub + (parity ? 0 : t.n);
     const CsrRhs rhs = K ? CsrRhs{K->row_ptr, K->col, K->val, src}
                          : CsrRhs{nullptr, nullptr, nullptr, nullptr};
-    return (int) trsv_chain<VT>(p.task_t, t.nb, 0, p.to_col, p.to_val, p.to_lr, p.ti_col, p.ti_val,
+    return (int) trsv_chain<VT>(p.task_t, 0, p.to_col, p.to_val, p.to_lr, p.ti_col, p.ti_val,
         p.ti_lr, pub, next, t, x, rhs, (hipStream_t) stream);
 }
 

@@ -128,15 +128,15 @@ def test_solve_error_reported_once(hip_device):
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])
-@pytest.mark.parametrize("kind", ["kkt", "dense_pivots"])
+@pytest.mark.parametrize("kind", ["kkt", "many_rows", "dense_pivots"])
 def test_solve_that_gives_up_waiting_leaves_nan(hip_device, kind, prec):
     """A single-launch solve whose waits give up at once (the testing hook's
     limit of no polls; every wave still runs to its end): each row is either
     the solution bit for bit or NaN, never a partial sum; the next call says
     so once, and the solve after it is whole again."""
     import torch
-    if kind == "kkt":
-        _, p = _system(2000, 801, B=32)
+    if kind != "dense_pivots":   # few and many block rows per level
+        _, p = _system(2000, 801, B=32) if kind == "kkt" else _system(4000, 1601, B=1)
         csr, piv, blocks = (p.row_ptr, p.col, p.val), p.piv_starts, p.block_starts
     else:   # inverses of more than 64 entries, 2x2 pivots
         csr, piv, blocks, _ = sym_problem(n_blocks=15, bmax=32, density=0.1, seed=15)

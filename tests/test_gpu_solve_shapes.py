@@ -90,6 +90,38 @@ def test_single_launch_equals_levels(hip_device, shape, prec):
             assert np.linalg.norm(out[0] - ref) <= 1e-12 * np.linalg.norm(ref), side
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("shape,rows_per_level", [
+    ((2000, 801, 4, 3, 32), (1, 128)),      # three waves per CU
+    ((1500, 601, 4, 3, 1), (128, 384)),     # four
+    ((4000, 1601, 4, 3, 1), (384, 4000)),   # rows walked one group after the other
+    ((20000, 8003, 4, 3, 4), (384, 4000)),
+])
+def test_single_launch_forms_equal_levels(hip_device, shape, rows_per_level, prec):
+    """The forms of the single-launch solve, chosen by block rows per level (of
+    256 CUs), and the product folded into them: the level launches' bits."""
+    import torch
+    csr, piv, bs = _kkt(*shape)
+    g = ca.BlockiLDLt(*csr, piv, bs, prec)
+    g.compute(0, 1.0, 1e-4)
+    lo, hi = rows_per_level
+    assert lo < bs.size / (g.get_int("lvl_off").size - 1) <= hi
+    A = ca.CSRMatrixSPMV(*csr)
+    b = torch.tensor(np.random.default_rng(8).normal(size=csr[0].size - 1), device=hip_device)
+    out = {}
+    for algo in ("levels", "single"):
+        g.set_solve_algorithm(algo)
+        for op in ("left", "right", "product"):
+            x = torch.zeros_like(b)
+            if op == "product":
+                assert g.left_product(A, b, x) == (algo == "single")
+            else:
+                getattr(g, f"solve_{op}")(b, x)
+            out[algo, op] = x.cpu().numpy()
+    for op in ("left", "right", "product"):
+        assert np.array_equal(out["levels", op], out["single", op]), op
+
+
 @pytest.mark.parametrize("algo,sweeps", [("levels", 0), ("single", 0), ("jacobi", 2)])
 def test_iterates_do_not_depend_on_check_period(hip_device, algo, sweeps):
     import torch
