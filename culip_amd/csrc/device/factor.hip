@@ -705,6 +705,62 @@ __device__ __forceinline__ bool light_update(const Dep& d, const RowOf& w, const
     return ok && o.noff <= LIGHT_OFF;
 }
 
+// The same for a block with a 2x2 pivot among its rows and at most COL_E entries,
+// all in one column c: it updates T[c][c] alone, the rows above and below coupled
+// by D. Among static 2x2 pivots two blocks in five are such; staged as tiles
+// instead, a refactor at n = 5,000 in blocks of up to 8 rows took 11.6 ms
+// instead of 7.0 (f64).
+constexpr int COL_E = 4;
+
+template<typename VT>
+__device__ __forceinline__ bool column_update(const Dep& d, const RowOf& w, const int32_t* ixs,
+    const VT* vals, const double* tri, LightUpd<VT>& o)
+{
+    if(d.fmt != FMT_SPARSE || d.nnz > COL_E || d.nnz == 0) return false;
+    constexpr int NONE = 1 << 20;
+    int key[COL_E];          // 32 row + column, ascending
+    VT v[COL_E];
+#pragma unroll
+    for(int e = 0; e < COL_E; ++e) {
+        const int at = min(e, d.nnz - 1);
+        const int ix = ixs[(int64_t) d.cp + at];
+        v[e] = vals[(int64_t) d.vp + at];
+        key[e] = (e < d.nnz && v[e] != (VT) 0) ? w.at(ix) : NONE;
+    }
+    auto order = [&](int x, int y) {
+        if(key[y] < key[x]) {
+            const int tk = key[x]; key[x] = key[y]; key[y] = tk;
+            const VT tv = v[x]; v[x] = v[y]; v[y] = tv;
+        }
+    };
+    static_assert(COL_E == 4, "sorting network on four");
+    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+    bool ok = true;
+    VT acc = (VT) 0;
+#pragma unroll
+    for(int e = 0; e < COL_E; ++e) {
+        if(key[e] == NONE) continue;
+        const double* t = tri + 3 * (int64_t) (d.rb + (key[e] >> 5));
+        const VT sup = (VT) t[0], dia = (VT) t[1], sub = (VT) t[2];
+        ok = ok && (key[e] & 31) == (key[0] & 31) && finite_value(sup) && finite_value(dia) &&
+            finite_value(sub) && finite_value(v[e]);
+        const VT left = (e > 0 && key[max(e - 1, 0)] == key[e] - 32) ? v[max(e - 1, 0)] : (VT) 0;
+        const VT right = (e + 1 < COL_E && key[min(e + 1, COL_E - 1)] == key[e] + 32)
+            ? v[min(e + 1, COL_E - 1)] : (VT) 0;
+        acc = fma(v[e], fma(sub, right, fma(dia, v[e], sup * left)), acc);
+    }
+    if(!ok) return false;
+    o.cols = (key[0] != NONE) ? 1u << (key[0] & 31) : 0u;
+    o.noff = 0;
+#pragma unroll
+    for(int e = 0; e < LIGHT_E; ++e) o.head[e] = -1;
+    if(o.cols) {
+        o.head[0] = key[0] & 31;
+        o.acc[0] = acc;
+    }
+    return true;
+}
+
 // T -= A' D A for the block staged in h.X by all NW waves: the arithmetic and
 // order of product() with R = A
 template<typename VT, int NW>
@@ -854,7 +910,10 @@ constexpr uint32_t PIV_ANY = 1, PIV_2X2 = 2, PIV_NONFINITE = 4, PIV_PERM = 8;
 // change nothing else, so they are done together last.
 // FP64 refactor, blocks above taken by rounds of one wave -> at once: 7.1 ->
 // 5.2 ms at n = 2,000, 8.3 -> 6.4 ms at n = 400,000.
-template<typename VT, int NW>
+// TWO: there may be 2x2 pivots, static ones or numerically chosen. Without them
+// their code stays out: a level's kernels follow each other through the
+// instruction cache (n = 400,000: 4.16 ms, with it 4.21).
+template<typename VT, int NW, bool TWO>
 __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
     PivLds<VT, NW>& s)
 {
@@ -913,6 +972,9 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
             light = blk >= 0 && light_update<VT, 2>(d, width, a.ix_out, a.val_out, a.tri, up);
         else
             light = blk >= 0 && light_update<VT, LIGHT_E>(d, width, a.ix_out, a.val_out, a.tri, up);
+        if(TWO && wave_ballot(blk >= 0 && !light && d.fmt == FMT_SPARSE && d.nnz <= COL_E))
+            light = light || (blk >= 0 &&
+                column_update<VT>(d, width, a.ix_out, a.val_out, a.tri, up));
         const uint64_t hm = wave_ballot(blk >= 0 && !light);
         if(lane == 0) s.heavy[wv] = hm;
         __syncthreads();
@@ -944,7 +1006,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
     if(wv == 0) {
         int32_t rflag = 0;
         uint32_t plain = 0, tiny = 0;
-        if(a.pivoting) {
+        if(TWO && a.pivoting) {
             int32_t* fpiv = a.is_piv + fr;
             int32_t* bperm = s.perm;
             if(lane < 32) bperm[lane] = lane;
@@ -989,7 +1051,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
             const VT d0 = T0[33 * (lane & 31)];
             if(d0 != d0) M = right;
             const uint32_t starts = (uint32_t) wave_ballot(lane < 32 && lane < len && piv != 0);
-            const uint32_t two = (~starts & live) >> 1;    // rows where a 2x2 pivot starts
+            const uint32_t two = TWO ? (~starts & live) >> 1 : 0u;   // rows where a 2x2 pivot starts
             uint32_t done = 0;
             for(int p = 0; p < len;) {
                 const uint32_t cand = ((uint32_t) wave_ballot(lane < len && M != 0u) | two) &
@@ -997,7 +1059,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
                 if(!cand) break;
                 p = __ffs(cand) - 1;
                 uint32_t bad;
-                if((two >> p) & 1u) {
+                if(TWO && ((two >> p) & 1u)) {
                     bad = a.piv64 ? step_2x2<VT, double>(T0, tri, p, len)
                                   : step_2x2<VT, VT>(T0, tri, p, len);
                     rflag |= ROW_2X2;
@@ -1073,7 +1135,7 @@ __device__ __forceinline__ void pivots_one(const FactorArgs<VT>& a, const LevelR
         if(s.rflag & ROW_2X2) flags |= PIV_2X2;
         if(s.rflag & ROW_NONFINITE) flags |= PIV_NONFINITE;
         const bool unbounded = wave_ballot(!bounded) != 0ull;
-        if(a.pivoting) {
+        if(TWO && a.pivoting) {
             const int p = (lane < len) ? s.perm[lane] : lane;
             if(wave_ballot(lane < len && p != lane)) flags |= PIV_PERM;
             if(lane < len) {
@@ -2023,14 +2085,14 @@ union PivPairsLds {
     TinyLds<VT, TINY_P, 64 * NW> tiny;
 };
 
-template<typename VT, int NW>
+template<typename VT, int NW, bool TWO>
 __device__ __forceinline__ void pivots_pairs_body(const FactorArgs<VT>& a, const LevelRange& lr,
     int bid_)
 {
     __shared__ PivPairsLds<VT, NW> u;
     const int w = bid_;
     if(w < lr.npiv) {
-        pivots_one<VT, NW>(a, lr, w, u.piv);
+        pivots_one<VT, NW, TWO>(a, lr, w, u.piv);
         return;
     }
     const int q0 = lr.npiv + (w - lr.npiv) * 64 * NW;
@@ -2612,10 +2674,10 @@ __global__ __launch_bounds__(TINY_TPB) void k_offdiag_tiny_scale(FactorArgs<VT> 
     offdiag_tiny_scale_body<VT>(a, lr, blockIdx.x);
 }
 
-template<typename VT, int NW>
+template<typename VT, int NW, bool TWO>
 __global__ __launch_bounds__(64 * NW, PP_WAVES<VT>) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
 {
-    pivots_pairs_body<VT, NW>(a, lr, blockIdx.x);
+    pivots_pairs_body<VT, NW, TWO>(a, lr, blockIdx.x);
 }
 
 template<typename VT>
@@ -2720,14 +2782,14 @@ __global__ void bk_gather(const FactorSys<VT>* fs, const int2* items)
     if(q < F.nnz && F.value_slot[q] >= 0) F.val_in[F.value_slot[q]] = (VT) F.vals[q];
 }
 
-template<typename VT>
+template<typename VT, bool TWO>
 __global__ __launch_bounds__(64, PP_WAVES<VT>) void bk_pivots_pairs(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
     const int2 it = items[blockIdx.x];
     const FactorSys<VT>& F = fs[it.x];
     const LevelRange lr = F.lr[level];
-    pivots_pairs_body<VT, 1>(F.a, lr, it.y);
+    pivots_pairs_body<VT, 1, TWO>(F.a, lr, it.y);
 }
 
 template<typename VT>
@@ -2830,10 +2892,10 @@ void factor_level(const FactorArgs<VT>& a, const LevelRange& r, void* stream)
     const int noff = r.size - r.npiv;
     const int tiny_blocks = fl_tiny_blocks(r);
     if(r.size > 0) {
-        if(r.piv_waves == 4)
-            k_pivots_pairs<VT, 4><<<fl_grid_pivots_pairs(r, 4), 256, 0, st>>>(a, r);
-        else
-            k_pivots_pairs<VT, 1><<<fl_grid_pivots_pairs(r, 1), 64, 0, st>>>(a, r);
+        const bool four = r.piv_waves == 4;
+        auto k = four ? (a.two ? k_pivots_pairs<VT, 4, true> : k_pivots_pairs<VT, 4, false>)
+                      : (a.two ? k_pivots_pairs<VT, 1, true> : k_pivots_pairs<VT, 1, false>);
+        k<<<fl_grid_pivots_pairs(r, r.piv_waves), 64 * r.piv_waves, 0, st>>>(a, r);
     }
     if(noff > 0) {
         const int grid = fl_grid_tasks(noff, 2048);
@@ -2878,7 +2940,10 @@ void factor_batch_level(const FactorSys<VT>* fs, const FactorBatchLevel& L, int3
     hipStream_t st)
 {
     auto grid = [](const FactorItems& f) { return (unsigned) f.count; };
-    if(L.pp.count) bk_pivots_pairs<VT><<<grid(L.pp), 64, 0, st>>>(fs, L.pp.items, level);
+    if(L.pp.count) {
+        auto k = L.two ? bk_pivots_pairs<VT, true> : bk_pivots_pairs<VT, false>;
+        k<<<grid(L.pp), 64, 0, st>>>(fs, L.pp.items, level);
+    }
     if(L.ts.count) bk_offdiag_tiny_scale<VT><<<grid(L.ts), TINY_TPB, 0, st>>>(fs, L.ts.items, level);
     if(L.off.count) {
         bk_offdiag<VT><<<grid(L.off), 64, 0, st>>>(fs, L.off.items, level);

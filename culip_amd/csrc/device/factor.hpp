@@ -21,6 +21,7 @@ struct FactorArgs {
     // numeric pivoting); pivoting: 0 static, 1 Bunch-Kaufman, 2 rook
     int32_t* perm = nullptr;
     int32_t pivoting = 0;
+    bool two = true;                      // 2x2 pivots: static ones or numeric pivoting
     // 1: 2x2 pivot steps and the Givens-form D solves in FP64 (an FP32
     // factor's default); 0: in the factor's type, as BlockiLDLt<T>
     int32_t piv64 = 0;
@@ -177,6 +178,7 @@ struct FactorBatchLevel {
     FactorItems off;   // k_offdiag and k_offdiag_general (BATCH_TASK_GRID per system)
     FactorItems dr;    // k_drop
     FactorItems st;    // k_store (BATCH_TASK_GRID per system)
+    bool two = true;   // a listed system may have 2x2 pivots
 };
 
 // Host entry points (factor.hip). All launches go to `stream`.

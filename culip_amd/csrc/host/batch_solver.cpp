@@ -438,11 +438,13 @@ void BatchSolver::build_factor()
     std::vector<FactorSys<VT>> F(S);
     std::vector<PlanSys<VT>> P(S);
     std::vector<int2> chunks, blk, scan, task;
+    bool two = false;
     for(int32_t s = 0; s < S; ++s) {
         Bildlt& f = *sys_[s]->f;
         f.threshold = o_.threshold;
         FactorSys<VT>& q = F[s];
         q.a = f.factor_args<VT>();
+        two = two || q.a.two;
         q.lr = d_lr_.as<LevelRange>() + lr_off[s];
         q.vals = f.d_vals.as<double>();
         q.value_slot = f.d_value_slot.as<int64_t>();
@@ -498,6 +500,7 @@ void BatchSolver::build_factor()
     FactorItems all[5];
     for(int k = 0; k < 5; ++k) all[k] = put(d_fit_[k], it[k]);
     flevels_.assign(max_levels, FactorBatchLevel{});
+    for(FactorBatchLevel& L : flevels_) L.two = two;
     for(int32_t l = 0; l < max_levels; ++l) {
         FactorItems* dst[5] = {&flevels_[l].pp, &flevels_[l].ts, &flevels_[l].off,
             &flevels_[l].dr, &flevels_[l].st};

@@ -195,6 +195,7 @@ void BildltPattern::build_levels()
         CULIP_REQUIRE(q == r.size, "factor: level list does not end with its last block row");
     }
     num_groups = (int32_t) (groups.size() / 4);
+    two_by_two = std::find(s.is_piv.begin(), s.is_piv.end(), 0) != s.is_piv.end();
     upload(d_lq, lq);
     upload(d_lq_val, lv);
     upload(d_groups, groups);
@@ -290,6 +291,7 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.is_piv = d_fis_piv.as<int32_t>();
     a.perm = d_perm.as<int32_t>();
     a.pivoting = (int32_t) pivoting;
+    a.two = pat->two_by_two || pivoting != CULIP_PIVOT_STATIC;
     a.piv64 = (f32() && pivot_precision == CULIP_PIVOT2_F64) ? 1 : 0;
     a.bin = d_bin.as<BlockMeta>();
     a.bout = d_bout.as<BlockMeta>();

@@ -131,6 +131,7 @@ struct BildltPattern {
     DevBuf d_lq, d_lq_val, d_groups, d_off_task, d_upd4;
     std::vector<LevelRange> levels;
     int32_t num_groups = 0;
+    bool two_by_two = false;   // static 2x2 pivots
     void build_levels();
     void upload_static();
     int64_t device_bytes() const;

@@ -56,3 +56,15 @@ def test_kkt_factor_equals_oracle(hip_device, n, m, o, c, B, order, prec, pivoti
 def test_two_by_two_factor_equals_oracle(hip_device, n_blocks, bmax, density, fill, ff, thr, prec):
     csr, piv, bs, _ = sym_problem(n_blocks=n_blocks, bmax=bmax, density=density, seed=n_blocks)
     _compare(csr, piv, bs, prec, fill=fill, ff=ff, thr=thr)
+
+
+@pytest.mark.parametrize("n_blocks,bmax,density,prec,pivoting", [
+    (200, 4, 0.03, "f64", "static"), (200, 4, 0.03, "f32", "static"),
+    (150, 8, 0.02, "f64", "static"), (90, 12, 0.01, "f32", "static"), (90, 12, 0.01, "f64", "bk"),
+])
+def test_columns_beside_two_by_two_pivots_equal_oracle(hip_device, n_blocks, bmax, density, prec,
+                                                       pivoting):
+    """Blocks of one to four entries in a single column whose rows belong to
+    2x2 pivots (most blocks of these sparse patterns)."""
+    csr, piv, bs, _ = sym_problem(n_blocks=n_blocks, bmax=bmax, density=density, seed=7)
+    _compare(csr, piv, bs, prec, pivoting=pivoting)
