@@ -2645,15 +2645,11 @@ __device__ __forceinline__ void store_body(const FactorArgs<VT>& a, const LevelR
     }
 }
 
-// k_pivot_col_blocks (kernels :1352-1418) with d_col_pivot_block
-// (:1290-1348): one wave per block row of the level; the stored blocks above
-// its pivot block (earlier levels, final storage) take its pivoting order in
-// their columns: sparse entries get new column indices in place, dense rows
-// are gathered column by column.
-// waves per SIMD the pivot, pair and one-wave off-diagonal kernels are compiled
-// for: as many as their registers allow with few spills
-template<typename VT>
-constexpr int PP_WAVES = sizeof(VT) == 4 ? 3 : 2;
+// Waves per SIMD the pivot, pair and one-wave off-diagonal kernels are compiled
+// for at least: as many as their registers allow with few spills. With three, FP32
+// spills too (k_offdiag 45 registers, bk_offdiag 18): refactor at n = 2,000 2.98
+// ms, with two 2.86; a burst of 24 requests 44.0 and 41.5 ms.
+constexpr int PP_WAVES = 2;
 
 // the single-system kernels: the bodies at their own grid position
 template<typename VT>
@@ -2663,7 +2659,7 @@ __global__ __launch_bounds__(64) void k_offdiag_general(FactorArgs<VT> a, LevelR
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64, PP_WAVES<VT>) void k_offdiag(FactorArgs<VT> a, LevelRange lr)
+__global__ __launch_bounds__(64, PP_WAVES) void k_offdiag(FactorArgs<VT> a, LevelRange lr)
 {
     offdiag_body<VT>(a, lr, blockIdx.x, gridDim.x);
 }
@@ -2675,7 +2671,7 @@ __global__ __launch_bounds__(TINY_TPB) void k_offdiag_tiny_scale(FactorArgs<VT> 
 }
 
 template<typename VT, int NW, bool TWO>
-__global__ __launch_bounds__(64 * NW, PP_WAVES<VT>) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
+__global__ __launch_bounds__(64 * NW, PP_WAVES) void k_pivots_pairs(FactorArgs<VT> a, LevelRange lr)
 {
     pivots_pairs_body<VT, NW, TWO>(a, lr, blockIdx.x);
 }
@@ -2692,6 +2688,11 @@ __global__ __launch_bounds__(64) void k_store(FactorArgs<VT> a, LevelRange lr)
     store_body<VT>(a, lr, blockIdx.x, gridDim.x);
 }
 
+// k_pivot_col_blocks (kernels :1352-1418) with d_col_pivot_block
+// (:1290-1348): one wave per block row of the level; the stored blocks above
+// its pivot block (earlier levels, final storage) take its pivoting order in
+// their columns: sparse entries get new column indices in place, dense rows
+// are gathered column by column.
 template<typename VT>
 __global__ __launch_bounds__(64) void k_pivot_cols(FactorArgs<VT> a, LevelRange lr)
 {
@@ -2783,7 +2784,7 @@ __global__ void bk_gather(const FactorSys<VT>* fs, const int2* items)
 }
 
 template<typename VT, bool TWO>
-__global__ __launch_bounds__(64, PP_WAVES<VT>) void bk_pivots_pairs(const FactorSys<VT>* fs, const int2* items,
+__global__ __launch_bounds__(64, PP_WAVES) void bk_pivots_pairs(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
     const int2 it = items[blockIdx.x];
@@ -2803,7 +2804,7 @@ __global__ __launch_bounds__(TINY_TPB) void bk_offdiag_tiny_scale(const FactorSy
 }
 
 template<typename VT>
-__global__ __launch_bounds__(64, PP_WAVES<VT>) void bk_offdiag(const FactorSys<VT>* fs, const int2* items,
+__global__ __launch_bounds__(64, PP_WAVES) void bk_offdiag(const FactorSys<VT>* fs, const int2* items,
     int32_t level)
 {
     const int2 it = items[blockIdx.x];
