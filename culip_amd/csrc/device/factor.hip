@@ -1730,7 +1730,7 @@ __device__ __forceinline__ void offdiag_small_one(const FactorArgs<VT>& a, const
     offdiag_output(a, q, s.X, !(flags & PIV_2X2), flags & PIV_NONFINITE, d_row, hgt, wid, t1.x);
 }
 
-// the positions k_offdiag_tiny leaves to the wave form, grid-stride
+// the positions the one-lane form leaves to the wave form, grid-stride
 template<typename VT>
 __device__ __forceinline__ void offdiag_body(const FactorArgs<VT>& a, const LevelRange& lr,
     int bid_, int nblk_)
@@ -1775,8 +1775,8 @@ __device__ __forceinline__ void to_wave_form(const FactorArgs<VT>& a, const Leve
 // One-lane form, first phase: the Schur updates of the off-diagonal block at
 // level position q (thread tid of its workgroup), which read only blocks of
 // earlier levels and so run beside the level's pivot blocks. The tile list
-// is parked in the position's compact store (if_idx / if_val, count in
-// if_cnt); if_cnt[q] = -1 marks a position left to the other kernels.
+// is parked as the position's entry list (EntryList: the first LIST_C in c_idx /
+// c_val, the others in if_idx / if_val, count in if_cnt); if_cnt[q] = -1 marks a position left to the other kernels.
 template<typename VT, int TPB>
 __device__ __forceinline__ void tiny_pairs_one(const FactorArgs<VT>& a, const LevelRange& lr, const int q,
     const int tid, TinyLds<VT, TINY_P, TPB>& s)

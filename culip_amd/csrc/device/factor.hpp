@@ -34,7 +34,6 @@ struct FactorArgs {
     const int32_t* upd_ki = nullptr;
     const int32_t* upd_kj = nullptr;
     const int32_t* lvlb_idx = nullptr;    // level block list
-    const int32_t* block_in_lvl = nullptr;
     const int32_t* lvl_rows = nullptr;
     const int32_t* ix_in = nullptr;       // input stores
     const VT* val_in = nullptr;

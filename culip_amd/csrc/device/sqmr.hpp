@@ -40,10 +40,10 @@ struct SqmrWork {
     double* xacc = nullptr;     // refinement: accumulated solution
     double* rhs = nullptr;      // refinement: current residual
     double* part = nullptr;     // PART_SLOTS * grid partial sums
-    double* scal = nullptr;     // 32 scalars
+    double* scal = nullptr;     // 64 doubles: the recurrence's 32, norms and eta above
     int32_t* flags = nullptr;   // 4 ints: test[0], test[1]
     int32_t* host_flags = nullptr;  // pinned
-    double* host_scal = nullptr;    // pinned, 32 doubles
+    double* host_scal = nullptr;    // pinned, 64 doubles
 };
 
 // scalar slots of SqmrWork::scal the host reads: the recurrence's gamma and

@@ -42,7 +42,7 @@ int64_t BildltPattern::device_bytes() const
 {
     int64_t b = 0;
     for(const DevBuf* d : {&d_bs, &d_is_piv, &d_bin, &d_csr_off, &d_csc_off, &d_csc_idx, &d_upd_off,
-            &d_upd_ki, &d_upd_kj, &d_lvlb_idx, &d_block_in_lvl, &d_lvl_rows, &d_ix_in,
+            &d_upd_ki, &d_upd_kj, &d_lvlb_idx, &d_lvl_rows, &d_ix_in,
             &d_value_slot, &d_lq, &d_lq_val, &d_groups, &d_off_task, &d_upd4})
         b += (int64_t) d->bytes;
     return b;
@@ -61,7 +61,6 @@ void BildltPattern::upload_static()
     upload(d_upd_ki, s.upd_ki);
     upload(d_upd_kj, s.upd_kj);
     upload(d_lvlb_idx, s.lvlb_idx);
-    upload(d_block_in_lvl, s.block_in_lvl);
     upload(d_lvl_rows, s.lvl_rows);
     upload(d_ix_in, s.ix_store);
     upload(d_value_slot, s.value_slot);
@@ -302,7 +301,6 @@ FactorArgs<VT> Bildlt::factor_args() const
     a.upd_ki = d_upd_ki.as<int32_t>();
     a.upd_kj = d_upd_kj.as<int32_t>();
     a.lvlb_idx = d_lvlb_idx.as<int32_t>();
-    a.block_in_lvl = d_block_in_lvl.as<int32_t>();
     a.lvl_rows = d_lvl_rows.as<int32_t>();
     a.ix_in = d_ix_in.as<int32_t>();
     a.val_in = d_val_in.as<VT>();
@@ -479,7 +477,7 @@ void Bildlt::factor(const double* vals, bool on_device, double thr, hipStream_t 
 
 void Bildlt::after_factor()
 {
-    // a level's dropping scan whose bounded wait gave up leaves the object
+    // a row group's bounded wait (dropping step) that gave up leaves the object
     // unfactored
     factored = false;
     take_async_error();
@@ -636,7 +634,7 @@ void Bildlt::take_async_error() const
 {
     const int32_t e = h_trsv_err.take();
     if(e == 2)
-        fail(CULIP_ERR_HIP, "factor: a chunk wait of a level's dropping scan timed out");
+        fail(CULIP_ERR_HIP, "factor: a row group's wait in a level's dropping step timed out");
     if(e)
         fail(CULIP_ERR_HIP, "triangular solve: a dependency wait of a single-launch solve timed "
                             "out (its x holds NaN)");

@@ -127,7 +127,7 @@ struct BildltPattern {
     bool uploaded = false;
     culip_prec prec = CULIP_PREC_F64;
     DevBuf d_bs, d_is_piv, d_bin, d_csr_off, d_csc_off, d_csc_idx, d_upd_off, d_upd_ki, d_upd_kj,
-        d_lvlb_idx, d_block_in_lvl, d_lvl_rows, d_ix_in, d_value_slot;
+        d_lvlb_idx, d_lvl_rows, d_ix_in, d_value_slot;
     DevBuf d_lq, d_lq_val, d_groups, d_off_task, d_upd4;
     std::vector<LevelRange> levels;
     int32_t num_groups = 0;
@@ -146,7 +146,7 @@ struct Bildlt final : Precond {
     Symbolic& sym;
     bool& have_sym;
     DevBuf &d_bs, &d_is_piv, &d_bin, &d_csr_off, &d_csc_off, &d_csc_idx, &d_upd_off, &d_upd_ki,
-        &d_upd_kj, &d_lvlb_idx, &d_block_in_lvl, &d_lvl_rows, &d_ix_in, &d_value_slot;
+        &d_upd_kj, &d_lvlb_idx, &d_lvl_rows, &d_ix_in, &d_value_slot;
     DevBuf &d_lq, &d_lq_val, &d_groups, &d_off_task, &d_upd4;
 
     culip_prec prec = CULIP_PREC_F64;
@@ -204,7 +204,7 @@ struct Bildlt final : Precond {
           have_sym(p->have_sym), d_bs(p->d_bs), d_is_piv(p->d_is_piv), d_bin(p->d_bin),
           d_csr_off(p->d_csr_off), d_csc_off(p->d_csc_off), d_csc_idx(p->d_csc_idx),
           d_upd_off(p->d_upd_off), d_upd_ki(p->d_upd_ki), d_upd_kj(p->d_upd_kj),
-          d_lvlb_idx(p->d_lvlb_idx), d_block_in_lvl(p->d_block_in_lvl), d_lvl_rows(p->d_lvl_rows),
+          d_lvlb_idx(p->d_lvlb_idx), d_lvl_rows(p->d_lvl_rows),
           d_ix_in(p->d_ix_in), d_value_slot(p->d_value_slot),
           d_lq(p->d_lq), d_lq_val(p->d_lq_val), d_groups(p->d_groups), d_off_task(p->d_off_task),
           d_upd4(p->d_upd4), prec(p->prec)
