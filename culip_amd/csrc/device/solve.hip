@@ -17,6 +17,7 @@
 #include "solve.hpp"
 #include "batch.hpp"
 #include "wave.hpp"
+#include <atomic>
 
 #include <hip/hip_runtime.h>
 
@@ -1603,10 +1604,12 @@ struct ChainRoom {
 template<typename VT>
 ChainRoom chain_room()
 {
-    static ChainRoom room[64] = {};
+    // both numbers in one word, since threads may get here at the same time
+    static std::atomic<int> room[64] = {};
     int dev = 0;
     if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return {};
-    if(room[dev].cus == 0) {
+    int r = room[dev].load(std::memory_order_relaxed);
+    if(r == 0) {
         hipDeviceProp_t pr;
         if(hipGetDeviceProperties(&pr, dev) != hipSuccess) return {};
         int per = CHAIN_WAVES_PER_CU;
@@ -1617,9 +1620,10 @@ ChainRoom chain_room()
                 return {};
             per = min(per, o / TRSV_SINGLE_MAX_CONCURRENT);
         }
-        room[dev] = {pr.multiProcessorCount, max(1, per)};
+        r = 8 * pr.multiProcessorCount + max(1, per);
+        room[dev].store(r, std::memory_order_relaxed);
     }
-    return room[dev];
+    return {r / 8, r % 8};
 }
 
 // The form of a solve by its block rows per level. Few (up to 3 in 2 CUs): the
